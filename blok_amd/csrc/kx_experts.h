@@ -12,8 +12,15 @@ struct KxExpertSlots {
   int4 *tiles = nullptr;
   int *n_tiles = nullptr;
 };
-// slots per tile of a step (those of the GEMM that will read them), and the most tiles its pairs make
-inline int kx_expert_tile(bool f32, int tokens, int top, int experts) { return !f32 && (long)tokens * top >= 96L * experts ? 128 : 64; }
+// slots per tile of a step (those of the GEMM that will read them), and the most tiles its pairs make.  bf16: 32 where an expert
+// has fewer than 8 pairs on average (the kernel for few tokens, 64 rows a workgroup: 50 and 24 us where the one with tiles of
+// 64 takes 75 and 38 us for 64 pairs on 64 experts of 3 x 2048 x 1024), 128 from 96 on
+constexpr int KX_EXPERT_TILE_MIN = 32;
+inline int kx_expert_tile(bool f32, int tokens, int top, int experts) {
+  const long pairs = (long)tokens * top;
+  if (f32) return 64;
+  return pairs >= 96L * experts ? 128 : pairs >= 8L * experts ? 64 : KX_EXPERT_TILE_MIN;
+}
 inline int kx_expert_tiles(int tokens, int top, int experts, int tile) {
   const int pairs = tokens * top;
   return (pairs + tile - 1) / tile + (experts < pairs ? experts : pairs);

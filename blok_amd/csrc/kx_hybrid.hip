@@ -89,6 +89,9 @@ struct HybridModel : kx_model {
   int proj_ld = 0, mid_ld = 0, part_tokens = 0;
   size_t part_floats = 0;
   int *want = nullptr;           // token rows of row_logits
+  float *split_part = nullptr;   // of products that split their columns over workgroups
+  int *split_arrived = nullptr;
+  size_t split_floats = 0;
   float init_sigma_ = 0;
   int hist_cur = 0;              // which of the two convolution histories the next step reads
   float *record = nullptr;       // [n_layers][max_context][max_batch][width]
@@ -116,7 +119,12 @@ struct HybridModel : kx_model {
   int fill(const KxTensorMap &files, const kx_open_options &o);
   int pack(const Slot &s, const void *src, bool src_f32);
   int logits_of(const float *x, const int *map, int n, float *d_out);
+  void split(KxLinArgs &g) const;
+  int product(KxLinArgs &g, void *row_buf) const;
 };
+
+// partial sums of a split product: two workgroups per CU with 64 rows of up to KX_NARROW_TOKENS tokens each
+constexpr int SPLIT_GROUPS = 512;
 
 // ---- kernels ----
 template <class T>
@@ -365,7 +373,7 @@ size_t HybridModel::layout(char *base) {
       const size_t pairs = std::max(T, B) * l.top;
       expert_slots = std::max(expert_slots, pairs);
       expert_mid = std::max(expert_mid, pairs * w.down.ld);
-      tiles = std::max(tiles, (size_t)kx_expert_tiles((int)std::max(T, B), l.top, l.experts, 64));
+      tiles = std::max(tiles, (size_t)kx_expert_tiles((int)std::max(T, B), l.top, l.experts, KX_EXPERT_TILE_MIN));
     }
   }
   final_norm = model_norm("final.norm");
@@ -425,6 +433,9 @@ size_t HybridModel::layout(char *base) {
   next = (uint32_t *)at(B * 4);
   history = (uint32_t *)at((size_t)max_context * B * 4);
   want = (int *)at((size_t)logit_rows() * 4);
+  split_floats = f32 ? 0 : (size_t)SPLIT_GROUPS * 64 * std::min<size_t>(std::max(T, (size_t)logit_rows()), KX_NARROW_TOKENS);
+  split_part = (float *)at(split_floats * 4);
+  split_arrived = (int *)at(SPLIT_GROUPS * 4);
   scratch_bytes = p.total - weight_bytes - cache_bytes;
   return p.total;
 }
@@ -511,6 +522,15 @@ int HybridModel::restart(int batch_) {
   return KX_OK;
 }
 
+void HybridModel::split(KxLinArgs &g) const {
+  g.part = split_part; g.part_floats = split_floats;
+  g.arrived = split_arrived; g.arrivals = SPLIT_GROUPS;
+}
+int HybridModel::product(KxLinArgs &g, void *row_buf) const {
+  split(g);
+  return kx_linear_launch(f32, g, row_buf, st);
+}
+
 int HybridModel::logits_of(const float *x, const int *map, int n, float *d_out) {
   KxLinArgs g;
   g.m = head;
@@ -519,7 +539,7 @@ int HybridModel::logits_of(const float *x, const int *map, int n, float *d_out) 
   g.row.w = final_norm; g.row.eps = c.eps;
   g.out = d_out;
   g.out_ld = c.vocab;
-  return kx_linear_launch(f32, g, rows, st);
+  return product(g, rows);
 }
 
 // latent attention of a layer, from proj into att
@@ -530,7 +550,7 @@ int HybridModel::latent(const KxHybridLayer &l, const LayerW &w, int C) {
   g.row.kind = KX_ROW_NORM; g.row.cols = l.q_rank; g.row.streams = proj + w.q_off; g.row.streams_ld = proj_ld; g.row.w = w.dq_norm; g.row.eps = c.eps;
   g.out = lat_q;
   g.out_ld = w.uq.rows;
-  KX_DO(kx_linear_launch(f32, g, out_rows, st));
+  KX_DO(product(g, out_rows));
   KxLatentArgs a;
   a.s = l.latent;
   a.rows = w.rows; a.cap = max_context;
@@ -585,7 +605,7 @@ int HybridModel::step(const uint32_t *d_ids, bool sample, int C) {
       in.mid = in_memory ? (char *)att + w.o_ld * es : mid;
       in.mid_ld = in_memory ? w.o.ld : w.o.ld - w.o_ld;
     }
-    KX_DO(kx_linear_launch(f32, in, rows, st));
+    KX_DO(product(in, rows));
     write(out, w.o, w.hc[0]);
     if (in_memory) {
       out.row.x = att;
@@ -644,6 +664,7 @@ int HybridModel::step(const uint32_t *d_ids, bool sample, int C) {
       KxExpertFf f;
       read(f.gu, w.gu, w.norm1, w.hc[0]);
       f.gu.limit = l.limit; f.gu.alpha = l.alpha; f.gu.bias = l.bias;
+      split(out);
       f.out = out;
       f.down = w.down; f.gu_stride = w.gu_stride; f.down_stride = w.down_stride;
       f.e.experts = l.experts; f.e.top = l.top; f.e.logits = proj + w.router_off; f.e.logits_ld = proj_ld; f.e.bias = w.router_b;
@@ -652,18 +673,18 @@ int HybridModel::step(const uint32_t *d_ids, bool sample, int C) {
       f.h_buf = rows; f.row_buf = out_rows; f.mid = mid; f.y = expert_y;
       KX_DO(kx_expert_ff_launch(f32, f, T, st));
     } else {
-      KX_DO(kx_linear_launch(f32, out, out_rows, st));
+      KX_DO(product(out, out_rows));
     }
     if (l.ff_kind == KxHybridLayer::GLU) {
       KxLinArgs gu, down;
       read(gu, w.gu, w.norm2, w.hc[1]);
       gu.epi = KX_LIN_GLU;
       gu.mid = mid; gu.mid_ld = mid_ld; gu.limit = l.limit; gu.alpha = l.alpha; gu.bias = l.bias;
-      KX_DO(kx_linear_launch(f32, gu, rows, st));
+      KX_DO(product(gu, rows));
       write(down, w.down, w.hc[1]);
       down.row.x = mid;
       down.row.x_ld = mid_ld;
-      KX_DO(kx_linear_launch(f32, down, out_rows, st));
+      KX_DO(product(down, out_rows));
     }
     if (record) {
       hipLaunchKernelGGL(sum_streams_k, dim3(T), dim3(256), 0, st, streams, record + ((size_t)i * max_context + pos) * max_batch * W, W, S, batch, max_batch);

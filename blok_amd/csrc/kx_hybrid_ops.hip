@@ -373,7 +373,7 @@ extern "C" int kx_experts_create(const kx_experts_config *c, int f32, int32_t ma
   f.e.experts = c->experts; f.e.top = c->top; f.e.logits_ld = c->experts;
   OpMem &m = d->mem;
   const size_t logits = m.take(T * c->experts * 4), ids = m.take(pairs * 4), gather = m.take(pairs * 4), slot_of = m.take(pairs * 4), weights = m.take(pairs * 4),
-               slot_weight = m.take(pairs * 4), tiles = m.take((size_t)kx_expert_tiles(max_tokens, c->top, c->experts, 64) * sizeof(int4)), n_tiles = m.take(4),
+               slot_weight = m.take(pairs * 4), tiles = m.take((size_t)kx_expert_tiles(max_tokens, c->top, c->experts, KX_EXPERT_TILE_MIN) * sizeof(int4)), n_tiles = m.take(4),
                h = m.take(T * f.gu.m.ld * es), mid = m.take(pairs * f.down.ld * es), y = m.take(pairs * c->width * 4);
   const int rc = m.alloc("kx_experts_create");
   if (rc) {

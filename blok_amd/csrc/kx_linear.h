@@ -80,6 +80,12 @@ struct KxLinArgs {
   // SHIFT rows: the matrix rows [var_row[v], var_row[v + 1]) meet variant v; multiples of KX_VARIANT_ROWS
   int n_var = 1;
   int var_row[KX_MAX_VARIANTS] = {};
+  // scratch of products that split their columns over workgroups (KX_NARROW_TOKENS); without it they do not.  One launch at
+  // a time uses it.
+  float *part = nullptr;
+  size_t part_floats = 0;
+  int *arrived = nullptr;    // [arrivals], zero between launches
+  int arrivals = 0;
 };
 constexpr int KX_MAX_STREAMS = 8;
 
@@ -108,6 +114,8 @@ constexpr int KX_MAX_EXPERTS = 1024, KX_MAX_TOP = 64;
 // f32: the model's type is float, else bf16.  row_buf: tokens * m.ld elements of scratch, where the rows of a step of
 // more than KX_GEMV_TOKENS tokens are built (not used for PLAIN).
 constexpr int KX_GEMV_TOKENS = 4;
+// bf16: up to this many tokens the matrix is streamed by workgroups that hold all tokens
+constexpr int KX_NARROW_TOKENS = 64;
 int kx_linear_launch(bool f32, const KxLinArgs &a, void *row_buf, hipStream_t st);
 // The rows alone, [variant][token][ld], into `out`.
 int kx_rows_launch(bool f32, const KxRowArgs &r, int tokens, void *out, int ld, hipStream_t st);
