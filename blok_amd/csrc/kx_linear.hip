@@ -248,7 +248,7 @@ lin_gemv_k(KxLinArgs a, KxExpertArgs x) {
 }
 
 template <class T, int KIND>
-__global__ void __launch_bounds__(256) row_k(KxRowArgs a, T *out, int ld) {
+__global__ void __launch_bounds__(512) row_k(KxRowArgs a, T *out, int ld) {
   extern __shared__ float row_lds[];
   kxr::build_row<T, KIND>(a, blockIdx.x, out + (size_t)blockIdx.x * ld, ld, row_lds, (size_t)gridDim.x * ld, true);
 }
@@ -596,7 +596,8 @@ int rows_kind(const KxRowArgs &r, int tokens, T *out, int ld, hipStream_t st) {
     KX_HIP(hipFuncSetAttribute((const void *)row_k<T, KIND>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 1024));
     attr = true;
   }
-  hipLaunchKernelGGL((row_k<T, KIND>), dim3(tokens), dim3(256), scratch, st, r, out, ld);
+  // a workgroup per token: twice the threads where the tokens do not fill the chip
+  hipLaunchKernelGGL((row_k<T, KIND>), dim3(tokens), dim3(tokens <= 256 ? 512 : 256), scratch, st, r, out, ld);
   KX_LAUNCH_CHECK();
   return KX_OK;
 }

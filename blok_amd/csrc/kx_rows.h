@@ -103,6 +103,10 @@ __device__ __forceinline__ void group_scales(float *part, int groups, int spg, i
 // with a barrier.  keep: this workgroup writes what the row's kind carries over to the next step.  need: the variants
 // to build, a bit each.
 // KIND: the row's kind where it is known when the kernel is compiled.
+// A row is a few KB and the time to build one is the time of its loads one after the other: every loop asks for what UB of its
+// turns read before the first of them stores anything (a store through `dst` would keep the compiler from doing so), and what
+// comes behind a sum is asked for in front of it.
+constexpr int UB = 4;
 template <class T, int KIND = -1>
 __device__ __forceinline__ void build_row(const KxRowArgs &a, int tok, T *dst, int ld, float *u, size_t vstride = 0, bool keep = false,
                                           uint32_t need = ~0u) {
@@ -113,91 +117,211 @@ __device__ __forceinline__ void build_row(const KxRowArgs &a, int tok, T *dst, i
     float *part = u + a.cols;
     const float *x = a.streams + (size_t)tok * xld;
     const int gs = a.cols / a.groups, spg = max(1, nw / a.groups), units = a.groups * spg, per = (gs + spg - 1) / spg;
+    float wf[UB];
+#pragma unroll
+    for (int k = 0; k < UB; ++k) wf[k] = a.w[min(tid + k * n, a.cols - 1)];
     for (int k = wave; k < units; k += nw) {  // a wave takes a slice of one group
       const int g = k / spg, s = k - g * spg, hi = min(gs, (s + 1) * per);
       float v = 0.0f;
-      for (int j = s * per + lane; j < hi; j += 64) {
-        const int c = g * gs + j;
-        float y = 0.0f;
-        for (int t = 0; t < a.n_streams; ++t) y = __builtin_fmaf(a.in ? a.in[t] : 1.0f, x[(size_t)t * a.cols + c], y);
-        u[c] = y;
-        v = __builtin_fmaf(y, y, v);
+      for (int j0 = s * per + lane; j0 < hi; j0 += 64 * UB) {
+        float y[UB] = {};
+        for (int t = 0; t < a.n_streams; ++t) {
+          const float in = a.in ? a.in[t] : 1.0f;
+#pragma unroll
+          for (int i = 0; i < UB; ++i) y[i] = __builtin_fmaf(in, x[(size_t)t * a.cols + g * gs + min(j0 + 64 * i, hi - 1)], y[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < UB; ++i)
+          if (j0 + 64 * i < hi) {
+            u[g * gs + j0 + 64 * i] = y[i];
+            v = __builtin_fmaf(y[i], y[i], v);
+          }
       }
       v = wave_sum(v);
       if (lane == 0) part[k] = v;
     }
     __syncthreads();
     group_scales(part, a.groups, spg, gs, a.eps);
-    for (int c = tid; c < ld; c += n) dst[c] = Elem<T>::make(c < a.cols ? u[c] * part[(c / gs) * spg] * a.w[c] : 0.0f);
+    for (int c0 = tid; c0 < ld; c0 += n * UB) {
+      if (c0 != tid)
+#pragma unroll
+        for (int k = 0; k < UB; ++k) wf[k] = a.w[min(c0 + k * n, a.cols - 1)];
+#pragma unroll
+      for (int k = 0; k < UB; ++k) {
+        const int c = c0 + k * n;
+        if (c < ld) dst[c] = Elem<T>::make(c < a.cols ? u[c] * part[(c / gs) * spg] * wf[k] : 0.0f);
+      }
+    }
   } else if (kind == KX_ROW_SHIFT) {
     const bool first = tok < a.batch;
     const float *x = a.streams + (size_t)tok * xld, *x1 = first ? a.prev + (size_t)tok * a.cols : x - (size_t)a.batch * xld;
+    float xv[UB], yv[UB], wv[UB];  // of the present UB columns
+    auto ask = [&](int c0) {
+#pragma unroll
+      for (int k = 0; k < UB; ++k) {
+        const int c = min(c0 + k * n, a.cols - 1);
+        xv[k] = x[c];
+        yv[k] = x1[c];
+        wv[k] = a.w[c];
+      }
+    };
     float v = 0.0f, v1 = 0.0f;
-    for (int c = tid; c < a.cols; c += n) {
-      v = __builtin_fmaf(x[c], x[c], v);
-      v1 = __builtin_fmaf(x1[c], x1[c], v1);
+    for (int c0 = tid; c0 < a.cols; c0 += n * UB) {
+      ask(c0);
+#pragma unroll
+      for (int k = 0; k < UB; ++k)
+        if (c0 + k * n < a.cols) {
+          v = __builtin_fmaf(xv[k], xv[k], v);
+          v1 = __builtin_fmaf(yv[k], yv[k], v1);
+        }
     }
     const float sc = kx_rsqrtf(block_sum(v, u) / (float)a.cols + a.eps), sc1 = kx_rsqrtf(block_sum(v1, u) / (float)a.cols + a.eps);
     const bool last = keep && tok + a.batch >= a.tokens;
-    for (int c = tid; c < ld; c += n) {
-      float h = 0.0f, d = 0.0f;
-      if (c < a.cols) {
-        const float w = a.w[c];
-        h = x[c] * sc * w;
-        d = (first ? x1[c] : x1[c] * sc1 * w) - h;
-        if (last) a.prev_out[(size_t)(tok + a.batch - a.tokens) * a.cols + c] = h;
+    for (int c0 = tid; c0 < ld; c0 += n * UB) {
+      if (a.cols > n * UB) ask(c0);  // otherwise they are still there
+      float h[UB], d[UB];
+#pragma unroll
+      for (int k = 0; k < UB; ++k) {
+        const int c = c0 + k * n;
+        h[k] = c < a.cols ? xv[k] * sc * wv[k] : 0.0f;
+        d[k] = c < a.cols ? (first ? yv[k] : yv[k] * sc1 * wv[k]) - h[k] : 0.0f;
+        if (last && c < a.cols) a.prev_out[(size_t)(tok + a.batch - a.tokens) * a.cols + c] = h[k];
       }
       for (int m = 0; m < a.n_mix; ++m)
-        if (need >> m & 1) dst[m * vstride + c] = Elem<T>::make(c < a.cols ? __builtin_fmaf(d, a.mu[(size_t)m * a.cols + c], h) : 0.0f);
-      dst[a.n_mix * vstride + c] = Elem<T>::make(h);
+        if (need >> m & 1) {
+          float mu[UB];
+#pragma unroll
+          for (int k = 0; k < UB; ++k) mu[k] = a.mu[(size_t)m * a.cols + min(c0 + k * n, a.cols - 1)];
+#pragma unroll
+          for (int k = 0; k < UB; ++k)
+            if (c0 + k * n < ld) dst[m * vstride + c0 + k * n] = Elem<T>::make(c0 + k * n < a.cols ? __builtin_fmaf(d[k], mu[k], h[k]) : 0.0f);
+        }
+#pragma unroll
+      for (int k = 0; k < UB; ++k)
+        if (c0 + k * n < ld) dst[a.n_mix * vstride + c0 + k * n] = Elem<T>::make(h[k]);
     }
   } else if (kind == KX_ROW_GATED) {
     const int cols = a.heads * a.vdim, hl = a.tail ? a.head_ld : ld;
     const float *o = a.o + (size_t)tok * cols, *gate = a.gate + (size_t)tok * a.gate_ld;
-    auto gated = [&](int c) { return a.gate_first ? o[c] * gate[c] * sigmoid_for<T>(gate[c]) : o[c]; };
-    auto out = [&](int c, int d, float y) {
-      y *= a.w[a.w_per_column ? c : d];
-      dst[c] = Elem<T>::make(a.gate_first ? y : y * gate[c] * sigmoid_for<T>(gate[c]));
+    auto gated = [&](float y, float g) { return a.gate_first ? y * g * sigmoid_for<T>(g) : y; };
+    auto out = [&](int c, float y, float g, float w) {
+      y *= w;
+      dst[c] = Elem<T>::make(a.gate_first ? y : y * g * sigmoid_for<T>(g));
     };
+    auto weight = [&](int c, int d) { return a.w[a.w_per_column ? c : d]; };
     if (a.heads < 8) {  // a few long parts: several waves each
       float *part = u + cols;
       const int spg = max(1, nw / a.heads), units = a.heads * spg, per = (a.vdim + spg - 1) / spg;
       for (int k = wave; k < units; k += nw) {
         const int h = k / spg, s = k - h * spg, hi = min(a.vdim, (s + 1) * per);
         float v = 0.0f;
-        for (int d = s * per + lane; d < hi; d += 64) {
-          const float y = gated(h * a.vdim + d);
-          u[h * a.vdim + d] = y;
-          v = __builtin_fmaf(y, y, v);
+        for (int d0 = s * per + lane; d0 < hi; d0 += 64 * UB) {
+          float ov[UB], gv[UB];
+#pragma unroll
+          for (int i = 0; i < UB; ++i) {
+            const int c = h * a.vdim + min(d0 + 64 * i, hi - 1);
+            ov[i] = o[c];
+            gv[i] = a.gate_first ? gate[c] : 0.0f;
+          }
+#pragma unroll
+          for (int i = 0; i < UB; ++i)
+            if (d0 + 64 * i < hi) {
+              const float y = gated(ov[i], gv[i]);
+              u[h * a.vdim + d0 + 64 * i] = y;
+              v = __builtin_fmaf(y, y, v);
+            }
         }
         v = wave_sum(v);
         if (lane == 0) part[k] = v;
       }
       __syncthreads();
       group_scales(part, a.heads, spg, a.vdim, a.eps);
-      for (int c = tid; c < cols; c += n) out(c, c % a.vdim, u[c] * part[(c / a.vdim) * spg]);
+      for (int c0 = tid; c0 < cols; c0 += n * UB) {
+        float wv[UB], gv[UB];
+#pragma unroll
+        for (int i = 0; i < UB; ++i) {
+          const int c = min(c0 + i * n, cols - 1);
+          wv[i] = weight(c, c % a.vdim);
+          gv[i] = a.gate_first ? 0.0f : gate[c];
+        }
+#pragma unroll
+        for (int i = 0; i < UB; ++i) {
+          const int c = c0 + i * n;
+          if (c < cols) out(c, u[c] * part[(c / a.vdim) * spg], gv[i], wv[i]);
+        }
+      }
+    } else if (a.vdim <= 128) {  // a wave takes UB heads at a time, two columns of each per lane
+      const int two = a.vdim > 64;
+      for (int h0 = wave; h0 < a.heads; h0 += nw * UB) {
+        float ov[UB][2], gv[UB][2], wv[UB][2];
+#pragma unroll
+        for (int i = 0; i < UB; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            if (j && !two) continue;
+            const int d = min(lane + 64 * j, a.vdim - 1), c = min(h0 + i * nw, a.heads - 1) * a.vdim + d;
+            ov[i][j] = o[c];
+            gv[i][j] = gate[c];
+            wv[i][j] = weight(c, d);
+          }
+#pragma unroll
+        for (int i = 0; i < UB; ++i) {
+          const int h = h0 + i * nw;
+          if (h >= a.heads) break;
+          float v = 0.0f, y[2];
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            if (lane + 64 * j < a.vdim) {
+              y[j] = gated(ov[i][j], gv[i][j]);
+              v = __builtin_fmaf(y[j], y[j], v);
+            }
+          const float sc = kx_rsqrtf(wave_sum(v) / (float)a.vdim + a.eps);
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            if (lane + 64 * j < a.vdim) out(h * a.vdim + lane + 64 * j, y[j] * sc, gv[i][j], wv[i][j]);
+        }
+      }
     } else {
       for (int h = wave; h < a.heads; h += nw) {
         float v = 0.0f;
         for (int d = lane; d < a.vdim; d += 64) {
-          const float y = gated(h * a.vdim + d);
+          const int c = h * a.vdim + d;
+          const float y = gated(o[c], gate[c]);
           v = __builtin_fmaf(y, y, v);
         }
         const float sc = kx_rsqrtf(wave_sum(v) / (float)a.vdim + a.eps);
-        for (int d = lane; d < a.vdim; d += 64) out(h * a.vdim + d, d, gated(h * a.vdim + d) * sc);
+        for (int d = lane; d < a.vdim; d += 64) {
+          const int c = h * a.vdim + d;
+          out(c, gated(o[c], gate[c]) * sc, gate[c], weight(c, d));
+        }
       }
     }
     for (int c = cols + tid; c < hl; c += n) dst[c] = Elem<T>::make(0.0f);
     if (a.tail) {
       const T *x = (const T *)a.tail + (size_t)tok * a.tail_ld;
-      for (int c = tid * 8; c < ld - hl; c += n * 8) *(typename Elem<T>::Raw *)(dst + hl + c) = Elem<T>::cached(x + c);
+#pragma unroll 1
+      for (int c0 = tid * 8; c0 < ld - hl; c0 += n * 8 * UB) {
+        typename Elem<T>::Raw r[UB];
+#pragma unroll
+        for (int k = 0; k < UB; ++k) r[k] = Elem<T>::cached(x + min(c0 + k * n * 8, ld - hl - 8));
+#pragma unroll
+        for (int k = 0; k < UB; ++k)
+          if (c0 + k * n * 8 < ld - hl) *(typename Elem<T>::Raw *)(dst + hl + c0 + k * n * 8) = r[k];
+      }
     }
   } else if (kind == KX_ROW_TANH) {
     const float *x = a.streams + (size_t)tok * xld;
     for (int c = tid; c < ld; c += n) dst[c] = Elem<T>::make(c < a.cols ? tanhf(x[c]) : 0.0f);
   } else {
     const T *x = (const T *)a.x + (size_t)tok * a.x_ld;
-    for (int c = tid * 8; c < ld; c += n * 8) *(typename Elem<T>::Raw *)(dst + c) = Elem<T>::cached(x + c);
+    for (int c0 = tid * 8; c0 < ld; c0 += n * 8 * UB) {
+      typename Elem<T>::Raw r[UB];
+#pragma unroll
+      for (int k = 0; k < UB; ++k) r[k] = Elem<T>::cached(x + min(c0 + k * n * 8, ld - 8));
+#pragma unroll
+      for (int k = 0; k < UB; ++k)
+        if (c0 + k * n * 8 < ld) *(typename Elem<T>::Raw *)(dst + c0 + k * n * 8) = r[k];
+    }
   }
   __syncthreads();
 }
