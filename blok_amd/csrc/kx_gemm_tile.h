@@ -1,0 +1,210 @@
+// kx_gemm_tile.h -- one tile of a bf16 matrix product on the matrix cores, y[t][r] = sum_k x[t][k] w[r][k]: the main loop that
+// the products of the hybrid decoder (kx_linear.hip) and the dense ones of Kimi-K2 (kx_dense_gemm.hip) share, and the
+// hand-over between workgroups that split a tile's columns.  No counterpart in the reference, whose products are mat-vecs
+// (src/kimi_exec.cu:272-298).
+//
+// A workgroup of WM x WN waves owns BM tokens and BN rows; wave (wm, wn) holds MI x NI blocks of 32 x 32
+// (v_mfma_f32_32x32x16_bf16).  Both operands are staged through LDS in blocks of 64 columns by global -> LDS copies, 128-byte rows
+// (whole lines: with 64-byte rows the copies cost as much a row and everything 10 to 15 % more) with the 16-byte pieces xor-ed by
+// the row, so that row-per-lane reads are free of bank conflicts.
+// The LDS is a ring of SLOTS half blocks -- tokens, matrix rows, tokens, ... --, two of the block that is multiplied and the others
+// on their way:
+//   operands of piece q + 1 are read while piece q is multiplied; between the last two pieces of a block the workgroup waits
+//   for the next block (a half that was asked for behind it may still be on its way), passes its one barrier per block
+//   -- behind it nobody reads the present block any more, its last operands are in registers --, asks for two more halves
+//   in its place and reads the next block's first operands.
+// What bounds it: a wave reads (MI + NI) KB of operands for MI NI products of 32 cycles, and LDS gives a CU about 128 bytes a
+// cycle: waves of 2 x 4 blocks stay below that with the copies' writes, waves of 2 x 2 do not; and a block of the 256 x 256 tile is
+// 64 KB for 2048 cycles of products and takes about as long to arrive.  2048 x 36864 x 7168 (32-bit result): 1026 us, the copies
+// alone 833, the products alone 710, everything but the copies 795.  A fifth slot, which keeps the queue of copies from
+// running dry, is worth 2 to 8 % to two workgroups per CU with few tiles and costs the large tile 4 %.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+#include "kx_arrive.h"
+#include "kx_lds_copy.h"
+
+namespace kxg {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+template <int WM_, int WN_, int MI_, int NI_, int SLOTS_>
+struct Tile {
+  static constexpr int SLOTS = SLOTS_, WM = WM_, WN = WN_, MI = MI_, NI = NI_, WAVES = WM * WN, THREADS = WAVES * 64;
+  static constexpr int BM = WM * MI * 32, BN = WN * NI * 32, SLOT = (BM > BN ? BM : BN) * 128, LDS = SLOTS * SLOT;
+  static constexpr int WAVES_PER_SIMD = MI * NI >= 16 ? 1 : 2;
+  static constexpr int CX = BM / 8 / WAVES, CW = BN / 8 / WAVES;  // copy instructions of a wave for half a block, 8 rows each
+  static constexpr size_t PART = (size_t)BM * BN;          // floats of a part's sums
+  static_assert(SLOTS == 4 || SLOTS == 5, "two blocks, and half of a third");
+  static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "the copies of a block are spread evenly over the waves");
+
+  // Columns 64 kb0 .. 64 kb1 - 1 (kb0 < kb1).  row(r): where staged row r begins, tokens 0 .. BM - 1, then BN rows of the
+  // matrix; every row has to be readable, what a row past the end holds only reaches sums that are not used.
+  template <class Row>
+  static __device__ __forceinline__ void run(uint8_t *lds, int kb0, int kb1, Row row, f32x16 (&acc)[MI][NI]) {
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wave / WN, wn = wave % WN, lr = lane & 31, h = lane >> 5, sub = lane >> 3, n = kb1 - kb0;
+    const uint16_t *src[CX + CW];
+#pragma unroll
+    for (int i = 0; i < CX + CW; ++i)
+      src[i] = row(i < CX ? (i * WAVES + wave) * 8 + sub : BM + ((i - CX) * WAVES + wave) * 8 + sub) + kb0 * 64 + ((lane & 7) ^ sub) * 8;
+    auto copy_x = [&](int b, int slot) {
+#pragma unroll
+      for (int i = 0; i < CX; ++i) kx_copy16_to_lds(src[i] + b * 64, __builtin_amdgcn_readfirstlane(lds0 + slot * SLOT + (i * WAVES + wave) * 1024));
+    };
+    auto copy_w = [&](int b, int slot) {
+#pragma unroll
+      for (int i = 0; i < CW; ++i) kx_copy16_to_lds(src[CX + i] + b * 64, __builtin_amdgcn_readfirstlane(lds0 + slot * SLOT + (i * WAVES + wave) * 1024));
+    };
+    struct Frag {
+      bf16x8 x[MI], w[NI];
+    };
+    const uint8_t *const xs = lds + (wm * MI * 32 + lr) * 128, *const ws = lds + (wn * NI * 32 + lr) * 128;
+    int sx = 0, sw = 1;  // slots of the present block
+    auto next = [](int slot) { return slot >= SLOTS - 2 ? slot - (SLOTS - 2) : slot + 2; };
+    auto read = [&](Frag &f, int q) {
+      const int p = ((2 * q + h) ^ (lr & 7)) * 16;
+#pragma unroll
+      for (int i = 0; i < MI; ++i) f.x[i] = *(const bf16x8 *)(xs + sx * SLOT + p + i * 4096);
+#pragma unroll
+      for (int j = 0; j < NI; ++j) f.w[j] = *(const bf16x8 *)(ws + sw * SLOT + p + j * 4096);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto multiply = [&](const Frag &f) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NI; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.x[i], f.w[j], acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+    Frag f0, f1;
+    copy_x(0, 0);
+    copy_w(0, 1);
+    if (n > 1) {
+      copy_x(1, 2);
+      copy_w(1, 3);
+    }
+    if (SLOTS == 5 && n > 2) {
+      copy_x(2, 4);
+      kx_wait_copies<CX + CW + CX>();
+    } else if (n > 1) {
+      kx_wait_copies<CX + CW>();
+    } else {
+      kx_wait_copies<0>();
+    }
+    kx_lds_barrier();
+    read(f0, 0);
+    for (int b = 0; b < n; ++b) {
+      read(f1, 1);
+      multiply(f0);
+      read(f0, 2);
+      multiply(f1);
+      read(f1, 3);
+      multiply(f0);
+      if (b + 1 < n) {
+        if (SLOTS == 5 && b + 2 < n) kx_wait_copies<CX>();  // the tokens of block b + 2 are behind block b + 1
+        else kx_wait_copies<0>();
+        kx_lds_barrier();
+        if (SLOTS == 5) {
+          if (b + 2 < n) copy_w(b + 2, sx);
+          if (b + 3 < n) copy_x(b + 3, sw);
+        } else if (b + 2 < n) {
+          copy_x(b + 2, sx);
+          copy_w(b + 2, sw);
+        }
+        sx = next(sx);
+        sw = next(sw);
+        read(f0, 0);
+      }
+      multiply(f1);
+    }
+  }
+  // Element v of block (i, j) of the present lane: matrix row col(j) and token row(i, v) of the tile.
+  static __device__ __forceinline__ int col(int j) { return (((int)threadIdx.x >> 6) % WN * NI + j) * 32 + (threadIdx.x & 31); }
+  static __device__ __forceinline__ int row(int i, int v) {
+    return (((int)threadIdx.x >> 6) / WN * MI + i) * 32 + 8 * (v >> 2) + 4 * (threadIdx.x >> 5 & 1) + (v & 3);
+  }
+
+  // The sums of `parts` workgroups that hold a part of the columns each, added in the parts' order by the one that arrives last
+  // (kx_arrive.h); false for the others.  part: parts * PART floats of this tile; arrived: its counter.
+  static __device__ __forceinline__ bool gather(uint8_t *lds, f32x16 (&acc)[MI][NI], float *part, int *arrived, int parts, int p) {
+    int &last = *(int *)lds;  // behind the barrier below nobody reads operands any more
+    uint64_t *at = (uint64_t *)part;
+    constexpr size_t PER = PART / 2;
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          const float a = acc[i][j][2 * q], b = acc[i][j][2 * q + 1];
+          kx_arrive_store(at + p * PER + ((i * NI + j) * 8 + q) * THREADS + threadIdx.x,
+                          (uint64_t)__builtin_bit_cast(uint32_t, a) | (uint64_t)__builtin_bit_cast(uint32_t, b) << 32);
+        }
+    kx_arrive_writes_done();
+    __syncthreads();
+    if (threadIdx.x == 0) last = kx_arrive_is_last(arrived, parts);
+    __syncthreads();
+    if (!last) return false;
+    if (threadIdx.x == 0) kx_arrive_reset(arrived);
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+        for (int s = 0; s < parts; ++s) {
+          uint64_t y[8];
+#pragma unroll
+          for (int q = 0; q < 8; ++q) y[q] = kx_arrive_load(at + s * PER + ((i * NI + j) * 8 + q) * THREADS + threadIdx.x);
+#pragma unroll
+          for (int q = 0; q < 8; ++q) {
+            const float a = __builtin_bit_cast(float, (uint32_t)y[q]), b = __builtin_bit_cast(float, (uint32_t)(y[q] >> 32));
+            acc[i][j][2 * q] = s ? acc[i][j][2 * q] + a : a;
+            acc[i][j][2 * q + 1] = s ? acc[i][j][2 * q + 1] + b : b;
+          }
+        }
+    return true;
+  }
+};
+
+// Workgroup id -> work item: consecutive ids go to the chip's eight dies in turn, each with its own L2, so every die takes a
+// run of consecutive items, which share rows of tokens and of the matrix.
+__device__ __forceinline__ int item_of(int id, int n) {
+  const int die = id & 7, q = n >> 3, r = n & 7;
+  return die * q + min(die, r) + (id >> 3);
+}
+
+typedef Tile<4, 2, 2, 4, 4> Large;   // 256 x 256, 8 waves, a CU each
+typedef Tile<2, 2, 2, 2, 5> Medium;  // 128 x 128, 4 waves, two workgroups per CU
+
+// Which tile, and in how many parts of the columns, for one product of `tokens` x `rows` with `blocks` blocks of 64 columns.
+// Where the medium tiles leave CUs idle they take parts, of at least 16 blocks; beyond that the shorter of two estimates, in
+// us: a round of large tiles takes 12 + 1.55 per block on 256 CUs, of medium ones (two per CU) 6 + 1.22.  Measured against it (us,
+// 32-bit results, large / medium): 2048 x 16384 x 2048 150 / 214, 2048 x 8448 x 2048 116 / 94, 2048 x 5120 x 2048 64 / 61,
+// 2048 x 36864 x 7168 1026 / 1265, 2048 x 7168 x 8192 252 / 329, 952 x 7168 x 18432 455 / 353; in parts: 300 x 2048 x 8192 71 alone,
+// 32 in four, 100 x 2048 x 8192 73 and 29 in eight, 2048 x 384 x 7168 65 and 32 in four.
+struct Choice {
+  bool large;
+  int parts;
+};
+inline Choice choose(int tokens, int rows, int blocks, size_t part_floats, int arrivals, int cus) {
+  auto tiles = [&](int m, int n) { return (long)((tokens + m - 1) / m) * ((rows + n - 1) / n); };
+  const long medium = tiles(Medium::BM, Medium::BN), large = tiles(Large::BM, Large::BN);
+  if (medium <= cus) {
+    long p = cus / medium;
+    if (p > blocks / 16) p = blocks / 16;
+    if ((size_t)p > part_floats / Medium::PART / medium) p = part_floats / Medium::PART / medium;
+    return {false, p < 2 || medium > arrivals ? 1 : (int)p};
+  }
+  const double l = (double)((large + cus - 1) / cus) * (12 + 1.55 * blocks), m = (medium > 2 * cus ? medium / (2.0 * cus) : 1.0) * (6 + 1.22 * blocks);
+  return {l < m, 1};
+}
+
+}  // namespace kxg

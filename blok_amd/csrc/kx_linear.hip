@@ -8,8 +8,8 @@
 // streams two rows of the matrix at a time, 8 columns per lane and load, the next pieces in flight while the present
 // ones are multiplied; the epilogue stores the product, forms the gated activation of a (gate, up) pair, or updates
 // all residual streams of the row.
-// lin_gemm_k (bf16, more tokens): tiles of BM tokens x 128 rows, v_mfma_f32_32x32x16_bf16, both operands staged through
-// LDS by global -> LDS copies in blocks of 64 columns, two stages, 16-byte pieces xor-swizzled by the row.
+// lin_narrow_k (bf16, up to 64 tokens): all tokens against 64 rows, the columns split over waves and workgroups.
+// lin_gemm_k (bf16, more tokens): tiles of 256 x 256 or 128 x 128 on the matrix cores (kx_gemm_tile.h).
 // lin_gemm_f32_k (f32): tiles of 64 x 64 on the vector ALU; true 32-bit products.
 //
 // Products with experts: up to 4 tokens lin_gemv_k with a matrix per (token, choice), the routing in its prologue, and with
@@ -17,18 +17,17 @@
 // the GEMMs with tiles of slots sorted by expert.
 #include <algorithm>
 #include <atomic>
-#include "kx_arrive.h"
 #include "kx_common.h"
 #include "kx_experts.h"
-#include "kx_lds_copy.h"
+#include "kx_gemm_tile.h"
 #include "kx_linear.h"
 #include "kx_rows.h"
 
 namespace {
 
 using kxr::Elem;
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
+using kxg::bf16x8;
+using kxg::f32x16;
 
 // ---- epilogues, one output element (or pair) at a time ----
 template <class T>
@@ -254,8 +253,8 @@ __global__ void __launch_bounds__(512) row_k(KxRowArgs a, T *out, int ld) {
 }
 
 // ---- bf16 GEMM ----
-// 4 waves as 2 x 2: wave (wm, wn) owns MI blocks of 32 tokens and 64 rows (two blocks of 32: with GLU rows, gate and up).
-// GROUP: blockIdx.y is a tile of slots of one expert.
+// Tiles of kx_gemm_tile.h; with GLU rows a wave's blocks are gate and up in turn.  GROUP: blockIdx.y is a tile of slots of one
+// expert.
 struct Tile {
   int m0, end;  // rows of the result
   size_t w;     // offset of the matrix
@@ -281,93 +280,65 @@ __device__ __forceinline__ size_t source_row(const KxExpertArgs &e, const Tile &
   return GROUP && e.gather ? e.gather[s] : s;
 }
 
-template <int MI, int EPI, bool GROUP>
-__global__ void __launch_bounds__(256, 2) lin_gemm_k(KxLinArgs a, KxExpertArgs e, const uint16_t *__restrict__ x, int x_ld) {
-  constexpr int BM = MI * 64, BN = 128, ROWS = BM + BN, STAGE = ROWS * 128, CPW = ROWS / 32;
+template <class TL, int EPI, bool GROUP>
+__global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) lin_gemm_k(KxLinArgs a, KxExpertArgs e, const uint16_t *__restrict__ x, int x_ld, int parts) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm = wave >> 1, wn = wave & 1, lr = lane & 31, h = lane >> 5;
-  const int n0 = blockIdx.x * BN;
   Tile tl;
-  if (!tile_of<GROUP>(a, e, BM, tl)) return;
-  const int m0 = tl.m0;
+  int n0, part = 0, tile = 0;
+  if constexpr (GROUP) {
+    if (!tile_of<true>(a, e, TL::BM, tl)) return;
+    n0 = blockIdx.x * TL::BN;
+  } else {
+    const int tm = (a.tokens + TL::BM - 1) / TL::BM, tiles = (int)gridDim.x / parts, item = kxg::item_of(blockIdx.x, gridDim.x);
+    part = item / tiles;
+    tile = item - part * tiles;
+    n0 = tile / tm * TL::BN;
+    tl.m0 = tile % tm * TL::BM;
+    tl.end = a.tokens;
+    tl.w = 0;
+  }
   x += (size_t)variant_of(a, n0) * a.tokens * x_ld;
   const int nb = a.m.ld >> 6;  // blocks of 64 columns
-  // copy instruction i of this wave moves 8 rows of 128 bytes: lane l the piece (l % 8) ^ (row % 8) of row l / 8
-  const uint16_t *src[CPW];
-  uint32_t dst[CPW];
+  f32x16 acc[TL::MI][TL::NI];
+  TL::run(lds, (int)((long)nb * part / parts), (int)((long)nb * (part + 1) / parts), [&](int r) {
+    return r < TL::BM ? x + source_row<GROUP>(e, tl, r) * x_ld : (const uint16_t *)a.m.w + tl.w + (size_t)min(n0 + r - TL::BM, a.m.rows - 1) * a.m.ld;
+  }, acc);
+  if (!GROUP && parts > 1 && !TL::gather(lds, acc, a.part + (size_t)tile * parts * TL::PART, a.arrived + tile, parts, part)) return;
 #pragma unroll
-  for (int i = 0; i < CPW; ++i) {
-    const int r0 = (i * 4 + wave) * 8, row = r0 + (lane >> 3), piece = (lane & 7) ^ (row & 7);
-    src[i] = (row < BM ? x + source_row<GROUP>(e, tl, row) * x_ld
-                       : (const uint16_t *)a.m.w + tl.w + (size_t)min(n0 + row - BM, a.m.rows - 1) * a.m.ld) + piece * 8;
-    dst[i] = r0 * 128;
-  }
-  auto copy = [&](int b) {
-    const uint32_t st = lds0 + (b & 1) * STAGE;
-#pragma unroll
-    for (int i = 0; i < CPW; ++i) kx_copy16_to_lds(src[i] + b * 64, __builtin_amdgcn_readfirstlane(st + dst[i]));
-  };
-  f32x16 acc[MI][2];
-#pragma unroll
-  for (int i = 0; i < MI; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-  copy(0);
-  for (int b = 0; b < nb; ++b) {
-    kx_wait_copies<0>();
-    kx_lds_barrier();  // block b is in LDS for every wave, and every wave is done with block b - 1
-    if (b + 1 < nb) copy(b + 1);
-    const uint8_t *st = lds + (b & 1) * STAGE;
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      const int p = ((2 * kk + h) ^ (lr & 7)) * 16;  // rows of a block of 32 start at a multiple of 8
-      bf16x8 xa[MI], wb[2];
-#pragma unroll
-      for (int i = 0; i < MI; ++i) xa[i] = *(const bf16x8 *)(st + ((wm * MI + i) * 32 + lr) * 128 + p);
-#pragma unroll
-      for (int j = 0; j < 2; ++j) wb[j] = *(const bf16x8 *)(st + (BM + (wn * 2 + j) * 32 + lr) * 128 + p);
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa[i], wb[j], acc[i][j], 0, 0, 0);
-    }
-  }
-  // D[i][j]: j = lane % 32 (row of the matrix), i = 8 (v / 4) + 4 (lane / 32) + v % 4 (token)
-  const int rg = n0 + wn * 64 + lr;
-  auto token = [&](int i, int v) { return m0 + (wm * MI + i) * 32 + 8 * (v >> 2) + 4 * h + (v & 3); };
-#pragma unroll
-  for (int i = 0; i < MI; ++i) {
+  for (int i = 0; i < TL::MI; ++i) {
     if constexpr (EPI == KX_LIN_GLU) {
 #pragma unroll
-      for (int v = 0; v < 16; ++v)
-        if (token(i, v) < tl.end && rg < a.m.rows)
-          put_glu<uint16_t>(a, token(i, v), (n0 + wn * 64) / 2 + lr, acc[i][0][v], acc[i][1][v], GROUP ? e.slot_weight[token(i, v)] : 1.0f);
+      for (int j = 0; j < TL::NI; j += 2) {
+        const int r = n0 + TL::col(j);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int t = tl.m0 + TL::row(i, v);
+          if (t < tl.end && r < a.m.rows)
+            put_glu<uint16_t>(a, t, (r >> 6) * KX_GLU_BLOCK + (r & 31), acc[i][j][v], acc[i][j + 1][v], GROUP ? e.slot_weight[t] : 1.0f);
+        }
+      }
     } else {
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int r = rg + 32 * j;
+      for (int j = 0; j < TL::NI; ++j) {
+        const int r = n0 + TL::col(j);
         if constexpr (EPI == KX_LIN_F32) {
 #pragma unroll
           for (int v = 0; v < 16; ++v)
-            if (token(i, v) < tl.end && r < a.m.rows) put_f32<uint16_t>(a, token(i, v), r, acc[i][j][v]);
+            if (tl.m0 + TL::row(i, v) < tl.end && r < a.m.rows) put_f32<uint16_t>(a, tl.m0 + TL::row(i, v), r, acc[i][j][v]);
         } else if constexpr (EPI == KX_LIN_HEADS) {
 #pragma unroll
           for (int v = 0; v < 16; ++v)
-            if (token(i, v) < tl.end && r < a.m.rows) put_head<uint16_t>(a, token(i, v), r, acc[i][j][v]);
+            if (tl.m0 + TL::row(i, v) < tl.end && r < a.m.rows) put_head<uint16_t>(a, tl.m0 + TL::row(i, v), r, acc[i][j][v]);
         } else {
           constexpr int G = most_streams(EPI) > 2 ? 4 : 16;  // elements read before the first is written
 #pragma unroll
           for (int v0 = 0; v0 < 16; v0 += G) {
             Streams<EPI> res[G];
 #pragma unroll
-            for (int v = 0; v < G; ++v) res[v].load(a, min(token(i, v0 + v), a.tokens - 1), min(r, a.m.rows - 1));
+            for (int v = 0; v < G; ++v) res[v].load(a, min(tl.m0 + TL::row(i, v0 + v), a.tokens - 1), min(r, a.m.rows - 1));
 #pragma unroll
             for (int v = 0; v < G; ++v)
-              if (token(i, v0 + v) < a.tokens && r < a.m.rows) res[v].store(a, token(i, v0 + v), r, acc[i][j][v0 + v]);
+              if (tl.m0 + TL::row(i, v0 + v) < a.tokens && r < a.m.rows) res[v].store(a, tl.m0 + TL::row(i, v0 + v), r, acc[i][j][v0 + v]);
           }
         }
       }
@@ -638,6 +609,21 @@ int narrow_launch(const KxLinArgs &a, const KxExpertArgs &e, const uint16_t *x, 
   return KX_OK;
 }
 
+typedef kxg::Tile<2, 2, 1, 2, 4> SmallSlots;  // 64 slots of an expert
+template <class TL, int EPI, bool GROUP>
+int tile_launch(const KxLinArgs &a, const KxExpertArgs &e, const uint16_t *x, int x_ld, int parts, hipStream_t st) {
+  static std::atomic<bool> attr{false};
+  if (!attr) {
+    KX_HIP(hipFuncSetAttribute((const void *)lin_gemm_k<TL, EPI, GROUP>, hipFuncAttributeMaxDynamicSharedMemorySize, TL::LDS));
+    attr = true;
+  }
+  const int tn = kx_cdiv(a.m.rows, TL::BN);
+  const dim3 grid = GROUP ? dim3(tn, e.max_tiles) : dim3(tn * kx_cdiv(a.tokens, TL::BM) * parts);
+  hipLaunchKernelGGL((lin_gemm_k<TL, EPI, GROUP>), grid, dim3(TL::THREADS), TL::LDS, st, a, e, x, x_ld, parts);
+  KX_LAUNCH_CHECK();
+  return KX_OK;
+}
+
 // GEMM over rows in memory; GROUP: e.max_tiles tiles of slots
 template <class T, int EPI, bool GROUP>
 int gemm_launch(const KxLinArgs &a, const KxExpertArgs &e, const T *x, int x_ld, hipStream_t st) {
@@ -646,19 +632,15 @@ int gemm_launch(const KxLinArgs &a, const KxExpertArgs &e, const T *x, int x_ld,
     if (e.tile_slots <= 32) return narrow_launch<EPI, true>(a, e, x, x_ld, st);
   if constexpr (sizeof(T) == 4) {
     hipLaunchKernelGGL((lin_gemm_f32_k<EPI, GROUP>), dim3(kx_cdiv(a.m.rows, 64), GROUP ? e.max_tiles : kx_cdiv(a.tokens, 64)), dim3(256), 0, st, a, e, x, x_ld);
+    KX_LAUNCH_CHECK();
+    return KX_OK;
+  } else if constexpr (GROUP) {
+    return e.tile_slots > 64 ? tile_launch<kxg::Medium, EPI, true>(a, e, x, x_ld, 1, st) : tile_launch<SmallSlots, EPI, true>(a, e, x, x_ld, 1, st);
   } else {
-    static std::atomic<bool> attr{false};
-    if (!attr) {
-      KX_HIP(hipFuncSetAttribute((const void *)lin_gemm_k<2, EPI, GROUP>, hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024));
-      attr = true;
-    }
-    const bool wide = GROUP ? e.tile_slots > 64 : a.tokens > 64;
-    const int tiles = GROUP ? e.max_tiles : kx_cdiv(a.tokens, wide ? 128 : 64);
-    if (wide) hipLaunchKernelGGL((lin_gemm_k<2, EPI, GROUP>), dim3(kx_cdiv(a.m.rows, 128), tiles), dim3(256), 2 * 256 * 128, st, a, e, x, x_ld);
-    else hipLaunchKernelGGL((lin_gemm_k<1, EPI, GROUP>), dim3(kx_cdiv(a.m.rows, 128), tiles), dim3(256), 2 * 192 * 128, st, a, e, x, x_ld);
+    const kxg::Choice c = kxg::choose(a.tokens, a.m.rows, a.m.ld >> 6, a.part ? a.part_floats : 0, a.arrived ? a.arrivals : 0, std::max(1, kx_device_cus()));
+    if (c.large && a.n_var == 1) return tile_launch<kxg::Large, EPI, false>(a, e, x, x_ld, 1, st);  // variants begin at multiples of 128 rows
+    return tile_launch<kxg::Medium, EPI, false>(a, e, x, x_ld, c.parts, st);
   }
-  KX_LAUNCH_CHECK();
-  return KX_OK;
 }
 
 template <class T, int EPI>

@@ -1,11 +1,15 @@
 """Products of the hybrid decoder where their kernels change: few tokens with the columns split over workgroups, experts with
-few slots.  Against the plain forward passes, with the bars of the whole-model tests."""
+few slots, large tiles.  Against the plain forward passes, with the bars of the whole-model tests."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import kagalorn_case as KC
 import kagalorn_oracle as K
-from test_gpu_kagalorn import BF16_LOGITS, rel
+from blok_amd.lib import DevBuf, KxLinearArgs, check
+from kxt import dev
+from test_gpu_kagalorn import BF16_LOGITS, _matrix, rel
 from test_gpu_rapitar import Experts
 
 pytestmark = pytest.mark.gpu
@@ -13,13 +17,14 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("ff", [4200, 4130], ids=["whole blocks", "half a block left"])
 def test_few_tokens_against_wide_matrices(kxlib, tmp_path, ff):
-    """5 to 64 tokens a step: up to eight parts of 66 and 65 pieces of 64 columns, and the last part shorter than the others."""
+    """5 to 64 tokens a step: up to eight parts of 66 and 65 pieces of 64 columns, and the last part shorter than the others;
+    66 to 192 tokens: tiles in up to four parts."""
     cfg = KC.config([KC.delta(heads=4, kv_heads=2, dim=32, vdim=640, ff=ff), KC.attention(ff=ff)], width=192, vocab=300)
     w = KC.weights(cfg, ff)
     ids = np.stack([KC.tokens(cfg, 6, 100 + b) for b in range(64)])
     want = np.stack([K.forward(cfg, w, s) for s in ids], 1)
     with KC.Model(KC.write(tmp_path, cfg, w), "bfloat16", batch=64, context=6) as m:
-        for batch, cuts in ((5, [1]), (8, [4, 1]), (31, [2, 1]), (33, [1]), (63, [1]), (64, [1]), (5, [1])):
+        for batch, cuts in ((5, [1]), (8, [4, 1]), (31, [2, 1]), (33, [1]), (63, [1]), (64, [1]), (5, [1]), (33, [2]), (64, [2]), (43, [3]), (64, [3])):
             first = m.run(ids[:batch], cuts, batch)
             assert KC.logit_error(first, want[:, :batch]).max() < BF16_LOGITS, (batch, cuts)
             assert (m.run(ids[:batch], cuts, batch) == first).all(), "the parts' order does not depend on who comes last"
@@ -38,3 +43,53 @@ def test_experts_of_more_slots_than_a_small_tile(kxlib, tokens):
     assert (np.sort(ids, 1) == [5, 40, 99]).all()
     assert rel(got, a.oracle(x, rows, ids)) < 2e-2
     a.close()
+
+
+def _put(x):
+    """bf16 values in memory as the rows of a product"""
+    return dev((np.ascontiguousarray(x, np.float32).view(np.uint32) >> 16).astype(np.uint16))
+
+
+@pytest.mark.parametrize("tokens, rows, cols", [(1985, 8000, 64), (2048, 8192, 128), (1793, 7937, 192)], ids=lambda v: str(v))
+def test_large_tiles(kxlib, tokens, rows, cols):
+    """Tiles of 256 x 256, whole and with remainders of tokens and rows, through every epilogue that a prompt meets."""
+    r = np.random.default_rng(rows)
+    w, x = KC.bf16(r.standard_normal((rows, cols)) * cols ** -0.5), KC.bf16(r.standard_normal((tokens, cols)))
+    dw, ld = _matrix(w, 0)
+    dx, y = _put(x), (x @ w.T).astype(np.float64)
+    scratch = DevBuf(64)
+
+    def run(out, m=dw, n=rows, **kw):
+        a = KxLinearArgs(f32=0, tokens=tokens, rows=n, cols=cols, ld=ld, row_kind=0, streams=1, groups=1, d_w=m.ptr, d_x=dx.ptr, x_ld=ld)
+        for k, v in kw.items():
+            setattr(a, k, v)
+        a.d_out = out.ptr
+        check(kxlib.kx_linear_run(C.byref(a), scratch.ptr, None))
+        check(kxlib.kx_sync(None))
+
+    # stored; the last rows through gelu
+    acts = 70
+    out, mid = dev(np.full((tokens, rows), 7.0, np.float32)), dev(np.zeros((tokens, 96), np.uint16))
+    run(out, epilogue=0, out_ld=rows, act_rows=acts, d_mid=mid.ptr, mid_ld=96)
+    got, act = out.to_numpy(np.float32, (tokens, rows)), mid.to_numpy(np.uint16, (tokens, 96))
+    assert rel(got[:, :rows - acts], y[:, :rows - acts]) < 1e-5 and (got[:, rows - acts:] == 7.0).all()
+    z = y[:, rows - acts:]
+    gelu = 0.5 * z * (1 + np.tanh(np.sqrt(2 / np.pi) * (z + 0.044715 * z ** 3)))
+    assert rel((act[:, :acts].astype(np.uint32) << 16).view(np.float32), gelu) < 1e-2 and not act[:, acts:].any()
+    # two streams, and one
+    for streams in (2, 1):
+        s0 = r.standard_normal((tokens, streams, rows)).astype(np.float32)
+        mix, ow = r.standard_normal((streams, streams)).astype(np.float32), r.standard_normal(streams).astype(np.float32)
+        ds, dm, do = dev(s0), dev(mix), dev(ow)
+        run(ds, epilogue=2, streams=streams, d_mix=dm.ptr, d_outw=do.ptr)
+        want = K.hyper_write(s0.transpose(1, 0, 2).astype(np.float64), mix, ow, y).transpose(1, 0, 2)
+        assert rel(ds.to_numpy(np.float32, s0.shape), want) < 1e-5
+    # gate and up
+    ff = rows // 64 * 32
+    g, u = w[:ff], w[ff:2 * ff]
+    packed = np.stack([g.reshape(-1, 32, cols), u.reshape(-1, 32, cols)], 1).reshape(2 * ff, cols)
+    out = dev(np.zeros((tokens, ff), np.uint16))
+    run(out, m=_matrix(packed, 0)[0], n=2 * ff, epilogue=1, out_ld=ff, limit=1.5, alpha=1.702, bias=1.0)
+    gv, uv = np.minimum(y[:, :ff], 1.5), np.clip(y[:, ff:2 * ff], -1.5, 1.5)
+    want = gv * K.sigmoid(1.702 * gv) * (uv + 1.0)
+    assert rel((out.to_numpy(np.uint16, (tokens, ff)).astype(np.uint32) << 16).view(np.float32), want) < 1e-2
