@@ -107,13 +107,33 @@ int kx_route_launch(const float *logits, const float *bias, uint16_t *ids, float
 int kx_bucket_launch(const uint16_t *ids, int tokens, int experts, int topk, int *counts, int *offsets,
                      int *pairs, int4 *work, int *n_active, hipStream_t st, int4 *pair_work = nullptr);
 
-// kx_prefill.hip
-// outputs of the grouped GEMM: bf16; fp32 unrounded; fp32 holding the bf16-rounded value; bf16 residual add into out
+// outputs of the matrix-core products: bf16; fp32 unrounded; fp32 holding the bf16-rounded value; bf16 residual add into out
 enum { KX_GG_BF16 = 0, KX_GG_F32 = 1, KX_GG_F32_OF_BF16 = 2, KX_GG_RESID = 3 };
-int kx_grouped_gemm_launch(bool dual, bool i4, const void *w0, const uint16_t *s0, const void *w1, const uint16_t *s1,
-                           const uint16_t *x, void *out, int out_mode, const int4 *work, const int *pairs, int n_pairs,
-                           int n_slots, int N, int K, int x_div, size_t expert_w, size_t expert_s, int n_pairs_max,
-                           hipStream_t st, int cnt_lo = 0);
+// kx_prefill.hip: the pairs of each expert against its W4A16 matrix, out[pair] = W[expert] x[pair / x_div], or swiglu(W0 x, W1 x)
+int kx_grouped_gemm_launch(bool dual, const void *w0, const uint16_t *s0, const void *w1, const uint16_t *s1, const uint16_t *x, uint16_t *out,
+                           const int4 *work, const int *pairs, int n_slots, int N, int K, int x_div, size_t expert_w, size_t expert_s,
+                           int n_pairs_max, hipStream_t st, int cnt_lo = 0);
+// kx_dense_gemm.hip: out[t] = W x[t] for bf16 matrices and more than 32 tokens (any number is right), or swiglu(W0 x, W1 x).
+// With `work` the rows of x and out are pairs[i], each group {matrix, first, last, -} of them against a matrix of its own.
+struct KxDenseArgs {
+  const uint16_t *w0 = nullptr, *w1 = nullptr;  // [rows][cols]; w1: the second of a SwiGLU
+  const uint16_t *x = nullptr;                  // rows of x_stride
+  void *out = nullptr;                          // rows of out_stride, as mode says
+  int mode = KX_GG_BF16, tokens = 0, rows = 0, cols = 0, x_stride = 0, out_stride = 0;
+  const int4 *work = nullptr;
+  const int *pairs = nullptr;
+  int groups = 0;              // tokens is then the most a group has
+  size_t group_stride = 0;     // elements from one matrix to the next
+  // scratch of products that split their columns over workgroups; without it they do not.  One launch at a time uses it.
+  float *part = nullptr;
+  size_t part_floats = 0;
+  int *arrived = nullptr;      // [arrivals], zero between launches
+  int arrivals = 0;
+};
+inline int kx_pad32(int n) { return (n + 31) & ~31; }
+constexpr size_t KX_DENSE_PART_FLOATS = (size_t)256 * 128 * 128;  // what a device of 256 CUs makes use of
+constexpr int KX_DENSE_ARRIVALS = 256;
+int kx_dense_gemm_launch(const KxDenseArgs &a, hipStream_t st);
 // kx_i4mm.hip: the experts of the work list with cnt_lo .. cnt_hi pairs as W4A16 products on the matrix cores with the
 // weights streamed into registers, up to 32 tokens of an expert per pass (passes: grid depth; an expert's pairs beyond
 // 32 * passes are not computed).  out[pair][N] = W[expert] x[pair / x_div], or swiglu(W0 x, W1 x) with two matrices.

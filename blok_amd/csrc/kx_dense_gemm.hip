@@ -1,0 +1,135 @@
+// kx_dense_gemm.hip -- bf16 products of Kimi-K2 steps of more than 32 tokens: the dense projections, the shared expert, the router's
+// logits, W_UV per head, with the epilogues of the mat-vec kernels they stand for (matvec_bf16_k / matvec_bf16_f32_k with
+// add_k, silu_mul_k and the rounding of the logits, src/kimi_exec.cu:248-298, :718-734).
+//
+// The main loop is kx_gemm_tile.h's.  With two matrices (SwiGLU) a tile's rows are blocks of 32 gate rows and their 32 up rows in
+// turn, so that a wave holds both halves of a pair.  Before these tiles the products went through the W4A16 kernel's loop with 64
+// tokens a tile and every lane loading its own row of the matrix: 400 TFLOP/s where these reach 800 to 1050 (2048 tokens, gate
+// and up of 2 x 18432 x 7168 with SwiGLU 2.7 ms then).
+// fp32 sums over exact bf16 products: a tolerance path like every matrix-core path (max-rel 1e-2), not used where tokens
+// have to be identical.
+#include <atomic>
+#include "kx_common.h"
+#include "kx_dense.h"
+#include "kx_gemm_tile.h"
+#include "kx_math.h"
+
+namespace {
+
+using kxg::f32x16;
+
+typedef kxg::Tile<2, 2, 1, 2, 4> Short;  // 64 tokens x 128 rows: up to 64 tokens
+
+template <class TL, int MODE, bool DUAL, bool GROUP>
+__global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) dense_gemm_k(KxDenseArgs a, int parts) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  constexpr int COLS = DUAL ? TL::BN / 2 : TL::BN;  // results per token of a tile
+  int m0, m_end, n0, part = 0, tile = 0;
+  const uint16_t *w0 = a.w0, *w1 = a.w1;
+  if constexpr (GROUP) {
+    const int4 g = a.work[blockIdx.y];
+    if (g.x < 0) return;
+    m0 = g.y + blockIdx.z * TL::BM;
+    m_end = g.z;
+    if (m0 >= m_end) return;
+    n0 = blockIdx.x * COLS;
+    w0 += (size_t)g.x * a.group_stride;
+  } else {
+    const int tm = (a.tokens + TL::BM - 1) / TL::BM, tiles = (int)gridDim.x / parts, item = kxg::item_of(blockIdx.x, gridDim.x);
+    part = item / tiles;
+    tile = item - part * tiles;
+    m0 = tile % tm * TL::BM;
+    m_end = a.tokens;
+    n0 = tile / tm * COLS;
+  }
+  auto row_of = [&](int i) { return GROUP ? a.pairs[i] : i; };
+  const int nb = a.cols >> 6;
+  f32x16 acc[TL::MI][TL::NI];
+  TL::run(lds, (int)((long)nb * part / parts), (int)((long)nb * (part + 1) / parts), [&](int r) -> const uint16_t * {
+    if (r < TL::BM) return a.x + (size_t)row_of(min(m0 + r, m_end - 1)) * a.x_stride;
+    r -= TL::BM;
+    if constexpr (DUAL) return ((r >> 5 & 1) ? w1 : w0) + (size_t)min(n0 + (r >> 6) * 32 + (r & 31), a.rows - 1) * a.cols;
+    else return w0 + (size_t)min(n0 + r, a.rows - 1) * a.cols;
+  }, acc);
+  if (!GROUP && parts > 1 && !TL::gather(lds, acc, a.part + (size_t)tile * parts * TL::PART, a.arrived + tile, parts, part)) return;
+  // block (i, j) of the wave: results t(v) of this lane, in row at(v) of out
+  auto block = [&](int i, int j, auto &&put) {
+    const int c = TL::col(j), n = n0 + (DUAL ? (c >> 6) * 32 + (c & 31) : c);
+    if (n < a.rows) put([&](int v) { return m0 + TL::row(i, v) < m_end; }, [&](int v) { return (size_t)row_of(min(m0 + TL::row(i, v), m_end - 1)) * a.out_stride + n; });
+  };
+#pragma unroll
+  for (int i = 0; i < TL::MI; ++i) {
+#pragma unroll
+    for (int j = 0; j < TL::NI; j += DUAL ? 2 : 1) {
+      block(i, j, [&](auto &&in, auto &&at) {
+        if constexpr (DUAL) {
+#pragma unroll
+          for (int v = 0; v < 16; ++v)
+            if (in(v)) ((uint16_t *)a.out)[at(v)] = kx_bf16_rne(kx_swiglu(kx_bfround(acc[i][j][v]), kx_bfround(acc[i][j + 1][v])));
+        } else if constexpr (MODE == KX_GG_RESID) {  // x = bf(x + bf(y))  (add_k, :248-251); all are read before the first is written
+          uint16_t old[16];
+#pragma unroll
+          for (int v = 0; v < 16; ++v) old[v] = ((const uint16_t *)a.out)[at(v)];
+#pragma unroll
+          for (int v = 0; v < 16; ++v)
+            if (in(v)) ((uint16_t *)a.out)[at(v)] = kx_bf16_rne(kx_bf16_f32(old[v]) + kx_bfround(acc[i][j][v]));
+        } else {
+#pragma unroll
+          for (int v = 0; v < 16; ++v)
+            if (in(v)) {
+              if constexpr (MODE == KX_GG_BF16) ((uint16_t *)a.out)[at(v)] = kx_bf16_rne(acc[i][j][v]);
+              else ((float *)a.out)[at(v)] = MODE == KX_GG_F32 ? acc[i][j][v] : kx_bfround(acc[i][j][v]);
+            }
+        }
+      });
+    }
+  }
+}
+
+template <class TL, int MODE, bool DUAL, bool GROUP>
+int launch_as(const KxDenseArgs &a, int parts, hipStream_t st) {
+  static std::atomic<bool> attr{false};  // setting it twice from two threads is harmless
+  if (!attr) {
+    KX_HIP(hipFuncSetAttribute((const void *)dense_gemm_k<TL, MODE, DUAL, GROUP>, hipFuncAttributeMaxDynamicSharedMemorySize, TL::LDS));
+    attr = true;
+  }
+  const int tn = kx_cdiv(a.rows, DUAL ? TL::BN / 2 : TL::BN), tm = kx_cdiv(a.tokens, TL::BM);
+  const dim3 grid = GROUP ? dim3(tn, a.groups, tm) : dim3((unsigned)((long)tn * tm * parts));
+  hipLaunchKernelGGL((dense_gemm_k<TL, MODE, DUAL, GROUP>), grid, dim3(TL::THREADS), TL::LDS, st, a, parts);
+  KX_LAUNCH_CHECK();
+  return KX_OK;
+}
+template <class TL>
+int launch(const KxDenseArgs &a, int parts, hipStream_t st) {
+  if (a.w1) return launch_as<TL, KX_GG_BF16, true, false>(a, parts, st);
+  switch (a.mode) {
+    case KX_GG_BF16: return launch_as<TL, KX_GG_BF16, false, false>(a, parts, st);
+    case KX_GG_F32: return launch_as<TL, KX_GG_F32, false, false>(a, parts, st);
+    case KX_GG_RESID: return launch_as<TL, KX_GG_RESID, false, false>(a, parts, st);
+  }
+  return launch_as<TL, KX_GG_F32_OF_BF16, false, false>(a, parts, st);
+}
+
+}  // namespace
+
+int kx_dense_gemm_launch(const KxDenseArgs &a, hipStream_t st) {
+  KX_REQUIRE(a.w0 && a.x && a.out && a.tokens > 0 && a.rows > 0, "kx_dense_gemm: tokens=%d rows=%d", a.tokens, a.rows);
+  KX_REQUIRE(a.cols > 0 && a.cols % 128 == 0 && a.x_stride >= a.cols && a.x_stride % 8 == 0, "kx_dense_gemm: cols=%d must be a positive multiple of 128", a.cols);
+  KX_REQUIRE(a.mode >= KX_GG_BF16 && a.mode <= KX_GG_RESID && !((a.w1 || a.work) && a.mode != KX_GG_BF16) && !(a.w1 && a.work), "kx_dense_gemm: out_mode=%d", a.mode);
+  if (a.work) {
+    KX_REQUIRE(a.pairs && a.groups > 0 && kx_cdiv(a.tokens, kxg::Medium::BM) <= 65535, "kx_dense_gemm: %d groups", a.groups);
+    return launch_as<kxg::Medium, KX_GG_BF16, false, true>(a, 1, st);
+  }
+  const int cus = kx_device_cus() > 0 ? kx_device_cus() : 1, staged = a.w1 ? 2 * kx_pad32(a.rows) : a.rows, blocks = a.cols >> 6;
+  const size_t room = a.part && a.arrived ? a.part_floats : 0;
+  if (a.tokens <= Short::BM) {
+    const long tiles = kx_cdiv(staged, Short::BN);
+    long p = cus / tiles;
+    p = p > blocks / 16 ? blocks / 16 : p;
+    p = (size_t)p > room / Short::PART / tiles ? (long)(room / Short::PART / tiles) : p;
+    if (p < 2 || tiles > a.arrivals) p = 1;
+    return launch<Short>(a, (int)p, st);
+  }
+  const kxg::Choice c = kxg::choose(a.tokens, staged, blocks, room, a.arrivals, cus);
+  return c.large ? launch<kxg::Large>(a, 1, st) : launch<kxg::Medium>(a, c.parts, st);
+}

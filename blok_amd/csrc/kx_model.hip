@@ -83,6 +83,8 @@ struct KimiModel : kx_model {
   uint32_t back_tag = 0;
   int4 *head_work;                 // [heads], [step tokens * heads]: the groups of head_groups_k
   int *head_pairs;
+  float *split_part;               // partial sums of products that split their columns, and the counters of who has left his
+  int *split_arrived;
   uint32_t fusion = KX_FUSE_ALL;
   int mla_kernel = KX_MLA_AUTO;    // kx_model_set_attention_kernel
   float *route_logits = nullptr;   // routing record (kx_model_set_routing_record): [n_layers][max_batch][experts]
@@ -211,12 +213,15 @@ int layout(const kx_config *c, Plan &p, KimiModel *m) {
   auto *back_hand = KX_AT(uint32_t *, kx_back_hand_words((int)VD, c->hidden, c->experts) * 4);
   auto *head_work = KX_AT(int4 *, (size_t)c->heads * 16);
   auto *head_pairs = KX_AT(int *, BT * c->heads * 4);
+  auto *split_part = KX_AT(float *, KX_DENSE_PART_FLOATS * 4);
+  auto *split_arrived = KX_AT(int *, KX_DENSE_ARRIVALS * 4);
 #undef KX_AT
   p.scratch = p.total - p.weights - p.cache;
   if (m) {
     m->x = x; m->n = n; m->qkv = qkv; m->qa = qa; m->q = q; m->o_lat = o_lat; m->att = att; m->dmid = dmid;
     m->qabs = qabs; m->partial = partial; m->logits = logits; m->argmax_scratch = argmax_scratch; m->ids = ids; m->next = next; m->history = history;
     m->head_count = head_count; m->hand_err = hand_err; m->front_hand = front_hand; m->back_hand = back_hand; m->head_work = head_work; m->head_pairs = head_pairs;
+    m->split_part = split_part; m->split_arrived = split_arrived;
   }
   return KX_OK;
 }
@@ -314,9 +319,11 @@ int KimiModel::step(const uint32_t *d_ids, bool sample, int C) {
                                       g.cols, &done, st);
       if (rc2 || done) return rc2;
     }
-    KX_REQUIRE(g.x_stride == g.cols && g.out_stride == g.rows, "kx_model: the GEMM kernel takes dense activation and output rows");
-    return kx_grouped_gemm_launch(dual, false, g.w0, nullptr, dual ? g.w1 : nullptr, nullptr, g.x, g.out, mode, nullptr, nullptr,
-                                  g.tokens, 1, g.rows, g.cols, 1, 0, 0, g.tokens, st);
+    KxDenseArgs d;
+    d.w0 = g.w0; d.w1 = dual ? g.w1 : nullptr; d.x = g.x; d.x_stride = g.x_stride; d.out = g.out; d.out_stride = g.out_stride; d.mode = mode;
+    d.tokens = g.tokens; d.rows = g.rows; d.cols = g.cols;
+    d.part = m->split_part; d.part_floats = KX_DENSE_PART_FLOATS; d.arrived = m->split_arrived; d.arrivals = KX_DENSE_ARRIVALS;
+    return kx_dense_gemm_launch(d, st);
   };
   for (int l = 0; l < c.n_layers; ++l) {
     bool moe_head_done = false;  // the MoE layer's router + shared gate/up step rode in the attention block's last launch
@@ -380,9 +387,11 @@ int KimiModel::step(const uint32_t *d_ids, bool sample, int C) {
         hipLaunchKernelGGL(head_groups_k, dim3(kx_cdiv(B * c.heads, 256)), dim3(256), 0, st, B, c.heads, m->head_work, m->head_pairs);
         KX_LAUNCH_CHECK();
       }
-      KX_TRY(kx_grouped_gemm_launch(false, false, L.kvb + (size_t)c.qk_nope * c.kv_rank, nullptr, nullptr, nullptr, m->o_lat, m->att,
-                                    KX_GG_BF16, m->head_work, m->head_pairs, 0, c.heads, c.v_head, c.kv_rank, 1,
-                                    (size_t)(c.qk_nope + c.v_head) * c.kv_rank, 0, B, st));
+      KxDenseArgs d;
+      d.w0 = L.kvb + (size_t)c.qk_nope * c.kv_rank; d.x = m->o_lat; d.x_stride = c.kv_rank; d.out = m->att; d.out_stride = c.v_head;
+      d.tokens = B; d.rows = c.v_head; d.cols = c.kv_rank; d.work = m->head_work; d.pairs = m->head_pairs; d.groups = c.heads;
+      d.group_stride = (size_t)(c.qk_nope + c.v_head) * c.kv_rank;
+      KX_TRY(kx_dense_gemm_launch(d, st));
       KxGemvArgs go = {};
       go.w0 = L.o; go.x = m->att; go.x_stride = VD; go.out = m->x; go.out_stride = H; go.rows = H; go.cols = VD; go.tokens = B;
       KX_TRY(dense(KX_EPI_RESID, go));                                                                  // :826-827
@@ -528,6 +537,7 @@ static int model_new(const kx_config *cfg, const char *who, KimiModel **out) {
   if (!rc && m->moe_ws) kx_moe_workspace_set_err(m->moe_ws, m->hand_err);
   if (!rc && (hipMemsetAsync(m->head_count, 0, (size_t)cfg->heads * 4, m->st) != hipSuccess ||
               hipMemsetAsync(m->hand_err, 0, 4, m->st) != hipSuccess ||
+              hipMemsetAsync(m->split_arrived, 0, KX_DENSE_ARRIVALS * 4, m->st) != hipSuccess ||
               hipMemsetAsync(m->back_hand, 0, kx_back_hand_words(cfg->heads * cfg->v_head, cfg->hidden, cfg->experts) * 4, m->st) != hipSuccess ||
               hipMemsetAsync(m->front_hand, 0, kx_front_hand_words(cfg->q_rank, cfg->kv_rank + cfg->qk_rope, cfg->heads * (cfg->qk_nope + cfg->qk_rope)) * 4, m->st) != hipSuccess || hipStreamSynchronize(m->st) != hipSuccess))
     rc = KX_ERR_HIP;

@@ -41,6 +41,8 @@ struct kx_moe_workspace {
   uint16_t *eout;     // [T*topk, hidden]
   uint16_t *smid;     // [T, shared_inter]
   uint16_t *sy;       // [T, hidden] shared expert output (prefill path)
+  float *split_part[2] = {nullptr, nullptr};  // partial sums of dense products that split their columns: of this stream, of the side stream
+  int *split_arrived; // [2][KX_DENSE_ARRIVALS] zero between launches
   uint32_t *mid_hand; // [topk, moe_inter] tagged words: one token's mid values inside the resident routed launch
   uint32_t mid_tag = 0;
   int *err = nullptr; // the caller's flag for waits given up inside resident launches (not owned)
@@ -77,8 +79,10 @@ extern "C" int kx_moe_workspace_create(const kx_config *cfg, int32_t max_tokens,
       {(void **)&ws->work, E * 16}, {(void **)&ws->pair_work, T * K * 16}, {(void **)&ws->n_active, 64}, {(void **)&ws->tail_count, KX_TAIL_BLOCKS * 4},
       {(void **)&ws->mid, T * K * (size_t)cfg->moe_inter * 2}, {(void **)&ws->eout, T * K * (size_t)cfg->hidden * 2},
       {(void **)&ws->smid, T * (size_t)cfg->shared_inter * 2}, {(void **)&ws->sy, T * (size_t)cfg->hidden * 2},
-      {(void **)&ws->mid_hand, K * (size_t)cfg->moe_inter * 4}};
+      {(void **)&ws->mid_hand, K * (size_t)cfg->moe_inter * 4}, {(void **)&ws->split_arrived, 2 * KX_DENSE_ARRIVALS * 4},
+      {(void **)&ws->split_part[0], max_tokens > 32 ? KX_DENSE_PART_FLOATS * 4 : 0}, {(void **)&ws->split_part[1], max_tokens > 32 ? KX_DENSE_PART_FLOATS * 4 : 0}};
   for (auto &al : allocs) {
+    if (!al.bytes) continue;
     hipError_t e = hipMalloc(al.p, al.bytes);
     if (e != hipSuccess) {
       kx_set_error("kx_moe_workspace_create: hipMalloc(%zu): %s", al.bytes, hipGetErrorString(e));
@@ -93,6 +97,7 @@ extern "C" int kx_moe_workspace_create(const kx_config *cfg, int32_t max_tokens,
   if (e == hipSuccess) e = hipMemset(ws->pair_work, 0xff, T * K * 16);
   if (e == hipSuccess) e = hipMemset(ws->n_active, 0, 64);
   if (e == hipSuccess) e = hipMemset(ws->tail_count, 0, KX_TAIL_BLOCKS * 4);
+  if (e == hipSuccess) e = hipMemset(ws->split_arrived, 0, 2 * KX_DENSE_ARRIVALS * 4);
   if (e == hipSuccess) e = hipMemset(ws->mid_hand, 0, K * (size_t)cfg->moe_inter * 4);
   for (auto &ev : ws->ev)
     if (e == hipSuccess) e = hipEventCreate(&ev);
@@ -111,7 +116,8 @@ extern "C" int kx_moe_workspace_create(const kx_config *cfg, int32_t max_tokens,
 extern "C" int kx_moe_workspace_destroy(kx_moe_workspace *ws) {
   if (!ws) return KX_OK;
   void *ptrs[] = {ws->logits, ws->ids, ws->weights, ws->counts, ws->offsets, ws->pairs,
-                  ws->work, ws->pair_work, ws->n_active, ws->tail_count, ws->mid, ws->eout, ws->smid, ws->sy, ws->mid_hand};
+                  ws->work, ws->pair_work, ws->n_active, ws->tail_count, ws->mid, ws->eout, ws->smid, ws->sy, ws->mid_hand,
+                  ws->split_arrived, ws->split_part[0], ws->split_part[1]};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   for (auto &e : ws->ev)
@@ -332,8 +338,8 @@ static int moe_layer_body(const kx_config *c, const kx_moe_weights *w, kx_moe_wo
                              (const uint16_t *)w->d_up_scale, n, ws->mid, ws->work, ws->pairs, n_slots, I, H, K, (size_t)I * (H / 8),
                              (size_t)I * (H / 32), rmm_min, 1 << 30, kx_cdiv(tokens, 32), &mm_done, st))) return rc;
     if (!mm_done &&
-        (rc = kx_grouped_gemm_launch(true, true, w->d_gate_packed, (const uint16_t *)w->d_gate_scale, w->d_up_packed,
-                                     (const uint16_t *)w->d_up_scale, n, ws->mid, KX_GG_BF16, ws->work, ws->pairs, 0, n_slots, I, H,
+        (rc = kx_grouped_gemm_launch(true, w->d_gate_packed, (const uint16_t *)w->d_gate_scale, w->d_up_packed,
+                                     (const uint16_t *)w->d_up_scale, n, ws->mid, ws->work, ws->pairs, n_slots, I, H,
                                      K, (size_t)I * (H / 8), (size_t)I * (H / 32), tokens, st, rmm_min))) return rc;
     if ((rc = kx_i4_launch(true, (const uint32_t *)w->d_gate_packed, (const uint16_t *)w->d_gate_scale,
                            (const uint32_t *)w->d_up_packed, (const uint16_t *)w->d_up_scale, n, ws->mid, ws->work, ws->pairs, 0, I,
@@ -365,8 +371,8 @@ static int moe_layer_body(const kx_config *c, const kx_moe_weights *w, kx_moe_wo
                              ws->eout, ws->work, ws->pairs, n_slots, H, I, 1, (size_t)H * (I / 8), (size_t)H * (I / 32), rmm_min,
                              1 << 30, kx_cdiv(tokens, 32), &mm_done, st))) return rc;
     if (!mm_done &&
-        (rc = kx_grouped_gemm_launch(false, true, w->d_down_packed, (const uint16_t *)w->d_down_scale, nullptr, nullptr,
-                                     ws->mid, ws->eout, KX_GG_BF16, ws->work, ws->pairs, 0, n_slots, H, I, 1, (size_t)H * (I / 8),
+        (rc = kx_grouped_gemm_launch(false, w->d_down_packed, (const uint16_t *)w->d_down_scale, nullptr, nullptr,
+                                     ws->mid, ws->eout, ws->work, ws->pairs, n_slots, H, I, 1, (size_t)H * (I / 8),
                                      (size_t)H * (I / 32), tokens, st, rmm_min))) return rc;
     if ((rc = kx_i4_launch(false, (const uint32_t *)w->d_down_packed, (const uint16_t *)w->d_down_scale, nullptr, nullptr,
                            ws->mid, ws->eout, ws->work, ws->pairs, 0, H, I, 1, (size_t)H * (I / 8), (size_t)H * (I / 32),
@@ -437,10 +443,15 @@ extern "C" int kx_moe_prefill_layer(const kx_config *c, const kx_moe_weights *w,
   // while this one routes and runs the grouped GEMMs, and are joined before the combine.
   KX_HIP(hipEventRecord(ws->fork, st));
   KX_HIP(hipStreamWaitEvent(ws->side, ws->fork, 0));
-  if ((rc = kx_grouped_gemm_launch(true, false, w->d_shared_gate, nullptr, w->d_shared_up, nullptr, n, ws->smid, KX_GG_BF16,
-                                   nullptr, nullptr, tokens, 1, SI, H, 1, 0, 0, tokens, ws->side))) return rc;
-  if ((rc = kx_grouped_gemm_launch(false, false, w->d_shared_down, nullptr, nullptr, nullptr, ws->smid, ws->sy, KX_GG_BF16,
-                                   nullptr, nullptr, tokens, 1, H, SI, 1, 0, 0, tokens, ws->side))) return rc;
+  auto dense = [&](const void *w0, const void *w1, const uint16_t *x, void *out, int mode, int rows, int cols, int side) {
+    KxDenseArgs d;
+    d.w0 = (const uint16_t *)w0; d.w1 = (const uint16_t *)w1; d.x = x; d.x_stride = cols; d.out = out; d.out_stride = rows; d.mode = mode;
+    d.tokens = tokens; d.rows = rows; d.cols = cols;
+    d.part = ws->split_part[side]; d.part_floats = KX_DENSE_PART_FLOATS; d.arrived = ws->split_arrived + side * KX_DENSE_ARRIVALS; d.arrivals = KX_DENSE_ARRIVALS;
+    return kx_dense_gemm_launch(d, side ? ws->side : st);
+  };
+  if ((rc = dense(w->d_shared_gate, w->d_shared_up, n, ws->smid, KX_GG_BF16, SI, H, 1))) return rc;
+  if ((rc = dense(w->d_shared_down, nullptr, ws->smid, ws->sy, KX_GG_BF16, H, SI, 1))) return rc;
   KX_HIP(hipEventRecord(ws->join, ws->side));
   // router: fp32 logits (unrounded) as one GEMM of all tokens against the gate, top-k, bucketing.  Up to 32 tokens
   // the decode GEMV is used instead (its summation order is the decode path's).
@@ -450,8 +461,7 @@ extern "C" int kx_moe_prefill_layer(const kx_config *c, const kx_moe_weights *w,
     g.rows = E; g.cols = H; g.tokens = tokens;
     if ((rc = kx_gemv_launch(KX_EPI_F32, g, st))) return rc;
   } else {
-    if ((rc = kx_grouped_gemm_launch(false, false, w->d_router_gate, nullptr, nullptr, nullptr, n, ws->logits, KX_GG_F32, nullptr,
-                                     nullptr, tokens, 1, E, H, 1, 0, 0, tokens, st))) return rc;
+    if ((rc = dense(w->d_router_gate, nullptr, n, ws->logits, KX_GG_F32, E, H, 0))) return rc;
   }
   if ((rc = kx_router_topk_launch(ws->logits, (const float *)w->d_router_bias, ws->ids, ws->weights, tokens, E, K,
                                   c->routed_scale, st))) return rc;
@@ -459,11 +469,11 @@ extern "C" int kx_moe_prefill_layer(const kx_config *c, const kx_moe_weights *w,
     return rc;
   const int n_slots = (long)tokens * K < E ? tokens * K : E;
   // routed experts: gate/up + SwiGLU, then down
-  if ((rc = kx_grouped_gemm_launch(true, true, w->d_gate_packed, (const uint16_t *)w->d_gate_scale, w->d_up_packed,
-                                   (const uint16_t *)w->d_up_scale, n, ws->mid, KX_GG_BF16, ws->work, ws->pairs, 0, n_slots, I, H,
+  if ((rc = kx_grouped_gemm_launch(true, w->d_gate_packed, (const uint16_t *)w->d_gate_scale, w->d_up_packed,
+                                   (const uint16_t *)w->d_up_scale, n, ws->mid, ws->work, ws->pairs, n_slots, I, H,
                                    K, (size_t)I * (H / 8), (size_t)I * (H / 32), tokens, st))) return rc;
-  if ((rc = kx_grouped_gemm_launch(false, true, w->d_down_packed, (const uint16_t *)w->d_down_scale, nullptr, nullptr,
-                                   ws->mid, ws->eout, KX_GG_BF16, ws->work, ws->pairs, 0, n_slots, H, I, 1, (size_t)H * (I / 8),
+  if ((rc = kx_grouped_gemm_launch(false, w->d_down_packed, (const uint16_t *)w->d_down_scale, nullptr, nullptr,
+                                   ws->mid, ws->eout, ws->work, ws->pairs, n_slots, H, I, 1, (size_t)H * (I / 8),
                                    (size_t)H * (I / 32), tokens, st))) return rc;
   KX_HIP(hipStreamWaitEvent(st, ws->join, 0));  // the shared expert's output
   return kx_moe_combine_launch(ws->eout, ws->weights, ws->sy, (uint16_t *)d_x, tokens, H, K, flags, st);

@@ -1,0 +1,47 @@
+"""Prompts of the Kimi-K2 design in long steps on dense layers, against the token-by-token prefill of the same model: the
+tiles of the dense products (short, medium and large ones, columns in parts) and the attention of a step."""
+import numpy as np
+import pytest
+
+import oracle as O
+from blok_amd.lib import check, default_config
+from kxt import say
+from test_gpu_model import KxModel
+
+pytestmark = pytest.mark.gpu
+
+
+def _config(heads, batch, context):
+    cfg = default_config()
+    cfg.n_layers = cfg.first_dense = 2
+    cfg.hidden, cfg.heads, cfg.dense_inter, cfg.vocab = 1024, heads, 8192, 3000
+    cfg.max_batch, cfg.max_context, cfg.seed = batch, context, 11
+    return cfg
+
+
+@pytest.mark.parametrize("heads, batch, prompt, chunks", [
+    (16, 1, 1801, (1801, 1000, 129, 40)),   # large tiles for gate and up, medium ones in parts, short ones; a step that ends with one position
+    (64, 1, 700, (700, 333, 64)),
+    (20, 3, 301, (301, 100, 17)),           # several sequences, a number of heads that is no multiple of 16
+    (4, 33, 40, (40, 7, 1)),                # a batch that takes the step kernels of long prompts
+], ids=lambda v: str(v))
+def test_long_steps_against_token_by_token(kxlib, ox, heads, batch, prompt, chunks):
+    cfg = _config(heads, batch, prompt + 4)
+    ids = O.tokens_u32(batch * prompt, cfg.seed, 4, cfg.vocab).reshape(batch, prompt)
+    km = KxModel(kxlib, cfg)
+    check(kxlib.kx_model_set_exact(km.h, 15))
+    got = {}
+    for c in (0,) + chunks:
+        if c:
+            check(kxlib.kx_model_set_exact(km.h, 0))
+            check(kxlib.kx_model_set_prefill_chunk(km.h, c))
+        rc, out, _ = km.generate(ids, 1)
+        assert rc == 0, kxlib.kx_last_error()
+        got[c] = O.bf16_to_f32(np.stack([km.latent(1, b, prompt) for b in range(batch)])).astype(np.float64), km.logits(batch)
+    km.close()
+    rows, logits = got[0]
+    for c in chunks:
+        row_err = np.abs(got[c][0] - rows).max() / np.abs(rows).max()
+        log_err = max(O.max_rel(got[c][1][b], logits[b]) for b in range(batch))
+        say(f"heads={heads} batch={batch} prompt={prompt} chunk={c}: cache rows {row_err:.1e}, logits {log_err:.1e}")
+        assert row_err < 2e-2 and log_err < 3e-2, c
