@@ -108,7 +108,7 @@ int kx_bucket_launch(const uint16_t *ids, int tokens, int experts, int topk, int
                      int *pairs, int4 *work, int *n_active, hipStream_t st, int4 *pair_work = nullptr);
 
 // outputs of the matrix-core products: bf16; fp32 unrounded; fp32 holding the bf16-rounded value; bf16 residual add into out
-enum { KX_GG_BF16 = 0, KX_GG_F32 = 1, KX_GG_F32_OF_BF16 = 2, KX_GG_RESID = 3 };
+enum { KX_GG_BF16 = 0, KX_GG_F32 = 1, KX_GG_F32_OF_BF16 = 2, KX_GG_RESID = 3, KX_GG_KV = 4 /* kx_dense_gemm only */ };
 // kx_prefill.hip: the pairs of each expert against its W4A16 matrix, out[pair] = W[expert] x[pair / x_div], or swiglu(W0 x, W1 x)
 int kx_grouped_gemm_launch(bool dual, const void *w0, const uint16_t *s0, const void *w1, const uint16_t *s1, const uint16_t *x, uint16_t *out,
                            const int4 *work, const int *pairs, int n_slots, int N, int K, int x_div, size_t expert_w, size_t expert_s,
@@ -124,6 +124,11 @@ struct KxDenseArgs {
   const int *pairs = nullptr;
   int groups = 0;              // tokens is then the most a group has
   size_t group_stride = 0;     // elements from one matrix to the next
+  // KV: rows of the matrix are heads of k_dim key and v_dim value rows; the tokens are `seq` positions each of sequences whose
+  // rows of x begin seq_jump rows apart.  Key d of (sequence b, head h, position t) goes to
+  // out[((b heads + h) cap + t) k_ld + d], values to out_v with v_ld.
+  int seq = 0, seq_jump = 0, heads = 0, k_dim = 0, v_dim = 0, cap = 0, k_ld = 0, v_ld = 0;
+  uint16_t *out_v = nullptr;
   // scratch of products that split their columns over workgroups; without it they do not.  One launch at a time uses it.
   float *part = nullptr;
   size_t part_floats = 0;

@@ -16,9 +16,9 @@
 
 namespace {
 
-using kxg::f32x16;
+using kxtile::f32x16;
 
-typedef kxg::Tile<2, 2, 1, 2, 4> Short;  // 64 tokens x 128 rows: up to 64 tokens
+typedef kxtile::Tile<2, 2, 1, 2, 4> Short;  // 64 tokens x 128 rows: up to 64 tokens
 
 template <class TL, int MODE, bool DUAL, bool GROUP>
 __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) dense_gemm_k(KxDenseArgs a, int parts) {
@@ -35,14 +35,17 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) dense_gemm_k(
     n0 = blockIdx.x * COLS;
     w0 += (size_t)g.x * a.group_stride;
   } else {
-    const int tm = (a.tokens + TL::BM - 1) / TL::BM, tiles = (int)gridDim.x / parts, item = kxg::item_of(blockIdx.x, gridDim.x);
+    const int tm = (a.tokens + TL::BM - 1) / TL::BM, tiles = (int)gridDim.x / parts, item = kxtile::item_of(blockIdx.x, gridDim.x);
     part = item / tiles;
     tile = item - part * tiles;
     m0 = tile % tm * TL::BM;
     m_end = a.tokens;
     n0 = tile / tm * COLS;
   }
-  auto row_of = [&](int i) { return GROUP ? a.pairs[i] : i; };
+  auto row_of = [&](int i) {
+    if constexpr (MODE == KX_GG_KV) return i / a.seq * a.seq_jump + i % a.seq;
+    else return GROUP ? a.pairs[i] : i;
+  };
   const int nb = a.cols >> 6;
   f32x16 acc[TL::MI][TL::NI];
   TL::run(lds, (int)((long)nb * part / parts), (int)((long)nb * (part + 1) / parts), [&](int r) -> const uint16_t * {
@@ -62,7 +65,18 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) dense_gemm_k(
 #pragma unroll
     for (int j = 0; j < TL::NI; j += DUAL ? 2 : 1) {
       block(i, j, [&](auto &&in, auto &&at) {
-        if constexpr (DUAL) {
+        if constexpr (MODE == KX_GG_KV) {
+          const int n = n0 + TL::col(j), per = a.k_dim + a.v_dim, hd = n / per, d = n - hd * per;
+          const bool key = d < a.k_dim;
+          uint16_t *to = key ? (uint16_t *)a.out + d : a.out_v + (d - a.k_dim);
+          const int ld = key ? a.k_ld : a.v_ld;
+#pragma unroll
+          for (int v = 0; v < 16; ++v)
+            if (in(v)) {
+              const int t = m0 + TL::row(i, v), b = t / a.seq;
+              to[((size_t)(b * a.heads + hd) * a.cap + t - b * a.seq) * ld] = kx_bf16_rne(acc[i][j][v]);
+            }
+        } else if constexpr (DUAL) {
 #pragma unroll
           for (int v = 0; v < 16; ++v)
             if (in(v)) ((uint16_t *)a.out)[at(v)] = kx_bf16_rne(kx_swiglu(kx_bfround(acc[i][j][v]), kx_bfround(acc[i][j + 1][v])));
@@ -106,6 +120,7 @@ int launch(const KxDenseArgs &a, int parts, hipStream_t st) {
     case KX_GG_BF16: return launch_as<TL, KX_GG_BF16, false, false>(a, parts, st);
     case KX_GG_F32: return launch_as<TL, KX_GG_F32, false, false>(a, parts, st);
     case KX_GG_RESID: return launch_as<TL, KX_GG_RESID, false, false>(a, parts, st);
+    case KX_GG_KV: return launch_as<TL, KX_GG_KV, false, false>(a, parts, st);
   }
   return launch_as<TL, KX_GG_F32_OF_BF16, false, false>(a, parts, st);
 }
@@ -115,10 +130,13 @@ int launch(const KxDenseArgs &a, int parts, hipStream_t st) {
 int kx_dense_gemm_launch(const KxDenseArgs &a, hipStream_t st) {
   KX_REQUIRE(a.w0 && a.x && a.out && a.tokens > 0 && a.rows > 0, "kx_dense_gemm: tokens=%d rows=%d", a.tokens, a.rows);
   KX_REQUIRE(a.cols > 0 && a.cols % 128 == 0 && a.x_stride >= a.cols && a.x_stride % 8 == 0, "kx_dense_gemm: cols=%d must be a positive multiple of 128", a.cols);
-  KX_REQUIRE(a.mode >= KX_GG_BF16 && a.mode <= KX_GG_RESID && !((a.w1 || a.work) && a.mode != KX_GG_BF16) && !(a.w1 && a.work), "kx_dense_gemm: out_mode=%d", a.mode);
+  KX_REQUIRE(a.mode >= KX_GG_BF16 && a.mode <= KX_GG_KV && !((a.w1 || a.work) && a.mode != KX_GG_BF16) && !(a.w1 && a.work), "kx_dense_gemm: out_mode=%d", a.mode);
+  KX_REQUIRE(a.mode != KX_GG_KV || (a.seq > 0 && a.tokens % a.seq == 0 && a.heads > 0 && a.rows == a.heads * (a.k_dim + a.v_dim) && a.cap >= a.seq && a.k_ld >= a.k_dim &&
+                                    a.v_ld >= a.v_dim && a.out_v),
+             "kx_dense_gemm: %d rows for %d heads, %d tokens", a.rows, a.heads, a.tokens);
   if (a.work) {
-    KX_REQUIRE(a.pairs && a.groups > 0 && kx_cdiv(a.tokens, kxg::Medium::BM) <= 65535, "kx_dense_gemm: %d groups", a.groups);
-    return launch_as<kxg::Medium, KX_GG_BF16, false, true>(a, 1, st);
+    KX_REQUIRE(a.pairs && a.groups > 0 && kx_cdiv(a.tokens, kxtile::Medium::BM) <= 65535, "kx_dense_gemm: %d groups", a.groups);
+    return launch_as<kxtile::Medium, KX_GG_BF16, false, true>(a, 1, st);
   }
   const int cus = kx_device_cus() > 0 ? kx_device_cus() : 1, staged = a.w1 ? 2 * kx_pad32(a.rows) : a.rows, blocks = a.cols >> 6;
   const size_t room = a.part && a.arrived ? a.part_floats : 0;
@@ -130,6 +148,6 @@ int kx_dense_gemm_launch(const KxDenseArgs &a, hipStream_t st) {
     if (p < 2 || tiles > a.arrivals) p = 1;
     return launch<Short>(a, (int)p, st);
   }
-  const kxg::Choice c = kxg::choose(a.tokens, staged, blocks, room, a.arrivals, cus);
-  return c.large ? launch<kxg::Large>(a, 1, st) : launch<kxg::Medium>(a, c.parts, st);
+  const kxtile::Choice c = kxtile::choose(a.tokens, staged, blocks, room, a.arrivals, cus);
+  return c.large ? launch<kxtile::Large>(a, 1, st) : launch<kxtile::Medium>(a, c.parts, st);
 }

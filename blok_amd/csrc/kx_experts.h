@@ -13,7 +13,7 @@ struct KxExpertSlots {
   int *n_tiles = nullptr;
 };
 // slots per tile of a step (those of the GEMM that will read them), and the most tiles its pairs make.  bf16: 32 where an expert
-// has fewer than 8 pairs on average (the kernel for few tokens, 64 rows a workgroup: 50 and 24 us where the one with tiles of
+// has fewer than 8 pairs on average (the kernel for few tokens, 64 rows a workgroup: 71 and 37 us where the one with tiles of
 // 64 takes 75 and 38 us for 64 pairs on 64 experts of 3 x 2048 x 1024), 128 from 96 on
 constexpr int KX_EXPERT_TILE_MIN = 32;
 inline int kx_expert_tile(bool f32, int tokens, int top, int experts) {

@@ -24,7 +24,7 @@
 #include "kx_arrive.h"
 #include "kx_lds_copy.h"
 
-namespace kxg {
+namespace kxtile {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -207,4 +207,4 @@ inline Choice choose(int tokens, int rows, int blocks, size_t part_floats, int a
   return {l < m, 1};
 }
 
-}  // namespace kxg
+}  // namespace kxtile

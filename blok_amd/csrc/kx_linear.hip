@@ -26,8 +26,8 @@
 namespace {
 
 using kxr::Elem;
-using kxg::bf16x8;
-using kxg::f32x16;
+using kxtile::bf16x8;
+using kxtile::f32x16;
 
 // ---- epilogues, one output element (or pair) at a time ----
 template <class T>
@@ -289,7 +289,7 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) lin_gemm_k(Kx
     if (!tile_of<true>(a, e, TL::BM, tl)) return;
     n0 = blockIdx.x * TL::BN;
   } else {
-    const int tm = (a.tokens + TL::BM - 1) / TL::BM, tiles = (int)gridDim.x / parts, item = kxg::item_of(blockIdx.x, gridDim.x);
+    const int tm = (a.tokens + TL::BM - 1) / TL::BM, tiles = (int)gridDim.x / parts, item = kxtile::item_of(blockIdx.x, gridDim.x);
     part = item / tiles;
     tile = item - part * tiles;
     n0 = tile / tm * TL::BN;
@@ -609,7 +609,7 @@ int narrow_launch(const KxLinArgs &a, const KxExpertArgs &e, const uint16_t *x, 
   return KX_OK;
 }
 
-typedef kxg::Tile<2, 2, 1, 2, 4> SmallSlots;  // 64 slots of an expert
+typedef kxtile::Tile<2, 2, 1, 2, 4> SmallSlots;  // 64 slots of an expert
 template <class TL, int EPI, bool GROUP>
 int tile_launch(const KxLinArgs &a, const KxExpertArgs &e, const uint16_t *x, int x_ld, int parts, hipStream_t st) {
   static std::atomic<bool> attr{false};
@@ -635,11 +635,11 @@ int gemm_launch(const KxLinArgs &a, const KxExpertArgs &e, const T *x, int x_ld,
     KX_LAUNCH_CHECK();
     return KX_OK;
   } else if constexpr (GROUP) {
-    return e.tile_slots > 64 ? tile_launch<kxg::Medium, EPI, true>(a, e, x, x_ld, 1, st) : tile_launch<SmallSlots, EPI, true>(a, e, x, x_ld, 1, st);
+    return e.tile_slots > 64 ? tile_launch<kxtile::Medium, EPI, true>(a, e, x, x_ld, 1, st) : tile_launch<SmallSlots, EPI, true>(a, e, x, x_ld, 1, st);
   } else {
-    const kxg::Choice c = kxg::choose(a.tokens, a.m.rows, a.m.ld >> 6, a.part ? a.part_floats : 0, a.arrived ? a.arrivals : 0, std::max(1, kx_device_cus()));
-    if (c.large && a.n_var == 1) return tile_launch<kxg::Large, EPI, false>(a, e, x, x_ld, 1, st);  // variants begin at multiples of 128 rows
-    return tile_launch<kxg::Medium, EPI, false>(a, e, x, x_ld, c.parts, st);
+    const kxtile::Choice c = kxtile::choose(a.tokens, a.m.rows, a.m.ld >> 6, a.part ? a.part_floats : 0, a.arrived ? a.arrivals : 0, std::max(1, kx_device_cus()));
+    if (c.large && a.n_var == 1) return tile_launch<kxtile::Large, EPI, false>(a, e, x, x_ld, 1, st);  // variants begin at multiples of 128 rows
+    return tile_launch<kxtile::Medium, EPI, false>(a, e, x, x_ld, c.parts, st);
   }
 }
 

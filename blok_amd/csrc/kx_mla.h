@@ -32,3 +32,22 @@ int kx_mla_partials_launch(const kx_config *c, const uint16_t *cache, size_t seq
 int kx_mla_combine_launch(const KxMlaPartials &p, uint16_t *o_lat, int batch, int heads, hipStream_t st);
 int kx_mla_attend_launch(const kx_config *c, const uint16_t *cache, size_t seq_stride, const float *qabs, float *partial,
                          uint16_t *o_lat, int batch, int seq, hipStream_t st, int seqs = 0, int kernel = KX_MLA_AUTO);
+
+// kx_mla_prompt.hip: attention of a prefill step of `positions` positions of `seqs` sequences, from the q_b and kv_a outputs to the
+// heads' values; also writes the step's cache rows.
+struct KxDenseArgs;
+struct KxMlaPromptArgs {
+  uint16_t *q;                    // [positions * seqs][heads][nope + rope]; the rope part is rotated in place
+  const uint16_t *kva, *w_kv_ln, *rope_row, *kvb;
+  uint16_t *cache, *out;          // out [positions * seqs][heads * v_head]
+  void *expand;                   // room for expanded keys and values; what is in it is finite
+  size_t expand_bytes, seq_stride;
+  int heads, nope, rope, kv_rank, kva_stride, seqs, positions, pos;
+  float eps;
+};
+constexpr size_t KX_MLA_EXPAND_BYTES = (size_t)1 << 30;
+size_t kx_mla_prompt_bytes(const kx_config *c);
+// whether a step of `positions` positions per sequence takes this form
+bool kx_mla_prompt_fits(const kx_config *c, int positions, size_t expand_bytes);
+// split: scratch of the expanding product (KxDenseArgs::part and what follows)
+int kx_mla_prompt_launch(const kx_config *c, const KxMlaPromptArgs &a, const KxDenseArgs &split, hipStream_t st);

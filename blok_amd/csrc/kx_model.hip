@@ -85,6 +85,8 @@ struct KimiModel : kx_model {
   int *head_pairs;
   float *split_part;               // partial sums of products that split their columns, and the counters of who has left his
   int *split_arrived;
+  void *expand = nullptr;          // keys and values of a prompt's context, expanded (kx_mla_prompt.hip); where there was memory for it
+  size_t expand_bytes = 0;
   uint32_t fusion = KX_FUSE_ALL;
   int mla_kernel = KX_MLA_AUTO;    // kx_model_set_attention_kernel
   float *route_logits = nullptr;   // routing record (kx_model_set_routing_record): [n_layers][max_batch][experts]
@@ -309,6 +311,10 @@ int KimiModel::step(const uint32_t *d_ids, bool sample, int C) {
   // GEMV is bound by its fma count there.  Same values, another summation order (the bf16 rounding points stay).
   const bool mm = B >= 5 && !(m->exact & KX_EXACT_PROJECTIONS);
   const int mla_kernel = (m->exact & KX_EXACT_ATTENTION) ? KX_MLA_VALU : m->mla_kernel;
+  // a step of several positions attends to expanded keys and values where it is long enough
+  const bool expand = C > 1 && B > 32 && mla_kernel == KX_MLA_AUTO && m->expand && kx_mla_prompt_fits(&c, C, m->expand_bytes);
+  KxDenseArgs split;
+  split.part = m->split_part; split.part_floats = KX_DENSE_PART_FLOATS; split.arrived = m->split_arrived; split.arrivals = KX_DENSE_ARRIVALS;
   auto dense = [&](int epi, const KxGemvArgs &g) -> int {
     if (!mm) return kx_gemv_launch(epi, g, st);
     const bool dual = epi == KX_EPI_SWIGLU;
@@ -319,10 +325,9 @@ int KimiModel::step(const uint32_t *d_ids, bool sample, int C) {
                                       g.cols, &done, st);
       if (rc2 || done) return rc2;
     }
-    KxDenseArgs d;
+    KxDenseArgs d = split;
     d.w0 = g.w0; d.w1 = dual ? g.w1 : nullptr; d.x = g.x; d.x_stride = g.x_stride; d.out = g.out; d.out_stride = g.out_stride; d.mode = mode;
     d.tokens = g.tokens; d.rows = g.rows; d.cols = g.cols;
-    d.part = m->split_part; d.part_floats = KX_DENSE_PART_FLOATS; d.arrived = m->split_arrived; d.arrivals = KX_DENSE_ARRIVALS;
     return kx_dense_gemm_launch(d, st);
   };
   for (int l = 0; l < c.n_layers; ++l) {
@@ -357,7 +362,7 @@ int KimiModel::step(const uint32_t *d_ids, bool sample, int C) {
       if (fuse && (m->fusion & KX_FUSE_ABSORB)) KX_TRY(kx_gemv_absorb_launch(gb, qa, &absorbed, st));     // :815
       if (!absorbed) {
         KX_TRY(dense(KX_EPI_BF16, gb));                                                                   // :815
-        KX_TRY(kx_q_absorb_launch(m->q, L.kvb, rope_row, m->qabs, B, c.heads, c.qk_nope, c.qk_rope, c.v_head, c.kv_rank,
+        if (!expand) KX_TRY(kx_q_absorb_launch(m->q, L.kvb, rope_row, m->qabs, B, c.heads, c.qk_nope, c.qk_rope, c.v_head, c.kv_rank,
                                   m->qkv + c.q_rank, QKV, L.kv_ln, L.cache, seq_stride, pos, c.rms_eps, st, C > 1 ? NB : 0));
       }
     }
@@ -373,6 +378,13 @@ int KimiModel::step(const uint32_t *d_ids, bool sample, int C) {
       } else {               // long context, few sequences: more spans than the GEMV's merge takes
         KX_TRY(kx_mla_combine_launch(mp, m->o_lat, B, c.heads, st));
       }
+    } else if (expand) {
+      KxMlaPromptArgs pa = {};
+      pa.q = m->q; pa.kva = m->qkv + c.q_rank; pa.w_kv_ln = L.kv_ln; pa.rope_row = rope_row; pa.kvb = L.kvb; pa.cache = L.cache; pa.out = m->att;
+      pa.expand = m->expand; pa.expand_bytes = m->expand_bytes; pa.seq_stride = seq_stride;
+      pa.heads = c.heads; pa.nope = c.qk_nope; pa.rope = c.qk_rope; pa.kv_rank = c.kv_rank; pa.kva_stride = QKV; pa.seqs = NB; pa.positions = C; pa.pos = pos;
+      pa.eps = c.rms_eps;
+      KX_TRY(kx_mla_prompt_launch(&c, pa, split, st));
     } else {
       // at most ATT_ENTRIES entries a launch: whole positions, in order
       const int cs = NB >= ATT_ENTRIES ? 1 : ATT_ENTRIES / NB;
@@ -383,15 +395,17 @@ int KimiModel::step(const uint32_t *d_ids, bool sample, int C) {
       }
     }
     if (C > 1 && B > 32 && c.kv_rank % 128 == 0) {  // a long prefill step: one grouped GEMM over the heads
-      if (l == 0) {
+      if (l == 0 && !expand) {
         hipLaunchKernelGGL(head_groups_k, dim3(kx_cdiv(B * c.heads, 256)), dim3(256), 0, st, B, c.heads, m->head_work, m->head_pairs);
         KX_LAUNCH_CHECK();
       }
-      KxDenseArgs d;
-      d.w0 = L.kvb + (size_t)c.qk_nope * c.kv_rank; d.x = m->o_lat; d.x_stride = c.kv_rank; d.out = m->att; d.out_stride = c.v_head;
-      d.tokens = B; d.rows = c.v_head; d.cols = c.kv_rank; d.work = m->head_work; d.pairs = m->head_pairs; d.groups = c.heads;
-      d.group_stride = (size_t)(c.qk_nope + c.v_head) * c.kv_rank;
-      KX_TRY(kx_dense_gemm_launch(d, st));
+      if (!expand) {
+        KxDenseArgs d;
+        d.w0 = L.kvb + (size_t)c.qk_nope * c.kv_rank; d.x = m->o_lat; d.x_stride = c.kv_rank; d.out = m->att; d.out_stride = c.v_head;
+        d.tokens = B; d.rows = c.v_head; d.cols = c.kv_rank; d.work = m->head_work; d.pairs = m->head_pairs; d.groups = c.heads;
+        d.group_stride = (size_t)(c.qk_nope + c.v_head) * c.kv_rank;
+        KX_TRY(kx_dense_gemm_launch(d, st));
+      }
       KxGemvArgs go = {};
       go.w0 = L.o; go.x = m->att; go.x_stride = VD; go.out = m->x; go.out_stride = H; go.rows = H; go.cols = VD; go.tokens = B;
       KX_TRY(dense(KX_EPI_RESID, go));                                                                  // :826-827
@@ -491,6 +505,7 @@ int KimiModel::row_logits(const int *rows, int n_rows, float *d_out) {
 
 KimiModel::~KimiModel() {
   if (moe_ws) kx_moe_workspace_destroy(moe_ws);
+  if (expand) (void)hipFree(expand);
   if (route_logits) (void)hipFree(route_logits);
   if (route_distinct) (void)hipFree(route_distinct);
   if (route_history) (void)hipFree(route_history);
@@ -545,6 +560,17 @@ static int model_new(const kx_config *cfg, const char *who, KimiModel **out) {
     if (rc == KX_ERR_HIP && !kx_last_error()[0]) kx_set_error("%s: HIP resource creation failed", who);
     kx_model_destroy(m);
     return rc;
+  }
+  // Room for a prompt's expanded keys and values, if there is memory to spare; without it prompts attend as decode steps do.
+  const size_t want = kx_mla_prompt_bytes(cfg);
+  if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && want + ((size_t)2 << 30) <= free_b) {
+    if (hipMalloc(&m->expand, want) != hipSuccess) {
+      (void)hipGetLastError();
+      m->expand = nullptr;
+    } else {
+      m->expand_bytes = want;
+      KX_HIP(hipMemsetAsync(m->expand, 0, want, m->st));  // what lies behind a context's last position is multiplied by zeros
+    }
   }
   *out = m;
   return KX_OK;

@@ -294,7 +294,7 @@ __global__ void __launch_bounds__(256) win_flash_k(KxWindowArgs a) {
   const int h = blockIdx.y, b = blockIdx.z, g = h / (s.heads / s.kv_heads);
   const int i0 = blockIdx.x * FQ, i = i0 + wave * 32 + lq;  // this lane's position of the step
   const bool live = i < a.positions;
-  const int p = a.pos + min(i, a.positions - 1), tok = min(i, a.positions - 1) * a.batch + b;
+  const int p = a.pos + min(i, a.positions - 1), tok = min(i, a.positions - 1) * (a.tok_batch ? a.tok_batch : a.batch) + b;
   const int p_first = a.pos + i0, p_last = a.pos + min(i0 + FQ, a.positions) - 1;
   const int nb = seen_blocks(p, s.size, s.pool), lo = window_lo(p, s.size);
   const size_t head = (size_t)b * s.kv_heads + g;
@@ -302,7 +302,7 @@ __global__ void __launch_bounds__(256) win_flash_k(KxWindowArgs a) {
   const uint16_t *pkc = (const uint16_t *)c.pk + head * c.blocks * c.dp, *pvc = (const uint16_t *)c.pv + head * c.blocks * c.vp;
   bf16x8 q[ND * 2];
   {
-    const uint16_t *qr = (const uint16_t *)a.q + ((size_t)tok * s.heads + h) * c.dp;
+    const uint16_t *qr = (const uint16_t *)a.q + (size_t)tok * (a.q_ld ? a.q_ld : (size_t)s.heads * c.dp) + (size_t)h * c.dp;
 #pragma unroll
     for (int kk = 0; kk < ND * 2; ++kk) q[kk] = kk * 16 < c.dp ? *(const bf16x8 *)(qr + kk * 16 + hh * 8) : bf16x8{};
   }
@@ -540,6 +540,7 @@ int attend(const KxWindowArgs &a, hipStream_t st) {
     return nd == 1 ? flash_nv<1>(a, nv, st) : nd == 2 ? flash_nv<2>(a, nv, st) : nd <= 4 ? flash_nv<4>(a, nv, st)
          : nd <= 6 ? flash_nv<6>(a, nv, st) : flash_nv<8>(a, nv, st);
   }
+  KX_REQUIRE(!a.tok_batch && !a.q_ld, "window attention: a part of a step with keys of %d and values of %d", a.s.dim, a.s.vdim);
   return attend_parts<T>(a, false, st);
 }
 

@@ -45,3 +45,25 @@ def test_long_steps_against_token_by_token(kxlib, ox, heads, batch, prompt, chun
         log_err = max(O.max_rel(got[c][1][b], logits[b]) for b in range(batch))
         say(f"heads={heads} batch={batch} prompt={prompt} chunk={c}: cache rows {row_err:.1e}, logits {log_err:.1e}")
         assert row_err < 2e-2 and log_err < 3e-2, c
+
+
+@pytest.mark.parametrize("heads, batch, prompt, kernel", [(64, 1, 27000, 2), (60, 40, 750, 1)], ids=["heads in groups", "sequences in groups"])
+def test_expanded_keys_that_do_not_fit_at_once(kxlib, ox, heads, batch, prompt, kernel):
+    """A context whose expanded keys and values take more than their room: fewer heads, or fewer sequences, at a time.
+    Against the decode form of the attention in the same steps."""
+    cfg = _config(heads, batch, prompt + 1)
+    ids = O.tokens_u32(batch * prompt, cfg.seed, 4, cfg.vocab).reshape(batch, prompt)
+    assert batch * heads * ((prompt + 63) // 64 * 64) * 640 > 1 << 30
+    km = KxModel(kxlib, cfg)
+    check(kxlib.kx_model_set_prefill_chunk(km.h, 2048))
+    got = []
+    for k in (kernel, 0):
+        check(kxlib.kx_model_set_attention_kernel(km.h, k))
+        rc, _, _ = km.generate(ids, 1)
+        assert rc == 0, kxlib.kx_last_error()
+        got.append((O.bf16_to_f32(np.stack([km.latent(1, b, prompt) for b in range(batch)])).astype(np.float64), km.logits(batch)))
+    km.close()
+    row_err = np.abs(got[1][0] - got[0][0]).max() / np.abs(got[0][0]).max()
+    log_err = max(O.max_rel(got[1][1][b], got[0][1][b]) for b in range(batch))
+    say(f"heads={heads} batch={batch} prompt={prompt}: cache rows {row_err:.1e}, logits {log_err:.1e}")
+    assert row_err < 2e-2 and log_err < 3e-2
