@@ -18,7 +18,7 @@ namespace {
 
 using kxtile::f32x16;
 
-typedef kxtile::Tile<2, 2, 1, 2, 4> Short;  // 64 tokens x 128 rows: up to 64 tokens
+typedef kxtile::Tile<uint16_t, 2, 2, 1, 2, 4> Short;  // 64 tokens x 128 rows: up to 64 tokens
 
 template <class TL, int MODE, bool DUAL, bool GROUP>
 __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) dense_gemm_k(KxDenseArgs a, int parts) {

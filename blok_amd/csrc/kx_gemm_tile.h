@@ -1,10 +1,10 @@
-// kx_gemm_tile.h -- one tile of a bf16 matrix product on the matrix cores, y[t][r] = sum_k x[t][k] w[r][k]: the main loop that
+// kx_gemm_tile.h -- one tile of a bf16 or f32 matrix product on the matrix cores, y[t][r] = sum_k x[t][k] w[r][k]: the main loop that
 // the products of the hybrid decoder (kx_linear.hip) and the dense ones of Kimi-K2 (kx_dense_gemm.hip) share, and the
 // hand-over between workgroups that split a tile's columns.  No counterpart in the reference, whose products are mat-vecs
 // (src/kimi_exec.cu:272-298).
 //
 // A workgroup of WM x WN waves owns BM tokens and BN rows; wave (wm, wn) holds MI x NI blocks of 32 x 32
-// (v_mfma_f32_32x32x16_bf16).  Both operands are staged through LDS in blocks of 64 columns by global -> LDS copies, 128-byte rows
+// (v_mfma_f32_32x32x16_bf16; for float v_mfma_f32_32x32x2_f32, products and sums in 32 bits).  Both operands are staged through LDS in blocks of 64 (32) columns by global -> LDS copies, 128-byte rows
 // (whole lines: with 64-byte rows the copies cost as much a row and everything 10 to 15 % more) with the 16-byte pieces xor-ed by
 // the row, so that row-per-lane reads are free of bank conflicts.
 // The LDS is a ring of SLOTS half blocks -- tokens, matrix rows, tokens, ... --, two of the block that is multiplied and the others
@@ -27,10 +27,28 @@
 namespace kxtile {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-template <int WM_, int WN_, int MI_, int NI_, int SLOTS_>
+// 16 bytes of a row, as a lane holds them: lanes 0-31 have piece 2 q of their row, lanes 32-63 piece 2 q + 1; both operands
+// alike, so that it does not matter which of the columns meet in one instruction
+template <class T> struct Piece;
+template <> struct Piece<uint16_t> {
+  typedef bf16x8 Type;
+  static __device__ __forceinline__ f32x16 multiply(Type x, Type w, f32x16 acc) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, w, acc, 0, 0, 0); }
+};
+template <> struct Piece<float> {
+  typedef f32x4 Type;
+  static __device__ __forceinline__ f32x16 multiply(Type x, Type w, f32x16 acc) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], w[e], acc, 0, 0, 0);
+    return acc;
+  }
+};
+
+template <class T, int WM_, int WN_, int MI_, int NI_, int SLOTS_>
 struct Tile {
+  static constexpr int COLS = 128 / sizeof(T);  // columns of a block
   static constexpr int SLOTS = SLOTS_, WM = WM_, WN = WN_, MI = MI_, NI = NI_, WAVES = WM * WN, THREADS = WAVES * 64;
   static constexpr int BM = WM * MI * 32, BN = WN * NI * 32, SLOT = (BM > BN ? BM : BN) * 128, LDS = SLOTS * SLOT;
   static constexpr int WAVES_PER_SIMD = MI * NI >= 16 ? 1 : 2;
@@ -39,27 +57,27 @@ struct Tile {
   static_assert(SLOTS == 4 || SLOTS == 5, "two blocks, and half of a third");
   static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "the copies of a block are spread evenly over the waves");
 
-  // Columns 64 kb0 .. 64 kb1 - 1 (kb0 < kb1).  row(r): where staged row r begins, tokens 0 .. BM - 1, then BN rows of the
+  // Columns COLS kb0 .. COLS kb1 - 1 (kb0 < kb1).  row(r): where staged row r begins, tokens 0 .. BM - 1, then BN rows of the
   // matrix; every row has to be readable, what a row past the end holds only reaches sums that are not used.
   template <class Row>
   static __device__ __forceinline__ void run(uint8_t *lds, int kb0, int kb1, Row row, f32x16 (&acc)[MI][NI]) {
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave / WN, wn = wave % WN, lr = lane & 31, h = lane >> 5, sub = lane >> 3, n = kb1 - kb0;
-    const uint16_t *src[CX + CW];
+    const T *src[CX + CW];
 #pragma unroll
     for (int i = 0; i < CX + CW; ++i)
-      src[i] = row(i < CX ? (i * WAVES + wave) * 8 + sub : BM + ((i - CX) * WAVES + wave) * 8 + sub) + kb0 * 64 + ((lane & 7) ^ sub) * 8;
+      src[i] = row(i < CX ? (i * WAVES + wave) * 8 + sub : BM + ((i - CX) * WAVES + wave) * 8 + sub) + kb0 * COLS + ((lane & 7) ^ sub) * (COLS / 8);
     auto copy_x = [&](int b, int slot) {
 #pragma unroll
-      for (int i = 0; i < CX; ++i) kx_copy16_to_lds(src[i] + b * 64, __builtin_amdgcn_readfirstlane(lds0 + slot * SLOT + (i * WAVES + wave) * 1024));
+      for (int i = 0; i < CX; ++i) kx_copy16_to_lds(src[i] + b * COLS, __builtin_amdgcn_readfirstlane(lds0 + slot * SLOT + (i * WAVES + wave) * 1024));
     };
     auto copy_w = [&](int b, int slot) {
 #pragma unroll
-      for (int i = 0; i < CW; ++i) kx_copy16_to_lds(src[CX + i] + b * 64, __builtin_amdgcn_readfirstlane(lds0 + slot * SLOT + (i * WAVES + wave) * 1024));
+      for (int i = 0; i < CW; ++i) kx_copy16_to_lds(src[CX + i] + b * COLS, __builtin_amdgcn_readfirstlane(lds0 + slot * SLOT + (i * WAVES + wave) * 1024));
     };
     struct Frag {
-      bf16x8 x[MI], w[NI];
+      typename Piece<T>::Type x[MI], w[NI];
     };
     const uint8_t *const xs = lds + (wm * MI * 32 + lr) * 128, *const ws = lds + (wn * NI * 32 + lr) * 128;
     int sx = 0, sw = 1;  // slots of the present block
@@ -67,16 +85,16 @@ struct Tile {
     auto read = [&](Frag &f, int q) {
       const int p = ((2 * q + h) ^ (lr & 7)) * 16;
 #pragma unroll
-      for (int i = 0; i < MI; ++i) f.x[i] = *(const bf16x8 *)(xs + sx * SLOT + p + i * 4096);
+      for (int i = 0; i < MI; ++i) f.x[i] = *(const typename Piece<T>::Type *)(xs + sx * SLOT + p + i * 4096);
 #pragma unroll
-      for (int j = 0; j < NI; ++j) f.w[j] = *(const bf16x8 *)(ws + sw * SLOT + p + j * 4096);
+      for (int j = 0; j < NI; ++j) f.w[j] = *(const typename Piece<T>::Type *)(ws + sw * SLOT + p + j * 4096);
       __builtin_amdgcn_sched_barrier(0);
     };
     auto multiply = [&](const Frag &f) {
 #pragma unroll
       for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < NI; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.x[i], f.w[j], acc[i][j], 0, 0, 0);
+        for (int j = 0; j < NI; ++j) acc[i][j] = Piece<T>::multiply(f.x[i], f.w[j], acc[i][j]);
       __builtin_amdgcn_sched_barrier(0);
     };
 #pragma unroll
@@ -181,8 +199,8 @@ __device__ __forceinline__ int item_of(int id, int n) {
   return die * q + min(die, r) + (id >> 3);
 }
 
-typedef Tile<4, 2, 2, 4, 4> Large;   // 256 x 256, 8 waves, a CU each
-typedef Tile<2, 2, 2, 2, 5> Medium;  // 128 x 128, 4 waves, two workgroups per CU
+typedef Tile<uint16_t, 4, 2, 2, 4, 4> Large;   // 256 x 256, 8 waves, a CU each
+typedef Tile<uint16_t, 2, 2, 2, 2, 5> Medium;  // 128 x 128, 4 waves, two workgroups per CU
 
 // Which tile, and in how many parts of the columns, for one product of `tokens` x `rows` with `blocks` blocks of 64 columns.
 // Where the medium tiles leave CUs idle they take parts, of at least 16 blocks; beyond that the shorter of two estimates, in
@@ -205,6 +223,19 @@ inline Choice choose(int tokens, int rows, int blocks, size_t part_floats, int a
   }
   const double l = (double)((large + cus - 1) / cus) * (12 + 1.55 * blocks), m = (medium > 2 * cus ? medium / (2.0 * cus) : 1.0) * (6 + 1.22 * blocks);
   return {l < m, 1};
+}
+
+// The 32-bit tile: 64 x 128, 4 waves, two workgroups per CU.  A piece is 4 products of 64 cycles, so LDS and copies are far
+// from their limits and what counts is that every SIMD has a wave: 777 x 8192 x 1024 takes 142 us so, 181 with two waves a
+// workgroup; 777 x 1024 x 4096 140 us with 104 tiles, 79 with their columns in four parts, 11 x 5120 x 1024 38 and 19.  On the
+// vector ALU (64 x 64, 4 x 4 a thread) the first, with its activation, took 260 us and was a little further from the 64-bit result.
+typedef Tile<float, 2, 2, 1, 2, 4> Single;
+inline int choose_single(int tokens, int rows, int blocks, size_t part_floats, int arrivals, int cus) {
+  const long tiles = (long)((tokens + Single::BM - 1) / Single::BM) * ((rows + Single::BN - 1) / Single::BN);
+  long p = 2 * cus / tiles;
+  if (p > blocks / 8) p = blocks / 8;
+  if ((size_t)p > part_floats / Single::PART / tiles) p = part_floats / Single::PART / tiles;
+  return p < 2 || tiles > arrivals ? 1 : (int)p;
 }
 
 }  // namespace kxtile

@@ -10,7 +10,7 @@
 // all residual streams of the row.
 // lin_narrow_k (bf16, up to 64 tokens): all tokens against 64 rows, the columns split over waves and workgroups.
 // lin_gemm_k (bf16, more tokens): tiles of 256 x 256 or 128 x 128 on the matrix cores (kx_gemm_tile.h).
-// lin_gemm_f32_k (f32): tiles of 64 x 64 on the vector ALU; true 32-bit products.
+// In f32 the same with tiles of 64 x 64 and 32-bit matrix instructions; true 32-bit products.
 //
 // Products with experts: up to 4 tokens lin_gemv_k with a matrix per (token, choice), the routing in its prologue, and with
 // the residual update's own product and the chosen experts' as one sum over consecutive segments of columns; beyond that
@@ -280,8 +280,8 @@ __device__ __forceinline__ size_t source_row(const KxExpertArgs &e, const Tile &
   return GROUP && e.gather ? e.gather[s] : s;
 }
 
-template <class TL, int EPI, bool GROUP>
-__global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) lin_gemm_k(KxLinArgs a, KxExpertArgs e, const uint16_t *__restrict__ x, int x_ld, int parts) {
+template <class T, class TL, int EPI, bool GROUP>
+__global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) lin_gemm_k(KxLinArgs a, KxExpertArgs e, const T *__restrict__ x, int x_ld, int parts) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   Tile tl;
   int n0, part = 0, tile = 0;
@@ -298,10 +298,10 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) lin_gemm_k(Kx
     tl.w = 0;
   }
   x += (size_t)variant_of(a, n0) * a.tokens * x_ld;
-  const int nb = a.m.ld >> 6;  // blocks of 64 columns
+  const int nb = a.m.ld / TL::COLS;
   f32x16 acc[TL::MI][TL::NI];
   TL::run(lds, (int)((long)nb * part / parts), (int)((long)nb * (part + 1) / parts), [&](int r) {
-    return r < TL::BM ? x + source_row<GROUP>(e, tl, r) * x_ld : (const uint16_t *)a.m.w + tl.w + (size_t)min(n0 + r - TL::BM, a.m.rows - 1) * a.m.ld;
+    return r < TL::BM ? x + source_row<GROUP>(e, tl, r) * x_ld : (const T *)a.m.w + tl.w + (size_t)min(n0 + r - TL::BM, a.m.rows - 1) * a.m.ld;
   }, acc);
   if (!GROUP && parts > 1 && !TL::gather(lds, acc, a.part + (size_t)tile * parts * TL::PART, a.arrived + tile, parts, part)) return;
 #pragma unroll
@@ -314,7 +314,7 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) lin_gemm_k(Kx
         for (int v = 0; v < 16; ++v) {
           const int t = tl.m0 + TL::row(i, v);
           if (t < tl.end && r < a.m.rows)
-            put_glu<uint16_t>(a, t, (r >> 6) * KX_GLU_BLOCK + (r & 31), acc[i][j][v], acc[i][j + 1][v], GROUP ? e.slot_weight[t] : 1.0f);
+            put_glu<T>(a, t, (r >> 6) * KX_GLU_BLOCK + (r & 31), acc[i][j][v], acc[i][j + 1][v], GROUP ? e.slot_weight[t] : 1.0f);
         }
       }
     } else {
@@ -324,11 +324,11 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) lin_gemm_k(Kx
         if constexpr (EPI == KX_LIN_F32) {
 #pragma unroll
           for (int v = 0; v < 16; ++v)
-            if (tl.m0 + TL::row(i, v) < tl.end && r < a.m.rows) put_f32<uint16_t>(a, tl.m0 + TL::row(i, v), r, acc[i][j][v]);
+            if (tl.m0 + TL::row(i, v) < tl.end && r < a.m.rows) put_f32<T>(a, tl.m0 + TL::row(i, v), r, acc[i][j][v]);
         } else if constexpr (EPI == KX_LIN_HEADS) {
 #pragma unroll
           for (int v = 0; v < 16; ++v)
-            if (tl.m0 + TL::row(i, v) < tl.end && r < a.m.rows) put_head<uint16_t>(a, tl.m0 + TL::row(i, v), r, acc[i][j][v]);
+            if (tl.m0 + TL::row(i, v) < tl.end && r < a.m.rows) put_head<T>(a, tl.m0 + TL::row(i, v), r, acc[i][j][v]);
         } else {
           constexpr int G = most_streams(EPI) > 2 ? 4 : 16;  // elements read before the first is written
 #pragma unroll
@@ -477,65 +477,6 @@ __global__ void __launch_bounds__(512, MI == 1 ? 4 : 2) lin_narrow_k(KxLinArgs a
   }
 }
 
-// ---- f32 GEMM: 64 tokens x 64 rows, a thread owns 4 x 4; its rows are r, r + 16, ..., so that (gate, up) pairs, 32
-// rows apart, meet in one thread ----
-template <int EPI, bool GROUP>
-__global__ void __launch_bounds__(256) lin_gemm_f32_k(KxLinArgs a, KxExpertArgs e, const float *__restrict__ x, int x_ld) {
-  constexpr int BK = 16, STR = 68;
-  __shared__ float xs[BK][STR], ws[BK][STR];
-  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-  const int n0 = blockIdx.x * 64;
-  Tile tl;
-  if (!tile_of<GROUP>(a, e, 64, tl)) return;
-  const int m0 = tl.m0;
-  x += (size_t)variant_of(a, n0) * a.tokens * x_ld;
-  const int lrow = tid >> 2, lc = (tid & 3) * 4;
-  const float *xp = x + source_row<GROUP>(e, tl, lrow) * x_ld + lc;
-  const float *wp = (const float *)a.m.w + tl.w + (size_t)min(n0 + lrow, a.m.rows - 1) * a.m.ld + lc;
-  float acc[4][4] = {};
-  for (int k0 = 0; k0 < a.m.ld; k0 += BK) {
-    const float4 xv = *(const float4 *)(xp + k0), wv = *(const float4 *)(wp + k0);
-    __syncthreads();
-    xs[lc][lrow] = xv.x; xs[lc + 1][lrow] = xv.y; xs[lc + 2][lrow] = xv.z; xs[lc + 3][lrow] = xv.w;
-    ws[lc][lrow] = wv.x; ws[lc + 1][lrow] = wv.y; ws[lc + 2][lrow] = wv.z; ws[lc + 3][lrow] = wv.w;
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < BK; ++k) {
-      float xr[4], wr[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        xr[i] = xs[k][ty + 16 * i];
-        wr[i] = ws[k][tx + 16 * i];
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_fmaf(xr[i], wr[j], acc[i][j]);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int t = m0 + ty + 16 * i;
-    if (t >= tl.end) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int r = n0 + tx + 16 * j;
-      if (r >= a.m.rows) continue;
-      if constexpr (EPI == KX_LIN_F32) {
-        put_f32<float>(a, t, r, acc[i][j]);
-      } else if constexpr (EPI == KX_LIN_HEADS) {
-        put_head<float>(a, t, r, acc[i][j]);
-      } else if constexpr (EPI == KX_LIN_GLU) {
-        if (j < 2) put_glu<float>(a, t, n0 / 2 + tx + 16 * j, acc[i][j], acc[i][(j + 2) & 3], GROUP ? e.slot_weight[t] : 1.0f);
-      } else {
-        Streams<EPI> res;
-        res.load(a, t, r);
-        res.store(a, t, r, acc[i][j]);
-      }
-    }
-  }
-}
-
 constexpr size_t GEMV_LDS = 150 * 1024;
 
 // `lds` bytes of the dynamic part; grid_y: 1, or the tokens or (token, choice) pairs
@@ -609,17 +550,17 @@ int narrow_launch(const KxLinArgs &a, const KxExpertArgs &e, const uint16_t *x, 
   return KX_OK;
 }
 
-typedef kxtile::Tile<2, 2, 1, 2, 4> SmallSlots;  // 64 slots of an expert
-template <class TL, int EPI, bool GROUP>
-int tile_launch(const KxLinArgs &a, const KxExpertArgs &e, const uint16_t *x, int x_ld, int parts, hipStream_t st) {
+typedef kxtile::Tile<uint16_t, 2, 2, 1, 2, 4> SmallSlots;  // 64 slots of an expert
+template <class T, class TL, int EPI, bool GROUP>
+int tile_launch(const KxLinArgs &a, const KxExpertArgs &e, const T *x, int x_ld, int parts, hipStream_t st) {
   static std::atomic<bool> attr{false};
   if (!attr) {
-    KX_HIP(hipFuncSetAttribute((const void *)lin_gemm_k<TL, EPI, GROUP>, hipFuncAttributeMaxDynamicSharedMemorySize, TL::LDS));
+    KX_HIP(hipFuncSetAttribute((const void *)lin_gemm_k<T, TL, EPI, GROUP>, hipFuncAttributeMaxDynamicSharedMemorySize, TL::LDS));
     attr = true;
   }
   const int tn = kx_cdiv(a.m.rows, TL::BN);
   const dim3 grid = GROUP ? dim3(tn, e.max_tiles) : dim3(tn * kx_cdiv(a.tokens, TL::BM) * parts);
-  hipLaunchKernelGGL((lin_gemm_k<TL, EPI, GROUP>), grid, dim3(TL::THREADS), TL::LDS, st, a, e, x, x_ld, parts);
+  hipLaunchKernelGGL((lin_gemm_k<T, TL, EPI, GROUP>), grid, dim3(TL::THREADS), TL::LDS, st, a, e, x, x_ld, parts);
   KX_LAUNCH_CHECK();
   return KX_OK;
 }
@@ -630,16 +571,17 @@ int gemm_launch(const KxLinArgs &a, const KxExpertArgs &e, const T *x, int x_ld,
   KX_REQUIRE(x && x_ld >= a.m.ld, "kx_linear: activation rows of %d, the matrix has %d", x_ld, a.m.ld);
   if constexpr (sizeof(T) == 2 && GROUP)
     if (e.tile_slots <= 32) return narrow_launch<EPI, true>(a, e, x, x_ld, st);
+  const size_t room = a.part ? a.part_floats : 0;
+  const int arrivals = a.arrived ? a.arrivals : 0, cus = std::max(1, kx_device_cus());
   if constexpr (sizeof(T) == 4) {
-    hipLaunchKernelGGL((lin_gemm_f32_k<EPI, GROUP>), dim3(kx_cdiv(a.m.rows, 64), GROUP ? e.max_tiles : kx_cdiv(a.tokens, 64)), dim3(256), 0, st, a, e, x, x_ld);
-    KX_LAUNCH_CHECK();
-    return KX_OK;
+    const int parts = GROUP ? 1 : kxtile::choose_single(a.tokens, a.m.rows, a.m.ld / kxtile::Single::COLS, room, arrivals, cus);
+    return tile_launch<float, kxtile::Single, EPI, GROUP>(a, e, x, x_ld, parts, st);
   } else if constexpr (GROUP) {
-    return e.tile_slots > 64 ? tile_launch<kxtile::Medium, EPI, true>(a, e, x, x_ld, 1, st) : tile_launch<SmallSlots, EPI, true>(a, e, x, x_ld, 1, st);
+    return e.tile_slots > 64 ? tile_launch<uint16_t, kxtile::Medium, EPI, true>(a, e, x, x_ld, 1, st) : tile_launch<uint16_t, SmallSlots, EPI, true>(a, e, x, x_ld, 1, st);
   } else {
-    const kxtile::Choice c = kxtile::choose(a.tokens, a.m.rows, a.m.ld >> 6, a.part ? a.part_floats : 0, a.arrived ? a.arrivals : 0, std::max(1, kx_device_cus()));
-    if (c.large && a.n_var == 1) return tile_launch<kxtile::Large, EPI, false>(a, e, x, x_ld, 1, st);  // variants begin at multiples of 128 rows
-    return tile_launch<kxtile::Medium, EPI, false>(a, e, x, x_ld, c.parts, st);
+    const kxtile::Choice c = kxtile::choose(a.tokens, a.m.rows, a.m.ld >> 6, room, arrivals, cus);
+    if (c.large && a.n_var == 1) return tile_launch<uint16_t, kxtile::Large, EPI, false>(a, e, x, x_ld, 1, st);  // variants begin at multiples of 128 rows
+    return tile_launch<uint16_t, kxtile::Medium, EPI, false>(a, e, x, x_ld, c.parts, st);
   }
 }
 
@@ -709,9 +651,9 @@ int linear(const KxLinArgs &a, void *row_buf, hipStream_t st) {
   if (a.epi == KX_LIN_F32) return linear_epi<T, KX_LIN_F32>(a, row_buf, st);
   if (a.epi == KX_LIN_GLU) return linear_epi<T, KX_LIN_GLU>(a, row_buf, st);
   if (a.epi == KX_LIN_HEADS) return linear_epi<T, KX_LIN_HEADS>(a, row_buf, st);
+  if (a.n_streams == 1) return linear_epi<T, KX_LIN_STREAMS + 1>(a, row_buf, st);
+  if (a.n_streams == 2) return linear_epi<T, KX_LIN_STREAMS + 2>(a, row_buf, st);
   if constexpr (sizeof(T) == 2) {
-    if (a.n_streams == 1) return linear_epi<T, KX_LIN_STREAMS + 1>(a, row_buf, st);
-    if (a.n_streams == 2) return linear_epi<T, KX_LIN_STREAMS + 2>(a, row_buf, st);
     if (a.n_streams == 3) return linear_epi<T, KX_LIN_STREAMS + 3>(a, row_buf, st);
     if (a.n_streams == 4) return linear_epi<T, KX_LIN_STREAMS + 4>(a, row_buf, st);
   }

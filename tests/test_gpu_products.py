@@ -9,24 +9,25 @@ import kagalorn_case as KC
 import kagalorn_oracle as K
 from blok_amd.lib import DevBuf, KxLinearArgs, check
 from kxt import dev
-from test_gpu_kagalorn import BF16_LOGITS, _matrix, rel
+from test_gpu_kagalorn import BF16_LOGITS, F32_LOGITS, _matrix, rel
 from test_gpu_rapitar import Experts
 
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.parametrize("dtype, bar", [("bfloat16", BF16_LOGITS), ("float32", F32_LOGITS)])
 @pytest.mark.parametrize("ff", [4200, 4130], ids=["whole blocks", "half a block left"])
-def test_few_tokens_against_wide_matrices(kxlib, tmp_path, ff):
+def test_few_tokens_against_wide_matrices(kxlib, tmp_path, ff, dtype, bar):
     """5 to 64 tokens a step: up to eight parts of 66 and 65 pieces of 64 columns, and the last part shorter than the others;
-    66 to 192 tokens: tiles in up to four parts."""
+    66 to 192 tokens: tiles in up to four parts.  In 32 bits tiles in up to 16 parts throughout."""
     cfg = KC.config([KC.delta(heads=4, kv_heads=2, dim=32, vdim=640, ff=ff), KC.attention(ff=ff)], width=192, vocab=300)
     w = KC.weights(cfg, ff)
     ids = np.stack([KC.tokens(cfg, 6, 100 + b) for b in range(64)])
     want = np.stack([K.forward(cfg, w, s) for s in ids], 1)
-    with KC.Model(KC.write(tmp_path, cfg, w), "bfloat16", batch=64, context=6) as m:
+    with KC.Model(KC.write(tmp_path, cfg, w), dtype, batch=64, context=6) as m:
         for batch, cuts in ((5, [1]), (8, [4, 1]), (31, [2, 1]), (33, [1]), (63, [1]), (64, [1]), (5, [1]), (33, [2]), (64, [2]), (43, [3]), (64, [3])):
             first = m.run(ids[:batch], cuts, batch)
-            assert KC.logit_error(first, want[:, :batch]).max() < BF16_LOGITS, (batch, cuts)
+            assert KC.logit_error(first, want[:, :batch]).max() < bar, (batch, cuts)
             assert (m.run(ids[:batch], cuts, batch) == first).all(), "the parts' order does not depend on who comes last"
 
 
