@@ -27,12 +27,18 @@ struct KxDeltaArgs {
   float *o = nullptr;             // f32 [tokens][heads * vdim]
   float *work = nullptr;          // kx_delta_work_floats(s, batch, positions) floats (not used for one position)
 };
-// Tokens go through the state in blocks of KX_DELTA_BLOCK; per token and head there are KX_DELTA_COEF numbers.
-constexpr int KX_DELTA_BLOCK = 4, KX_DELTA_COEF = 12;
-// keys and queries lie in the scratch with rows of 32, 64, 128 or 256
-__host__ __device__ inline int kx_delta_row(const KxDeltaSpec &s) { return s.dim <= 32 ? 32 : s.dim <= 64 ? 64 : s.dim <= 128 ? 128 : 256; }
+// Tokens go through the state in blocks of KX_DELTA_BLOCK; per token and head there are KX_DELTA_COEF numbers, and per token and
+// key head the key twice and the query, with rows of whole multiples of 64.
+constexpr int KX_DELTA_BLOCK = 16, KX_DELTA_COEF = 34;
+__host__ __device__ inline int kx_delta_row(const KxDeltaSpec &s) { return (s.dim + 63) / 64 * 64; }
+// blocks whose numbers a wave holds in registers at a time, and which a step is filled up to: three where the row leaves room for them
+__host__ __device__ inline int kx_delta_sets(const KxDeltaSpec &s) { return s.dim <= 128 ? 3 : 2; }
+__host__ __device__ inline int kx_delta_blocks(const KxDeltaSpec &s, int positions) {
+  const int span = kx_delta_sets(s) * KX_DELTA_BLOCK;
+  return (positions + span - 1) / span * kx_delta_sets(s);
+}
 inline size_t kx_delta_work_floats(const KxDeltaSpec &s, int batch, int positions) {
-  const size_t padded = (size_t)batch * ((positions + KX_DELTA_BLOCK - 1) / KX_DELTA_BLOCK * KX_DELTA_BLOCK);
-  return padded * ((size_t)KX_DELTA_COEF * s.heads + kx_delta_channels(s) + 2 * s.kv_heads * kx_delta_row(s));
+  const size_t padded = (size_t)batch * kx_delta_blocks(s, positions) * KX_DELTA_BLOCK;
+  return padded * ((size_t)KX_DELTA_COEF * s.heads + kx_delta_channels(s) + 3 * s.kv_heads * kx_delta_row(s));
 }
 int kx_delta_launch(const KxDeltaArgs &a, hipStream_t st);

@@ -1,24 +1,25 @@
-// kx_delta.hip -- see kx_delta.h.  Everything here is 32-bit.  No counterpart in the reference, which has no recurrent layer.
+// kx_delta.hip -- see kx_delta.h.  Nothing here is less than 32-bit.  No counterpart in the reference, which has no recurrent layer.
 //
 // One token per sequence: delta_step_k.  A workgroup owns 32 columns of one head's state; it convolves and norms the
 // head's q and k itself, reads its columns once, and writes them once.
 //
-// Several positions: the convolutions (kx_conv.hip), delta_unit_k (unit norms and the numbers below) and delta_scan_k, which
-// keeps the state in registers:
-// the columns of a head's state do not meet, so a column is spread over dim / 8 lanes with 8 rows each, and a wave goes
-// through the tokens.  It takes them in blocks of four, so that the sums over a column's lanes do not wait for each
-// other: with S the state before the block, D(i, j) the product of the decays of tokens i + 1 .. j and D(j) that of tokens
-// 1 .. j of the block,
-//   u_j = beta_j (v_j - D(j) S^T k_j - sum_{i < j} D(i, j) (k_i . k_j) u_i)
-//   o_j = D(j) S^T q_j + sum_{i <= j} D(i, j) (k_i . q_j) u_i
-//   S  <- D(4) S + sum_i D(i, 4) k_i u_i^T,
-// which is the recurrence written out for four tokens.  The numbers that do not depend on the column -- per token D(j),
-// beta, D(j, 4), D(j - d, j) (k_{j-d} . k_j) for d = 1..3 and D(j - d, j) (k_{j-d} . q_j) for d = 0..3 -- are made
-// once per head by delta_unit_k.
+// Several positions: the convolutions (kx_conv.hip), then blocks of 16 tokens counted from the step's first position.  With S the
+// state before a block, D(i, j) the product of the decays of its tokens i + 1 .. j and G(j) that of tokens 1 .. j,
+//   u_j = beta_j (v_j - G(j) S^T k_j - sum_{i < j} D(i, j) (k_i . k_j) u_i)
+//   o_j = G(j) S^T q_j + sum_{i <= j} D(i, j) (k_i . q_j) u_i
+//   S  <- G(16) S + sum_i D(i, 16) k_i u_i^T,
+// which is the recurrence written out for sixteen tokens: only products of decays occur, never a quotient.  The first line is a
+// triangular system with the same matrix for every column, I + L, L(j, i) = beta_j D(i, j) (k_i . k_j); delta_block_k inverts it
+// once per block and head -- T = (I + L)^-1 diag(beta); its entries are those of products of contractions, beta being at
+// most 1 and the keys of unit length, and so do not grow -- and delta_scan_k is left with
+//   U = T (V - G K S),  O = G Q S + A U,  S <- G(16) S + (E K)^T U,
+// products of 32-bit matrix instructions on the state, which it keeps in registers.  Lengths, decays and T are computed in 64 bits and
+// rounded once, which pays for the sums over more tokens: the error is below that of the recurrence in 32 bits, token by token.
 #include <algorithm>
 #include <atomic>
 #include "kx_common.h"
 #include "kx_conv.h"
+#include "kx_lds_copy.h"
 #include "kx_rows.h"
 #include "kx_delta.h"
 
@@ -101,247 +102,289 @@ __global__ void __launch_bounds__(256) delta_step_k(KxDeltaArgs a, KxConvArgs cv
   }
 }
 
-constexpr int NB = KX_DELTA_BLOCK, NCF = KX_DELTA_COEF;
-enum { CF_GAMMA = 0, CF_BETA = 1, CF_END = 2, CF_KK = 3, CF_KQ = 6 };  // places of a token's numbers
+constexpr int NB = KX_DELTA_BLOCK, NCF = KX_DELTA_COEF * NB;  // numbers of a block and head:
+enum { CF_T = 0, CF_A = NB * NB, CF_GAMMA = 2 * NB * NB, CF_END = CF_GAMMA + NB };  // T, A [token][token], G(j), D(j, 16)
+static_assert(CF_END + NB == NCF, "room for a block's numbers");
 
 struct Work {
-  float *coef;  // [batch][heads][padded positions][NCF]
-  float *qk;    // [tokens][kv_heads][2][kx_delta_row]: unit k, unit q times dim^-1/2, zeros behind them
+  float *coef;  // [batch][heads][blocks][NCF]
+  float *qk;    // [batch][kv_heads][blocks][k, q, k^T][row / 16][lane][4]: unit k, unit q times dim^-1/2, zeros behind them, as delta_scan_k takes them
   float *raw;   // [tokens][channels]: q, k, v behind convolution and silu
-  int padded;
+  int blocks;
 };
 __host__ __device__ __forceinline__ Work work_of(const KxDeltaArgs &a) {
   Work w;
-  w.padded = (a.positions + NB - 1) / NB * NB;
+  w.blocks = kx_delta_blocks(a.s, a.positions);
   w.coef = a.work;
-  w.qk = w.coef + (size_t)a.batch * a.s.heads * w.padded * NCF;
-  w.raw = w.qk + (size_t)a.batch * a.positions * a.s.kv_heads * 2 * kx_delta_row(a.s);
+  w.qk = w.coef + (size_t)a.batch * a.s.heads * w.blocks * NCF;
+  w.raw = w.qk + (size_t)a.batch * a.s.kv_heads * w.blocks * 3 * NB * kx_delta_row(a.s);
   return w;
 }
 
-// one wave per (position, key head)
-__global__ void __launch_bounds__(256) delta_unit_k(KxDeltaArgs a) {
-  const KxDeltaSpec &s = a.s;
-  const int lane = threadIdx.x & 63, D = s.dim, nq = s.kv_heads * D, C = kx_delta_channels(s), ratio = s.heads / s.kv_heads;
-  const Work w = work_of(a);
-  const int item = blockIdx.x * 4 + (threadIdx.x >> 6), kvh = item % s.kv_heads, i = item / s.kv_heads, b = blockIdx.y;
-  if (i >= w.padded) return;
-  const int j = i % NB, t0 = i - j;  // place in the block, and the block's first position
-  float dot[NB + NB - 1] = {}, inv[NB] = {};  // kk of d = 1.., kq of d = 0..
-  if (i < a.positions) {
-    const float *row[NB];
+// 1 / sqrt of a sum over 16 lanes, in every one of them
+__device__ __forceinline__ double row_rsqrt(double v, float eps) {
 #pragma unroll
-    for (int d = 0; d < NB; ++d) row[d] = w.raw + (size_t)((i - min(d, j)) * a.batch + b) * C + kvh * D;
-    float qq = 0.0f, ss[NB] = {};
-    for (int x = lane; x < D; x += 64) {
-      const float q = row[0][x];
-      float k[NB];
-#pragma unroll
-      for (int d = 0; d < NB; ++d) k[d] = row[d][nq + x];
-      qq = __builtin_fmaf(q, q, qq);
-#pragma unroll
-      for (int d = 0; d < NB; ++d) {
-        ss[d] = __builtin_fmaf(k[d], k[d], ss[d]);
-        dot[NB - 1 + d] = __builtin_fmaf(k[d], q, dot[NB - 1 + d]);
-        if (d) dot[d - 1] = __builtin_fmaf(k[d], k[0], dot[d - 1]);
-      }
-    }
-    const float qsc = kx_rsqrtf(kxr::wave_sum(qq) + s.unit_eps) * kx_rsqrtf((float)D);
-#pragma unroll
-    for (int d = 0; d < NB; ++d) inv[d] = kx_rsqrtf(kxr::wave_sum(ss[d]) + s.unit_eps);
-#pragma unroll
-    for (int d = 0; d < NB; ++d) {
-      dot[NB - 1 + d] = kxr::wave_sum(dot[NB - 1 + d]) * inv[d] * qsc;
-      if (d) dot[d - 1] = kxr::wave_sum(dot[d - 1]) * inv[d] * inv[0];
-    }
-    const int DP = kx_delta_row(s);
-    float *out = w.qk + ((size_t)(i * a.batch + b) * s.kv_heads + kvh) * 2 * DP;
-    for (int x = lane; x < DP; x += 64) {
-      out[x] = x < D ? row[0][nq + x] * inv[0] : 0.0f;
-      out[DP + x] = x < D ? row[0][x] * qsc : 0.0f;
-    }
-  }
-  for (int r = lane; r < ratio; r += 64) {  // the heads that share the key
-    const int h = kvh * ratio + r;
-    float g[NB];  // decays of the block; a position past the end leaves the state as it is
-#pragma unroll
-    for (int d = 0; d < NB; ++d)
-      g[d] = t0 + d < a.positions ? decay_of(a, a.proj + (size_t)((t0 + d) * a.batch + b) * a.proj_ld, h) : 1.0f;
-    float *cf = w.coef + (((size_t)b * s.heads + h) * w.padded + i) * NCF;
-    float gamma = 1.0f, end = 1.0f;
-#pragma unroll
-    for (int d = 0; d < NB; ++d) {
-      if (d <= j) gamma *= g[d];
-      else end *= g[d];
-    }
-    cf[CF_GAMMA] = gamma;
-    cf[CF_BETA] = i < a.positions ? kx_sigmoidf(a.proj[(size_t)(i * a.batch + b) * a.proj_ld + a.b_off + h]) : 0.0f;
-    cf[CF_END] = end;
-    float down = 1.0f;  // D(j - d, j)
-#pragma unroll
-    for (int d = 0; d < NB; ++d) {
-      const bool in = d <= j;  // the other token is in the block
-      cf[CF_KQ + d] = in ? down * dot[NB - 1 + d] : 0.0f;
-      if (d) cf[CF_KK + d - 1] = in ? down * dot[d - 1] : 0.0f;
-#pragma unroll
-      for (int x = 0; x < NB; ++x)
-        if (x == j - d) down *= g[x];
-    }
-  }
+  for (int m = 1; m < 16; m <<= 1) v += __shfl_xor(v, m);
+  return 1.0 / sqrt(v + eps);
 }
 
-template <int LPC>
-__device__ __forceinline__ float column_sum(float v) {  // over the LPC lanes of a column, in every one of them
-  v += kxw::dpp_f<kxw::DPP_QUAD_XOR1>(v);
-  v += kxw::dpp_f<kxw::DPP_QUAD_XOR2>(v);
-  if (LPC >= 8) v += kxw::dpp_f<kxw::DPP_ROW_HALF_MIRROR>(v);
-  if (LPC >= 16) v += kxw::dpp_f<kxw::DPP_ROW_MIRROR>(v);
-  if (LPC >= 32) {
-    float t = v;
-    kxw::swap_rows16(v, t);
-    v += t;
-  }
-  return v;
-}
-
-// A block's numbers, one per lane as they are loaded, in scalar registers as they are used: they are the same for the whole
-// workgroup.  (Scalar loads would come from the memory side of the caches, 1-2 us away, once per block.)
-struct Coefs {
-  float v[NB][NCF];
-  __device__ __forceinline__ void from_lanes(float x) {
-#pragma unroll
-    for (int j = 0; j < NB; ++j)
-#pragma unroll
-      for (int y = 0; y < NCF; ++y) v[j][y] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), j * NCF + y));
-  }
-};
-static_assert(NB * NCF <= 64, "a block's numbers are one wave load");
-
-template <int LPC>  // lanes per column, 8 rows of the state each
-__global__ void __launch_bounds__(256) delta_scan_k(KxDeltaArgs a) {
-  constexpr int DP = LPC * 8, COLS = 256 / LPC, CT = LPC >= 16 ? 16 : 32;  // CT: tokens per staged block
-  __shared__ __attribute__((aligned(16))) float kq_s[2][CT][2][DP];
-  __shared__ float v_s[2][CT][COLS], o_s[2][CT][COLS];
+// One workgroup per (block, key head): unit norms, the products of the block's keys and queries (thread (j, i) those of tokens
+// j and i), then the numbers of each head that shares the key.
+__host__ __device__ constexpr int block_stride(int row) { return row + 4; }  // 16 rows at one column fall into different banks
+constexpr size_t block_lds(int row) { return (size_t)2 * NB * block_stride(row) * 4; }
+__global__ void __launch_bounds__(256) delta_block_k(KxDeltaArgs a) {
+  extern __shared__ __attribute__((aligned(16))) float bl_lds[];
+  __shared__ float g_s[NB], beta_s[NB];
+  __shared__ double L[NB][NB + 1];
   const KxDeltaSpec &s = a.s;
-  const int D = s.dim, V = s.vdim, tid = threadIdx.x;
-  const int h = blockIdx.y, b = blockIdx.z, c0 = blockIdx.x * COLS, kvh = h / (s.heads / s.kv_heads), nq = s.kv_heads * D;
-  const int C = kx_delta_channels(s), l4 = (tid % LPC) * 4, cl = tid / LPC, col = c0 + cl, n = a.positions;
+  const int D = s.dim, DP = kx_delta_row(s), STR = block_stride(DP), tid = threadIdx.x, sl = tid & 15, j = tid >> 4;
+  const int blk = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z, n = a.positions, nq = s.kv_heads * D, C = kx_delta_channels(s), ratio = s.heads / s.kv_heads;
   const Work w = work_of(a);
-  const float *coef = w.coef + ((size_t)b * s.heads + h) * w.padded * NCF;
-  float *st = a.state + ((size_t)b * s.heads + h) * D * V;
-  auto row = [&](int r) { return (r < 4 ? 0 : DP / 2 - 4) + l4 + r; };  // two runs of four rows: neighbouring lanes read neighbouring words
-  float S[8];
+  float *qs = bl_lds, *ks = qs + NB * STR;
+  {
+    const float *row = w.raw + (size_t)(min(blk * NB + j, n - 1) * a.batch + b) * C + kvh * D;
+    double qq = 0.0, kk = 0.0;  // the lengths in 64 bits: their error is one of every number of the row
+    for (int d0 = sl; d0 < DP; d0 += 64) {
+      float q[4], k[4];
 #pragma unroll
-  for (int r = 0; r < 8; ++r) S[r] = row(r) < D && col < V ? st[(size_t)row(r) * V + col] : 0.0f;
-  // A stage of tokens goes through registers into one of two LDS stages while the other is worked on.  Places past the last
-  // token repeat it: their numbers in `coef` make them leave the state alone.
-  constexpr int NK = CT * DP * 2 / 4 / 256, NV = (CT * COLS + 255) / 256;
-  f32x4 rk[NK];
-  float rv[NV], rc[CT / NB], rn[CT / NB];  // rc, rn: the numbers of this stage's blocks and of the next
-  auto fetch = [&](int t0) {
-#pragma unroll
-    for (int x = 0; x < NK; ++x) {
-      const int at = (x * 256 + tid) * 4, t = min(t0 + at / (2 * DP), n - 1);
-      rk[x] = *(const f32x4 *)(w.qk + ((size_t)(t * a.batch + b) * s.kv_heads + kvh) * 2 * DP + at % (2 * DP));
-    }
-#pragma unroll
-    for (int x = 0; x < NV; ++x) {
-      const int at = min(x * 256 + tid, CT * COLS - 1), t = min(t0 + at / COLS, n - 1), cc = min(c0 + at % COLS, V - 1);
-      rv[x] = w.raw[(size_t)(t * a.batch + b) * C + 2 * nq + h * V + cc];
-    }
-#pragma unroll
-    for (int x = 0; x < CT / NB; ++x) rn[x] = coef[(size_t)min(t0 + x * NB, w.padded - NB) * NCF + min(tid & 63, NB * NCF - 1)];
-  };
-  auto put = [&](int stage) {
-#pragma unroll
-    for (int x = 0; x < CT / NB; ++x) rc[x] = rn[x];
-#pragma unroll
-    for (int x = 0; x < NK; ++x) *(f32x4 *)(&kq_s[stage][0][0][0] + (x * 256 + tid) * 4) = rk[x];
-#pragma unroll
-    for (int x = 0; x < NV; ++x) {
-      const int at = x * 256 + tid;
-      if (at < CT * COLS) v_s[stage][at / COLS][at % COLS] = rv[x];
-    }
-  };
-  // keys, queries and values of a block, read from LDS while the block before it is worked on
-  float k[2][NB][8], q[2][NB][8], v[2][NB];
-  auto read = [&](int x, int stage, int tb) {
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-#pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        const f32x4 kk = *(const f32x4 *)&kq_s[stage][tb + j][0][half * (DP / 2) + l4], qq = *(const f32x4 *)&kq_s[stage][tb + j][1][half * (DP / 2) + l4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          k[x][j][half * 4 + e] = kk[e];
-          q[x][j][half * 4 + e] = qq[e];
-        }
+      for (int x = 0; x < 4; ++x) {
+        const int d = min(d0 + 16 * x, D - 1);
+        q[x] = row[d];
+        k[x] = row[nq + d];
       }
-      v[x][j] = v_s[stage][tb + j][cl];
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const bool in = d0 + 16 * x < D;
+        q[x] = in ? q[x] : 0.0f;
+        k[x] = in ? k[x] : 0.0f;
+        qs[j * STR + d0 + 16 * x] = q[x];
+        ks[j * STR + d0 + 16 * x] = k[x];
+        qq = __builtin_fma((double)q[x], (double)q[x], qq);
+        kk = __builtin_fma((double)k[x], (double)k[x], kk);
+      }
     }
-  };
-  fetch(0);
-  put(0);
+    const double qsc = row_rsqrt(qq, s.unit_eps) / sqrt((double)D), ksc = row_rsqrt(kk, s.unit_eps);
+    for (int d = sl; d < DP; d += 16) {
+      ks[j * STR + d] = (float)(ks[j * STR + d] * ksc);
+      qs[j * STR + d] = (float)(qs[j * STR + d] * qsc);
+    }
+  }
   __syncthreads();
-  for (int t0 = 0, stage = 0; t0 < n; t0 += CT, stage ^= 1) {
-    fetch(t0 + CT);  // past the end: the last token again
-    read(0, stage, 0);
+  f32x4 *out = (f32x4 *)(w.qk + (((size_t)b * s.kv_heads + kvh) * w.blocks + blk) * 3 * NB * DP);
+  for (int x = tid; x < 4 * DP; x += 256) {
+    const int c = x & 15, d = (x >> 6) * 16, t = (x >> 4 & 3) * 4;
+    out[x] = *(const f32x4 *)(ks + c * STR + d + t);
+    out[4 * DP + x] = *(const f32x4 *)(qs + c * STR + d + t);
+    f32x4 kt;
 #pragma unroll
-    for (int tb = 0; tb < CT; tb += NB) {
-      if (t0 + tb >= n) break;
-      const int x = (tb / NB) & 1;
-      float sk[NB], sq[NB];
+    for (int e = 0; e < 4; ++e) kt[e] = ks[(t + e) * STR + d + c];
+    out[8 * DP + x] = kt;
+  }
+  const int i = sl;
+  f32x4 kk4[4] = {}, kq4[4] = {};  // sixteen partial sums each: short chains, also of roundings
+  for (int d0 = 0; d0 < DP; d0 += 16)
 #pragma unroll
-      for (int j = 0; j < NB; ++j) {
-        sk[j] = sq[j] = 0.0f;
+    for (int x = 0; x < 4; ++x) {
+      const int d = d0 + 4 * x;
+      const f32x4 ki = *(const f32x4 *)(ks + i * STR + d), kj = *(const f32x4 *)(ks + j * STR + d), qj = *(const f32x4 *)(qs + j * STR + d);
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
-          sk[j] = __builtin_fmaf(S[r], k[x][j][r], sk[j]);
-          sq[j] = __builtin_fmaf(S[r], q[x][j][r], sq[j]);
-        }
-      }
-      if (tb + NB < CT) read(x ^ 1, stage, tb + NB);
-#pragma unroll
-      for (int j = 0; j < NB; ++j) {
-        sk[j] = column_sum<LPC>(sk[j]);
-        sq[j] = column_sum<LPC>(sq[j]);
-      }
-      Coefs now;
-      now.from_lanes(rc[tb / NB]);
-      float u[NB];
-#pragma unroll
-      for (int j = 0; j < NB; ++j) {
-        float e = __builtin_fmaf(-now.v[j][CF_GAMMA], sk[j], v[x][j]), o = now.v[j][CF_GAMMA] * sq[j];
-#pragma unroll
-        for (int d = 1; d <= j; ++d) {
-          e = __builtin_fmaf(-now.v[j][CF_KK + d - 1], u[j - d], e);
-          o = __builtin_fmaf(now.v[j][CF_KQ + d], u[j - d], o);
-        }
-        u[j] = now.v[j][CF_BETA] * e;
-        o = __builtin_fmaf(now.v[j][CF_KQ], u[j], o);
-        if (l4 == 0) o_s[stage][tb + j][cl] = o;
-      }
-#pragma unroll
-      for (int r = 0; r < 8; ++r) S[r] *= now.v[NB - 1][CF_GAMMA];
-#pragma unroll
-      for (int j = 0; j < NB; ++j) {
-        const float y = u[j] * now.v[j][CF_END];
-#pragma unroll
-        for (int r = 0; r < 8; ++r) S[r] = __builtin_fmaf(k[x][j][r], y, S[r]);
+      for (int e = 0; e < 4; ++e) {
+        kk4[x][e] = __builtin_fmaf(ki[e], kj[e], kk4[x][e]);
+        kq4[x][e] = __builtin_fmaf(ki[e], qj[e], kq4[x][e]);
       }
     }
-    put(stage ^ 1);
+  auto total = [](const f32x4 (&p)[4]) {
+    const f32x4 t = (p[0] + p[1]) + (p[2] + p[3]);
+    return (t[0] + t[1]) + (t[2] + t[3]);
+  };
+  const float kk = total(kk4), kq = total(kq4);  // k_i . k_j, k_i . q_j
+  for (int r = 0; r < ratio; ++r) {
+    const int h = kvh * ratio + r;
+    float *cf = w.coef + (((size_t)b * s.heads + h) * w.blocks + blk) * NCF;
+    __syncthreads();  // the head before has been worked on
+    if (tid < NB) {   // a position past the end leaves the state as it is
+      const bool in = blk * NB + tid < n;
+      const float *pr = a.proj + (size_t)(min(blk * NB + tid, n - 1) * a.batch + b) * a.proj_ld;
+      g_s[tid] = in ? decay_of(a, pr, h) : 1.0f;
+      beta_s[tid] = in ? kx_sigmoidf(pr[a.b_off + h]) : 0.0f;
+    }
     __syncthreads();
-    // the read-outs go to memory here, behind the wait for the next stage's rows, so that no wait is for a store just made
+    double d = 1.0;  // D(i, j): rounded once, not with each decay; a state that decays by it has fewer roundings than token by token
+    for (int m = i + 1; m <= j; ++m) d *= g_s[m];
+    L[j][i] = i < j ? beta_s[j] * d * kk : 0.0;
+    cf[CF_A + j * NB + i] = i <= j ? (float)(d * kq) : 0.0f;
+    if (i == 0) cf[CF_GAMMA + j] = (float)(d * g_s[0]);
+    if (j == NB - 1) cf[CF_END + i] = (float)d;
+    __syncthreads();
+    if (tid < NB) {  // column tid of the inverse
+      double t[NB];
 #pragma unroll
-    for (int x = 0; x < NV; ++x) {
-      const int at = x * 256 + tid, t = t0 + at / COLS, cc = c0 + at % COLS;
-      if (at < CT * COLS && t < n && cc < V) a.o[((size_t)(t * a.batch + b) * s.heads + h) * V + cc] = o_s[stage][at / COLS][at % COLS];
+      for (int y = 0; y < NB; ++y) {
+        double v = y == tid ? 1.0 : 0.0;
+#pragma unroll
+        for (int m = 0; m < y; ++m) v = __builtin_fma(-L[y][m], t[m], v);
+        t[y] = v;
+        cf[CF_T + y * NB + tid] = (float)(v * beta_s[tid]);
+      }
     }
   }
+}
+
+// A block's lower triangular matrix times a row per token, in 32-bit matrix instructions.  Those multiply the zeros above the
+// diagonal too, so a row that is not finite would reach the tokens before it; then the products are made token by token
+// from the rows up to it.
+__device__ __forceinline__ f32x4 lower(f32x4 m, f32x4 x) {
+  auto product = [&](f32x4 y) {
+    f32x4 p = __builtin_amdgcn_mfma_f32_16x16x4f32(m[0], y[0], f32x4{}, 0, 0, 0), q = __builtin_amdgcn_mfma_f32_16x16x4f32(m[2], y[2], f32x4{}, 0, 0, 0);
+    p = __builtin_amdgcn_mfma_f32_16x16x4f32(m[1], y[1], p, 0, 0, 0);
+    return p + __builtin_amdgcn_mfma_f32_16x16x4f32(m[3], y[3], q, 0, 0, 0);
+  };
+  const bool odd = !(__builtin_isfinite(x[0]) && __builtin_isfinite(x[1]) && __builtin_isfinite(x[2]) && __builtin_isfinite(x[3]));
+  if (__builtin_expect(__ballot(odd) == 0, 1)) return product(x);
+  const int g = (threadIdx.x & 63) >> 4;
+  f32x4 out = {};
+#pragma unroll 1
+  for (int j = 0; j < NB; ++j) {
+    f32x4 y;
 #pragma unroll
-  for (int r = 0; r < 8; ++r)
-    if (row(r) < D && col < V) st[(size_t)row(r) * V + col] = S[r];
+    for (int v = 0; v < 4; ++v) y[v] = 4 * g + v <= j ? x[v] : 0.0f;
+    y = product(y);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) out[v] = 4 * g + v == j ? y[v] : out[v];
+  }
+  return out;
+}
+
+// A workgroup owns 16 columns of a head's state, four waves a quarter of the rows each: row-block rb of wave w is rows 16 (w RB +
+// rb) .. + 15 as v_mfma_f32_16x16x4_f32 leaves its result -- lane (c, g) holds rows 4 g + v of column c --, which is also how
+// that instruction takes its second operand if the columns of a row-block meet in the order 4 g + v.
+// Bound by the chain of a block: 4 RB products for K S, their sums over the waves through LDS and a barrier, 4 products with
+// T, 4 RB with the keys' transpose.  Q S fills the time the exchange takes; a fifth wave makes the read-outs, a block
+// behind the others, which do not wait for it.  The numbers of the next SETS blocks are on their way meanwhile.
+// 2048 tokens of 16 heads of 128 x 128: 155 us, and 20 us for delta_block_k; on the vector ALU, four tokens per dependent step, 316 us
+// and 35 us.  Three sets in flight instead of two, and the slices of a head on one XCD, gave 3 %: it is the chain, not the loads.
+template <int RB>
+__global__ void __launch_bounds__(320, 2) delta_scan_k(KxDeltaArgs a) {
+  __shared__ f32x4 sk_s[2][4][64], sq_s[2][4][64], u_s[2][64];
+  const KxDeltaSpec &s = a.s;
+  const int D = s.dim, V = s.vdim, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, g = lane >> 4;
+  const int h = blockIdx.x, b = blockIdx.z, kvh = h / (s.heads / s.kv_heads), n = a.positions, C = kx_delta_channels(s);
+  const int col = blockIdx.y * 16 + c;
+  const Work w = work_of(a);
+  constexpr int DP = RB * 64, SETS = RB <= 2 ? 3 : 2;  // kx_delta_sets
+  const f32x4 *coef = (const f32x4 *)(w.coef + ((size_t)b * s.heads + h) * w.blocks * NCF);
+  if (wave == 4) {
+    auto numbers = [&](int blk, int at) { return coef[(size_t)min(blk, w.blocks - 1) * (NCF / 4) + at]; };
+    f32x4 A = numbers(0, CF_A / 4 + c * 4 + g), gamma = numbers(0, CF_GAMMA / 4 + g);
+    kx_lds_barrier();
+    for (int blk = 0; blk < w.blocks; ++blk) {
+      kx_lds_barrier();  // the sums and the rows u of block blk are there
+      const f32x4 nextA = numbers(blk + 1, CF_A / 4 + c * 4 + g), nextG = numbers(blk + 1, CF_GAMMA / 4 + g);
+      const f32x4(*q)[64] = sq_s[blk & 1];
+      const f32x4 qs = (q[0][lane] + q[1][lane]) + (q[2][lane] + q[3][lane]), au = lower(A, u_s[blk & 1][lane]);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int t = blk * NB + 4 * g + v;
+        if (t < n && col < V) a.o[((size_t)(t * a.batch + b) * s.heads + h) * V + col] = __builtin_fmaf(gamma[v], qs[v], au[v]);
+      }
+      A = nextA;
+      gamma = nextG;
+    }
+    return;
+  }
+  const int row0 = wave * RB * 16, last = (n - 1) / NB;
+  const f32x4 *qk = (const f32x4 *)(w.qk + ((size_t)b * s.kv_heads + kvh) * w.blocks * 3 * NB * DP) + wave * RB * 64 + lane;
+  const float *raw = w.raw + (size_t)b * C + (size_t)2 * s.kv_heads * D + h * V + min(col, V - 1);
+  float *st = a.state + ((size_t)b * s.heads + h) * D * V;
+  size_t row_at[4], last_at[4];  // of a token's values in their block; in the last one its last token stands for those past the end
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    row_at[v] = (size_t)(4 * g + v) * a.batch * C;
+    last_at[v] = (size_t)min(4 * g + v, n - 1 - last * NB) * a.batch * C;
+  }
+  struct Set {
+    f32x4 k[RB], q[RB], kt[RB], t, gamma, end, v;
+  };
+  auto load = [&](Set &x, int blk) {
+    blk = min(blk, w.blocks - 1);  // past the end: not used
+    const f32x4 *kp = qk + (size_t)blk * 12 * DP, *cf = coef + (size_t)blk * (NCF / 4);
+    const float *rows = raw + (size_t)min(blk, last) * NB * a.batch * C;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) x.v[v] = rows[blk < last ? row_at[v] : last_at[v]];
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+      x.k[r] = kp[r * 64];
+      x.q[r] = kp[4 * DP + r * 64];
+      x.kt[r] = kp[8 * DP + r * 64];
+    }
+    x.t = cf[(CF_T + c * NB) / 4 + g];
+    x.gamma = cf[CF_GAMMA / 4 + g];
+    x.end = cf[CF_END / 4 + g];
+  };
+  f32x4 S[RB];
+#pragma unroll
+  for (int r = 0; r < RB; ++r)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int row = row0 + r * 16 + 4 * g + v;
+      const float x = st[(size_t)min(row, D - 1) * V + min(col, V - 1)];
+      S[r][v] = row < D && col < V ? x : 0.0f;
+    }
+  // the wave's part of a product with the state; sums of four, then those of sums: no more roundings in a row than a sum over lanes has
+  auto times_state = [&](const f32x4 (&m)[RB]) {
+    f32x4 p[RB][4];
+#pragma unroll
+    for (int r = 0; r < RB; ++r)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) p[r][v] = __builtin_amdgcn_mfma_f32_16x16x4f32(m[r][v], S[r][v], f32x4{}, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < RB; ++r) p[r][0] = (p[r][0] + p[r][1]) + (p[r][2] + p[r][3]);
+    if constexpr (RB == 1) return p[0][0];
+    if constexpr (RB == 2) return p[0][0] + p[1][0];
+    if constexpr (RB == 3) return (p[0][0] + p[1][0]) + p[2][0];
+    if constexpr (RB == 4) return (p[0][0] + p[1][0]) + (p[2][0] + p[3][0]);
+  };
+  auto step = [&](Set &x, int blk) {
+    sk_s[blk & 1][wave][lane] = times_state(x.k);
+    kx_lds_barrier();  // the waves' sums; and everybody is done with the block before the last
+    const f32x4 sk = (sk_s[blk & 1][0][lane] + sk_s[blk & 1][1][lane]) + (sk_s[blk & 1][2][lane] + sk_s[blk & 1][3][lane]);
+    sq_s[blk & 1][wave][lane] = times_state(x.q);
+    f32x4 e;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) e[v] = __builtin_fmaf(-x.gamma[v], sk[v], x.v[v]);
+    const f32x4 u = lower(x.t, e);
+    if (wave == 0) u_s[blk & 1][lane] = u;
+    const float all = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, (float)x.gamma[3]), 48));  // G(16)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) e[v] = u[v] * x.end[v];
+    f32x4 p[RB];  // the block's sums first: the state is rounded once a block
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+      for (int r = 0; r < RB; ++r) p[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.kt[r][v], e[v], v ? p[r] : f32x4{}, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < RB; ++r)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) S[r][v] = __builtin_fmaf(all, S[r][v], p[r][v]);
+    load(x, blk + SETS);
+  };
+  Set x[SETS];
+#pragma unroll
+  for (int y = 0; y < SETS; ++y) load(x[y], y);
+  int blk = 0;
+  do {  // whole turns of the sets: the loads in flight stay in the registers that they arrive in
+#pragma unroll
+    for (int y = 0; y < SETS; ++y) step(x[y], blk + y);
+    blk += SETS;
+  } while (blk < w.blocks);
+  kx_lds_barrier();
+#pragma unroll
+  for (int r = 0; r < RB; ++r)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int row = row0 + r * 16 + 4 * g + v;
+      if (row < D && col < V) st[(size_t)row * V + col] = S[r][v];
+    }
 }
 
 }  // namespace
@@ -361,14 +404,14 @@ int kx_delta_launch(const KxDeltaArgs &a, hipStream_t st) {
   KX_REQUIRE(a.work, "delta rule: no scratch");
   const int rc = kx_conv_launch(conv_of(a), work_of(a).raw, st);
   if (rc) return rc;
-  hipLaunchKernelGGL(delta_unit_k, dim3(kx_cdiv(work_of(a).padded * s.kv_heads, 4), a.batch), dim3(256), 0, st, a);
+  const int row = kx_delta_row(s);
+  hipLaunchKernelGGL(delta_block_k, dim3(work_of(a).blocks, s.kv_heads, a.batch), dim3(256), block_lds(row), st, a);
   KX_LAUNCH_CHECK();
-#define KX_SCAN(LPC) hipLaunchKernelGGL(delta_scan_k<LPC>, dim3(kx_cdiv(s.vdim, 256 / LPC), s.heads, a.batch), dim3(256), 0, st, a)
-  if (s.dim <= 32) KX_SCAN(4);
-  else if (s.dim <= 64) KX_SCAN(8);
-  else if (s.dim <= 128) KX_SCAN(16);
-  else KX_SCAN(32);
-#undef KX_SCAN
+  const dim3 grid(s.heads, kx_cdiv(s.vdim, 16), a.batch);
+  if (row == 64) hipLaunchKernelGGL(delta_scan_k<1>, grid, dim3(320), 0, st, a);
+  else if (row == 128) hipLaunchKernelGGL(delta_scan_k<2>, grid, dim3(320), 0, st, a);
+  else if (row == 192) hipLaunchKernelGGL(delta_scan_k<3>, grid, dim3(320), 0, st, a);
+  else hipLaunchKernelGGL(delta_scan_k<4>, grid, dim3(320), 0, st, a);
   KX_LAUNCH_CHECK();
   return KX_OK;
 }

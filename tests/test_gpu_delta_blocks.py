@@ -1,0 +1,39 @@
+"""The delta rule where its blocks of 16 tokens, its rows of 64 and its slices of 16 columns end."""
+import numpy as np
+import pytest
+
+from kxt import say
+from test_gpu_kagalorn import Delta, rel
+
+pytestmark = pytest.mark.gpu
+# keys have unit length, so a sum of 256 products is off by at most 256 * 2^-24 of its terms, in what a token takes
+# out of the state and again in what it reads
+TOLERANCE = 2 * 256 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("shape", [(2, 1, 16, 15), (3, 1, 64, 16), (2, 2, 65, 17), (4, 2, 128, 33), (1, 1, 192, 1), (2, 1, 256, 16)], ids=lambda c: "-".join(map(str, c)))
+def test_delta_blocks(kxlib, shape):
+    d = Delta(kxlib, *shape, 3, batch=2)
+    for n in (2, 15, 16, 17, 32, 33, 49):
+        say(f"delta blocks {shape} {n}")
+        proj = np.random.default_rng(n).standard_normal((2, n + 5, d.cols[-1])).astype(np.float32)
+        got = d.run(proj, [n, 5], 2)
+        for b in range(2):
+            assert rel(got[b], d.oracle(proj[b])) < TOLERANCE, (n, b)
+    d.close()
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_delta_value_that_is_not_finite_reaches_no_token_before_it(kxlib, bad):
+    heads, kv, dim, vdim = 2, 1, 40, 20
+    d = Delta(kxlib, heads, kv, dim, vdim, 1)
+    proj = np.random.default_rng(1).standard_normal((1, 45, d.cols[-1])).astype(np.float32)
+    d.conv[:] = np.abs(d.conv)
+    d.d[0].upload(d.conv)
+    clean = d.run(proj, [45])[0].reshape(45, heads, vdim)
+    proj[0, 21, d.cols[2] + vdim + 3] = bad                       # head 1, column 3
+    got = d.run(proj, [45])[0].reshape(45, heads, vdim)
+    hit = np.zeros(got.shape, bool)
+    hit[21:, 1, 3] = True
+    assert np.array_equal(got[~hit], clean[~hit]) and not np.isfinite(got[hit]).any()
+    d.close()
