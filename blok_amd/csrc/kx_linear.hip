@@ -349,7 +349,7 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) lin_gemm_k(Kx
 // ---- bf16 products of few tokens ----
 // Bound by the stream of the matrix.  A workgroup of 8 waves owns 64 rows (with GLU rows a block of gate and its block of up),
 // all tokens, and one of `splits` parts of the columns, so that a matrix of few rows still has a workgroup or two for every CU:
-// a tile per 128 rows alone is 16 workgroups for 2048 rows (90 us for 8 tokens against 2048 x 10240; 14 us here).  The columns
+// a tile per 128 rows alone is 16 workgroups for 2048 rows (90 us for 8 tokens against 2048 x 10240; 11 us here).  The columns
 // are walked in blocks of 128, each two halves of 64 in the layout of the tiles above, through a ring of NS blocks; wave w
 // multiplies 16 columns of each half for row block w % 2, so that four waves hold sums of the same outputs, which meet in LDS.
 // With several parts the sums go to memory and the workgroup that arrives last (kx_arrive.h) adds the parts in their order,

@@ -6,7 +6,7 @@
 // reads every cached row once per position of the step; expanded they are 2 x 320, and 128 positions of a step share each
 // tile of keys.  What it costs is one product of the context with W_UK and W_UV per step, 2 x 512 x (128 + 128) per cached
 // row and head, as much as the attention of about 100 positions saves; hence the rule in kx_mla_prompt_fits.
-// 64 heads, 2048 + 952 positions of one sequence: 3.2 ms a layer in the decode form (with absorb, merge and W_UV), 0.8 ms here.
+// 64 heads, 2048 + 952 positions of one sequence: 3.25 ms a layer in the decode form (with absorb, merge and W_UV), 0.94 ms here.
 #include <algorithm>
 #include "kx_attn_parts.h"
 #include "kx_common.h"
@@ -37,9 +37,10 @@ __global__ void __launch_bounds__(256) prompt_prep_k(KxMlaPromptArgs a) {
   }
 }
 
-// the shared part of the keys (RoPE'd, 16-byte pieces) behind each head's own
+// the shared part of the keys (RoPE'd, 16-byte pieces) behind each head's own; zeros behind the last value, which meet weights of
+// zero: what an earlier context left there may not be finite
 __global__ void __launch_bounds__(256) share_key_k(const uint16_t *__restrict__ cache, size_t seq_stride, int row, int kv_rank, int pieces, uint16_t *__restrict__ k, int n,
-                                                   int heads, int cap, int ld, int at) {
+                                                   int heads, int cap, int ld, int at, uint16_t *__restrict__ v, int dv) {
   const size_t total = (size_t)n * heads * pieces;
   const int b = blockIdx.y;
   for (size_t x = (size_t)blockIdx.x * 256 + threadIdx.x; x < total; x += (size_t)gridDim.x * 256) {
@@ -48,6 +49,9 @@ __global__ void __launch_bounds__(256) share_key_k(const uint16_t *__restrict__ 
     const int t = (int)(y % n), h = (int)(y / n);
     *(uint4 *)(k + ((size_t)(b * heads + h) * cap + t) * ld + at + p * 8) = *(const uint4 *)(cache + b * seq_stride + (size_t)t * row + kv_rank + p * 8);
   }
+  const int tail = (cap - n) * (dv / 8);
+  for (int x = blockIdx.x * 256 + threadIdx.x; x < tail * heads; x += gridDim.x * 256)
+    *(uint4 *)(v + ((size_t)(b * heads + x / tail) * cap + n) * dv + (size_t)(x % tail) * 8) = uint4{0, 0, 0, 0};
 }
 
 }  // namespace
@@ -92,7 +96,7 @@ int kx_mla_prompt_launch(const kx_config *c, const KxMlaPromptArgs &a, const KxD
       if (rc) return rc;
       const size_t pieces = (size_t)n * nh * (a.rope / 8);
       hipLaunchKernelGGL(share_key_k, dim3((unsigned)std::min<size_t>((pieces + 255) / 256, 4096), nb), dim3(256), 0, st, rows, a.seq_stride, a.kv_rank + a.rope, a.kv_rank,
-                         a.rope / 8, k, n, nh, cap, dk, a.nope);
+                         a.rope / 8, k, n, nh, cap, dk, a.nope, v, dv);
       KX_LAUNCH_CHECK();
       KxWindowArgs w;
       w.s.heads = w.s.kv_heads = nh; w.s.dim = dk; w.s.vdim = dv; w.s.scale = rs * ms * ms;

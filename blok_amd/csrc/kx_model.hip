@@ -569,7 +569,6 @@ static int model_new(const kx_config *cfg, const char *who, KimiModel **out) {
       m->expand = nullptr;
     } else {
       m->expand_bytes = want;
-      KX_HIP(hipMemsetAsync(m->expand, 0, want, m->st));  // what lies behind a context's last position is multiplied by zeros
     }
   }
   *out = m;

@@ -7,7 +7,7 @@
 // combine (:868,:871), the shared expert (:872-875) and the residual add (:877) --
 // with the tokens of each expert gathered into one GEMM.
 //
-// The only place MFMA is used.  Per workgroup (8 waves): one expert, 256 weight rows, the
+// Per workgroup (8 waves): one expert, 256 weight rows, the
 // expert's tokens in tiles of 128.  Wave w owns weight rows 32 w .. +31 for all 128 tokens
 // (fp32 accumulators of v_mfma_f32_32x32x16_bf16).  Per K step of 64 columns:
 //  * INT4 weights reach the lanes through LDS as packed words: for every two K steps the

@@ -6,8 +6,8 @@
 //
 // A GEMV kernel streams the weights once per block of four tokens and is bound by its fma count from about 16 tokens
 // on (every weight meets every token on the VALU), and
-// the grouped prefill GEMM of kx_prefill.hip, built for 128-token tiles of many experts, leaves most of the chip idle
-// on one 32-token tile.  Here a workgroup of 8 waves owns 32 weight rows and all (up to 32) tokens, the eight waves
+// the prefill GEMM of kx_dense_gemm.hip, built for tiles of 64 tokens and more, leaves most of the chip idle on one of
+// 32.  Here a workgroup of 8 waves owns 32 weight rows and all (up to 32) tokens, the eight waves
 // split the columns, and their partial 32 x 32 tiles (v_mfma_f32_32x32x16_bf16) are summed through LDS in wave
 // order before the epilogue.
 //
