@@ -224,7 +224,7 @@ __global__ void __launch_bounds__(256) delta_block_k(KxDeltaArgs a) {
 #pragma unroll
         for (int m = 0; m < y; ++m) v = __builtin_fma(-L[y][m], t[m], v);
         t[y] = v;
-        cf[CF_T + y * NB + tid] = (float)(v * beta_s[tid]);
+        cf[CF_T + y * NB + tid] = y < tid ? 0.0f : (float)(v * beta_s[tid]);  // nothing of a token in the rows before it, whatever its numbers are
       }
     }
   }

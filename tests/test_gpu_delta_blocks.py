@@ -37,3 +37,31 @@ def test_delta_value_that_is_not_finite_reaches_no_token_before_it(kxlib, bad):
     hit[21:, 1, 3] = True
     assert np.array_equal(got[~hit], clean[~hit]) and not np.isfinite(got[hit]).any()
     d.close()
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf])
+@pytest.mark.parametrize("at", [0, 16, 21, 31, 44])
+def test_delta_token_that_is_not_finite_reaches_no_token_before_it(kxlib, at, bad):
+    """The query, the key, a value, the step size, the decay or the whole row of a token at the first, a middle or the last place
+    of a block or of the step; with more heads than key heads, so that a key head's neighbour has to stay as it is too."""
+    heads, kv, dim, vdim = 4, 2, 40, 20
+    d = Delta(kxlib, heads, kv, dim, vdim, 1)
+    clean = np.random.default_rng(2).standard_normal((1, 45, d.cols[-1])).astype(np.float32)
+    want = d.run(clean, [45])[0].reshape(45, heads, vdim)
+    assert np.isfinite(want).all()
+    c = [int(x) for x in d.cols]
+    # columns of a token, and the heads that read them
+    cases = {"query": (c[0] + 3, [0, 1]), "key": (c[1] + dim + 5, [2, 3]), "value": (c[2] + vdim + 3, [1]), "step size": (c[3] + 2, [2]), "decay": (c[4] + 3, [3]),
+             "row": (slice(None), [0, 1, 2, 3])}
+    for name, (col, hit) in cases.items():
+        say(f"delta {name} {bad} at {at}")
+        proj = clean.copy()
+        proj[0, at, col] = bad
+        got = d.run(proj, [45])[0].reshape(45, heads, vdim)
+        others = [h for h in range(heads) if h not in hit]
+        assert np.array_equal(got[:at], want[:at]) and np.array_equal(got[:, others], want[:, others]), name
+        if name in ("query", "key", "value", "row"):  # the sigmoid and the decay are finite for every number and for none
+            assert not np.isfinite(got[at, hit]).all(), name
+        if name == "query":  # is read by its own token alone
+            assert np.array_equal(got[at + 1:], want[at + 1:]), name
+    d.close()
