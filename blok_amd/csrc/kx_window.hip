@@ -10,6 +10,7 @@
 // blocks that complete, and then win_flash_k (bf16; matrix cores) or win_partial_k<T, false> + win_merge_k (f32) attend.
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 #include "kx_common.h"
 #include "kx_rows.h"
 #include "kx_window.h"
@@ -279,6 +280,11 @@ __global__ void __launch_bounds__(MERGE_THREADS) win_merge_k(KxWindowArgs a, int
 // h = 0 and 4-7, 12-15 for h = 1.  The 8-key pieces of a V^T row are xor-swizzled by the row, which spreads the
 // transposing writes over the banks.  The next tile's rows are on their way to registers while a tile is multiplied;
 // scores are in units of log 2, so that a weight is one exp2.
+// A key that a query does not see has a weight of zero, and its value is multiplied all the same; zero times a value that is not
+// finite would make the query's output follow a position behind it, or one that its window has left.  So a workgroup whose sums
+// are not all finite makes them once more: in tiles that not every query sees as a whole, such values are replaced by zeros, and
+// added at the end by the queries that see them.  This costs a launch 0 to 1 % (64 heads of 192, 2048 positions behind 952: 612 us, 618
+// with it); looking for such values as each tile is written to LDS took 857.
 constexpr int FQ = 128, FK = 64;
 __device__ __forceinline__ int vt_piece(int d, int piece) { return (piece ^ (d >> 1) ^ (d >> 4)) & 7; }
 
@@ -286,6 +292,7 @@ template <int ND, int NV>  // 32-column blocks of a key and of a value
 __global__ void __launch_bounds__(256) win_flash_k(KxWindowArgs a) {
   constexpr int KSTR = ND * 32 + 8, VSTR = FK + 8;
   extern __shared__ __attribute__((aligned(16))) uint16_t fl_lds[];
+  __shared__ int odd_s;                 // a sum that is not finite
   uint16_t *ks = fl_lds;                // [FK][KSTR]
   uint16_t *vt = ks + FK * KSTR;        // [NV * 32][VSTR]
   const KxWindowSpec &s = a.s;
@@ -307,11 +314,7 @@ __global__ void __launch_bounds__(256) win_flash_k(KxWindowArgs a) {
     for (int kk = 0; kk < ND * 2; ++kk) q[kk] = kk * 16 < c.dp ? *(const bf16x8 *)(qr + kk * 16 + hh * 8) : bf16x8{};
   }
   f32x16 o[NV];
-#pragma unroll
-  for (int j = 0; j < NV; ++j)
-#pragma unroll
-    for (int v = 0; v < 16; ++v) o[j][v] = 0.0f;
-  float m = s.sink ? (a.sinks ? a.sinks[h] * 1.44269504088896341f : 0.0f) : NEG_INF, z = s.sink && hh == 0 ? 1.0f : 0.0f;  // z: this lane's half of the keys
+  float m, z;  // z: of this lane's half of the keys
   const float scale2 = s.scale * 1.44269504088896341f;
 
   // tiles: the blocks the last query sees, then the positions from the first query's window on
@@ -322,6 +325,9 @@ __global__ void __launch_bounds__(256) win_flash_k(KxWindowArgs a) {
   const int q1 = __builtin_amdgcn_readfirstlane(a.pos + min(i0 + wave * 32 + 31, a.positions - 1));
   const int nb0 = seen_blocks(q0, s.size, s.pool), nb1 = seen_blocks(q1, s.size, s.pool), lo0 = window_lo(q0, s.size), lo1 = window_lo(q1, s.size);
   auto first_key = [&](int t) { return t < tb ? t * FK : j0 + (t - tb) * FK; };
+  auto seen_by_all = [&](int t) {
+    return t < tb ? (t + 1) * FK <= seen_blocks(p_first, s.size, s.pool) : first_key(t) >= window_lo(p_last, s.size) && first_key(t) + FK - 1 <= p_first;
+  };
   constexpr int VT = (FK / 8) * NV * 16, VN = (VT + 255) / 256;  // V is taken by 8 keys x 2 columns
   u32x4 kreg[ND];
   uint32_t vreg[VN][8];
@@ -344,7 +350,12 @@ __global__ void __launch_bounds__(256) win_flash_k(KxWindowArgs a) {
       for (int r = 0; r < 8; ++r) vreg[y][r] = *(const uint32_t *)(vr + (size_t)min(oct * 8 + r, last) * c.vp + d);
     }
   };
-  auto put = [&]() {
+  auto put = [&](bool as_it_is) {
+    if (!as_it_is)
+#pragma unroll
+      for (int y = 0; y < VN; ++y)
+#pragma unroll
+        for (int r = 0; r < 8; ++r) vreg[y][r] &= ~(((((vreg[y][r] & 0x7f807f80u) + 0x00800080u) & 0x80008000u) >> 15) * 0xffffu);  // an exponent of all ones carries into the sign's place
 #pragma unroll
     for (int y = 0; y < ND; ++y) {
       const int x = y * 256 + tid, r = x / (ND * 4), d = (x - r * (ND * 4)) * 8;
@@ -364,102 +375,142 @@ __global__ void __launch_bounds__(256) win_flash_k(KxWindowArgs a) {
       }
     }
   };
-  fetch(0);
-  for (int t = 0; t < tiles; ++t) {
-    const bool pooled = t < tb;
-    const int k0 = first_key(t);
-    __syncthreads();  // the tile before has been multiplied
-    put();
-    __syncthreads();
-    fetch(min(t + 1, tiles - 1));
-    const bool none = pooled ? k0 >= nb1 : k0 > q1 || k0 + FK - 1 < lo0;
-    const bool all = pooled ? k0 + FK <= nb0 : k0 >= lo1 && k0 + FK - 1 <= q0;
-    if (none) continue;
-    f32x16 sc[2];
+  auto attend = [&](auto replace) {
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
+    for (int j = 0; j < NV; ++j)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) sc[kt][v] = 0.0f;
+      for (int v = 0; v < 16; ++v) o[j][v] = 0.0f;
+    m = s.sink ? (a.sinks ? a.sinks[h] * 1.44269504088896341f : 0.0f) : NEG_INF;
+    z = s.sink && hh == 0 ? 1.0f : 0.0f;
+    fetch(0);
+    for (int t = 0; t < tiles; ++t) {
+      const bool pooled = t < tb;
+      const int k0 = first_key(t);
+      __syncthreads();  // the tile before has been multiplied
+      put(!decltype(replace)::value || seen_by_all(t));
+      __syncthreads();
+      fetch(min(t + 1, tiles - 1));
+      const bool none = pooled ? k0 >= nb1 : k0 > q1 || k0 + FK - 1 < lo0;
+      const bool all = pooled ? k0 + FK <= nb0 : k0 >= lo1 && k0 + FK - 1 <= q0;
+      if (none) continue;
+      f32x16 sc[2];
 #pragma unroll
-      for (int kk = 0; kk < ND * 2; ++kk) {
-        const bf16x8 kf = *(const bf16x8 *)(ks + (kt * 32 + lq) * KSTR + kk * 16 + hh * 8);
-        sc[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, q[kk], sc[kt], 0, 0, 0);
+      for (int kt = 0; kt < 2; ++kt) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) sc[kt][v] = 0.0f;
+#pragma unroll
+        for (int kk = 0; kk < ND * 2; ++kk) {
+          const bf16x8 kf = *(const bf16x8 *)(ks + (kt * 32 + lq) * KSTR + kk * 16 + hh * 8);
+          sc[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, q[kk], sc[kt], 0, 0, 0);
+        }
       }
-    }
-    const int from = (pooled ? 0 : lo) - k0 - 4 * hh, to = (pooled ? nb - 1 : p) - k0 - 4 * hh;  // the keys this lane's query sees, from its first one on
+      const int from = (pooled ? 0 : lo) - k0 - 4 * hh, to = (pooled ? nb - 1 : p) - k0 - 4 * hh;  // the keys this lane's query sees, from its first one on
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
+      for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) sc[kt][v] *= scale2;
-    if (!all) {
+        for (int v = 0; v < 16; ++v) sc[kt][v] *= scale2;
+      if (!all) {
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) {
+            const int e = kt * 32 + 8 * (v >> 2) + (v & 3);
+            sc[kt][v] = ((e < from) | (e > to)) ? NEG_INF : sc[kt][v];
+          }
+      }
+      float tm = NEG_INF;
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) tm = fmaxf(tm, sc[kt][v]);
+      tm = fmaxf(tm, __shfl_xor(tm, 32));
+      if (__any(tm > m)) {
+        const float m1 = fmaxf(m, tm), al = m == NEG_INF ? 0.0f : __builtin_amdgcn_exp2f(m - m1);
+        m = m1;
+        z *= al;
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) o[j][v] *= al;
+      }
+      const float mm = m == NEG_INF ? 0.0f : m;  // nothing seen so far
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-          const int e = kt * 32 + 8 * (v >> 2) + (v & 3);
-          sc[kt][v] = ((e < from) | (e > to)) ? NEG_INF : sc[kt][v];
+          sc[kt][v] = __builtin_amdgcn_exp2f(sc[kt][v] - mm);
+          z += sc[kt][v];
         }
+#pragma unroll
+      for (int ss = 0; ss < FK / 16; ++ss) {
+        const f32x16 &f = sc[ss >> 1];
+        const int v0 = (ss & 1) * 8;
+        uint32_t pw[4];
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+          const f32x2 two = {f[v0 + 2 * y], f[v0 + 2 * y + 1]};
+          pw[y] = __builtin_bit_cast(uint32_t, __builtin_convertvector(two, bf16x2));
+        }
+        const bf16x8 pf = __builtin_bit_cast(bf16x8, make_uint4(pw[0], pw[1], pw[2], pw[3]));
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+          const int d = j * 32 + lq;
+          const bf16x8 vf = *(const bf16x8 *)(vt + d * VSTR + vt_piece(d, ss * 2 + hh) * 8);
+          o[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf, o[j], 0, 0, 0);
+        }
+      }
     }
-    float tm = NEG_INF;
+  };
+  auto store = [&]() {
+    z += __shfl_xor(z, 32);
+    if (!live) return;
+    const float inv = 1.0f / z;
+    uint16_t *out = (uint16_t *)a.out + (size_t)tok * a.out_ld + h * s.vdim;
+    const float *gate = a.g_off >= 0 ? a.proj + (size_t)tok * a.proj_ld + a.g_off + h * s.vdim : nullptr;
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
+    for (int j = 0; j < NV; ++j) {
+      float gt[16];
 #pragma unroll
-      for (int v = 0; v < 16; ++v) tm = fmaxf(tm, sc[kt][v]);
-    tm = fmaxf(tm, __shfl_xor(tm, 32));
-    if (__any(tm > m)) {
-      const float m1 = fmaxf(m, tm), al = m == NEG_INF ? 0.0f : __builtin_amdgcn_exp2f(m - m1);
-      m = m1;
-      z *= al;
+      for (int v = 0; v < 16; ++v) gt[v] = gate ? gate[min(j * 32 + 8 * (v >> 2) + 4 * hh + (v & 3), s.vdim - 1)] : 0.0f;
 #pragma unroll
-      for (int j = 0; j < NV; ++j)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) o[j][v] *= al;
-    }
-    const float mm = m == NEG_INF ? 0.0f : m;  // nothing seen so far
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
+      for (int v = 0; v < 16; ++v) asm volatile("" : "+v"(gt[v]));  // all sixteen are asked for before the first is used
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
-        sc[kt][v] = __builtin_amdgcn_exp2f(sc[kt][v] - mm);
-        z += sc[kt][v];
-      }
-#pragma unroll
-    for (int ss = 0; ss < FK / 16; ++ss) {
-      const f32x16 &f = sc[ss >> 1];
-      const int v0 = (ss & 1) * 8;
-      uint32_t pw[4];
-#pragma unroll
-      for (int y = 0; y < 4; ++y) {
-        const f32x2 two = {f[v0 + 2 * y], f[v0 + 2 * y + 1]};
-        pw[y] = __builtin_bit_cast(uint32_t, __builtin_convertvector(two, bf16x2));
-      }
-      const bf16x8 pf = __builtin_bit_cast(bf16x8, make_uint4(pw[0], pw[1], pw[2], pw[3]));
-#pragma unroll
-      for (int j = 0; j < NV; ++j) {
-        const int d = j * 32 + lq;
-        const bf16x8 vf = *(const bf16x8 *)(vt + d * VSTR + vt_piece(d, ss * 2 + hh) * 8);
-        o[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf, o[j], 0, 0, 0);
+        const int d = j * 32 + 8 * (v >> 2) + 4 * hh + (v & 3);
+        const float y = o[j][v] * inv * (gate ? kxr::sigmoid_for<uint16_t>(gt[v]) : 1.0f);
+        if (d < s.vdim) out[d] = kx_bf16_rne(y);
       }
     }
-  }
-  z += __shfl_xor(z, 32);
-  if (!live) return;
-  const float inv = 1.0f / z;
-  uint16_t *out = (uint16_t *)a.out + (size_t)tok * a.out_ld + h * s.vdim;
-  const float *gate = a.g_off >= 0 ? a.proj + (size_t)tok * a.proj_ld + a.g_off + h * s.vdim : nullptr;
+  };
+  if (tid == 0) odd_s = 0;
+  attend(std::false_type{});
+  store();
+  float odd[4] = {};  // zero, unless a sum is not finite
 #pragma unroll
-  for (int j = 0; j < NV; ++j) {
-    float gt[16];
+  for (int j = 0; j < NV; ++j)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) gt[v] = gate ? gate[min(j * 32 + 8 * (v >> 2) + 4 * hh + (v & 3), s.vdim - 1)] : 0.0f;
+    for (int v = 0; v < 16; ++v) odd[v & 3] = __builtin_fmaf(o[j][v], 0.0f, odd[v & 3]);
+  if ((odd[0] + odd[1]) + (odd[2] + odd[3]) != 0.0f) odd_s = 1;
+  __syncthreads();
+  if (__builtin_expect(odd_s, 0)) {
+    attend(std::true_type{});
 #pragma unroll
-    for (int v = 0; v < 16; ++v) asm volatile("" : "+v"(gt[v]));  // all sixteen are asked for before the first is used
+    for (int j = 0; j < NV; ++j)
+#pragma unroll 1
+      for (int t = 0; t < tiles; ++t) {
+        if (seen_by_all(t)) continue;
+        const bool pooled = t < tb;
+        const int k0 = first_key(t), e1 = min(FK - 1, (pooled ? nb - 1 : p) - k0);
+        const uint16_t *vr = pooled ? pvc + (size_t)k0 * c.vp : vc + (size_t)(k0 % c.cap) * c.vp;
+#pragma unroll 1
+        for (int e = max(0, (pooled ? 0 : lo) - k0); e <= e1; ++e)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int d = j * 32 + 8 * (v >> 2) + 4 * hh + (v & 3);
-      const float y = o[j][v] * inv * (gate ? kxr::sigmoid_for<uint16_t>(gt[v]) : 1.0f);
-      if (d < s.vdim) out[d] = kx_bf16_rne(y);
-    }
+          for (int v = 0; v < 16; ++v) {
+            const float x = kx_bf16_f32(vr[(size_t)e * c.vp + min(j * 32 + 8 * (v >> 2) + 4 * hh + (v & 3), c.vp - 1)]);
+            o[j][v] = __builtin_isfinite(x) ? o[j][v] : o[j][v] + x;
+          }
+      }
+    store();
   }
 }
 
