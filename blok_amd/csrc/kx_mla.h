@@ -40,14 +40,12 @@ struct KxMlaPromptArgs {
   uint16_t *q;                    // [positions * seqs][heads][nope + rope]; the rope part is rotated in place
   const uint16_t *kva, *w_kv_ln, *rope_row, *kvb;
   uint16_t *cache, *out;          // out [positions * seqs][heads * v_head]
-  void *expand;                   // room for expanded keys and values; what is in it is finite
+  void *expand;                   // room for expanded keys and values; anything may be in it
   size_t expand_bytes, seq_stride;
   int heads, nope, rope, kv_rank, kva_stride, seqs, positions, pos;
   float eps;
 };
-constexpr size_t KX_MLA_EXPAND_BYTES = (size_t)1 << 30;
-size_t kx_mla_prompt_bytes(const kx_config *c);
-// whether a step of `positions` positions per sequence takes this form
+// whether a step of `positions` positions per sequence takes this form; expand_bytes: the room for keys and values
 bool kx_mla_prompt_fits(const kx_config *c, int positions, size_t expand_bytes);
 // split: scratch of the expanding product (KxDenseArgs::part and what follows)
 int kx_mla_prompt_launch(const kx_config *c, const KxMlaPromptArgs &a, const KxDenseArgs &split, hipStream_t st);

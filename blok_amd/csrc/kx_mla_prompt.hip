@@ -38,7 +38,7 @@ __global__ void __launch_bounds__(256) prompt_prep_k(KxMlaPromptArgs a) {
 }
 
 // the shared part of the keys (RoPE'd, 16-byte pieces) behind each head's own; zeros behind the last value, which meet weights of
-// zero: what an earlier context left there may not be finite
+// zero: what lies there may not be finite, and the attention would make its sums twice
 __global__ void __launch_bounds__(256) share_key_k(const uint16_t *__restrict__ cache, size_t seq_stride, int row, int kv_rank, int pieces, uint16_t *__restrict__ k, int n,
                                                    int heads, int cap, int ld, int at, uint16_t *__restrict__ v, int dv) {
   const size_t total = (size_t)n * heads * pieces;
@@ -56,13 +56,6 @@ __global__ void __launch_bounds__(256) share_key_k(const uint16_t *__restrict__ 
 
 }  // namespace
 
-// Room for the keys and values of one head at least; more heads and sequences at once as far as KX_MLA_EXPAND_BYTES goes.
-size_t kx_mla_prompt_bytes(const kx_config *c) {
-  const size_t row = (size_t)(c->qk_nope + c->qk_rope + c->v_head) * 2, cap = kx_pad(c->max_context, 64);
-  const size_t all = (size_t)c->max_batch * c->heads * cap * row;
-  return all <= KX_MLA_EXPAND_BYTES ? all : std::max<size_t>(KX_MLA_EXPAND_BYTES, cap * row);
-}
-
 bool kx_mla_prompt_fits(const kx_config *c, int positions, size_t expand_bytes) {
   const int half = c->qk_rope / 2;
   if ((c->qk_nope + c->qk_rope) % 32 || c->v_head % 32 || c->qk_nope % 32 || c->qk_nope + c->qk_rope > 256 || c->v_head > 256 || half > 64 || (half & (half - 1)) || c->kv_rank % 128) return false;
@@ -78,7 +71,7 @@ int kx_mla_prompt_launch(const kx_config *c, const KxMlaPromptArgs &a, const KxD
   const size_t head = (size_t)cap * (dk + dv) * 2;  // bytes
   const int most = (int)std::min<size_t>(a.expand_bytes / head, (size_t)a.heads * a.seqs);
   KX_REQUIRE(most > 0, "kx_mla: no room for the keys of %d positions", n);
-  const int hg = std::min(most, a.heads), bg = hg == a.heads ? most / hg : 1;
+  const int hg = kx_cdiv(a.heads, kx_cdiv(a.heads, std::min(most, a.heads))), bg = hg == a.heads ? most / hg : 1;
   float rs, ms;
   kx_softmax_scale(c, &rs, &ms);
   for (int b0 = 0; b0 < a.seqs; b0 += bg)

@@ -85,8 +85,7 @@ struct KimiModel : kx_model {
   int *head_pairs;
   float *split_part;               // partial sums of products that split their columns, and the counters of who has left his
   int *split_arrived;
-  void *expand = nullptr;          // keys and values of a prompt's context, expanded (kx_mla_prompt.hip); where there was memory for it
-  size_t expand_bytes = 0;
+  size_t expand_bytes;             // from qabs to the end of partial: room for expanded keys and values in steps that need neither
   uint32_t fusion = KX_FUSE_ALL;
   int mla_kernel = KX_MLA_AUTO;    // kx_model_set_attention_kernel
   float *route_logits = nullptr;   // routing record (kx_model_set_routing_record): [n_layers][max_batch][experts]
@@ -204,6 +203,7 @@ int layout(const kx_config *c, Plan &p, KimiModel *m) {
   auto *dmid = KX_AT(uint16_t *, BT * inter * 2);
   auto *qabs = KX_AT(float *, BT * (size_t)c->heads * KVA * 4);
   auto *partial = KX_AT(float *, kx_mla_partial_floats(att_entries(c), c->heads, c->kv_rank, c->max_context) * 4);
+  const size_t expand_bytes = base + p.total - (char *)qabs;  // the two are neighbours
   auto *logits = KX_AT(float *, B * V * 4);
   auto *argmax_scratch = KX_AT(float *, KX_ARGMAX_SCRATCH_FLOATS(B) * 4);
   auto *ids = KX_AT(uint32_t *, (size_t)c->max_context * B * 4);
@@ -223,7 +223,7 @@ int layout(const kx_config *c, Plan &p, KimiModel *m) {
     m->x = x; m->n = n; m->qkv = qkv; m->qa = qa; m->q = q; m->o_lat = o_lat; m->att = att; m->dmid = dmid;
     m->qabs = qabs; m->partial = partial; m->logits = logits; m->argmax_scratch = argmax_scratch; m->ids = ids; m->next = next; m->history = history;
     m->head_count = head_count; m->hand_err = hand_err; m->front_hand = front_hand; m->back_hand = back_hand; m->head_work = head_work; m->head_pairs = head_pairs;
-    m->split_part = split_part; m->split_arrived = split_arrived;
+    m->split_part = split_part; m->split_arrived = split_arrived; m->expand_bytes = expand_bytes;
   }
   return KX_OK;
 }
@@ -312,7 +312,7 @@ int KimiModel::step(const uint32_t *d_ids, bool sample, int C) {
   const bool mm = B >= 5 && !(m->exact & KX_EXACT_PROJECTIONS);
   const int mla_kernel = (m->exact & KX_EXACT_ATTENTION) ? KX_MLA_VALU : m->mla_kernel;
   // a step of several positions attends to expanded keys and values where it is long enough
-  const bool expand = C > 1 && B > 32 && mla_kernel == KX_MLA_AUTO && m->expand && kx_mla_prompt_fits(&c, C, m->expand_bytes);
+  const bool expand = C > 1 && B > 32 && mla_kernel == KX_MLA_AUTO && kx_mla_prompt_fits(&c, C, m->expand_bytes);
   KxDenseArgs split;
   split.part = m->split_part; split.part_floats = KX_DENSE_PART_FLOATS; split.arrived = m->split_arrived; split.arrivals = KX_DENSE_ARRIVALS;
   auto dense = [&](int epi, const KxGemvArgs &g) -> int {
@@ -381,7 +381,7 @@ int KimiModel::step(const uint32_t *d_ids, bool sample, int C) {
     } else if (expand) {
       KxMlaPromptArgs pa = {};
       pa.q = m->q; pa.kva = m->qkv + c.q_rank; pa.w_kv_ln = L.kv_ln; pa.rope_row = rope_row; pa.kvb = L.kvb; pa.cache = L.cache; pa.out = m->att;
-      pa.expand = m->expand; pa.expand_bytes = m->expand_bytes; pa.seq_stride = seq_stride;
+      pa.expand = m->qabs; pa.expand_bytes = m->expand_bytes; pa.seq_stride = seq_stride;
       pa.heads = c.heads; pa.nope = c.qk_nope; pa.rope = c.qk_rope; pa.kv_rank = c.kv_rank; pa.kva_stride = QKV; pa.seqs = NB; pa.positions = C; pa.pos = pos;
       pa.eps = c.rms_eps;
       KX_TRY(kx_mla_prompt_launch(&c, pa, split, st));
@@ -505,7 +505,6 @@ int KimiModel::row_logits(const int *rows, int n_rows, float *d_out) {
 
 KimiModel::~KimiModel() {
   if (moe_ws) kx_moe_workspace_destroy(moe_ws);
-  if (expand) (void)hipFree(expand);
   if (route_logits) (void)hipFree(route_logits);
   if (route_distinct) (void)hipFree(route_distinct);
   if (route_history) (void)hipFree(route_history);
@@ -560,16 +559,6 @@ static int model_new(const kx_config *cfg, const char *who, KimiModel **out) {
     if (rc == KX_ERR_HIP && !kx_last_error()[0]) kx_set_error("%s: HIP resource creation failed", who);
     kx_model_destroy(m);
     return rc;
-  }
-  // Room for a prompt's expanded keys and values, if there is memory to spare; without it prompts attend as decode steps do.
-  const size_t want = kx_mla_prompt_bytes(cfg);
-  if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && want + ((size_t)2 << 30) <= free_b) {
-    if (hipMalloc(&m->expand, want) != hipSuccess) {
-      (void)hipGetLastError();
-      m->expand = nullptr;
-    } else {
-      m->expand_bytes = want;
-    }
   }
   *out = m;
   return KX_OK;

@@ -258,8 +258,6 @@ int kx_mla_decode(const kx_config *cfg, const void *d_cache, size_t seq_stride, 
  * kx_generate    : the loops at :885-890; h_out u32 [batch][n_tokens], h_counts i32 [batch] ids
  *                  emitted per sequence (stops before eos_id unless ignore_eos).              */
 typedef struct kx_model kx_model;
-/* kx_model_bytes: what the arena of such a model takes.  Where it is free when the model is created, up to 1 GiB more (a head's
- * keys and values of the whole context, if those are more) is taken for prompts in long steps; without it they take longer. */
 int kx_model_bytes(const kx_config *cfg, uint64_t *weights, uint64_t *kv_cache, uint64_t *scratch);
 int kx_model_create(const kx_config *cfg, kx_model **model);
 int kx_model_destroy(kx_model *model);

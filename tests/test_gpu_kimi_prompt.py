@@ -1,5 +1,7 @@
 """Prompts of the Kimi-K2 design in long steps on dense layers, against the token-by-token prefill of the same model: the
 tiles of the dense products (short, medium and large ones, columns in parts) and the attention of a step."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -47,7 +49,8 @@ def test_long_steps_against_token_by_token(kxlib, ox, heads, batch, prompt, chun
         assert row_err < 2e-2 and log_err < 3e-2, c
 
 
-@pytest.mark.parametrize("heads, batch, prompt, kernel", [(64, 1, 27000, 2), (60, 40, 750, 1)], ids=["heads in groups", "sequences in groups"])
+@pytest.mark.parametrize("heads, batch, prompt, kernel", [(64, 1, 27000, 2), (60, 40, 750, 1), (64, 1, 62000, 2)],
+                         ids=["all at once", "sequences in groups", "heads in groups"])
 def test_expanded_keys_that_do_not_fit_at_once(kxlib, ox, heads, batch, prompt, kernel):
     """A context whose expanded keys and values take more than their room: fewer heads, or fewer sequences, at a time.
     Against the decode form of the attention in the same steps."""
@@ -63,7 +66,30 @@ def test_expanded_keys_that_do_not_fit_at_once(kxlib, ox, heads, batch, prompt, 
         assert rc == 0, kxlib.kx_last_error()
         got.append((O.bf16_to_f32(np.stack([km.latent(1, b, prompt) for b in range(batch)])).astype(np.float64), km.logits(batch)))
     km.close()
+    assert (got[0][0] != got[1][0]).any(), "the same bits: both runs took the decode form"
     row_err = np.abs(got[1][0] - got[0][0]).max() / np.abs(got[0][0]).max()
     log_err = max(O.max_rel(got[1][1][b], got[0][1][b]) for b in range(batch))
     say(f"heads={heads} batch={batch} prompt={prompt}: cache rows {row_err:.1e}, logits {log_err:.1e}")
     assert row_err < 2e-2 and log_err < 3e-2
+
+
+def _free(lib):
+    free, total = C.c_size_t(), C.c_size_t()
+    assert lib.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def test_a_model_takes_the_memory_that_its_size_is_given_as(kxlib):
+    """Also where a prompt's expanded keys and values would take a gigabyte."""
+    cfg = _config(64, 33, 1000)
+    parts = [C.c_uint64() for _ in range(3)]
+    check(kxlib.kx_model_bytes(C.byref(cfg), *map(C.byref, parts)))
+    KxModel(kxlib, _config(16, 1, 64)).close()                    # what the first model of a process loads
+    before = _free(kxlib)
+    km = KxModel(kxlib, cfg)
+    check(kxlib.kx_model_set_prefill_chunk(km.h, 2048))
+    rc, _, _ = km.generate(O.tokens_u32(33 * 130, 3, 4, cfg.vocab).reshape(33, 130), 1)
+    assert rc == 0, kxlib.kx_last_error()
+    taken = before - _free(kxlib)
+    km.close()
+    assert taken < sum(p.value for p in parts) + (64 << 20)
