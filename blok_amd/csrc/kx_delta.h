@@ -25,7 +25,7 @@ struct KxDeltaArgs {
   float *hist_out = nullptr;      // the same after this step (another buffer)
   int batch = 0, positions = 0;   // token i * batch + b is the i-th new position of sequence b
   float *o = nullptr;             // f32 [tokens][heads * vdim]
-  float *work = nullptr;          // kx_delta_work_floats(s, batch, positions) floats (not used for one position)
+  float *work = nullptr;          // kx_delta_work_floats(s, batch, positions) floats, 16-byte aligned (not used for one position)
 };
 // Tokens go through the state in blocks of KX_DELTA_BLOCK; per token and head there are KX_DELTA_COEF numbers, and per token and
 // key head the key twice and the query, with rows of whole multiples of 64.

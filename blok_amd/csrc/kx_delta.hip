@@ -401,7 +401,7 @@ int kx_delta_launch(const KxDeltaArgs &a, hipStream_t st) {
     KX_LAUNCH_CHECK();
     return KX_OK;
   }
-  KX_REQUIRE(a.work, "delta rule: no scratch");
+  KX_REQUIRE(a.work && (uintptr_t)a.work % 16 == 0, "delta rule: no scratch, or none for pieces of 16 bytes");
   const int rc = kx_conv_launch(conv_of(a), work_of(a).raw, st);
   if (rc) return rc;
   const int row = kx_delta_row(s);

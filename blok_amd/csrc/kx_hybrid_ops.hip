@@ -16,14 +16,6 @@ struct kx_window {
   int max_batch = 0, max_context = 0, max_positions = 0;
   char *mem = nullptr;
 };
-struct kx_delta {
-  KxDeltaArgs a;
-  int max_batch = 0, max_positions = 0, cur = 0;
-  size_t state_bytes = 0, hist_bytes = 0;
-  char *mem = nullptr;
-  float *hist[2] = {nullptr, nullptr};
-};
-
 // device memory of an operator: offsets first, then one zeroed allocation
 struct OpMem {
   char *p = nullptr;
@@ -43,6 +35,13 @@ struct OpMem {
   ~OpMem() {
     if (p) (void)hipFree(p);
   }
+};
+struct kx_delta {
+  KxDeltaArgs a;
+  int max_batch = 0, max_positions = 0, cur = 0;
+  size_t kept = 0;  // bytes of state and inputs at the start of mem
+  float *hist[2] = {nullptr, nullptr};
+  OpMem mem;
 };
 struct kx_ssd {
   KxSsdArgs a;
@@ -143,30 +142,26 @@ extern "C" int kx_delta_create(const kx_delta_config *c, int32_t max_batch, int3
   KxDeltaSpec &s = d->a.s;
   s.heads = c->heads; s.kv_heads = c->kv_heads; s.dim = c->dim; s.vdim = c->vdim; s.taps = c->taps; s.unit_eps = c->unit_eps;
   d->max_batch = max_batch; d->max_positions = max_positions;
-  d->state_bytes = (size_t)max_batch * s.heads * s.dim * s.vdim * 4;
-  d->hist_bytes = (size_t)max_batch * (s.taps - 1) * kx_delta_channels(s) * 4;
-  const size_t total = d->state_bytes + 2 * d->hist_bytes + kx_delta_work_floats(s, max_batch, max_positions) * 4;
-  if (hipMalloc((void **)&d->mem, total) != hipSuccess || hipMemset(d->mem, 0, total) != hipSuccess) {
-    kx_set_error("kx_delta_create: no device memory for %zu bytes", total);
-    kx_delta_destroy(d);
-    return KX_ERR_HIP;
+  const size_t hist = (size_t)max_batch * (s.taps - 1) * kx_delta_channels(s) * 4;
+  const size_t state = d->mem.take((size_t)max_batch * s.heads * s.dim * s.vdim * 4), h0 = d->mem.take(hist), h1 = d->mem.take(hist);
+  d->kept = d->mem.total;
+  const size_t work = d->mem.take(kx_delta_work_floats(s, max_batch, max_positions) * 4);
+  const int rc = d->mem.alloc("kx_delta_create");
+  if (rc) {
+    delete d;
+    return rc;
   }
-  d->a.state = (float *)d->mem;
-  d->hist[0] = (float *)(d->mem + d->state_bytes);
-  d->hist[1] = (float *)(d->mem + d->state_bytes + d->hist_bytes);
-  d->a.work = (float *)(d->mem + d->state_bytes + 2 * d->hist_bytes);
+  d->a.state = (float *)(d->mem.p + state); d->hist[0] = (float *)(d->mem.p + h0); d->hist[1] = (float *)(d->mem.p + h1); d->a.work = (float *)(d->mem.p + work);
   *out = d;
   return KX_OK;
 }
 extern "C" int kx_delta_destroy(kx_delta *d) {
-  if (!d) return KX_OK;
-  if (d->mem) (void)hipFree(d->mem);
   delete d;
   return KX_OK;
 }
 extern "C" int kx_delta_restart(kx_delta *d, void *stream) {
   KX_REQUIRE(d, "kx_delta_restart: null argument");
-  KX_HIP(hipMemsetAsync(d->mem, 0, d->state_bytes + 2 * d->hist_bytes, kx_stream(stream)));
+  KX_HIP(hipMemsetAsync(d->mem.p, 0, d->kept, kx_stream(stream)));
   return KX_OK;
 }
 extern "C" int kx_delta_run(kx_delta *d, const void *d_proj, int32_t proj_ld, int32_t q_off, int32_t k_off, int32_t v_off, int32_t b_off, int32_t a_off,

@@ -23,6 +23,16 @@ def test_delta_blocks(kxlib, shape):
     d.close()
 
 
+@pytest.mark.parametrize("shape", [(1, 1, 3, 1, 2), (3, 1, 5, 7, 4)], ids=lambda c: "-".join(map(str, c)))
+def test_delta_state_that_is_no_multiple_of_16_bytes(kxlib, shape):
+    """The scratch, which is accessed in pieces of 16 bytes, does not begin where the state and the inputs end."""
+    d = Delta(kxlib, *shape)
+    proj = np.random.default_rng(5).standard_normal((1, 40, d.cols[-1])).astype(np.float32)
+    for cuts in ([40], [2, 17, 1, 20]):
+        assert rel(d.run(proj, cuts)[0], d.oracle(proj[0])) < TOLERANCE
+    d.close()
+
+
 @pytest.mark.parametrize("bad", [np.nan, np.inf])
 def test_delta_value_that_is_not_finite_reaches_no_token_before_it(kxlib, bad):
     heads, kv, dim, vdim = 2, 1, 40, 20
