@@ -31,14 +31,9 @@ struct KxDeltaArgs {
 // key head the key twice and the query, with rows of whole multiples of 64.
 constexpr int KX_DELTA_BLOCK = 16, KX_DELTA_COEF = 34;
 __host__ __device__ inline int kx_delta_row(const KxDeltaSpec &s) { return (s.dim + 63) / 64 * 64; }
-// blocks whose numbers a wave holds in registers at a time, and which a step is filled up to: three where the row leaves room for them
-__host__ __device__ inline int kx_delta_sets(const KxDeltaSpec &s) { return s.dim <= 128 ? 3 : 2; }
-__host__ __device__ inline int kx_delta_blocks(const KxDeltaSpec &s, int positions) {
-  const int span = kx_delta_sets(s) * KX_DELTA_BLOCK;
-  return (positions + span - 1) / span * kx_delta_sets(s);
-}
+__host__ __device__ inline int kx_delta_blocks(int positions) { return (positions + KX_DELTA_BLOCK - 1) / KX_DELTA_BLOCK; }
 inline size_t kx_delta_work_floats(const KxDeltaSpec &s, int batch, int positions) {
-  const size_t padded = (size_t)batch * kx_delta_blocks(s, positions) * KX_DELTA_BLOCK;
+  const size_t padded = (size_t)batch * kx_delta_blocks(positions) * KX_DELTA_BLOCK;
   return padded * ((size_t)KX_DELTA_COEF * s.heads + kx_delta_channels(s) + 3 * s.kv_heads * kx_delta_row(s));
 }
 int kx_delta_launch(const KxDeltaArgs &a, hipStream_t st);

@@ -114,7 +114,7 @@ struct Work {
 };
 __host__ __device__ __forceinline__ Work work_of(const KxDeltaArgs &a) {
   Work w;
-  w.blocks = kx_delta_blocks(a.s, a.positions);
+  w.blocks = kx_delta_blocks(a.positions);
   w.coef = a.work;
   w.qk = w.coef + (size_t)a.batch * a.s.heads * w.blocks * NCF;
   w.raw = w.qk + (size_t)a.batch * a.s.kv_heads * w.blocks * 3 * NB * kx_delta_row(a.s);
@@ -141,7 +141,12 @@ __global__ void __launch_bounds__(256) delta_block_k(KxDeltaArgs a) {
   const int blk = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z, n = a.positions, nq = s.kv_heads * D, C = kx_delta_channels(s), ratio = s.heads / s.kv_heads;
   const Work w = work_of(a);
   float *qs = bl_lds, *ks = qs + NB * STR;
-  {
+  // tokens of this block; a wave without any makes zeros, which meet step sizes of zero
+  const int cnt = min(NB, n - blk * NB);
+  const bool any = __builtin_amdgcn_readfirstlane(j) < cnt;
+  if (!any) {
+    for (int d = sl; d < DP; d += 16) qs[j * STR + d] = ks[j * STR + d] = 0.0f;
+  } else {
     const float *row = w.raw + (size_t)(min(blk * NB + j, n - 1) * a.batch + b) * C + kvh * D;
     double qq = 0.0, kk = 0.0;  // the lengths in 64 bits: their error is one of every number of the row
     for (int d0 = sl; d0 < DP; d0 += 64) {
@@ -182,7 +187,7 @@ __global__ void __launch_bounds__(256) delta_block_k(KxDeltaArgs a) {
   }
   const int i = sl;
   f32x4 kk4[4] = {}, kq4[4] = {};  // sixteen partial sums each: short chains, also of roundings
-  for (int d0 = 0; d0 < DP; d0 += 16)
+  for (int d0 = 0; d0 < (any ? DP : 0); d0 += 16)
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
       const int d = d0 + 4 * x;
@@ -261,9 +266,14 @@ __device__ __forceinline__ f32x4 lower(f32x4 m, f32x4 x) {
 // Bound by the chain of a block: 4 RB products for K S, their sums over the waves through LDS and a barrier, 4 products with
 // T, 4 RB with the keys' transpose.  Q S fills the time the exchange takes; a fifth wave makes the read-outs, a block
 // behind the others, which do not wait for it.  The numbers of the next SETS blocks are on their way meanwhile.
-// 2048 tokens of 16 heads of 128 x 128: 155 us, and 20 us for delta_block_k; on the vector ALU, four tokens per dependent step, 316 us
-// and 35 us.  Three sets in flight instead of two, and the slices of a head on one XCD, gave 3 %: it is the chain, not the loads.
-template <int RB>
+// The whole operator, us: 2048 tokens of 16 heads of 128 x 128 175 with two sets, 190 with three, 198 with one (the registers of three
+// leave a CU one workgroup instead of two); on the vector ALU, four tokens per dependent step, 370.  With 32 sequences of 512
+// tokens, where workgroups hide each other's waits, 894 with one set (three workgroups per CU), 1015 with two, 1085 with three;
+// rows of 64, 192 and 256 columns keep two (867, 943 and 1469 of 32 sequences against 981, 1105 and 1568).  A step of few tokens
+// is the state's way through the chip and little else: 32 sequences of 2 tokens 68 with one set, 94 with two; four tokens per
+// dependent step took 64 there, and 35 for 32 heads of 64 x 64, which take 50 here: steps of up to 8 tokens of 8 and more sequences
+// with such heads are what blocks of 16 do not pay for.
+template <int RB, int SETS>
 __global__ void __launch_bounds__(320, 2) delta_scan_k(KxDeltaArgs a) {
   __shared__ f32x4 sk_s[2][4][64], sq_s[2][4][64], u_s[2][64];
   const KxDeltaSpec &s = a.s;
@@ -271,7 +281,7 @@ __global__ void __launch_bounds__(320, 2) delta_scan_k(KxDeltaArgs a) {
   const int h = blockIdx.x, b = blockIdx.z, kvh = h / (s.heads / s.kv_heads), n = a.positions, C = kx_delta_channels(s);
   const int col = blockIdx.y * 16 + c;
   const Work w = work_of(a);
-  constexpr int DP = RB * 64, SETS = RB <= 2 ? 3 : 2;  // kx_delta_sets
+  constexpr int DP = RB * 64;
   const f32x4 *coef = (const f32x4 *)(w.coef + ((size_t)b * s.heads + h) * w.blocks * NCF);
   if (wave == 4) {
     auto numbers = [&](int blk, int at) { return coef[(size_t)min(blk, w.blocks - 1) * (NCF / 4) + at]; };
@@ -308,7 +318,7 @@ __global__ void __launch_bounds__(320, 2) delta_scan_k(KxDeltaArgs a) {
   auto load = [&](Set &x, int blk) {
     blk = min(blk, w.blocks - 1);  // past the end: not used
     const f32x4 *kp = qk + (size_t)blk * 12 * DP, *cf = coef + (size_t)blk * (NCF / 4);
-    const float *rows = raw + (size_t)min(blk, last) * NB * a.batch * C;
+    const float *rows = raw + (size_t)blk * NB * a.batch * C;
 #pragma unroll
     for (int v = 0; v < 4; ++v) x.v[v] = rows[blk < last ? row_at[v] : last_at[v]];
 #pragma unroll
@@ -368,15 +378,15 @@ __global__ void __launch_bounds__(320, 2) delta_scan_k(KxDeltaArgs a) {
       for (int v = 0; v < 4; ++v) S[r][v] = __builtin_fmaf(all, S[r][v], p[r][v]);
     load(x, blk + SETS);
   };
-  Set x[SETS];
+  Set x[SETS];  // the loads in flight stay in the registers that they arrive in
 #pragma unroll
   for (int y = 0; y < SETS; ++y) load(x[y], y);
   int blk = 0;
-  do {  // whole turns of the sets: the loads in flight stay in the registers that they arrive in
+  for (; blk + SETS <= w.blocks; blk += SETS) {
 #pragma unroll
     for (int y = 0; y < SETS; ++y) step(x[y], blk + y);
-    blk += SETS;
-  } while (blk < w.blocks);
+  }
+  if (SETS == 2 && blk < w.blocks) step(x[0], blk);
   kx_lds_barrier();
 #pragma unroll
   for (int r = 0; r < RB; ++r)
@@ -385,6 +395,14 @@ __global__ void __launch_bounds__(320, 2) delta_scan_k(KxDeltaArgs a) {
       const int row = row0 + r * 16 + 4 * g + v;
       if (row < D && col < V) st[(size_t)row * V + col] = S[r][v];
     }
+}
+
+template <int RB>
+void scan(const KxDeltaArgs &a, dim3 grid, hipStream_t st) {
+  // one set where there is one block, and where rows of 128 make more workgroups than the chip has CUs (figures at delta_scan_k)
+  const bool one = work_of(a).blocks == 1 || (RB == 2 && (long)grid.x * grid.y * grid.z > kx_device_cus());
+  if (one) hipLaunchKernelGGL((delta_scan_k<RB, 1>), grid, dim3(320), 0, st, a);
+  else hipLaunchKernelGGL((delta_scan_k<RB, 2>), grid, dim3(320), 0, st, a);
 }
 
 }  // namespace
@@ -408,10 +426,10 @@ int kx_delta_launch(const KxDeltaArgs &a, hipStream_t st) {
   hipLaunchKernelGGL(delta_block_k, dim3(work_of(a).blocks, s.kv_heads, a.batch), dim3(256), block_lds(row), st, a);
   KX_LAUNCH_CHECK();
   const dim3 grid(s.heads, kx_cdiv(s.vdim, 16), a.batch);
-  if (row == 64) hipLaunchKernelGGL(delta_scan_k<1>, grid, dim3(320), 0, st, a);
-  else if (row == 128) hipLaunchKernelGGL(delta_scan_k<2>, grid, dim3(320), 0, st, a);
-  else if (row == 192) hipLaunchKernelGGL(delta_scan_k<3>, grid, dim3(320), 0, st, a);
-  else hipLaunchKernelGGL(delta_scan_k<4>, grid, dim3(320), 0, st, a);
+  if (row == 64) scan<1>(a, grid, st);
+  else if (row == 128) scan<2>(a, grid, st);
+  else if (row == 192) scan<3>(a, grid, st);
+  else scan<4>(a, grid, st);
   KX_LAUNCH_CHECK();
   return KX_OK;
 }

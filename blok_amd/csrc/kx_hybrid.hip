@@ -297,7 +297,7 @@ size_t HybridModel::layout(char *base) {
       w.a_log = vec(m + "A_log", d.heads, 0, 0.0f, 0.5f);
       w.dt_bias = vec(m + "dt_bias", d.heads, 0, -2.0f, 0.5f);
       w.o_norm = vec(m + "norm", d.vdim, 0, 1.0f, 0.02f);
-      work_floats = std::max(work_floats, kx_delta_work_floats(d, 1, step_tokens + max_batch * (kx_delta_sets(d) * KX_DELTA_BLOCK - 1)));
+      work_floats = std::max(work_floats, kx_delta_work_floats(d, 1, step_tokens + max_batch * (KX_DELTA_BLOCK - 1)));
       w.state_floats = (size_t)d.heads * d.dim * d.vdim;
       w.hist_floats = (size_t)(d.taps - 1) * C;
     } else if (l.mixer == KxHybridLayer::SSD) {

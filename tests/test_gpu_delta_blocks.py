@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 TOLERANCE = 2 * 256 * 2.0 ** -24
 
 
-@pytest.mark.parametrize("shape", [(2, 1, 16, 15), (3, 1, 64, 16), (2, 2, 65, 17), (4, 2, 128, 33), (1, 1, 192, 1), (2, 1, 256, 16)], ids=lambda c: "-".join(map(str, c)))
+@pytest.mark.parametrize("shape", [(2, 1, 16, 15), (3, 1, 64, 16), (2, 2, 65, 17), (4, 2, 128, 33), (1, 1, 192, 1), (2, 1, 256, 16), (32, 2, 70, 80)], ids=lambda c: "-".join(map(str, c)))
 def test_delta_blocks(kxlib, shape):
     d = Delta(kxlib, *shape, 3, batch=2)
     for n in (2, 15, 16, 17, 32, 33, 49):
