@@ -48,7 +48,7 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) dense_gemm_k(
   };
   const int nb = a.cols >> 6;
   f32x16 acc[TL::MI][TL::NI];
-  TL::run(lds, (int)((long)nb * part / parts), (int)((long)nb * (part + 1) / parts), [&](int r) -> const uint16_t * {
+  TL::run(lds, kxtile::cut(nb, part, parts), kxtile::cut(nb, part + 1, parts), [&](int r) -> const uint16_t * {
     if (r < TL::BM) return a.x + (size_t)row_of(min(m0 + r, m_end - 1)) * a.x_stride;
     r -= TL::BM;
     if constexpr (DUAL) return ((r >> 5 & 1) ? w1 : w0) + (size_t)min(n0 + (r >> 6) * 32 + (r & 31), a.rows - 1) * a.cols;

@@ -51,11 +51,15 @@ struct Tile {
   static constexpr int COLS = 128 / sizeof(T);  // columns of a block
   static constexpr int SLOTS = SLOTS_, WM = WM_, WN = WN_, MI = MI_, NI = NI_, WAVES = WM * WN, THREADS = WAVES * 64;
   static constexpr int BM = WM * MI * 32, BN = WN * NI * 32, SLOT = (BM > BN ? BM : BN) * 128, LDS = SLOTS * SLOT;
+  static constexpr int PAIR = (BM + BN) * 128, LEAST_LDS = SLOTS == 4 ? 2 * PAIR : LDS;  // with LDS a CU has two workgroups of four waves, with less of it three
   static constexpr int WAVES_PER_SIMD = MI * NI >= 16 ? 1 : 2;
   static constexpr int CX = BM / 8 / WAVES, CW = BN / 8 / WAVES;  // copy instructions of a wave for half a block, 8 rows each
   static constexpr size_t PART = (size_t)BM * BN;          // floats of a part's sums
   static_assert(SLOTS == 4 || SLOTS == 5, "two blocks, and half of a third");
   static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "the copies of a block are spread evenly over the waves");
+
+  // Where a slot begins: with four, tokens have the even ones and the matrix the odd ones; with five each takes every one in turn.
+  static __device__ __forceinline__ int at(int slot) { return SLOTS == 4 ? (slot >> 1) * PAIR + (slot & 1) * (BM * 128) : slot * SLOT; }
 
   // Columns COLS kb0 .. COLS kb1 - 1 (kb0 < kb1).  row(r): where staged row r begins, tokens 0 .. BM - 1, then BN rows of the
   // matrix; every row has to be readable, what a row past the end holds only reaches sums that are not used.
@@ -70,11 +74,11 @@ struct Tile {
       src[i] = row(i < CX ? (i * WAVES + wave) * 8 + sub : BM + ((i - CX) * WAVES + wave) * 8 + sub) + kb0 * COLS + ((lane & 7) ^ sub) * (COLS / 8);
     auto copy_x = [&](int b, int slot) {
 #pragma unroll
-      for (int i = 0; i < CX; ++i) kx_copy16_to_lds(src[i] + b * COLS, __builtin_amdgcn_readfirstlane(lds0 + slot * SLOT + (i * WAVES + wave) * 1024));
+      for (int i = 0; i < CX; ++i) kx_copy16_to_lds(src[i] + b * COLS, __builtin_amdgcn_readfirstlane(lds0 + at(slot) + (i * WAVES + wave) * 1024));
     };
     auto copy_w = [&](int b, int slot) {
 #pragma unroll
-      for (int i = 0; i < CW; ++i) kx_copy16_to_lds(src[CX + i] + b * COLS, __builtin_amdgcn_readfirstlane(lds0 + slot * SLOT + (i * WAVES + wave) * 1024));
+      for (int i = 0; i < CW; ++i) kx_copy16_to_lds(src[CX + i] + b * COLS, __builtin_amdgcn_readfirstlane(lds0 + at(slot) + (i * WAVES + wave) * 1024));
     };
     struct Frag {
       typename Piece<T>::Type x[MI], w[NI];
@@ -85,9 +89,9 @@ struct Tile {
     auto read = [&](Frag &f, int q) {
       const int p = ((2 * q + h) ^ (lr & 7)) * 16;
 #pragma unroll
-      for (int i = 0; i < MI; ++i) f.x[i] = *(const typename Piece<T>::Type *)(xs + sx * SLOT + p + i * 4096);
+      for (int i = 0; i < MI; ++i) f.x[i] = *(const typename Piece<T>::Type *)(xs + at(sx) + p + i * 4096);
 #pragma unroll
-      for (int j = 0; j < NI; ++j) f.w[j] = *(const typename Piece<T>::Type *)(ws + sw * SLOT + p + j * 4096);
+      for (int j = 0; j < NI; ++j) f.w[j] = *(const typename Piece<T>::Type *)(ws + at(sw) + p + j * 4096);
       __builtin_amdgcn_sched_barrier(0);
     };
     auto multiply = [&](const Frag &f) {
@@ -198,6 +202,10 @@ __device__ __forceinline__ int item_of(int id, int n) {
   const int die = id & 7, q = n >> 3, r = n & 7;
   return die * q + min(die, r) + (id >> 3);
 }
+
+// Where part `part` of `parts` of `blocks` blocks begins.  In 32 bits (the products that fit a device stay below 2^31): two divisions
+// in 64 bits cost a workgroup 0.3 us, 2 % of a product of 16 blocks.
+__device__ __forceinline__ int cut(int blocks, int part, int parts) { return (uint32_t)blocks * part / (uint32_t)parts; }
 
 typedef Tile<uint16_t, 4, 2, 2, 4, 4> Large;   // 256 x 256, 8 waves, a CU each
 typedef Tile<uint16_t, 2, 2, 2, 2, 5> Medium;  // 128 x 128, 4 waves, two workgroups per CU

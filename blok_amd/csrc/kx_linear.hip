@@ -300,7 +300,7 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) lin_gemm_k(Kx
   x += (size_t)variant_of(a, n0) * a.tokens * x_ld;
   const int nb = a.m.ld / TL::COLS;
   f32x16 acc[TL::MI][TL::NI];
-  TL::run(lds, (int)((long)nb * part / parts), (int)((long)nb * (part + 1) / parts), [&](int r) {
+  TL::run(lds, kxtile::cut(nb, part, parts), kxtile::cut(nb, part + 1, parts), [&](int r) {
     return r < TL::BM ? x + source_row<GROUP>(e, tl, r) * x_ld : (const T *)a.m.w + tl.w + (size_t)min(n0 + r - TL::BM, a.m.rows - 1) * a.m.ld;
   }, acc);
   if (!GROUP && parts > 1 && !TL::gather(lds, acc, a.part + (size_t)tile * parts * TL::PART, a.arrived + tile, parts, part)) return;
@@ -550,9 +550,20 @@ int narrow_launch(const KxLinArgs &a, const KxExpertArgs &e, const uint16_t *x, 
   return KX_OK;
 }
 
-typedef kxtile::Tile<uint16_t, 2, 2, 1, 2, 4> SmallSlots;  // 64 slots of an expert
+// 64 slots of an expert.  Three workgroups per CU, or two by asking for more LDS where even routing then ends sooner: bound by the
+// stream of the matrices, a round of workgroups takes as long as there are of them per CU.  Experts of 3 x 2048 x 1024, 64 to 256
+// tokens to 8 of 64, which make 1024 tiles: 225 to 260 us with two, 244 to 276 with three; 3 x 1536 x 768, 768 tiles: 149 and 138.
+// Where few experts have the tokens three are better throughout (1000 tokens to 4 of 128, all among 8: 422 with two, 375 with
+// three), but that is known on the device alone.
+typedef kxtile::Tile<uint16_t, 2, 2, 1, 2, 4> SmallSlots;
+int small_slots_lds(const KxLinArgs &a, const KxExpertArgs &e) {
+  const long pairs = (long)a.tokens * e.top, used = std::min<long>(pairs, e.experts), cus = std::max(1, kx_device_cus());
+  const long tiles = std::max(used, (pairs + 32 * used) / 64) * kx_cdiv(a.m.rows, SmallSlots::BN);  // an expert's last tile is half full
+  const long two = (tiles + 2 * cus - 1) / (2 * cus) * 2, three = (tiles + 3 * cus - 1) / (3 * cus) * 3;
+  return two < three ? SmallSlots::LDS : SmallSlots::LEAST_LDS;
+}
 template <class T, class TL, int EPI, bool GROUP>
-int tile_launch(const KxLinArgs &a, const KxExpertArgs &e, const T *x, int x_ld, int parts, hipStream_t st) {
+int tile_launch(const KxLinArgs &a, const KxExpertArgs &e, const T *x, int x_ld, int parts, hipStream_t st, int lds = TL::LDS) {
   static std::atomic<bool> attr{false};
   if (!attr) {
     KX_HIP(hipFuncSetAttribute((const void *)lin_gemm_k<T, TL, EPI, GROUP>, hipFuncAttributeMaxDynamicSharedMemorySize, TL::LDS));
@@ -560,7 +571,7 @@ int tile_launch(const KxLinArgs &a, const KxExpertArgs &e, const T *x, int x_ld,
   }
   const int tn = kx_cdiv(a.m.rows, TL::BN);
   const dim3 grid = GROUP ? dim3(tn, e.max_tiles) : dim3(tn * kx_cdiv(a.tokens, TL::BM) * parts);
-  hipLaunchKernelGGL((lin_gemm_k<T, TL, EPI, GROUP>), grid, dim3(TL::THREADS), TL::LDS, st, a, e, x, x_ld, parts);
+  hipLaunchKernelGGL((lin_gemm_k<T, TL, EPI, GROUP>), grid, dim3(TL::THREADS), lds, st, a, e, x, x_ld, parts);
   KX_LAUNCH_CHECK();
   return KX_OK;
 }
@@ -577,7 +588,7 @@ int gemm_launch(const KxLinArgs &a, const KxExpertArgs &e, const T *x, int x_ld,
     const int parts = GROUP ? 1 : kxtile::choose_single(a.tokens, a.m.rows, a.m.ld / kxtile::Single::COLS, room, arrivals, cus);
     return tile_launch<float, kxtile::Single, EPI, GROUP>(a, e, x, x_ld, parts, st);
   } else if constexpr (GROUP) {
-    return e.tile_slots > 64 ? tile_launch<uint16_t, kxtile::Medium, EPI, true>(a, e, x, x_ld, 1, st) : tile_launch<uint16_t, SmallSlots, EPI, true>(a, e, x, x_ld, 1, st);
+    return e.tile_slots > 64 ? tile_launch<uint16_t, kxtile::Medium, EPI, true>(a, e, x, x_ld, 1, st) : tile_launch<uint16_t, SmallSlots, EPI, true>(a, e, x, x_ld, 1, st, small_slots_lds(a, e));
   } else {
     const kxtile::Choice c = kxtile::choose(a.tokens, a.m.rows, a.m.ld >> 6, room, arrivals, cus);
     if (c.large && a.n_var == 1) return tile_launch<uint16_t, kxtile::Large, EPI, false>(a, e, x, x_ld, 1, st);  // variants begin at multiples of 128 rows
