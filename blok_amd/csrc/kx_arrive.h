@@ -1,7 +1,8 @@
 // kx_arrive.h -- "the last one in finishes the job": how workgroups of one launch hand results to each other
 // without anybody waiting.  Used by the q_b GEMV that completes a head's query (kx_dense.hip), the router GEMV
-// whose last workgroup does top-k and bucketing (kx_dense.hip) and the routed down GEMV that combines a block
-// of rows (kx_i4.hip).  No counterpart in the reference, which runs each of these steps as a launch of its own
+// whose last workgroup does top-k and bucketing (kx_dense.hip), the routed down GEMV that combines a block
+// of rows (kx_i4.hip) and the products that split a tile's columns (kx_gemm_tile.h in kx_linear.hip and kx_dense_gemm.hip,
+// lin_narrow_k in kx_linear.hip).  No counterpart in the reference, which runs each of these steps as a launch of its own
 // (src/kimi_exec.cu:812-877).
 //
 // Protocol.  Every group (a workgroup on the GPU, a thread in the host model of it) first writes its results,
@@ -40,8 +41,9 @@
 //      increment's return value has arrived (the branch on it needs the value; loads are not speculated).
 // The plain accesses on these paths (routing weights, the residual row that is read, modified and written, the
 // counter reset) touch only data that an earlier launch wrote or that no other workgroup of this launch touches.
-// The GPU tests hold every kernel that uses the protocol to the oracle's bits in both forms of launch (fused and
-// separate), which would differ if a finisher ever read a stale value.
+// The GPU tests hold the kernels of kx_dense.hip and kx_i4.hip to the oracle's bits in both forms of launch (fused and
+// separate), which would differ if a finisher ever read a stale value; the split products, which are held to a tolerance, have to
+// give the same bits again and again.  All of them are compared to the bit with the library compiled in form (1).
 //
 // The same header compiles for the host (tests build a thread model of the protocol under ThreadSanitizer: in
 // form (1) it is race-free, with relaxed operations it is reported).

@@ -1,15 +1,20 @@
 """Products of the hybrid decoder where their kernels change: few tokens with the columns split over workgroups, experts with
 few slots, large tiles.  Against the plain forward passes, with the bars of the whole-model tests."""
 import ctypes as C
+import os
 
 import numpy as np
 import pytest
 
+import blok_amd.lib as kxl
 import kagalorn_case as KC
 import kagalorn_oracle as K
+import oracle as O
 from blok_amd.lib import DevBuf, KxLinearArgs, check
-from kxt import dev
+from kxt import dev, say
 from test_gpu_kagalorn import BF16_LOGITS, F32_LOGITS, _matrix, rel
+from test_gpu_kimi_prompt import _config
+from test_gpu_model import KxModel
 from test_gpu_rapitar import Experts
 
 pytestmark = pytest.mark.gpu
@@ -29,6 +34,43 @@ def test_few_tokens_against_wide_matrices(kxlib, tmp_path, ff, dtype, bar):
             first = m.run(ids[:batch], cuts, batch)
             assert KC.logit_error(first, want[:, :batch]).max() < bar, (batch, cuts)
             assert (m.run(ids[:batch], cuts, batch) == first).all(), "the parts' order does not depend on who comes last"
+
+
+@pytest.fixture(scope="module")
+def strict():
+    """The library with the hand-over between workgroups in its memory-model form (kx_arrive.h)."""
+    return kxl.load_library(os.path.join(os.path.dirname(kxl.lib_path()), "libkx_strict.so"))
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+def test_parts_of_the_hybrid_decoder_in_both_forms_of_the_hand_over(kxlib, strict, tmp_path, monkeypatch, dtype):
+    """All tokens against 64 rows in parts of the columns, and tiles in parts, bf16 and f32."""
+    cfg = KC.config([KC.delta(heads=4, kv_heads=2, dim=32, vdim=640, ff=4200), KC.attention(ff=4130)], width=192, vocab=300)
+    path, ids = KC.write(tmp_path, cfg, KC.weights(cfg, 3)), np.stack([KC.tokens(cfg, 6, 50 + b) for b in range(64)])
+    got = []
+    for lib in (kxlib, strict):
+        monkeypatch.setattr(KC, "kx", lambda lib=lib: lib)
+        with KC.Model(path, dtype, batch=64, context=6) as m:
+            got.append([m.run(ids[:b], cuts, b) for b, cuts in ((5, [1]), (8, [4, 1]), (33, [2]), (64, [1]), (64, [3]))])
+    for a, b in zip(*got):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+def test_parts_of_kimi_in_both_forms_of_the_hand_over(kxlib, strict, ox):
+    """Steps of 40 to 300 tokens: short and medium tiles in parts."""
+    cfg = _config(16, 1, 310)
+    ids = O.tokens_u32(300, 9, 4, cfg.vocab).reshape(1, 300)
+    for chunk in (300, 129, 40):
+        got = []
+        for lib in (kxlib, strict):
+            km = KxModel(lib, cfg)
+            check(lib.kx_model_set_prefill_chunk(km.h, chunk))
+            rc, _, _ = km.generate(ids, 1)
+            assert rc == 0, lib.kx_last_error()
+            got.append((km.logits(1), km.latent(1, 0, 300)))
+            km.close()
+        say(f"kimi, steps of {chunk}")
+        assert np.array_equal(got[0][0].view(np.uint32), got[1][0].view(np.uint32)) and np.array_equal(got[0][1], got[1][1]), chunk
 
 
 @pytest.mark.parametrize("tokens", [31, 32, 33, 200])
