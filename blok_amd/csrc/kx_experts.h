@@ -12,14 +12,16 @@ struct KxExpertSlots {
   int4 *tiles = nullptr;
   int *n_tiles = nullptr;
 };
-// slots per tile of a step (those of the GEMM that will read them), and the most tiles its pairs make.  bf16: 32 where an expert
-// has fewer than 8 pairs on average (the kernel for few tokens, 64 rows a workgroup: 71 and 37 us where the one with tiles of
-// 64 takes 75 and 38 us for 64 pairs on 64 experts of 3 x 2048 x 1024), 128 from 96 on
-constexpr int KX_EXPERT_TILE_MIN = 32;
+// slots per tile of a step (those of the GEMM that will read them), and the most tiles its pairs make.  bf16: 128 where an expert
+// has 96 pairs and more on average; 32, those of the kernel for few tokens, where it has fewer than 8 and no expert can have
+// more than three tiles, each of which reads its matrix again.  The operator with 32 / 64 slots, us: 8 to 8 of 64 of 3 x 2048 x 1024
+// 153 / 180, 63 tokens 211 / 230, all among 8 experts 83 / 90; 4 of 128 of 3 x 4096 x 1536, even 96 tokens 891 / 921, 192 tokens 982 /
+// 985; among 8 experts 96 tokens 174 / 183, 128 tokens 190 / 186, 192 tokens 215 / 187, 255 tokens 239 / 207.
+constexpr int KX_EXPERT_TILE_MIN = 32, KX_EXPERT_TILE_MIN_TOKENS = 3 * KX_EXPERT_TILE_MIN;
 inline int kx_expert_tile(bool f32, int tokens, int top, int experts) {
   const long pairs = (long)tokens * top;
   if (f32) return 64;
-  return pairs >= 96L * experts ? 128 : pairs >= 8L * experts ? 64 : KX_EXPERT_TILE_MIN;
+  return pairs >= 96L * experts ? 128 : pairs >= 8L * experts || tokens > KX_EXPERT_TILE_MIN_TOKENS ? 64 : KX_EXPERT_TILE_MIN;
 }
 inline int kx_expert_tiles(int tokens, int top, int experts, int tile) {
   const int pairs = tokens * top;

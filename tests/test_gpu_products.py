@@ -73,9 +73,9 @@ def test_parts_of_kimi_in_both_forms_of_the_hand_over(kxlib, strict, ox):
         assert np.array_equal(got[0][0].view(np.uint32), got[1][0].view(np.uint32)) and np.array_equal(got[0][1], got[1][1]), chunk
 
 
-@pytest.mark.parametrize("tokens", [31, 32, 33, 200])
+@pytest.mark.parametrize("tokens", [31, 32, 33, 96, 97, 200])
 def test_experts_of_more_slots_than_a_small_tile(kxlib, tokens):
-    """All tokens on three of 100 experts: one to seven tiles of 32 slots each, the last one short."""
+    """All tokens on three of 100 experts: one to three tiles of 32 slots each, and from 97 tokens on of 64, the last one short."""
     a = Experts(kxlib, 192, 72, 100, 3, 64, 0, 200)
     a.router[:], a.bias[:] = 0.0, 0.0
     a.bias[[99, 5, 40]] = 3.0
