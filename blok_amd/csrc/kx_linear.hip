@@ -552,13 +552,16 @@ int narrow_launch(const KxLinArgs &a, const KxExpertArgs &e, const uint16_t *x, 
 
 // 64 slots of an expert.  Three workgroups per CU, or two by asking for more LDS where even routing then ends sooner: bound by the
 // stream of the matrices, a round of workgroups takes as long as there are of them per CU.  Experts of 3 x 2048 x 1024, 64 to 256
-// tokens to 8 of 64, which make 1024 tiles: 225 to 260 us with two, 244 to 276 with three; 3 x 1536 x 768, 768 tiles: 149 and 138.
+// and 128 tokens to 8 of 64, which make 1024 tiles: 228 and 251 us with two, 244 and 268 with three; 3 x 1536 x 768, 768 tiles: 149 and 138.
 // Where few experts have the tokens three are better throughout (1000 tokens to 4 of 128, all among 8: 422 with two, 375 with
-// three), but that is known on the device alone.
+// three), but that is known on the device alone.  How many tiles there are is only certain while nearly every expert makes do
+// with one: with more than 16 pairs per expert two are not taken (256 tokens, even 262 with two, 281 with three, a few experts with more
+// tokens 293 and 277; 760 tokens 343 and 327).
 typedef kxtile::Tile<uint16_t, 2, 2, 1, 2, 4> SmallSlots;
 int small_slots_lds(const KxLinArgs &a, const KxExpertArgs &e) {
   const long pairs = (long)a.tokens * e.top, used = std::min<long>(pairs, e.experts), cus = std::max(1, kx_device_cus());
-  const long tiles = std::max(used, (pairs + 32 * used) / 64) * kx_cdiv(a.m.rows, SmallSlots::BN);  // an expert's last tile is half full
+  if (pairs > 16 * used) return SmallSlots::LEAST_LDS;
+  const long tiles = used * kx_cdiv(a.m.rows, SmallSlots::BN);
   const long two = (tiles + 2 * cus - 1) / (2 * cus) * 2, three = (tiles + 3 * cus - 1) / (3 * cus) * 3;
   return two < three ? SmallSlots::LDS : SmallSlots::LEAST_LDS;
 }
