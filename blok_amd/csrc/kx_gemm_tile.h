@@ -212,10 +212,13 @@ typedef Tile<uint16_t, 2, 2, 2, 2, 5> Medium;  // 128 x 128, 4 waves, two workgr
 
 // Which tile, and in how many parts of the columns, for one product of `tokens` x `rows` with `blocks` blocks of 64 columns.
 // Where the medium tiles leave CUs idle they take parts, of at least 16 blocks; beyond that the shorter of two estimates, in
-// us: a round of large tiles takes 12 + 1.55 per block on 256 CUs, of medium ones (two per CU) 6 + 1.22.  Measured against it (us,
-// 32-bit results, large / medium): 2048 x 16384 x 2048 150 / 214, 2048 x 8448 x 2048 116 / 94, 2048 x 5120 x 2048 64 / 61,
-// 2048 x 36864 x 7168 1026 / 1265, 2048 x 7168 x 8192 252 / 329, 952 x 7168 x 18432 455 / 353; in parts: 300 x 2048 x 8192 71 alone,
-// 32 in four, 100 x 2048 x 8192 73 and 29 in eight, 2048 x 384 x 7168 65 and 32 in four.
+// us: a round of large tiles takes 12 + 1.6 per block on 256 CUs, of medium ones (two per CU) 4.5 + 1.09; a last round of medium tiles
+// that is not full takes its share of that, but no less than half, the time of one per CU.  Measured against it (us, 32-bit
+// results, large / medium): large tiles in 1.5 rounds, medium ones in 3: 1536 x 16384 x 1024 75 / 69, x 2048 127 / 116, x 4096 228 / 211,
+// x 8192 453 / 434, x 16384 855 / 886; 2048 x 16384 x 2048 150 / 214, 2048 x 8448 x 2048 116 / 94, 2048 x 5120 x 2048 64 / 61, 2048 x 36864 x
+// 7168 1026 / 1265, 2048 x 7168 x 8192 252 / 329, 952 x 7168 x 18432 455 / 353, 700 x 12288 x 16384 379 / 428, 1024 x 36864 x 4096 359 / 345;
+// over 250 products of 300 to 2048 tokens with 2048 to 36864 x 1024 to 16384 the choice is at most 6 % behind the other one.
+// In parts: 300 x 2048 x 8192 71 alone, 32 in four, 100 x 2048 x 8192 73 and 29 in eight, 2048 x 384 x 7168 65 and 32 in four.
 struct Choice {
   bool large;
   int parts;
@@ -229,8 +232,9 @@ inline Choice choose(int tokens, int rows, int blocks, size_t part_floats, int a
     if ((size_t)p > part_floats / Medium::PART / medium) p = part_floats / Medium::PART / medium;
     return {false, p < 2 || medium > arrivals ? 1 : (int)p};
   }
-  const double l = (double)((large + cus - 1) / cus) * (12 + 1.55 * blocks), m = (medium > 2 * cus ? medium / (2.0 * cus) : 1.0) * (6 + 1.22 * blocks);
-  return {l < m, 1};
+  const long full = medium / (2 * cus), rest = medium % (2 * cus);
+  const double rounds = full == 0 ? 1.0 : full + (rest == 0 ? 0.0 : rest <= cus ? 0.5 : rest / (2.0 * cus));
+  return {(large + cus - 1) / cus * (12 + 1.6 * blocks) < rounds * (4.5 + 1.09 * blocks), 1};
 }
 
 // The 32-bit tile: 64 x 128, 4 waves, two workgroups per CU.  A piece is 4 products of 64 cycles, so LDS and copies are far
