@@ -45,7 +45,7 @@ struct KxMlaPromptArgs {
   int heads, nope, rope, kv_rank, kva_stride, seqs, positions, pos;
   float eps;
 };
-// whether a step of `positions` positions per sequence takes this form; expand_bytes: the room for keys and values
-bool kx_mla_prompt_fits(const kx_config *c, int positions, size_t expand_bytes);
+// whether a step of `positions` positions of `seqs` sequences, from `pos` on, takes this form; expand_bytes: the room for keys and values
+bool kx_mla_prompt_fits(const kx_config *c, int seqs, int positions, int pos, size_t expand_bytes);
 // split: scratch of the expanding product (KxDenseArgs::part and what follows)
 int kx_mla_prompt_launch(const kx_config *c, const KxMlaPromptArgs &a, const KxDenseArgs &split, hipStream_t st);

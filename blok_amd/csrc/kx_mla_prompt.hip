@@ -5,7 +5,7 @@
 // split_kv_k :364-370).  The decode form on the latent rows (kx_mla.hip) costs 2 x 1088 products per query, key and head and
 // reads every cached row once per position of the step; expanded they are 2 x 320, and 128 positions of a step share each
 // tile of keys.  What it costs is one product of the context with W_UK and W_UV per step, 2 x 512 x (128 + 128) per cached
-// row and head, as much as the attention of about 100 positions saves; hence the rule in kx_mla_prompt_fits.
+// row and head, so that a short step behind a long context is better off with the decode form (kx_mla_prompt_fits).
 // 64 heads, 2048 + 952 positions of one sequence: 3.25 ms a layer in the decode form (with absorb, merge and W_UV), 0.94 ms here.
 #include <algorithm>
 #include "kx_attn_parts.h"
@@ -54,24 +54,48 @@ __global__ void __launch_bounds__(256) share_key_k(const uint16_t *__restrict__ 
     *(uint4 *)(v + ((size_t)(b * heads + x / tail) * cap + n) * dv + (size_t)(x % tail) * 8) = uint4{0, 0, 0, 0};
 }
 
+// How the heads and sequences of a launch take turns with the room for their keys and values.
+struct Turns {
+  int heads, seqs;  // of a turn
+};
+Turns turns_of(const kx_config *c, int seqs, int context, size_t expand_bytes) {
+  const size_t head = (size_t)kx_pad(context, 64) * (c->qk_nope + c->qk_rope + c->v_head) * 2;  // bytes
+  const int most = (int)std::min<size_t>(expand_bytes / head, (size_t)c->heads * seqs);
+  if (most == 0) return {0, 0};
+  const int heads = kx_cdiv(c->heads, kx_cdiv(c->heads, std::min(most, c->heads)));
+  return {heads, heads == c->heads ? most / heads : 1};
+}
+
 }  // namespace
 
-bool kx_mla_prompt_fits(const kx_config *c, int positions, size_t expand_bytes) {
+// The shorter of two estimates, in us per layer, measured with 8 to 128 heads, 1 to 16 sequences and contexts of up to 60000 positions.  The
+// decode form does its work per position, cached row and head (with 64 heads, on the matrix cores, per position and row) and
+// some per position; expanded, a cached row costs its share of the product per head and sequence, and of the way of a workgroup
+// through all keys, alone on its CU, as often as there are more of them than CUs.  Figures, decode form / this one: 64 heads, 96
+// positions behind 1000 377 / 303, behind 4000 418 / 542, behind 16000 609 / 1499; 256 positions 433 / 314, 584 / 584, 1109 / 1521; 512
+// positions behind 16000 2080 / 1572, behind 60000, in two turns, 6117 / 7417; 8 heads, 33 positions behind 16000 540 / 829, of 4 sequences
+// behind 8000 916 / 675.  With no context the decode form is behind from 96 positions on (16 where heads is not 64) at the latest.
+bool kx_mla_prompt_fits(const kx_config *c, int seqs, int positions, int pos, size_t expand_bytes) {
   const int half = c->qk_rope / 2;
   if ((c->qk_nope + c->qk_rope) % 32 || c->v_head % 32 || c->qk_nope % 32 || c->qk_nope + c->qk_rope > 256 || c->v_head > 256 || half > 64 || (half & (half - 1)) || c->kv_rank % 128) return false;
-  // the matrix-core decode kernel (64 heads) is as fast below about 100 positions, the other one far behind at any number
-  if (positions < (c->heads == 64 ? 96 : 16)) return false;
-  return expand_bytes >= (size_t)kx_pad(c->max_context, 64) * (c->qk_nope + c->qk_rope + c->v_head) * 2;
+  const bool matrix_cores = c->heads == 64;
+  if (positions < (matrix_cores ? 96 : 16)) return false;
+  if (expand_bytes < (size_t)kx_pad(c->max_context, 64) * (c->qk_nope + c->qk_rope + c->v_head) * 2) return false;
+  const Turns t = turns_of(c, seqs, pos + positions, expand_bytes);
+  const int cus = std::max(1, kx_device_cus());
+  const double trips = (double)kx_cdiv(c->heads, t.heads) * kx_cdiv(seqs, t.seqs) * kx_cdiv(t.heads * t.seqs * kx_cdiv(positions, 128), cus);
+  const double expanded = (pos + positions) * (0.041 * trips + 0.00063 * c->heads * seqs);
+  const double decode = (double)seqs * positions * ((matrix_cores ? 0.00017 : 0.00009 * c->heads) * (pos + positions / 2) + (matrix_cores ? 0.8 : 0.4));
+  return expanded < decode;
 }
 
 int kx_mla_prompt_launch(const kx_config *c, const KxMlaPromptArgs &a, const KxDenseArgs &split, hipStream_t st) {
   const int n = a.pos + a.positions, cap = kx_pad(n, 64), dk = a.nope + a.rope, dv = c->v_head;
   hipLaunchKernelGGL(prompt_prep_k, dim3(a.positions * a.seqs), dim3(256), 0, st, a);
   KX_LAUNCH_CHECK();
-  const size_t head = (size_t)cap * (dk + dv) * 2;  // bytes
-  const int most = (int)std::min<size_t>(a.expand_bytes / head, (size_t)a.heads * a.seqs);
-  KX_REQUIRE(most > 0, "kx_mla: no room for the keys of %d positions", n);
-  const int hg = kx_cdiv(a.heads, kx_cdiv(a.heads, std::min(most, a.heads))), bg = hg == a.heads ? most / hg : 1;
+  const Turns turn = turns_of(c, a.seqs, n, a.expand_bytes);
+  KX_REQUIRE(turn.heads > 0, "kx_mla: no room for the keys of %d positions", n);
+  const int hg = turn.heads, bg = turn.seqs;
   float rs, ms;
   kx_softmax_scale(c, &rs, &ms);
   for (int b0 = 0; b0 < a.seqs; b0 += bg)

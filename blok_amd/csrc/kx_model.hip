@@ -312,7 +312,7 @@ int KimiModel::step(const uint32_t *d_ids, bool sample, int C) {
   const bool mm = B >= 5 && !(m->exact & KX_EXACT_PROJECTIONS);
   const int mla_kernel = (m->exact & KX_EXACT_ATTENTION) ? KX_MLA_VALU : m->mla_kernel;
   // a step of several positions attends to expanded keys and values where it is long enough
-  const bool expand = C > 1 && B > 32 && mla_kernel == KX_MLA_AUTO && kx_mla_prompt_fits(&c, C, m->expand_bytes);
+  const bool expand = C > 1 && B > 32 && mla_kernel == KX_MLA_AUTO && kx_mla_prompt_fits(&c, NB, C, pos, m->expand_bytes);
   KxDenseArgs split;
   split.part = m->split_part; split.part_floats = KX_DENSE_PART_FLOATS; split.arrived = m->split_arrived; split.arrivals = KX_DENSE_ARRIVALS;
   auto dense = [&](int epi, const KxGemvArgs &g) -> int {

@@ -73,6 +73,27 @@ def test_expanded_keys_that_do_not_fit_at_once(kxlib, ox, heads, batch, prompt, 
     assert row_err < 2e-2 and log_err < 3e-2
 
 
+@pytest.mark.parametrize("heads, kernel, short, long", [(64, 2, 100, 600), (8, 1, 40, 300)], ids=lambda v: str(v))
+def test_short_steps_behind_a_long_context_take_the_decode_form(kxlib, heads, kernel, short, long):
+    """Which of the two forms a step took shows in its bits: those of the decode form where that is the shorter one, others where not."""
+    behind = 16000
+    cfg = _config(heads, 1, behind + long)
+    ids = O.tokens_u32(behind + long, cfg.seed, 4, cfg.vocab).astype(np.uint32)
+    km = KxModel(kxlib, cfg)
+    check(kxlib.kx_model_set_prefill_chunk(km.h, 2048))
+    check(kxlib.kx_restart(km.h, 1))
+    check(kxlib.kx_extend(km.h, ids.ctypes.data, behind, None, 0, None))
+    for n, decode in ((short, True), (long, False)):
+        got = []
+        for k in (kernel, 0):
+            check(kxlib.kx_model_set_attention_kernel(km.h, k))
+            check(kxlib.kx_extend(km.h, ids[behind:].ctypes.data, n, None, 0, None))
+            got.append(km.latent(1, 0, behind + n)[behind:])
+            check(kxlib.kx_model_rewind(km.h, n))
+        assert np.array_equal(got[0], got[1]) == decode, (n, decode)
+    km.close()
+
+
 def _free(lib):
     free, total = C.c_size_t(), C.c_size_t()
     assert lib.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
