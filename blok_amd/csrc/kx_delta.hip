@@ -17,6 +17,7 @@
 // rounded once, which pays for the sums over more tokens: the error is below that of the recurrence in 32 bits, token by token.
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 #include "kx_common.h"
 #include "kx_conv.h"
 #include "kx_lds_copy.h"
@@ -29,9 +30,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int SC = 32;  // columns per workgroup of delta_step_k
 
-__device__ __forceinline__ float decay_of(const KxDeltaArgs &a, const float *pr, int h) {
-  return kx_expf(-kx_expf(a.a_log[h]) * kxr::softplus(pr[a.a_off + h] + a.dt_bias[h]));
-}
+__device__ __forceinline__ float decay_of(float proj, float a_log, float dt_bias) { return kx_expf(-kx_expf(a_log) * kxr::softplus(proj + dt_bias)); }
 
 __host__ __device__ __forceinline__ KxConvArgs conv_of(const KxDeltaArgs &a) {
   const int nq = a.s.kv_heads * a.s.dim;
@@ -71,7 +70,7 @@ __global__ void __launch_bounds__(256) delta_step_k(KxDeltaArgs a, KxConvArgs cv
   kk = kxr::block_sum(kk, red);
   const float qsc = kx_rsqrtf(qq + s.unit_eps) * kx_rsqrtf((float)D), ksc = kx_rsqrtf(kk + s.unit_eps);
   const float *pr = a.proj + (size_t)b * a.proj_ld;
-  const float beta = kx_sigmoidf(pr[a.b_off + h]), g = decay_of(a, pr, h);
+  const float beta = kx_sigmoidf(pr[a.b_off + h]), g = decay_of(pr[a.a_off + h], a.a_log[h], a.dt_bias[h]);
   // the convolutions' inputs for the next token: this workgroup's value channels, and q and k once per head of theirs
   if (s.taps > 1) {
     if (tid < SC && c0 + tid < V) kxc::shift(cv, b, 2 * nq + h * V + c0 + tid);
@@ -134,7 +133,7 @@ __host__ __device__ constexpr int block_stride(int row) { return row + 4; }  // 
 constexpr size_t block_lds(int row) { return (size_t)2 * NB * block_stride(row) * 4; }
 __global__ void __launch_bounds__(256) delta_block_k(KxDeltaArgs a) {
   extern __shared__ __attribute__((aligned(16))) float bl_lds[];
-  __shared__ float g_s[NB], beta_s[NB];
+  __shared__ float g_s[NB][NB], beta_s[NB][NB];  // [head of the key's][token]
   __shared__ double L[NB][NB + 1];
   const KxDeltaSpec &s = a.s;
   const int D = s.dim, DP = kx_delta_row(s), STR = block_stride(DP), tid = threadIdx.x, sl = tid & 15, j = tid >> 4;
@@ -144,6 +143,22 @@ __global__ void __launch_bounds__(256) delta_block_k(KxDeltaArgs a) {
   // tokens of this block; a wave without any makes zeros, which meet step sizes of zero
   const int cnt = min(NB, n - blk * NB);
   const bool any = __builtin_amdgcn_readfirstlane(j) < cnt;
+  // decays and step sizes of NB heads at a time, thread (j, sl) those of head r0 + j and token sl, asked for ahead of the rows; a position
+  // past the end leaves the state as it is
+  float pb = 0.0f, pa = 0.0f, pl = 0.0f, pt = 0.0f;
+  auto ask = [&](int r0) {
+    const int h = kvh * ratio + min(r0 + j, ratio - 1);
+    const float *pr = a.proj + (size_t)(min(blk * NB + sl, n - 1) * a.batch + b) * a.proj_ld;
+    pb = pr[a.b_off + h];
+    pa = pr[a.a_off + h];
+    pl = a.a_log[h];
+    pt = a.dt_bias[h];
+  };
+  auto keep = [&]() {
+    g_s[j][sl] = sl < cnt ? decay_of(pa, pl, pt) : 1.0f;
+    beta_s[j][sl] = sl < cnt ? kx_sigmoidf(pb) : 0.0f;
+  };
+  ask(0);
   if (!any) {
     for (int d = sl; d < DP; d += 16) qs[j * STR + d] = ks[j * STR + d] = 0.0f;
   } else {
@@ -174,6 +189,7 @@ __global__ void __launch_bounds__(256) delta_block_k(KxDeltaArgs a) {
       qs[j * STR + d] = (float)(qs[j * STR + d] * qsc);
     }
   }
+  keep();
   __syncthreads();
   f32x4 *out = (f32x4 *)(w.qk + (((size_t)b * s.kv_heads + kvh) * w.blocks + blk) * 3 * NB * DP);
   for (int x = tid; x < 4 * DP; x += 256) {
@@ -207,30 +223,38 @@ __global__ void __launch_bounds__(256) delta_block_k(KxDeltaArgs a) {
     const int h = kvh * ratio + r;
     float *cf = w.coef + (((size_t)b * s.heads + h) * w.blocks + blk) * NCF;
     __syncthreads();  // the head before has been worked on
-    if (tid < NB) {   // a position past the end leaves the state as it is
-      const bool in = blk * NB + tid < n;
-      const float *pr = a.proj + (size_t)(min(blk * NB + tid, n - 1) * a.batch + b) * a.proj_ld;
-      g_s[tid] = in ? decay_of(a, pr, h) : 1.0f;
-      beta_s[tid] = in ? kx_sigmoidf(pr[a.b_off + h]) : 0.0f;
+    if (r && r % NB == 0) {
+      ask(r);
+      keep();
+      __syncthreads();
     }
-    __syncthreads();
+    const float *const g = g_s[r % NB], *const beta = beta_s[r % NB];
     double d = 1.0;  // D(i, j): rounded once, not with each decay; a state that decays by it has fewer roundings than token by token
-    for (int m = i + 1; m <= j; ++m) d *= g_s[m];
-    L[j][i] = i < j ? beta_s[j] * d * kk : 0.0;
+    for (int m = i + 1; m <= min(j, cnt - 1); ++m) d *= g[m];
+    L[j][i] = i < j ? beta[j] * d * kk : 0.0;
     cf[CF_A + j * NB + i] = i <= j ? (float)(d * kq) : 0.0f;
-    if (i == 0) cf[CF_GAMMA + j] = (float)(d * g_s[0]);
+    if (i == 0) cf[CF_GAMMA + j] = (float)(d * g[0]);
     if (j == NB - 1) cf[CF_END + i] = (float)d;
     __syncthreads();
-    if (tid < NB) {  // column tid of the inverse
-      double t[NB];
+    if (tid < NB) {  // column tid of the inverse; rows past the end are zero
+      auto invert = [&](auto few) {
+        constexpr int ROWS = decltype(few)::value ? 4 : NB;
+        double t[ROWS];
 #pragma unroll
-      for (int y = 0; y < NB; ++y) {
-        double v = y == tid ? 1.0 : 0.0;
+        for (int y = 0; y < NB; ++y) {
+          float c = 0.0f;
+          if (y < ROWS) {
+            double v = y == tid ? 1.0 : 0.0;
 #pragma unroll
-        for (int m = 0; m < y; ++m) v = __builtin_fma(-L[y][m], t[m], v);
-        t[y] = v;
-        cf[CF_T + y * NB + tid] = y < tid ? 0.0f : (float)(v * beta_s[tid]);  // nothing of a token in the rows before it, whatever its numbers are
-      }
+            for (int m = 0; m < y; ++m) v = __builtin_fma(-L[y][m], t[m], v);
+            t[y] = v;
+            c = (float)(v * beta[tid]);
+          }
+          cf[CF_T + y * NB + tid] = y < tid ? 0.0f : c;  // nothing of a token in the rows before it, whatever its numbers are
+        }
+      };
+      if (cnt <= 4) invert(std::true_type{});
+      else invert(std::false_type{});
     }
   }
 }
