@@ -294,10 +294,11 @@ __device__ __forceinline__ f32x4 lower(f32x4 m, f32x4 x) {
 // leave a CU one workgroup instead of two); on the vector ALU, four tokens per dependent step, 370.  With 32 sequences of 512
 // tokens, where workgroups hide each other's waits, 894 with one set (three workgroups per CU), 1015 with two, 1085 with three;
 // rows of 64, 192 and 256 columns keep two (867, 943 and 1469 of 32 sequences against 981, 1105 and 1568).  A step of few tokens
-// is the state's way through the chip and little else: 32 sequences of 2 tokens 68 with one set, 94 with two; four tokens per
-// dependent step took 64 there, and 35 for 32 heads of 64 x 64, which take 50 here: steps of up to 8 tokens of 8 and more sequences
-// with such heads are what blocks of 16 do not pay for.
-template <int RB, int SETS>
+// is the state's way through the chip and little else: 32 sequences of 2 tokens 64 with one set, 94 with two (four tokens per
+// dependent step 64), and 38 for 32 heads of 64 x 64 -- 50 if the block after the only one is asked for -- where four tokens per
+// dependent step took 33.  Steps of 17 tokens, a block of them and one token, are what blocks of 16 pay least for: 32 sequences, 64 heads
+// of 128 x 128 338 (302), 32 of 64 x 64 73 (66), at 32 tokens 368 (407) and 76 (85).
+template <int RB, int SETS, bool MORE>  // MORE: the step may have more than SETS blocks
 __global__ void __launch_bounds__(320, 2) delta_scan_k(KxDeltaArgs a) {
   __shared__ f32x4 sk_s[2][4][64], sq_s[2][4][64], u_s[2][64];
   const KxDeltaSpec &s = a.s;
@@ -313,7 +314,11 @@ __global__ void __launch_bounds__(320, 2) delta_scan_k(KxDeltaArgs a) {
     kx_lds_barrier();
     for (int blk = 0; blk < w.blocks; ++blk) {
       kx_lds_barrier();  // the sums and the rows u of block blk are there
-      const f32x4 nextA = numbers(blk + 1, CF_A / 4 + c * 4 + g), nextG = numbers(blk + 1, CF_GAMMA / 4 + g);
+      f32x4 nextA = A, nextG = gamma;
+      if constexpr (MORE) {
+        nextA = numbers(blk + 1, CF_A / 4 + c * 4 + g);
+        nextG = numbers(blk + 1, CF_GAMMA / 4 + g);
+      }
       const f32x4(*q)[64] = sq_s[blk & 1];
       const f32x4 qs = (q[0][lane] + q[1][lane]) + (q[2][lane] + q[3][lane]), au = lower(A, u_s[blk & 1][lane]);
 #pragma unroll
@@ -400,7 +405,7 @@ __global__ void __launch_bounds__(320, 2) delta_scan_k(KxDeltaArgs a) {
     for (int r = 0; r < RB; ++r)
 #pragma unroll
       for (int v = 0; v < 4; ++v) S[r][v] = __builtin_fmaf(all, S[r][v], p[r][v]);
-    load(x, blk + SETS);
+    if constexpr (MORE) load(x, blk + SETS);
   };
   Set x[SETS];  // the loads in flight stay in the registers that they arrive in
 #pragma unroll
@@ -410,7 +415,7 @@ __global__ void __launch_bounds__(320, 2) delta_scan_k(KxDeltaArgs a) {
 #pragma unroll
     for (int y = 0; y < SETS; ++y) step(x[y], blk + y);
   }
-  if (SETS == 2 && blk < w.blocks) step(x[0], blk);
+  if (MORE && SETS == 2 && blk < w.blocks) step(x[0], blk);
   kx_lds_barrier();
 #pragma unroll
   for (int r = 0; r < RB; ++r)
@@ -423,10 +428,13 @@ __global__ void __launch_bounds__(320, 2) delta_scan_k(KxDeltaArgs a) {
 
 template <int RB>
 void scan(const KxDeltaArgs &a, dim3 grid, hipStream_t st) {
-  // one set where there is one block, and where rows of 128 make more workgroups than the chip has CUs (figures at delta_scan_k)
-  const bool one = work_of(a).blocks == 1 || (RB == 2 && (long)grid.x * grid.y * grid.z > kx_device_cus());
-  if (one) hipLaunchKernelGGL((delta_scan_k<RB, 1>), grid, dim3(320), 0, st, a);
-  else hipLaunchKernelGGL((delta_scan_k<RB, 2>), grid, dim3(320), 0, st, a);
+  const int blocks = work_of(a).blocks;
+  auto run = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(320), 0, st, a); };
+  if (blocks == 1) return run(delta_scan_k<RB, 1, false>);
+  // one set where rows of 128 make more workgroups than the chip has CUs (figures at delta_scan_k)
+  if constexpr (RB == 2)
+    if ((long)grid.x * grid.y * grid.z > kx_device_cus()) return run(delta_scan_k<RB, 1, true>);
+  run(delta_scan_k<RB, 2, true>);
 }
 
 }  // namespace
