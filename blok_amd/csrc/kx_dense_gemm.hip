@@ -4,7 +4,7 @@
 //
 // The main loop is kx_gemm_tile.h's.  With two matrices (SwiGLU) a tile's rows are blocks of 32 gate rows and their 32 up rows in
 // turn, so that a wave holds both halves of a pair.  Before these tiles the products went through the W4A16 kernel's loop with 64
-// tokens a tile and every lane loading its own row of the matrix: 400 TFLOP/s where these reach 800 to 1050 (2048 tokens, gate
+// tokens a tile and every lane loading its own row of the matrix: 400 TFLOP/s where these reach 1030 (2048 tokens, gate
 // and up of 2 x 18432 x 7168 with SwiGLU 2.7 ms then).
 // fp32 sums over exact bf16 products: a tolerance path like every matrix-core path (max-rel 1e-2), not used where tokens
 // have to be identical.

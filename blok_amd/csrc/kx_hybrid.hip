@@ -124,7 +124,7 @@ struct HybridModel : kx_model {
 };
 
 // partial sums of products that split their columns: two workgroups per CU with 64 rows of up to KX_NARROW_TOKENS tokens each, or
-// one with a tile of 128 x 128 (f32: four with one of 64 x 64)
+// one with a tile of 128 x 128 (f32: two with one of 64 x 128)
 constexpr int SPLIT_GROUPS = 512;
 constexpr size_t SPLIT_NARROW = (size_t)SPLIT_GROUPS * 64, SPLIT_TILES = (size_t)SPLIT_GROUPS / 2 * 128 * 128;
 

@@ -80,8 +80,8 @@ struct KxLinArgs {
   // SHIFT rows: the matrix rows [var_row[v], var_row[v + 1]) meet variant v; multiples of KX_VARIANT_ROWS
   int n_var = 1;
   int var_row[KX_MAX_VARIANTS] = {};
-  // scratch of products that split their columns over workgroups (KX_NARROW_TOKENS); without it they do not.  One launch at
-  // a time uses it.
+  // scratch of products that split their columns over workgroups: those of 5 to KX_NARROW_TOKENS tokens, and tiles where they
+  // leave CUs idle; without it they do not.  One launch at a time uses it.
   float *part = nullptr;
   size_t part_floats = 0;
   int *arrived = nullptr;    // [arrivals], zero between launches

@@ -10,7 +10,7 @@
 // all residual streams of the row.
 // lin_narrow_k (bf16, up to 64 tokens): all tokens against 64 rows, the columns split over waves and workgroups.
 // lin_gemm_k (bf16, more tokens): tiles of 256 x 256 or 128 x 128 on the matrix cores (kx_gemm_tile.h).
-// In f32 the same with tiles of 64 x 64 and 32-bit matrix instructions; true 32-bit products.
+// In f32 from 5 tokens on tiles of 64 x 128 on the 32-bit matrix instructions; true 32-bit products.
 //
 // Products with experts: up to 4 tokens lin_gemv_k with a matrix per (token, choice), the routing in its prologue, and with
 // the residual update's own product and the chosen experts' as one sum over consecutive segments of columns; beyond that
@@ -551,7 +551,7 @@ int narrow_launch(const KxLinArgs &a, const KxExpertArgs &e, const uint16_t *x, 
 }
 
 // 64 slots of an expert.  Three workgroups per CU, or two by asking for more LDS where even routing then ends sooner: bound by the
-// stream of the matrices, a round of workgroups takes as long as there are of them per CU.  Experts of 3 x 2048 x 1024, 64 to 256
+// stream of the matrices, a round of workgroups takes as long as there are of them per CU.  Experts of 3 x 2048 x 1024, 64
 // and 128 tokens to 8 of 64, which make 1024 tiles: 228 and 251 us with two, 244 and 268 with three; 3 x 1536 x 768, 768 tiles: 149 and 138.
 // Where few experts have the tokens three are better throughout (1000 tokens to 4 of 128, all among 8: 422 with two, 375 with
 // three), but that is known on the device alone.  How many tiles there are is only certain while nearly every expert makes do

@@ -283,8 +283,9 @@ __global__ void __launch_bounds__(MERGE_THREADS) win_merge_k(KxWindowArgs a, int
 // A key that a query does not see has a weight of zero, and its value is multiplied all the same; zero times a value that is not
 // finite would make the query's output follow a position behind it, or one that its window has left.  So a workgroup whose sums
 // are not all finite makes them once more: in tiles that not every query sees as a whole, such values are replaced by zeros, and
-// added at the end by the queries that see them.  This costs a launch 0 to 1 % (64 heads of 192, 2048 positions behind 952: 612 us, 618
-// with it); looking for such values as each tile is written to LDS took 857.
+// added at the end by the queries that see them.  This costs a launch 0 to 4 % (64 heads of 192, 2048 positions behind 952: 612 us, 618
+// with it; 4 sequences, 32 heads of 128, 2048 positions with a window of 4096 behind 3000: 1278 and 1327); looking for such values as
+// each tile is written to LDS took 857.
 constexpr int FQ = 128, FK = 64;
 __device__ __forceinline__ int vt_piece(int d, int piece) { return (piece ^ (d >> 1) ^ (d >> 4)) & 7; }
 

@@ -511,7 +511,8 @@ int kx_model_set_fusion(kx_model *model, uint32_t mask);
  * kx_model_set_fusion.  The flag stays set: the model is only good for kx_model_destroy afterwards.              */
 int kx_model_debug_fail_waits(kx_model *model);
 /* The attention kernel this model's steps use: KX_MLA_AUTO (default), KX_MLA_VALU or KX_MLA_MATRIX_CORES, as for
- * kx_mla_decode.  A property of the model: other models of the process keep theirs.                          */
+ * kx_mla_decode; with one of the latter two, long prompt steps attend to the cached rows as well (kx_model_set_prefill_chunk).
+ * A property of the model: other models of the process keep theirs.                                          */
 int kx_model_set_attention_kernel(kx_model *model, int32_t kernel);
 /* kx_model_set_exact(model, KX_EXACT_ALL): every step takes the kernels of the bit-reproducible path -- the GEMV
  * kernels, the VALU attention kernel, one prompt position per prefill step -- whatever the batch size, instead of
@@ -548,8 +549,9 @@ int kx_model_routing_history(kx_model *model, int32_t layer, int32_t pos0, int32
  * and the bit-reproducible path.  With n > 1, kx_prefill and kx_generate take up to n consecutive positions of
  * every sequence in one step (at most 2048 tokens a step, so min(n, 2048 / batch) positions): the projections, the
  * shared expert and the attention then run on the matrix cores as they do for a batch of that many sequences, and
- * from 33 tokens a step on the routed experts too (the grouped GEMMs of kx_moe_prefill_layer).  Same values, another
- * summation order: logits within the stack-level tolerance of the token-by-token prefill.  Each position attends to
+ * from 33 tokens a step on the routed experts too (the grouped GEMMs of kx_moe_prefill_layer).  Another summation order, and
+ * in steps of 96 positions and more (16 where heads is not 64), if they are long enough for their context, attention to keys
+ * and values that are expanded from the cache and rounded to bf16: logits within the stack-level tolerance of the token-by-token prefill.  Each position attends to
  * the cache rows up to its own, and only the last position is sampled.  1 <= n <= 2048. */
 int kx_model_set_prefill_chunk(kx_model *model, int32_t positions);
 /* bf(mean + sigma*z) fill used for the norm weights */
