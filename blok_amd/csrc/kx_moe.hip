@@ -35,6 +35,8 @@ struct kx_moe_workspace {
   int4 *work;         // [E] {expert, first, last, first pair}
   int4 *pair_work;    // [T*topk] one record per pair {expert, q, q + 1, pairs[q]}
   int *n_active;      // [1]
+  int4 *tiles;        // the grouped GEMMs' tiles where an expert may have more than one; n_tiles: how many
+  int *n_tiles;
   int *route_counter; // [10] zero between launches: workgroups of the router GEMV count themselves in (one counter, or one and one per block of four tokens)
   int *tail_count;    // [KX_TAIL_BLOCKS] zero between launches: arrivals per block of output rows (routed down + shared down)
   uint16_t *mid;      // [T*topk, moe_inter]
@@ -76,7 +78,7 @@ extern "C" int kx_moe_workspace_create(const kx_config *cfg, int32_t max_tokens,
   struct { void **p; size_t bytes; } allocs[] = {
       {(void **)&ws->logits, T * E * 4}, {(void **)&ws->ids, T * K * 2}, {(void **)&ws->weights, T * K * 4},
       {(void **)&ws->counts, E * 4}, {(void **)&ws->offsets, (E + 1) * 4}, {(void **)&ws->pairs, T * K * 4},
-      {(void **)&ws->work, E * 16}, {(void **)&ws->pair_work, T * K * 16}, {(void **)&ws->n_active, 64}, {(void **)&ws->tail_count, KX_TAIL_BLOCKS * 4},
+      {(void **)&ws->work, E * 16}, {(void **)&ws->pair_work, T * K * 16}, {(void **)&ws->n_active, 64}, {(void **)&ws->tiles, kx_grouped_tiles_max(T * K, E) * 16}, {(void **)&ws->n_tiles, 64}, {(void **)&ws->tail_count, KX_TAIL_BLOCKS * 4},
       {(void **)&ws->mid, T * K * (size_t)cfg->moe_inter * 2}, {(void **)&ws->eout, T * K * (size_t)cfg->hidden * 2},
       {(void **)&ws->smid, T * (size_t)cfg->shared_inter * 2}, {(void **)&ws->sy, T * (size_t)cfg->hidden * 2},
       {(void **)&ws->mid_hand, K * (size_t)cfg->moe_inter * 4}, {(void **)&ws->split_arrived, 2 * KX_DENSE_ARRIVALS * 4},
@@ -116,7 +118,7 @@ extern "C" int kx_moe_workspace_create(const kx_config *cfg, int32_t max_tokens,
 extern "C" int kx_moe_workspace_destroy(kx_moe_workspace *ws) {
   if (!ws) return KX_OK;
   void *ptrs[] = {ws->logits, ws->ids, ws->weights, ws->counts, ws->offsets, ws->pairs,
-                  ws->work, ws->pair_work, ws->n_active, ws->tail_count, ws->mid, ws->eout, ws->smid, ws->sy, ws->mid_hand,
+                  ws->work, ws->pair_work, ws->n_active, ws->tiles, ws->n_tiles, ws->tail_count, ws->mid, ws->eout, ws->smid, ws->sy, ws->mid_hand,
                   ws->split_arrived, ws->split_part[0], ws->split_part[1]};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
@@ -297,6 +299,11 @@ static int moe_layer_body(const kx_config *c, const kx_moe_weights *w, kx_moe_wo
   }
   if (timed) KX_HIP(hipEventRecord(ws->ev[1], st));
   const int n_slots = (long)tokens * K < E ? tokens * K : E;
+  // the grouped GEMMs' records: the experts', which are tiles while none can have more pairs than one holds
+  const bool tiled = rmm && tokens > KX_GROUPED_TILE;
+  const int4 *grouped = tiled ? ws->tiles : ws->work;
+  const int *n_tiles = tiled ? ws->n_tiles : nullptr;
+  const int tiles_max = tiled ? (int)kx_grouped_tiles_max((size_t)tokens * K, E) : n_slots;
   // one token: the routed experts and the layer's tail as one resident launch
   bool resident = false;
   if ((flags & KX_MOE_ROUTED_RESIDENT) && ws->err && paired && tokens == 1 && !(flags & KX_MOE_SEPARATE_TAIL) && H / 16 <= KX_TAIL_BLOCKS) {
@@ -333,14 +340,15 @@ static int moe_layer_body(const kx_config *c, const kx_moe_weights *w, kx_moe_wo
     KX_HIP(hipStreamWaitEvent(ws->side, ws->fork, 0));
     forked = true;
     bool mm_done = false;
+    if (tiled && (rc = kx_grouped_tiles_launch(ws->work, n_slots, rmm_min, ws->tiles, ws->n_tiles, st))) return rc;
     if (i4mm &&
         (rc = kx_i4mm_launch(true, (const uint32_t *)w->d_gate_packed, (const uint16_t *)w->d_gate_scale, (const uint32_t *)w->d_up_packed,
                              (const uint16_t *)w->d_up_scale, n, ws->mid, ws->work, ws->pairs, n_slots, I, H, K, (size_t)I * (H / 8),
                              (size_t)I * (H / 32), rmm_min, 1 << 30, kx_cdiv(tokens, 32), &mm_done, st))) return rc;
     if (!mm_done &&
         (rc = kx_grouped_gemm_launch(true, w->d_gate_packed, (const uint16_t *)w->d_gate_scale, w->d_up_packed,
-                                     (const uint16_t *)w->d_up_scale, n, ws->mid, ws->work, ws->pairs, n_slots, I, H,
-                                     K, (size_t)I * (H / 8), (size_t)I * (H / 32), tokens, st, rmm_min))) return rc;
+                                     (const uint16_t *)w->d_up_scale, n, ws->mid, grouped, n_tiles, ws->pairs, tiles_max, I, H,
+                                     K, (size_t)I * (H / 8), (size_t)I * (H / 32), st, tiled ? 0 : rmm_min))) return rc;
     if ((rc = kx_i4_launch(true, (const uint32_t *)w->d_gate_packed, (const uint16_t *)w->d_gate_scale,
                            (const uint32_t *)w->d_up_packed, (const uint16_t *)w->d_up_scale, n, ws->mid, ws->work, ws->pairs, 0, I,
                            H, K, (size_t)I * (H / 8), (size_t)I * (H / 32), 1, n_slots, 1, rmm_min - 1, ws->side))) return rc;
@@ -372,8 +380,8 @@ static int moe_layer_body(const kx_config *c, const kx_moe_weights *w, kx_moe_wo
                              1 << 30, kx_cdiv(tokens, 32), &mm_done, st))) return rc;
     if (!mm_done &&
         (rc = kx_grouped_gemm_launch(false, w->d_down_packed, (const uint16_t *)w->d_down_scale, nullptr, nullptr,
-                                     ws->mid, ws->eout, ws->work, ws->pairs, n_slots, H, I, 1, (size_t)H * (I / 8),
-                                     (size_t)H * (I / 32), tokens, st, rmm_min))) return rc;
+                                     ws->mid, ws->eout, grouped, n_tiles, ws->pairs, tiles_max, H, I, 1, (size_t)H * (I / 8),
+                                     (size_t)H * (I / 32), st, tiled ? 0 : rmm_min))) return rc;
     if ((rc = kx_i4_launch(false, (const uint32_t *)w->d_down_packed, (const uint16_t *)w->d_down_scale, nullptr, nullptr,
                            ws->mid, ws->eout, ws->work, ws->pairs, 0, H, I, 1, (size_t)H * (I / 8), (size_t)H * (I / 32),
                            1, n_slots, 1, rmm_min - 1, ws->side, 2))) return rc;
@@ -469,12 +477,14 @@ extern "C" int kx_moe_prefill_layer(const kx_config *c, const kx_moe_weights *w,
     return rc;
   const int n_slots = (long)tokens * K < E ? tokens * K : E;
   // routed experts: gate/up + SwiGLU, then down
+  const int tiles_max = (int)kx_grouped_tiles_max((size_t)tokens * K, E);
+  if ((rc = kx_grouped_tiles_launch(ws->work, n_slots, 0, ws->tiles, ws->n_tiles, st))) return rc;
   if ((rc = kx_grouped_gemm_launch(true, w->d_gate_packed, (const uint16_t *)w->d_gate_scale, w->d_up_packed,
-                                   (const uint16_t *)w->d_up_scale, n, ws->mid, ws->work, ws->pairs, n_slots, I, H,
-                                   K, (size_t)I * (H / 8), (size_t)I * (H / 32), tokens, st))) return rc;
+                                   (const uint16_t *)w->d_up_scale, n, ws->mid, ws->tiles, ws->n_tiles, ws->pairs, tiles_max, I, H,
+                                   K, (size_t)I * (H / 8), (size_t)I * (H / 32), st))) return rc;
   if ((rc = kx_grouped_gemm_launch(false, w->d_down_packed, (const uint16_t *)w->d_down_scale, nullptr, nullptr,
-                                   ws->mid, ws->eout, ws->work, ws->pairs, n_slots, H, I, 1, (size_t)H * (I / 8),
-                                   (size_t)H * (I / 32), tokens, st))) return rc;
+                                   ws->mid, ws->eout, ws->tiles, ws->n_tiles, ws->pairs, tiles_max, H, I, 1, (size_t)H * (I / 8),
+                                   (size_t)H * (I / 32), st))) return rc;
   KX_HIP(hipStreamWaitEvent(st, ws->join, 0));  // the shared expert's output
   return kx_moe_combine_launch(ws->eout, ws->weights, ws->sy, (uint16_t *)d_x, tokens, H, K, flags, st);
 }

@@ -7,11 +7,11 @@
 // combine (:868,:871), the shared expert (:872-875) and the residual add (:877) --
 // with the tokens of each expert gathered into one GEMM.
 //
-// Per workgroup (8 waves): one expert, 256 weight rows, the
-// expert's tokens in tiles of 128.  Wave w owns weight rows 32 w .. +31 for all 128 tokens
+// Per workgroup (8 waves) and tile: one expert, 256 weight rows (of a prompt's down product 512), up to 128 of the
+// expert's tokens.  Wave w owns weight rows 32 w .. +31 for all 128 tokens
 // (fp32 accumulators of v_mfma_f32_32x32x16_bf16).  Per K step of 64 columns:
 //  * INT4 weights reach the lanes through LDS as packed words: for every two K steps the
-//    64-byte runs of the 256 rows (both matrices) are copied by global -> LDS loads, which
+//    64-byte runs of the 256 rows (of both matrices, or of both halves of the 512) are copied by global -> LDS loads, which
 //    take no registers and use every byte they fetch, into a ring of two stages; lane
 //    (r, h) = (lane % 32, lane / 32) reads the 16 bytes of row r that hold columns 32 h .. +31
 //    of the step -- one quantization group, four packed words -- and dequantizes word j to
@@ -33,6 +33,7 @@
 //
 // MFMA's internal summation order is not documented, so this path is held to the
 // max-rel 1e-2 bar and is never used for the token-identity runs.
+#include <algorithm>
 #include <atomic>
 #include "kx_common.h"
 #include "kx_lds_copy.h"
@@ -49,7 +50,7 @@ typedef float kx_f32x2 __attribute__((ext_vector_type(2)));
 typedef float kx_f32x16 __attribute__((ext_vector_type(16)));
 typedef _Float16 kx_h2 __attribute__((ext_vector_type(2)));
 
-constexpr int BN = 256, BK = 64;  // a token tile has up to 4 blocks of 32 tokens (PfArgs::nb_max)
+constexpr int BN = 256, BK = 64, XT = 128 * BK;  // XT: elements of an activation tile
 constexpr int W_STAGE = BN * 64;               // bytes of one matrix's packed words for two K steps
 constexpr int SC_BLOCK = 16;                   // K steps per staged block of group scales
 constexpr int SC_STRIDE = SC_BLOCK * 4;        // bytes per (row, matrix) of a block: 32 bf16, one 64-byte sector of the row
@@ -59,12 +60,13 @@ struct PfArgs {
   const uint16_t *s0, *s1;      // bf16 scales [E][N][K/32]
   const uint16_t *x;            // bf16 activation rows of K
   uint16_t *out;                // bf16 [pairs][N]
-  const int4 *work;             // {expert, first, last, _} per expert with work
+  const int4 *tiles;            // {expert, first, last, _} of up to 128 pairs
+  const int *n_tiles;           // how many; nullptr: tiles_max
+  int tiles_max, cnt_lo;        // records with fewer pairs are left to another launch
+  int row_tiles;                // of 256 rows, WIDE 512
   const int *pairs;             // pair ids sorted by expert
   int N, K, x_div;              // activation row = pair / x_div
   size_t expert_w, expert_s;    // elements between experts (words; scales)
-  int nb_max;                   // 32-token blocks per token tile (1..4): sizes the activation tiles in LDS
-  int cnt_lo;                   // groups with fewer pairs are left to another launch
 };
 
 __device__ __forceinline__ uint32_t pf_and_or(uint32_t a, uint32_t mask, uint32_t magic) {
@@ -104,65 +106,101 @@ __device__ __forceinline__ kx_bf16x8 dequant_word(uint32_t w, float sc, float sc
   return __builtin_bit_cast(kx_bf16x8, make_uint4(pf_pack(f0, f1), pf_pack(f2, f3), pf_pack(f4, f5), pf_pack(f6, f7)));
 }
 
-// 8 waves per workgroup, 32 weight rows each
-template <bool DUAL>
+// The tiles of up to 128 pairs of every group with at least cnt_lo pairs, {expert, first, last, -}, those of four 32-token
+// blocks first and those of one last (a last round of the short ones ends sooner): tiles of a group in turn, so that workgroups which run at
+// the same time share its weights.  One workgroup, a thread per group; n_tiles[0]: how many.
+__global__ void __launch_bounds__(1024) grouped_tiles_k(const int4 *__restrict__ work, int n_slots, int cnt_lo, int4 *__restrict__ tiles, int *__restrict__ n_tiles) {
+  __shared__ int4 sum[2][1024];
+  const int i = threadIdx.x;
+  const int4 w = i < n_slots ? work[i] : make_int4(-1, 0, 0, 0);
+  const int cnt = w.x >= 0 && w.z - w.y >= cnt_lo ? w.z - w.y : 0;
+  const int rest = cnt & 127, cls = rest ? (rest + 31) >> 5 : 0, full = (cnt >> 7) + (cls == 4);
+  const int4 own = make_int4(full, cls == 3, cls == 2, cls == 1);
+  int cur = 0;
+  sum[0][i] = own;
+  __syncthreads();
+  for (int d = 1; d < 1024; d <<= 1, cur ^= 1) {  // inclusive sums
+    int4 v = sum[cur][i];
+    if (i >= d) {
+      const int4 u = sum[cur][i - d];
+      v = make_int4(v.x + u.x, v.y + u.y, v.z + u.z, v.w + u.w);
+    }
+    sum[cur ^ 1][i] = v;
+    __syncthreads();
+  }
+  const int4 at = sum[cur][i], all = sum[cur][1023];
+  for (int t = 0; t < full; ++t) tiles[at.x - full + t] = make_int4(w.x, w.y + t * 128, min(w.y + t * 128 + 128, w.z), 0);
+  const int last = cls == 3 ? all.x + at.y : cls == 2 ? all.x + all.y + at.z : all.x + all.y + all.z + at.w;
+  if (cls >= 1 && cls <= 3) tiles[last - 1] = make_int4(w.x, w.z - rest, w.z, 0);
+  if (i == 0) *n_tiles = all.x + all.y + all.z + all.w;
+}
+
+// 8 waves per workgroup, 32 weight rows each: of two matrices (DUAL), of 256 rows of one (SINGLE), or twice 256 of them (WIDE).  An activation
+// operand meets two weight operands in DUAL and WIDE: with one a wave reads a KB of LDS for every product of 32 cycles, all of
+// LDS' rate.  7168 rows of 2048 columns, 8 experts of 2048 tokens: 0.80 ms as SINGLE with a workgroup per possible tile, 0.61 as WIDE over a
+// list.  Records without a list are SINGLE (a few tokens per expert, beside other kernels): twice as many workgroups, of less LDS.
+enum { GG_SINGLE = 0, GG_WIDE = 1, GG_DUAL = 2 };
+template <int MODE>
 __global__ void __launch_bounds__(512, 1) grouped_gemm_k(PfArgs a) {
-  constexpr int MATS = DUAL ? 2 : 1;
+  constexpr bool DUAL = MODE == GG_DUAL;
+  constexpr int MATS = MODE == GG_SINGLE ? 1 : 2;
   extern __shared__ __attribute__((aligned(16))) uint8_t pf_lds[];
-  const int BM = a.nb_max * 32, XT = BM * BK;  // tokens and elements of one activation tile
   uint16_t *xs_lds = (uint16_t *)pf_lds;                 // two activation tiles
   uint8_t *w_ring = pf_lds + 2 * XT * 2;                 // [2 stages][MATS][256 rows][4 pieces of 16 B]
   uint8_t *sc_lds = w_ring + 2 * MATS * W_STAGE;         // [2 blocks][MATS][256 rows][SC_STRIDE]
   const uint32_t ring0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)w_ring;  // LDS address of the ring
   const uint32_t sc0 = ring0 + 2 * MATS * W_STAGE;                                                  // of the scale blocks
   const uint32_t xs0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)pf_lds;    // and of the activation tiles
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lr = lane & 31, lh = lane >> 5;
-  const int n0 = blockIdx.x * BN;
-  const int4 wk = a.work[blockIdx.y];
-  const int e = __builtin_amdgcn_readfirstlane(wk.x);
-  if (e < 0) return;
-  const int p_begin = __builtin_amdgcn_readfirstlane(wk.y), p_end = __builtin_amdgcn_readfirstlane(wk.z);
-  if (p_end - p_begin < a.cnt_lo) return;
-  uint32_t magic;
-  asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(magic));
   const int nk = a.K / BK;
-  const int trow = wave * 32 + lr;                       // this lane's weight row within the tile
-  // global -> LDS copies of this wave for one stage: MATS*2 instructions of 64 pieces
-  const uint32_t *dma_src[MATS * 2];
-  int dma_dst[MATS * 2];
+  const int items = (a.n_tiles ? *a.n_tiles : a.tiles_max) * a.row_tiles;
+  for (int item = blockIdx.x; item < items; item += gridDim.x) {
+    const int n0 = item % a.row_tiles * (MODE == GG_WIDE ? 2 * BN : BN);
+    const int4 wk = a.tiles[item / a.row_tiles];
+    const int e = __builtin_amdgcn_readfirstlane(wk.x);
+    const int m0 = __builtin_amdgcn_readfirstlane(wk.y), p_end = __builtin_amdgcn_readfirstlane(wk.z);
+    if (e < 0 || p_end - m0 < a.cnt_lo) continue;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));  // what follows from it is not worked out, and spilled, in front of the loop
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 31, lh = lane >> 5;
+    const int trow = wave * 32 + lr;                       // this lane's weight row within the tile
+    uint32_t magic;
+    asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(magic));
+    // row r of matrix m: of the second matrix, or 256 rows further down the same one
+    auto row_of = [&](int m, int r) { return min(n0 + r + (DUAL ? 0 : m * BN), a.N - 1); };
+    // global -> LDS copies of this wave for one stage: MATS*2 instructions of 64 pieces
+    const uint32_t *dma_src[MATS * 2];
+    int dma_dst[MATS * 2];
 #pragma unroll
-  for (int u = 0; u < MATS * 2; ++u) {
-    const int g = (wave * MATS * 2 + u) * 64 + lane;     // piece index over [MATS][256 rows][4]
-    const int m = g >> 10, sl = g & 1023, row = sl >> 2, ps = sl & 3;
-    const int p = ps ^ ((row >> 2) & 3);                 // the piece of the row that lives in slot ps
-    dma_src[u] = (m ? a.w1 : a.w0) + (size_t)e * a.expert_w + (size_t)min(n0 + row, a.N - 1) * (a.K >> 3) + p * 4;
-    dma_dst[u] = (wave * MATS * 2 + u) * 1024;           // byte offset within a stage, the same for the whole wave
-  }
-  auto dma_stage = [&](int ss) {  // packed words of K steps 2 ss, 2 ss + 1 into stage ss % 2
+    for (int u = 0; u < MATS * 2; ++u) {
+      const int g = (wave * MATS * 2 + u) * 64 + lane;     // piece index over [MATS][256 rows][4]
+      const int m = g >> 10, sl = g & 1023, row = sl >> 2, ps = sl & 3;
+      const int p = ps ^ ((row >> 2) & 3);                 // the piece of the row that lives in slot ps
+      dma_src[u] = (DUAL && m ? a.w1 : a.w0) + (size_t)e * a.expert_w + (size_t)row_of(m, row) * (a.K >> 3) + p * 4;
+      dma_dst[u] = (wave * MATS * 2 + u) * 1024;           // byte offset within a stage, the same for the whole wave
+    }
+    auto dma_stage = [&](int ss) {  // packed words of K steps 2 ss, 2 ss + 1 into stage ss % 2
 #pragma unroll
-    for (int u = 0; u < MATS * 2; ++u) pf_copy16_to_lds(dma_src[u] + ss * 16, ring0 + (ss & 1) * MATS * W_STAGE + dma_dst[u]);
-  };
-  // group scales: blocks of SC_BLOCK K steps, 64 bytes per row and matrix -- whole sectors -- copied global -> LDS.
-  // Instruction c = wave * 2 MATS + i covers pieces 64 c .. +63 of [MATS][256 rows][4 slots]; slot s of row r holds
-  // piece s ^ ((r / 2) % 4): a wave reads one 2-byte scale per row at the same offset of 32 consecutive rows, and with
-  // the pieces in place (64-byte rows) those fall into two banks; xor-ed by the row they fall into eight.  A last block of
-  // half the steps (K / 64 an odd multiple of 8) repeats its two pieces, the copies land in slots that are never read.
-  const uint16_t *sc_src[MATS * 2];
+      for (int u = 0; u < MATS * 2; ++u) pf_copy16_to_lds(dma_src[u] + ss * 16, ring0 + (ss & 1) * MATS * W_STAGE + dma_dst[u]);
+    };
+    // group scales: blocks of SC_BLOCK K steps, 64 bytes per row and matrix -- whole sectors -- copied global -> LDS.
+    // Instruction c = wave * 2 MATS + i covers pieces 64 c .. +63 of [MATS][256 rows][4 slots]; slot s of row r holds
+    // piece s ^ ((r / 2) % 4): a wave reads one 2-byte scale per row at the same offset of 32 consecutive rows, and with
+    // the pieces in place (64-byte rows) those fall into two banks; xor-ed by the row they fall into eight.  A last block of
+    // half the steps (K / 64 an odd multiple of 8) repeats its two pieces, the copies land in slots that are never read.
+    const uint16_t *sc_src[MATS * 2];
 #pragma unroll
-  for (int i = 0; i < MATS * 2; ++i) {
-    const int c = wave * MATS * 2 + i, m = c >> 4, row = (c & 15) * 16 + (lane >> 2);
-    sc_src[i] = (m ? a.s1 : a.s0) + (size_t)e * a.expert_s + (size_t)min(n0 + row, a.N - 1) * (a.K >> 5);
-  }
-  auto copy_scales = [&](int blk) {
-    const int left = (nk - blk * SC_BLOCK) >> 2;  // 16-byte pieces of the row from this block on: 2 or at least 4
-    const int piece = min((lane & 3) ^ ((lane >> 3) & 3), left - 1);  // row = 16 (c % 16) + lane / 4
+    for (int i = 0; i < MATS * 2; ++i) {
+      const int c = wave * MATS * 2 + i, m = c >> 4, row = (c & 15) * 16 + (lane >> 2);
+      sc_src[i] = (DUAL && m ? a.s1 : a.s0) + (size_t)e * a.expert_s + (size_t)row_of(m, row) * (a.K >> 5);
+    }
+    auto copy_scales = [&](int blk) {
+      const int left = (nk - blk * SC_BLOCK) >> 2;  // 16-byte pieces of the row from this block on: 2 or at least 4
+      const int piece = min((lane & 3) ^ ((lane >> 3) & 3), left - 1);  // row = 16 (c % 16) + lane / 4
 #pragma unroll
-    for (int i = 0; i < MATS * 2; ++i)
-      pf_copy16_to_lds(sc_src[i] + blk * (SC_BLOCK * 2) + piece * 8, sc0 + (blk & 1) * (BN * MATS * SC_STRIDE) + (wave * MATS * 2 + i) * 1024);
-  };
-  for (int m0 = p_begin + blockIdx.z * BM; m0 < p_end; m0 += gridDim.z * BM) {
-    const int nb = min(a.nb_max, (p_end - m0 + 31) >> 5);  // 32-token blocks that hold tokens
+      for (int i = 0; i < MATS * 2; ++i)
+        pf_copy16_to_lds(sc_src[i] + blk * (SC_BLOCK * 2) + piece * 8, sc0 + (blk & 1) * (BN * MATS * SC_STRIDE) + (wave * MATS * 2 + i) * 1024);
+    };
+    const int nb = (p_end - m0 + 31) >> 5;  // 32-token blocks that hold tokens
     // The activation tile goes global -> LDS like the weights.  A row of a K step is 128 B = 8 pieces;
     // copy instruction ii covers rows 8 ii .. 8 ii + 7, slot (row, p') holding piece p' ^ ((row >> 1) & 7), so that
     // the row-per-lane operand reads are free of bank conflicts without padding.  Rows past the expert's tokens
@@ -172,7 +210,7 @@ __global__ void __launch_bounds__(512, 1) grouped_gemm_k(PfArgs a) {
     int xc_dst[XCMAX];
 #pragma unroll
     for (int q = 0; q < XCMAX; ++q) {
-      const int ii = min(wave + 8 * q, a.nb_max * 4 - 1);
+      const int ii = wave + 8 * q;
       const int slot = ii * 64 + lane, row = slot >> 3, piece = (slot & 7) ^ ((row >> 1) & 7);
       const int pi = m0 + row;
       const int pair = pi < p_end ? a.pairs[pi] : 0;
@@ -287,21 +325,22 @@ __global__ void __launch_bounds__(512, 1) grouped_gemm_k(PfArgs a) {
         }
       }
       // epilogue: D[i][j], j = lane % 32 (weight row), i = 8*(v/4) + 4*(lane/32) + v%4 (token of the 32-token block)
-      const int n = n0 + trow;
-      if (n < a.N) {
 #pragma unroll
-        for (int t = 0; t < NB; ++t)
+      for (int t = 0; t < NB; ++t)
 #pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            const int po = m0 + t * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
-            if (po < p_end) {
-              float r = acc[0][t][v];
-              if (DUAL) r = kx_swiglu(kx_bfround(r), kx_bfround(acc[MATS - 1][t][v]));
-              a.out[(size_t)a.pairs[po] * a.N + n] = kx_bf16_rne(r);
+        for (int v = 0; v < 16; ++v) {
+          const int po = m0 + t * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
+          if (po < p_end) {
+            uint16_t *out = a.out + (size_t)a.pairs[po] * a.N;
+            if constexpr (DUAL) {
+              if (n0 + trow < a.N) out[n0 + trow] = kx_bf16_rne(kx_swiglu(kx_bfround(acc[0][t][v]), kx_bfround(acc[MATS - 1][t][v])));
+            } else {
+#pragma unroll
+              for (int m = 0; m < MATS; ++m)
+                if (n0 + m * BN + trow < a.N) out[n0 + m * BN + trow] = kx_bf16_rne(acc[m][t][v]);
             }
           }
-      }
-      __syncthreads();  // the next token tile starts by overwriting the LDS tiles
+        }
     };
     if (nb == 1) run(std::integral_constant<int, 1>{});
     else if (nb == 2) run(std::integral_constant<int, 2>{});
@@ -326,30 +365,44 @@ __global__ void __launch_bounds__(256) moe_combine_k(const uint16_t *__restrict_
 
 }  // namespace
 
+int kx_grouped_tiles_launch(const int4 *work, int n_slots, int cnt_lo, int4 *tiles, int *n_tiles, hipStream_t st) {
+  KX_REQUIRE(n_slots > 0 && n_slots <= 1024, "kx_grouped_tiles: %d groups", n_slots);
+  hipLaunchKernelGGL(grouped_tiles_k, dim3(1), dim3(1024), 0, st, work, n_slots, cnt_lo, tiles, n_tiles);
+  KX_LAUNCH_CHECK();
+  return KX_OK;
+}
+
 int kx_grouped_gemm_launch(bool dual, const void *w0, const uint16_t *s0, const void *w1, const uint16_t *s1, const uint16_t *x, uint16_t *out,
-                           const int4 *work, const int *pairs, int n_slots, int N, int K, int x_div, size_t expert_w, size_t expert_s,
-                           int n_pairs_max, hipStream_t st, int cnt_lo) {
+                           const int4 *tiles, const int *n_tiles, const int *pairs, int tiles_max, int N, int K, int x_div, size_t expert_w, size_t expert_s,
+                           hipStream_t st, int cnt_lo) {
   KX_REQUIRE(K > 0 && K % 512 == 0, "kx_grouped_gemm: K=%d must be a positive multiple of 512", K);
   KX_REQUIRE(N > 0, "kx_grouped_gemm: N=%d must be positive", N);
   PfArgs a;
-  a.w0 = (const uint32_t *)w0; a.w1 = (const uint32_t *)w1; a.s0 = s0; a.s1 = s1; a.x = x; a.out = out; a.work = work; a.pairs = pairs;
-  a.N = N; a.K = K; a.x_div = x_div; a.expert_w = expert_w; a.expert_s = expert_s;
+  a.w0 = (const uint32_t *)w0; a.w1 = (const uint32_t *)w1; a.s0 = s0; a.s1 = s1; a.x = x; a.out = out; a.tiles = tiles; a.pairs = pairs;
+  a.n_tiles = n_tiles;
+  a.tiles_max = tiles_max;
   a.cnt_lo = cnt_lo;
-  a.nb_max = 4;  // 128 tokens a tile: the dequant work per weight tile is amortised over the tokens
-  const int BM = a.nb_max * 32;
-  int mz = kx_cdiv(n_pairs_max, BM);
-  mz = mz < 1 ? 1 : mz > 64 ? 64 : mz;
-  const dim3 g(kx_cdiv(N, BN), n_slots, mz), b(512);
-  const int mats = dual ? 2 : 1;
-  const size_t lds = (size_t)2 * BM * BK * 2 + (size_t)2 * mats * W_STAGE + (size_t)2 * BN * mats * SC_STRIDE;
+  a.N = N; a.K = K; a.x_div = x_div; a.expert_w = expert_w; a.expert_s = expert_s;
+  const int mode = dual ? GG_DUAL : n_tiles ? GG_WIDE : GG_SINGLE, mats = mode == GG_SINGLE ? 1 : 2;
+  a.row_tiles = kx_cdiv(N, mode == GG_WIDE ? 2 * BN : BN);
+  const long items = (long)tiles_max * a.row_tiles;
+  KX_REQUIRE(tiles_max > 0 && items < (1L << 31), "kx_grouped_gemm: %d tiles of %d rows", tiles_max, N);
+  // With a list a workgroup per CU goes over it, since only the device knows how long it is: a workgroup per possible tile (128
+  // tokens of every expert) were 170000 for 2048 tokens to 384 experts, nearly all of them without work and each waiting for a CU of
+  // its own, whose registers it takes whole.  A few tokens per expert beside other kernels gain
+  // nothing by it (16 tokens 580 us, 583 with a list and its launch).
+  const dim3 g((unsigned)(n_tiles ? std::min<long>(items, std::max(1, kx_device_cus())) : items)), b(512);
+  const size_t lds = (size_t)2 * XT * 2 + (size_t)2 * mats * W_STAGE + (size_t)2 * BN * mats * SC_STRIDE;
   static std::atomic<bool> attr_set{false};  // setting it twice from two threads is harmless
   if (!attr_set) {  // more than 64 KB of dynamic LDS has to be allowed per kernel
-    KX_HIP(hipFuncSetAttribute((const void *)grouped_gemm_k<true>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-    KX_HIP(hipFuncSetAttribute((const void *)grouped_gemm_k<false>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    KX_HIP(hipFuncSetAttribute((const void *)grouped_gemm_k<GG_SINGLE>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    KX_HIP(hipFuncSetAttribute((const void *)grouped_gemm_k<GG_WIDE>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    KX_HIP(hipFuncSetAttribute((const void *)grouped_gemm_k<GG_DUAL>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     attr_set = true;
   }
-  if (dual) hipLaunchKernelGGL(grouped_gemm_k<true>, g, b, lds, st, a);
-  else hipLaunchKernelGGL(grouped_gemm_k<false>, g, b, lds, st, a);
+  if (mode == GG_DUAL) hipLaunchKernelGGL(grouped_gemm_k<GG_DUAL>, g, b, lds, st, a);
+  else if (mode == GG_WIDE) hipLaunchKernelGGL(grouped_gemm_k<GG_WIDE>, g, b, lds, st, a);
+  else hipLaunchKernelGGL(grouped_gemm_k<GG_SINGLE>, g, b, lds, st, a);
   KX_LAUNCH_CHECK();
   return KX_OK;
 }

@@ -1,0 +1,35 @@
+"""The list of tiles that the grouped W4A16 GEMMs go over: every expert has exactly T pairs, T on both sides of a 32-token block
+and of a tile's 128 tokens, through the prefill layer and through the decode layer with its matrix-core classes (flags 0x600, where
+the list is made from 129 tokens on).  Oracle: the layer in the reference's schedule (src/kimi_exec.cu:835-877); bound: 1e-2 of the
+largest element, which the bf16 roundings of a layer stay below (0.5e-2 measured with other orders of the sums)."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import oracle as O
+from blok_amd.lib import check
+from kxt import dev, moe_case, moe_cfg, moe_device_weights, moe_oracle_weights
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("path,T", [("prefill", t) for t in (31, 97, 128, 129, 257)] + [("decode", t) for t in (6, 128, 129, 161)])
+def test_every_expert_has_all_tokens(kxlib, ox, path, T):
+    H, I, SI, E, K = 1024, 1024, 512, 3, 3
+    print(f"grouped tiles {path} T={T}", flush=True)
+    host, n, x = moe_case(kxlib, H, I, SI, E, K, T, 77)
+    cfg = moe_cfg(H, I, SI, E, K)
+    w, bufs = moe_device_weights(host)
+    ws = C.c_void_p()
+    check(kxlib.kx_moe_workspace_create(C.byref(cfg), T, C.byref(ws)))
+    dn, dx = dev(n), dev(x)
+    call, flags = (kxlib.kx_moe_prefill_layer, 0) if path == "prefill" else (kxlib.kx_moe_decode_layer, 0x600)
+    check(call(C.byref(cfg), C.byref(w), ws, dn.ptr, dx.ptr, T, flags, None))
+    check(kxlib.kx_sync(None))
+    got = dx.to_numpy(np.uint16, (T, H))
+    check(kxlib.kx_moe_workspace_destroy(ws))
+    want, wo = x.copy(), moe_oracle_weights(host)
+    ox.ox_moe_layer(C.byref(wo), n.ctypes.data, want.ctypes.data, T, H, I, SI, E, K, 2.827, 0, 0, None, None, None, None, None)
+    err = O.max_rel(O.bf16_to_f32(got), O.bf16_to_f32(want))
+    assert err < 1e-2, err
