@@ -100,33 +100,36 @@ __device__ __forceinline__ int unit_row(int k, int i) {
   return EPI == KX_LIN_GLU ? (k / KX_GLU_BLOCK) * (2 * KX_GLU_BLOCK) + (k % KX_GLU_BLOCK) + i * KX_GLU_BLOCK : 2 * k + i;
 }
 
-constexpr int GEMV_WAVES = 8, UP = 4;  // UP: pieces per row in flight
-constexpr int CHUNK = 64 * UP * 8;     // columns per pass of a wave
+constexpr int GEMV_WAVES = 8;
+constexpr int CHUNK = 64 * 4 * 8;      // columns per pass of a wave; half of them where waves share a unit
 __host__ __device__ __forceinline__ int gemv_row(int ld) { return (ld + CHUNK - 1) / CHUNK * CHUNK; }
 // what a launch of lin_gemv_k goes over: one matrix for all tokens, the same with several variants of the rows, a matrix per
 // (token, choice), or per token one matrix and then the chosen experts'
 enum { GV_PLAIN = 0, GV_VARIANTS = 1, GV_EXPERT_IN = 2, GV_EXPERT_OUT = 3 };
 
-template <class T, int NT, int EPI, int MODE>
+// SPLIT > 1: that many waves share a unit, each with every SPLIT-th pass of its columns (gemv_split says where); a workgroup then has
+// one block of units.
+template <class T, int NT, int EPI, int MODE, int SPLIT>
 __global__ void __launch_bounds__(GEMV_WAVES * 64) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 2 ? 4 : 2)))
 lin_gemv_k(KxLinArgs a, KxExpertArgs x) {
   using E = Elem<T>;
   constexpr bool OWN = MODE >= GV_EXPERT_IN;  // a token of its own per blockIdx.y
   static_assert(!OWN || NT == 1, "one token per workgroup");
+  constexpr int UP = SPLIT > 1 ? 2 : 4, PASS = 64 * UP * 8, UNITS = GEMV_WAVES / SPLIT;  // UP: pieces per row of a pass
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   __shared__ float red[GEMV_WAVES][2 * NT];
   __shared__ int eid[OWN ? KX_MAX_TOP : 1];
   __shared__ float ewt[MODE == GV_EXPERT_IN ? KX_MAX_TOP : 1];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int ld = a.m.ld, np = ld >> 3, nc0 = (np + 64 * UP - 1) / (64 * UP);
-  const int nce = MODE == GV_EXPERT_OUT ? gemv_row(x.ld) / CHUNK : 0, nc = nc0 + (MODE == GV_EXPERT_OUT ? x.top * nce : 0);
-  const int xl = nc * CHUNK;  // a row in LDS, with zeros up to whole passes of the wave
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, place = wave / SPLIT, share = wave % SPLIT;  // place: of the wave's unit in its block
+  const int ld = a.m.ld, np = ld >> 3, nc0 = gemv_row(ld) / PASS;
+  const int nce = MODE == GV_EXPERT_OUT ? gemv_row(x.ld) / PASS : 0, nc = nc0 + (MODE == GV_EXPERT_OUT ? x.top * nce : 0);
+  const int xl = nc * PASS;  // a row in LDS, with zeros up to whole passes of the wave
   const int nv = MODE == GV_VARIANTS ? a.n_var : 1;
   T *xs = (T *)lds;                                              // [NT][nv][xl]
   float *u = (float *)(lds + (size_t)NT * nv * xl * sizeof(T));  // row scratch
   const int tokens = OWN ? 1 : a.tokens, pair = MODE == GV_EXPERT_IN ? blockIdx.y : 0;
   const int tok0 = MODE == GV_EXPERT_IN ? pair / x.top : MODE == GV_EXPERT_OUT ? blockIdx.y : 0;
-  const int units = (a.m.rows + 1) >> 1, nblk = (units + GEMV_WAVES - 1) / GEMV_WAVES;
+  const int units = (a.m.rows + 1) >> 1, nblk = (units + UNITS - 1) / UNITS;
   const T *w = (const T *)a.m.w;
   float weight = 1.0f;
   if constexpr (MODE == GV_EXPERT_IN) {
@@ -144,16 +147,18 @@ lin_gemv_k(KxLinArgs a, KxExpertArgs x) {
   // Past the last block the first row is asked for once more, by every wave: the number of loads in flight has to be the
   // same on every path, or the compiler waits for all of them.
   auto load = [&](typename E::Raw (&b)[2][UP], int blk, int c) {
-    const int k = blk < nblk ? min(blk * GEMV_WAVES + wave, units - 1) : 0;
+    const int k = blk < nblk ? min(blk * UNITS + place, units - 1) : 0;
     if (blk >= nblk) c = 0;
     const T *base = w;
     int bld = ld, bnp = np;
-    if (MODE == GV_EXPERT_OUT && c >= nc0) {  // the columns go on with the experts' matrices
-      const int j = (c - nc0) / nce;
-      c -= nc0 + j * nce;
-      base = (const T *)x.w + (size_t)__builtin_amdgcn_readfirstlane(eid[j]) * x.stride;
-      bld = x.ld;
-      bnp = x.ld >> 3;
+    if constexpr (MODE == GV_EXPERT_OUT) {
+      if (c >= nc0) {  // the columns go on with the experts' matrices
+        const int j = (c - nc0) / nce;
+        c -= nc0 + j * nce;
+        base = (const T *)x.w + (size_t)__builtin_amdgcn_readfirstlane(eid[j]) * x.stride;
+        bld = x.ld;
+        bnp = x.ld >> 3;
+      }
     }
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -165,25 +170,25 @@ lin_gemv_k(KxLinArgs a, KxExpertArgs x) {
       }
     }
   };
-  int blk = blockIdx.x, c = 0;
-  load(bufA, blk, 0);
+  int blk = blockIdx.x, c = share;
+  load(bufA, blk, c);
   if (MODE == GV_EXPERT_OUT && (int)threadIdx.x < x.top) eid[threadIdx.x] = x.ids[tok0 * x.top + threadIdx.x];
   uint32_t need = ~0u;  // variants that this workgroup's rows meet
   if constexpr (MODE == GV_VARIANTS) {
     need = 0;
-    for (int k = blockIdx.x; k < nblk; k += gridDim.x) need |= 1u << variant_of(a, 2 * k * GEMV_WAVES);
+    for (int k = blockIdx.x; k < nblk; k += gridDim.x) need |= 1u << variant_of(a, 2 * k * UNITS);
   }
 #pragma unroll
   for (int t = 0; t < NT; ++t)
     if (t < tokens) {
       T *row = xs + (size_t)t * nv * xl;
       for (int v = 0; v < nv; ++v)
-        for (int y = ld + threadIdx.x; y < nc0 * CHUNK; y += GEMV_WAVES * 64) row[(size_t)v * xl + y] = E::make(0.0f);
+        for (int y = ld + threadIdx.x; y < nc0 * PASS; y += GEMV_WAVES * 64) row[(size_t)v * xl + y] = E::make(0.0f);
       if constexpr (MODE == GV_EXPERT_OUT) {
-        const int el = nce * CHUNK;
+        const int el = nce * PASS;
         for (int j = 0; j < x.top; ++j) {
           const T *m = (const T *)x.mid + (size_t)(tok0 * x.top + j) * x.mid_ld;
-          for (int y = threadIdx.x; y < el; y += GEMV_WAVES * 64) row[nc0 * CHUNK + j * el + y] = y < x.ld ? m[y] : E::make(0.0f);
+          for (int y = threadIdx.x; y < el; y += GEMV_WAVES * 64) row[nc0 * PASS + j * el + y] = y < x.ld ? m[y] : E::make(0.0f);
         }
       }
       kxr::build_row<T>(a.row, tok0 + t, row, ld, u, xl, blockIdx.x == 0, need);
@@ -191,17 +196,17 @@ lin_gemv_k(KxLinArgs a, KxExpertArgs x) {
   float acc[2 * NT];
 #pragma unroll
   for (int v = 0; v < 2 * NT; ++v) acc[v] = 0.0f;
-  auto step = [&](typename E::Raw (&cur)[2][UP], typename E::Raw (&nxt)[2][UP]) {  // one chunk of columns of one unit per wave
-    const bool last = c + 1 == nc;
-    const int nblk_ = last ? blk + gridDim.x : blk, nc_ = last ? 0 : c + 1;
+  auto step = [&](typename E::Raw (&cur)[2][UP], typename E::Raw (&nxt)[2][UP]) {  // one pass over columns of one unit per wave
+    const bool last = c + SPLIT >= nc;
+    const int nblk_ = last ? blk + (SPLIT > 1 ? nblk : (int)gridDim.x) : blk, nc_ = last ? share : c + SPLIT;
     // lane i * NT + t < 2 NT finishes row i of the unit for token t; what it updates is asked for ahead of the next weights
-    const int unit = blk * GEMV_WAVES + wave, row = unit_row<EPI>(unit, lane / NT & 1), tok = NT > 1 ? lane % NT : 0;
-    const bool finish = EPI == KX_LIN_GLU ? lane < NT && tok < tokens && unit < units : lane < 2 * NT && row < a.m.rows && tok < tokens;
+    const int unit = blk * UNITS + place, row = unit_row<EPI>(unit, lane / NT & 1), tok = NT > 1 ? lane % NT : 0;
+    const bool finish = (SPLIT == 1 || share == 0) && (EPI == KX_LIN_GLU ? lane < NT && tok < tokens && unit < units : lane < 2 * NT && row < a.m.rows && tok < tokens);
     Streams<EPI> res;
     if (EPI >= KX_LIN_STREAMS && last && finish) res.load(a, tok0 + tok, row);
     load(nxt, nblk_, nc_);
     __builtin_amdgcn_sched_barrier(0);  // these loads are on their way before the last ones are waited for
-    const T *xv = xs + (MODE == GV_VARIANTS ? (size_t)variant_of(a, 2 * blk * GEMV_WAVES) * xl : 0);
+    const T *xv = xs + (MODE == GV_VARIANTS ? (size_t)variant_of(a, 2 * blk * UNITS) * xl : 0);
 #pragma unroll
     for (int j = 0; j < UP; ++j) {
       const int p = (c * UP + j) * 64 + lane;
@@ -224,6 +229,12 @@ lin_gemv_k(KxLinArgs a, KxExpertArgs x) {
       if (kxw::reduce_writer<2 * NT, 64>(lane))
 #pragma unroll
         for (int j = 0; j < kxw::reduce_out<2 * NT, 64>(); ++j) red[wave][kxw::reduce_index<2 * NT, 64>(lane, j)] = acc[j];
+      if constexpr (SPLIT > 1) {
+        __syncthreads();
+        if (finish)
+#pragma unroll
+          for (int k = 1; k < SPLIT; ++k) red[wave][lane] += red[wave + k][lane];  // the shares in their order
+      }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave reads its own sums back
       if (finish) {
         if constexpr (EPI == KX_LIN_GLU) put_glu<T>(a, MODE == GV_EXPERT_IN ? pair : tok, unit, red[wave][lane], red[wave][NT + lane], weight);
@@ -479,16 +490,34 @@ __global__ void __launch_bounds__(512, MI == 1 ? 4 : 2) lin_narrow_k(KxLinArgs a
 
 constexpr size_t GEMV_LDS = 150 * 1024;
 
+// Waves per unit of two rows: a workgroup has 16 rows with one, 8 with two, 4 with four.  As many as let the CU with the most rows have
+// the fewest, without more workgroups than run at once and with a pass for every wave.  2048 x 2048 and 2048 x 8192, one token, are 128
+// workgroups of 16 rows: 8.0 us on average, 7.1 as 256 of 8.
+int gemv_split(int rows, int passes, int grid_y) {
+  const long cus = std::max(1, kx_device_cus());
+  long best = 1, least = 0;
+  for (int s = 1; s <= 4; s *= 2) {
+    const long groups = (long)kx_cdiv((rows + 1) / 2, GEMV_WAVES / s) * grid_y, most = (groups + cus - 1) / cus * (16 / s);
+    if (s > 1 && (groups > 2 * cus || passes < s)) break;
+    if (s == 1 || most < least) best = s, least = most;
+  }
+  return (int)best;
+}
 // `lds` bytes of the dynamic part; grid_y: 1, or the tokens or (token, choice) pairs
-template <class T, int NT, int EPI, int MODE>
+template <class T, int NT, int EPI, int MODE, int SPLIT = 1>
 int gemv_launch(const KxLinArgs &a, const KxExpertArgs &x, size_t lds, int grid_y, hipStream_t st) {
+  if constexpr (SPLIT == 1 && EPI >= KX_LIN_STREAMS) {
+    const int split = gemv_split(a.m.rows, kx_cdiv(a.m.ld, CHUNK / 2), grid_y);
+    if (split == 2) return gemv_launch<T, NT, EPI, MODE, 2>(a, x, lds, grid_y, st);
+    if (split == 4) return gemv_launch<T, NT, EPI, MODE, 4>(a, x, lds, grid_y, st);
+  }
   static std::atomic<bool> attr{false};  // setting it twice from two threads is harmless
   if (!attr) {
-    KX_HIP(hipFuncSetAttribute((const void *)lin_gemv_k<T, NT, EPI, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)GEMV_LDS));
+    KX_HIP(hipFuncSetAttribute((const void *)lin_gemv_k<T, NT, EPI, MODE, SPLIT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)GEMV_LDS));
     attr = true;
   }
-  const int nblk = kx_cdiv((a.m.rows + 1) / 2, GEMV_WAVES), most = std::max(1, 2 * std::max(1, kx_device_cus()) / grid_y);
-  hipLaunchKernelGGL((lin_gemv_k<T, NT, EPI, MODE>), dim3(std::min(nblk, most), grid_y), dim3(GEMV_WAVES * 64), lds, st, a, x);
+  const int nblk = kx_cdiv((a.m.rows + 1) / 2, GEMV_WAVES / SPLIT), most = SPLIT > 1 ? nblk : std::max(1, 2 * std::max(1, kx_device_cus()) / grid_y);
+  hipLaunchKernelGGL((lin_gemv_k<T, NT, EPI, MODE, SPLIT>), dim3(std::min(nblk, most), grid_y), dim3(GEMV_WAVES * 64), lds, st, a, x);
   KX_LAUNCH_CHECK();
   return KX_OK;
 }
