@@ -141,7 +141,7 @@ struct KxDenseArgs {
   int arrivals = 0;
 };
 inline int kx_pad32(int n) { return (n + 31) & ~31; }
-constexpr size_t KX_DENSE_PART_FLOATS = (size_t)256 * 128 * 128;  // what a device of 256 CUs makes use of
+constexpr size_t KX_DENSE_PART_FLOATS = (size_t)256 * 256 * 256;  // what a device of 256 CUs makes use of: a large tile's sums each
 constexpr int KX_DENSE_ARRIVALS = 256;
 int kx_dense_gemm_launch(const KxDenseArgs &a, hipStream_t st);
 // kx_i4mm.hip: the experts of the work list with cnt_lo .. cnt_hi pairs as W4A16 products on the matrix cores with the

@@ -21,10 +21,11 @@ using kxtile::f32x16;
 typedef kxtile::Tile<uint16_t, 2, 2, 1, 2, 4> Short;  // 64 tokens x 128 rows: up to 64 tokens
 
 template <class TL, int MODE, bool DUAL, bool GROUP>
-__global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) dense_gemm_k(KxDenseArgs a, int parts) {
+__global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) dense_gemm_k(KxDenseArgs a, kxtile::Share share) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   constexpr int COLS = DUAL ? TL::BN / 2 : TL::BN;  // results per token of a tile
-  int m0, m_end, n0, part = 0, tile = 0;
+  int m0, m_end, n0;
+  kxtile::Place place = {0, 0, 1};
   const uint16_t *w0 = a.w0, *w1 = a.w1;
   if constexpr (GROUP) {
     const int4 g = a.work[blockIdx.y];
@@ -35,12 +36,11 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) dense_gemm_k(
     n0 = blockIdx.x * COLS;
     w0 += (size_t)g.x * a.group_stride;
   } else {
-    const int tm = (a.tokens + TL::BM - 1) / TL::BM, tiles = (int)gridDim.x / parts, item = kxtile::item_of(blockIdx.x, gridDim.x);
-    part = item / tiles;
-    tile = item - part * tiles;
-    m0 = tile % tm * TL::BM;
+    const int tm = (a.tokens + TL::BM - 1) / TL::BM;
+    place = kxtile::place_of(blockIdx.x, tm * ((a.rows + COLS - 1) / COLS), share);
+    m0 = place.tile % tm * TL::BM;
     m_end = a.tokens;
-    n0 = tile / tm * COLS;
+    n0 = place.tile / tm * COLS;
   }
   auto row_of = [&](int i) {
     if constexpr (MODE == KX_GG_KV) return i / a.seq * a.seq_jump + i % a.seq;
@@ -48,13 +48,15 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) dense_gemm_k(
   };
   const int nb = a.cols >> 6;
   f32x16 acc[TL::MI][TL::NI];
-  TL::run(lds, kxtile::cut(nb, part, parts), kxtile::cut(nb, part + 1, parts), [&](int r) -> const uint16_t * {
+  TL::run(lds, kxtile::cut(nb, place.part, place.of), kxtile::cut(nb, place.part + 1, place.of), [&](int r) -> const uint16_t * {
     if (r < TL::BM) return a.x + (size_t)row_of(min(m0 + r, m_end - 1)) * a.x_stride;
     r -= TL::BM;
     if constexpr (DUAL) return ((r >> 5 & 1) ? w1 : w0) + (size_t)min(n0 + (r >> 6) * 32 + (r & 31), a.rows - 1) * a.cols;
     else return w0 + (size_t)min(n0 + r, a.rows - 1) * a.cols;
   }, acc);
-  if (!GROUP && parts > 1 && !TL::gather(lds, acc, a.part + (size_t)tile * parts * TL::PART, a.arrived + tile, parts, part)) return;
+  if (!GROUP && place.of > 1 &&
+      !TL::gather(lds, acc, a.part + (size_t)(place.tile - share.whole) * place.of * TL::PART, a.arrived + place.tile - share.whole, place.of, place.part))
+    return;
   // block (i, j) of the wave: results t(v) of this lane, in row at(v) of out
   auto block = [&](int i, int j, auto &&put) {
     const int c = TL::col(j), n = n0 + (DUAL ? (c >> 6) * 32 + (c & 31) : c);
@@ -101,28 +103,28 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) dense_gemm_k(
 }
 
 template <class TL, int MODE, bool DUAL, bool GROUP>
-int launch_as(const KxDenseArgs &a, int parts, hipStream_t st) {
+int launch_as(const KxDenseArgs &a, kxtile::Share share, hipStream_t st) {
   static std::atomic<bool> attr{false};  // setting it twice from two threads is harmless
   if (!attr) {
     KX_HIP(hipFuncSetAttribute((const void *)dense_gemm_k<TL, MODE, DUAL, GROUP>, hipFuncAttributeMaxDynamicSharedMemorySize, TL::LDS));
     attr = true;
   }
   const int tn = kx_cdiv(a.rows, DUAL ? TL::BN / 2 : TL::BN), tm = kx_cdiv(a.tokens, TL::BM);
-  const dim3 grid = GROUP ? dim3(tn, a.groups, tm) : dim3((unsigned)((long)tn * tm * parts));
-  hipLaunchKernelGGL((dense_gemm_k<TL, MODE, DUAL, GROUP>), grid, dim3(TL::THREADS), TL::LDS, st, a, parts);
+  const dim3 grid = GROUP ? dim3(tn, a.groups, tm) : dim3(share.grid(tn * tm));
+  hipLaunchKernelGGL((dense_gemm_k<TL, MODE, DUAL, GROUP>), grid, dim3(TL::THREADS), TL::LDS, st, a, share);
   KX_LAUNCH_CHECK();
   return KX_OK;
 }
 template <class TL>
-int launch(const KxDenseArgs &a, int parts, hipStream_t st) {
-  if (a.w1) return launch_as<TL, KX_GG_BF16, true, false>(a, parts, st);
+int launch(const KxDenseArgs &a, kxtile::Share share, hipStream_t st) {
+  if (a.w1) return launch_as<TL, KX_GG_BF16, true, false>(a, share, st);
   switch (a.mode) {
-    case KX_GG_BF16: return launch_as<TL, KX_GG_BF16, false, false>(a, parts, st);
-    case KX_GG_F32: return launch_as<TL, KX_GG_F32, false, false>(a, parts, st);
-    case KX_GG_RESID: return launch_as<TL, KX_GG_RESID, false, false>(a, parts, st);
-    case KX_GG_KV: return launch_as<TL, KX_GG_KV, false, false>(a, parts, st);
+    case KX_GG_BF16: return launch_as<TL, KX_GG_BF16, false, false>(a, share, st);
+    case KX_GG_F32: return launch_as<TL, KX_GG_F32, false, false>(a, share, st);
+    case KX_GG_RESID: return launch_as<TL, KX_GG_RESID, false, false>(a, share, st);
+    case KX_GG_KV: return launch_as<TL, KX_GG_KV, false, false>(a, share, st);
   }
-  return launch_as<TL, KX_GG_F32_OF_BF16, false, false>(a, parts, st);
+  return launch_as<TL, KX_GG_F32_OF_BF16, false, false>(a, share, st);
 }
 
 }  // namespace
@@ -136,7 +138,7 @@ int kx_dense_gemm_launch(const KxDenseArgs &a, hipStream_t st) {
              "kx_dense_gemm: %d rows for %d heads, %d tokens", a.rows, a.heads, a.tokens);
   if (a.work) {
     KX_REQUIRE(a.pairs && a.groups > 0 && kx_cdiv(a.tokens, kxtile::Medium::BM) <= 65535, "kx_dense_gemm: %d groups", a.groups);
-    return launch_as<kxtile::Medium, KX_GG_BF16, false, true>(a, 1, st);
+    return launch_as<kxtile::Medium, KX_GG_BF16, false, true>(a, {0, 1}, st);
   }
   const int cus = kx_device_cus() > 0 ? kx_device_cus() : 1, staged = a.w1 ? 2 * kx_pad32(a.rows) : a.rows, blocks = a.cols >> 6;
   const size_t room = a.part && a.arrived ? a.part_floats : 0;
@@ -146,8 +148,8 @@ int kx_dense_gemm_launch(const KxDenseArgs &a, hipStream_t st) {
     p = p > blocks / 16 ? blocks / 16 : p;
     p = (size_t)p > room / Short::PART / tiles ? (long)(room / Short::PART / tiles) : p;
     if (p < 2 || tiles > a.arrivals) p = 1;
-    return launch<Short>(a, (int)p, st);
+    return launch<Short>(a, {0, (int)p}, st);
   }
   const kxtile::Choice c = kxtile::choose(a.tokens, staged, blocks, room, a.arrivals, cus);
-  return c.large ? launch<kxtile::Large>(a, 1, st) : launch<kxtile::Medium>(a, c.parts, st);
+  return c.large ? launch<kxtile::Large>(a, c.s, st) : launch<kxtile::Medium>(a, c.s, st);
 }

@@ -124,9 +124,9 @@ struct HybridModel : kx_model {
 };
 
 // partial sums of products that split their columns: two workgroups per CU with 64 rows of up to KX_NARROW_TOKENS tokens each, or
-// one with a tile of 128 x 128 (f32: two with one of 64 x 128)
+// one with a tile of 256 x 256 (f32: two with one of 64 x 128)
 constexpr int SPLIT_GROUPS = 512;
-constexpr size_t SPLIT_NARROW = (size_t)SPLIT_GROUPS * 64, SPLIT_TILES = (size_t)SPLIT_GROUPS / 2 * 128 * 128;
+constexpr size_t SPLIT_NARROW = (size_t)SPLIT_GROUPS * 64, SPLIT_TILES = (size_t)SPLIT_GROUPS / 2 * 256 * 256, SPLIT_SINGLES = (size_t)SPLIT_GROUPS * 64 * 128;
 
 // ---- kernels ----
 template <class T>
@@ -436,7 +436,7 @@ size_t HybridModel::layout(char *base) {
   history = (uint32_t *)at((size_t)max_context * B * 4);
   want = (int *)at((size_t)logit_rows() * 4);
   const size_t most = std::max(T, (size_t)logit_rows());
-  split_floats = f32 || most > KX_NARROW_TOKENS ? SPLIT_TILES : SPLIT_NARROW * most;
+  split_floats = f32 ? SPLIT_SINGLES : most > KX_NARROW_TOKENS ? SPLIT_TILES : SPLIT_NARROW * most;
   split_part = (float *)at(split_floats * 4);
   split_arrived = (int *)at(SPLIT_GROUPS * 4);
   scratch_bytes = p.total - weight_bytes - cache_bytes;

@@ -292,29 +292,31 @@ __device__ __forceinline__ size_t source_row(const KxExpertArgs &e, const Tile &
 }
 
 template <class T, class TL, int EPI, bool GROUP>
-__global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) lin_gemm_k(KxLinArgs a, KxExpertArgs e, const T *__restrict__ x, int x_ld, int parts) {
+__global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) lin_gemm_k(KxLinArgs a, KxExpertArgs e, const T *__restrict__ x, int x_ld, kxtile::Share share) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   Tile tl;
-  int n0, part = 0, tile = 0;
+  int n0;
+  kxtile::Place at = {0, 0, 1};
   if constexpr (GROUP) {
     if (!tile_of<true>(a, e, TL::BM, tl)) return;
     n0 = blockIdx.x * TL::BN;
   } else {
-    const int tm = (a.tokens + TL::BM - 1) / TL::BM, tiles = (int)gridDim.x / parts, item = kxtile::item_of(blockIdx.x, gridDim.x);
-    part = item / tiles;
-    tile = item - part * tiles;
-    n0 = tile / tm * TL::BN;
-    tl.m0 = tile % tm * TL::BM;
+    const int tm = (a.tokens + TL::BM - 1) / TL::BM;
+    at = kxtile::place_of(blockIdx.x, tm * ((a.m.rows + TL::BN - 1) / TL::BN), share);
+    n0 = at.tile / tm * TL::BN;
+    tl.m0 = at.tile % tm * TL::BM;
     tl.end = a.tokens;
     tl.w = 0;
   }
   x += (size_t)variant_of(a, n0) * a.tokens * x_ld;
   const int nb = a.m.ld / TL::COLS;
   f32x16 acc[TL::MI][TL::NI];
-  TL::run(lds, kxtile::cut(nb, part, parts), kxtile::cut(nb, part + 1, parts), [&](int r) {
+  TL::run(lds, kxtile::cut(nb, at.part, at.of), kxtile::cut(nb, at.part + 1, at.of), [&](int r) {
     return r < TL::BM ? x + source_row<GROUP>(e, tl, r) * x_ld : (const T *)a.m.w + tl.w + (size_t)min(n0 + r - TL::BM, a.m.rows - 1) * a.m.ld;
   }, acc);
-  if (!GROUP && parts > 1 && !TL::gather(lds, acc, a.part + (size_t)tile * parts * TL::PART, a.arrived + tile, parts, part)) return;
+  if (!GROUP && at.of > 1 &&
+      !TL::gather(lds, acc, a.part + (size_t)(at.tile - share.whole) * at.of * TL::PART, a.arrived + at.tile - share.whole, at.of, at.part))
+    return;
 #pragma unroll
   for (int i = 0; i < TL::MI; ++i) {
     if constexpr (EPI == KX_LIN_GLU) {
@@ -595,15 +597,15 @@ int small_slots_lds(const KxLinArgs &a, const KxExpertArgs &e) {
   return two < three ? SmallSlots::LDS : SmallSlots::LEAST_LDS;
 }
 template <class T, class TL, int EPI, bool GROUP>
-int tile_launch(const KxLinArgs &a, const KxExpertArgs &e, const T *x, int x_ld, int parts, hipStream_t st, int lds = TL::LDS) {
+int tile_launch(const KxLinArgs &a, const KxExpertArgs &e, const T *x, int x_ld, kxtile::Share share, hipStream_t st, int lds = TL::LDS) {
   static std::atomic<bool> attr{false};
   if (!attr) {
     KX_HIP(hipFuncSetAttribute((const void *)lin_gemm_k<T, TL, EPI, GROUP>, hipFuncAttributeMaxDynamicSharedMemorySize, TL::LDS));
     attr = true;
   }
   const int tn = kx_cdiv(a.m.rows, TL::BN);
-  const dim3 grid = GROUP ? dim3(tn, e.max_tiles) : dim3(tn * kx_cdiv(a.tokens, TL::BM) * parts);
-  hipLaunchKernelGGL((lin_gemm_k<T, TL, EPI, GROUP>), grid, dim3(TL::THREADS), lds, st, a, e, x, x_ld, parts);
+  const dim3 grid = GROUP ? dim3(tn, e.max_tiles) : dim3(share.grid(tn * kx_cdiv(a.tokens, TL::BM)));
+  hipLaunchKernelGGL((lin_gemm_k<T, TL, EPI, GROUP>), grid, dim3(TL::THREADS), lds, st, a, e, x, x_ld, share);
   KX_LAUNCH_CHECK();
   return KX_OK;
 }
@@ -617,14 +619,16 @@ int gemm_launch(const KxLinArgs &a, const KxExpertArgs &e, const T *x, int x_ld,
   const size_t room = a.part ? a.part_floats : 0;
   const int arrivals = a.arrived ? a.arrivals : 0, cus = std::max(1, kx_device_cus());
   if constexpr (sizeof(T) == 4) {
-    const int parts = GROUP ? 1 : kxtile::choose_single(a.tokens, a.m.rows, a.m.ld / kxtile::Single::COLS, room, arrivals, cus);
-    return tile_launch<float, kxtile::Single, EPI, GROUP>(a, e, x, x_ld, parts, st);
+    const kxtile::Share s = GROUP ? kxtile::Share{0, 1} : kxtile::choose_single(a.tokens, a.m.rows, a.m.ld / kxtile::Single::COLS, room, arrivals, cus);
+    return tile_launch<float, kxtile::Single, EPI, GROUP>(a, e, x, x_ld, s, st);
   } else if constexpr (GROUP) {
-    return e.tile_slots > 64 ? tile_launch<uint16_t, kxtile::Medium, EPI, true>(a, e, x, x_ld, 1, st) : tile_launch<uint16_t, SmallSlots, EPI, true>(a, e, x, x_ld, 1, st, small_slots_lds(a, e));
+    return e.tile_slots > 64 ? tile_launch<uint16_t, kxtile::Medium, EPI, true>(a, e, x, x_ld, {0, 1}, st) : tile_launch<uint16_t, SmallSlots, EPI, true>(a, e, x, x_ld, {0, 1}, st, small_slots_lds(a, e));
   } else {
     const kxtile::Choice c = kxtile::choose(a.tokens, a.m.rows, a.m.ld >> 6, room, arrivals, cus);
-    if (c.large && a.n_var == 1) return tile_launch<uint16_t, kxtile::Large, EPI, false>(a, e, x, x_ld, 1, st);  // variants begin at multiples of 128 rows
-    return tile_launch<uint16_t, kxtile::Medium, EPI, false>(a, e, x, x_ld, c.parts, st);
+    if (c.large && a.n_var == 1) return tile_launch<uint16_t, kxtile::Large, EPI, false>(a, e, x, x_ld, c.s, st);  // variants begin at multiples of 128 rows
+    // with variants a choice of large tiles is taken as medium ones, whole
+    const kxtile::Share whole = {kx_cdiv(a.tokens, kxtile::Medium::BM) * kx_cdiv(a.m.rows, kxtile::Medium::BN), 1};
+    return tile_launch<uint16_t, kxtile::Medium, EPI, false>(a, e, x, x_ld, c.large ? whole : c.s, st);
   }
 }
 
