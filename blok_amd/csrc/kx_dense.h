@@ -110,8 +110,8 @@ int kx_bucket_launch(const uint16_t *ids, int tokens, int experts, int topk, int
 // outputs of the matrix-core products: bf16; fp32 unrounded; fp32 holding the bf16-rounded value; bf16 residual add into out
 enum { KX_GG_BF16 = 0, KX_GG_F32 = 1, KX_GG_F32_OF_BF16 = 2, KX_GG_RESID = 3, KX_GG_KV = 4 /* kx_dense_gemm only */ };
 // kx_prefill.hip: the pairs of each expert against its W4A16 matrix, out[pair] = W[expert] x[pair / x_div], or swiglu(W0 x, W1 x).
-// tiles: records {expert, first, last, -} of up to KX_GROUPED_TILE pairs, the first *n_tiles as kx_grouped_tiles_launch leaves them for the
-// experts of `work`; without n_tiles tiles_max of them, those of fewer than cnt_lo pairs passed over.
+// tiles: records {expert, first, last, -}, the first *n_tiles of up to KX_GROUPED_TILE pairs as kx_grouped_tiles_launch leaves them for the
+// experts of `work`; without n_tiles tiles_max of any number of pairs, those of fewer than cnt_lo passed over.
 constexpr int KX_GROUPED_TILE = 128;
 inline size_t kx_grouped_tiles_max(size_t pairs, size_t experts) { return pairs / KX_GROUPED_TILE + (pairs < experts ? pairs : experts); }
 int kx_grouped_tiles_launch(const int4 *work, int n_slots, int cnt_lo, int4 *tiles, int *n_tiles, hipStream_t st);  // of at least cnt_lo pairs

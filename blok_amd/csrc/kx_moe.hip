@@ -299,7 +299,7 @@ static int moe_layer_body(const kx_config *c, const kx_moe_weights *w, kx_moe_wo
   }
   if (timed) KX_HIP(hipEventRecord(ws->ev[1], st));
   const int n_slots = (long)tokens * K < E ? tokens * K : E;
-  // the grouped GEMMs' records: the experts', which are tiles while none can have more pairs than one holds
+  // the grouped GEMMs' records: the experts' while one with more pairs than a tile holds is an exception (a workgroup then goes over them)
   const bool tiled = rmm && tokens > KX_GROUPED_TILE;
   const int4 *grouped = tiled ? ws->tiles : ws->work;
   const int *n_tiles = tiled ? ws->n_tiles : nullptr;

@@ -60,7 +60,7 @@ struct PfArgs {
   const uint16_t *s0, *s1;      // bf16 scales [E][N][K/32]
   const uint16_t *x;            // bf16 activation rows of K
   uint16_t *out;                // bf16 [pairs][N]
-  const int4 *tiles;            // {expert, first, last, _} of up to 128 pairs
+  const int4 *tiles;            // {expert, first, last, _}: tiles of up to 128 pairs, or experts
   const int *n_tiles;           // how many; nullptr: tiles_max
   int tiles_max, cnt_lo;        // records with fewer pairs are left to another launch
   int row_tiles;                // of 256 rows, WIDE 512
@@ -157,8 +157,8 @@ __global__ void __launch_bounds__(512, 1) grouped_gemm_k(PfArgs a) {
     const int n0 = item % a.row_tiles * (MODE == GG_WIDE ? 2 * BN : BN);
     const int4 wk = a.tiles[item / a.row_tiles];
     const int e = __builtin_amdgcn_readfirstlane(wk.x);
-    const int m0 = __builtin_amdgcn_readfirstlane(wk.y), p_end = __builtin_amdgcn_readfirstlane(wk.z);
-    if (e < 0 || p_end - m0 < a.cnt_lo) continue;
+    const int p_begin = __builtin_amdgcn_readfirstlane(wk.y), p_end = __builtin_amdgcn_readfirstlane(wk.z);
+    if (e < 0 || p_end - p_begin < a.cnt_lo) continue;
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));  // what follows from it is not worked out, and spilled, in front of the loop
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 31, lh = lane >> 5;
@@ -200,152 +200,156 @@ __global__ void __launch_bounds__(512, 1) grouped_gemm_k(PfArgs a) {
       for (int i = 0; i < MATS * 2; ++i)
         pf_copy16_to_lds(sc_src[i] + blk * (SC_BLOCK * 2) + piece * 8, sc0 + (blk & 1) * (BN * MATS * SC_STRIDE) + (wave * MATS * 2 + i) * 1024);
     };
-    const int nb = (p_end - m0 + 31) >> 5;  // 32-token blocks that hold tokens
-    // The activation tile goes global -> LDS like the weights.  A row of a K step is 128 B = 8 pieces;
-    // copy instruction ii covers rows 8 ii .. 8 ii + 7, slot (row, p') holding piece p' ^ ((row >> 1) & 7), so that
-    // the row-per-lane operand reads are free of bank conflicts without padding.  Rows past the expert's tokens
-    // read pair 0: they only feed accumulator rows that are never stored.
-    constexpr int XCMAX = 2;  // copy instructions per wave and K step at 128 tokens
-    const uint16_t *xc_src[XCMAX];
-    int xc_dst[XCMAX];
+    // Once for a tile of the list.  An expert's record is no tile: where a token has fewer candidates than choices (the others' bias
+    // -inf, logits that are no numbers) expert 0 stands for the missing ones, and has more pairs than there are tokens.
+    for (int m0 = p_begin; m0 < p_end; m0 += 128) {
+      const int nb = (p_end - m0 + 31) >> 5;  // 32-token blocks that hold tokens, of which a tile takes four
+      // The activation tile goes global -> LDS like the weights.  A row of a K step is 128 B = 8 pieces;
+      // copy instruction ii covers rows 8 ii .. 8 ii + 7, slot (row, p') holding piece p' ^ ((row >> 1) & 7), so that
+      // the row-per-lane operand reads are free of bank conflicts without padding.  Rows past the expert's tokens
+      // read pair 0: they only feed accumulator rows that are never stored.
+      constexpr int XCMAX = 2;  // copy instructions per wave and K step at 128 tokens
+      const uint16_t *xc_src[XCMAX];
+      int xc_dst[XCMAX];
 #pragma unroll
-    for (int q = 0; q < XCMAX; ++q) {
-      const int ii = wave + 8 * q;
-      const int slot = ii * 64 + lane, row = slot >> 3, piece = (slot & 7) ^ ((row >> 1) & 7);
-      const int pi = m0 + row;
-      const int pair = pi < p_end ? a.pairs[pi] : 0;
-      xc_src[q] = a.x + (size_t)(pair / a.x_div) * a.K + piece * 8;
-      xc_dst[q] = ii * 1024;
-    }
-
-    // the tile with NB token blocks, NB a compile-time constant so that the K loop has no branches
-    auto run = [&](auto nb_c) {
-      constexpr int NB = decltype(nb_c)::value;
-      kx_f32x16 acc[MATS][NB];
-#pragma unroll
-      for (int m = 0; m < MATS; ++m)
-#pragma unroll
-        for (int t = 0; t < NB; ++t)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) acc[m][t][i] = 0.0f;
-      struct WRaw {
-        uint4 q[MATS];  // the group's four packed words
-        float sc[MATS];
-      };
-      constexpr int XC = (NB * 4 + 7) / 8;  // activation copies per wave and K step (every wave issues XC)
-      auto copy_x = [&](int ks) {            // activations of K step ks into tile ks % 2
-#pragma unroll
-        for (int q = 0; q < XC; ++q) pf_copy16_to_lds(xc_src[q] + ks * BK, xs0 + (ks & 1) * XT * 2 + xc_dst[q]);
-      };
-      // this lane's weights of K step ks, from the LDS ring and the staged scales
-      auto fetch_w = [&](WRaw &r, int ks) {
-#pragma unroll
-        for (int m = 0; m < MATS; ++m) {
-          const int q = (ks & 1) * 2 + lh;
-          const uint8_t *st = w_ring + ((ks >> 1) & 1) * MATS * W_STAGE + m * W_STAGE;
-          r.q[m] = *(const uint4 *)(st + (trow * 4 + (q ^ ((trow >> 2) & 3))) * 16);
-          const uint8_t *sb = sc_lds + ((ks / SC_BLOCK) & 1) * (BN * MATS * SC_STRIDE) + (m * BN + trow) * SC_STRIDE;
-          const int el = (ks % SC_BLOCK) * 2 + lh;  // the lane's group among the block's 32
-          r.sc[m] = kx_bf16_f32(*(const uint16_t *)(sb + (((el >> 3) ^ ((trow >> 1) & 3)) * 8 + (el & 7)) * 2));
-        }
-      };
-      auto dequant_j = [&](const WRaw &r, int j, kx_bf16x8 (&b)[MATS]) {
-#pragma unroll
-        for (int m = 0; m < MATS; ++m) {
-          const float sc = r.sc[m];
-          const uint32_t w = j == 0 ? r.q[m].x : j == 1 ? r.q[m].y : j == 2 ? r.q[m].z : r.q[m].w;
-          b[m] = dequant_word(w, sc, sc * 0.0625f, -1032.0f * sc, -72.0f * sc, magic);
-        }
-      };
-      auto read_a = [&](const uint16_t *xs, int j, kx_bf16x8 (&av)[NB]) {
-        const int off = lr * 128 + (((lh * 4 + j) ^ (lr >> 1)) & 7) * 16;  // 128-byte rows, pieces xor-swizzled by the row
-#pragma unroll
-        for (int t = 0; t < NB; ++t) av[t] = *(const kx_bf16x8 *)((const uint8_t *)xs + t * 32 * 128 + off);
-      };
-      constexpr int VPER = (34 * MATS + NB * MATS - 1) / (NB * MATS);  // VALU instructions per MFMA
-      auto mfma_group = [&](const kx_bf16x8 (&av)[NB], const kx_bf16x8 (&b)[MATS], auto with_valu) {
-#pragma unroll
-        for (int t = 0; t < NB; ++t)
-#pragma unroll
-          for (int m = 0; m < MATS; ++m) acc[m][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[t], b[m], acc[m][t], 0, 0, 0);
-        // scheduling: one MFMA, then a share of the VALU work that prepares the next group
-#pragma unroll
-        for (int i = 0; i < NB * MATS; ++i) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          if constexpr (decltype(with_valu)::value) __builtin_amdgcn_sched_group_barrier(0x002, VPER, 0);
-        }
-      };
-      // one K step.  MFMA j contracts over columns 8 j .. +7 (lanes 0-31) and 32 + 8 j .. +7 (lanes 32-63); the
-      // operands of group j+1 (LDS reads, dequant) are produced while the matrix cores run group j.
-      auto step = [&](const WRaw &r, int ks) {
-        const uint16_t *xs = xs_lds + (ks & 1) * XT;
-        kx_bf16x8 b0[MATS], b1[MATS], a0[NB], a1[NB];
-        dequant_j(r, 0, b0);
-        read_a(xs, 0, a0);
-        read_a(xs, 1, a1);
-        dequant_j(r, 1, b1);
-        mfma_group(a0, b0, std::true_type{});
-        read_a(xs, 2, a0);
-        dequant_j(r, 2, b0);
-        mfma_group(a1, b1, std::true_type{});
-        read_a(xs, 3, a1);
-        dequant_j(r, 3, b1);
-        mfma_group(a0, b0, std::true_type{});
-        mfma_group(a1, b1, std::false_type{});
-      };
-
-      // prologue: stage 0 of the ring, the first scale block, the first activation tile
-      WRaw w0, w1;
-      copy_scales(0);
-      copy_x(0);
-      dma_stage(0);
-      pf_wait_copies<0>();
-      pf_barrier();
-      for (int ks = 0; ks < nk; ks += 2) {
-        // even step: the other ring stage and the other activation tile were last read behind a barrier.  Order of
-        // issue: activations of the next step, the ring copies, then (every SC_BLOCK steps) the next scale block; the
-        // activations have to land by the end of this step, the copies behind them stay in flight until the end of
-        // the odd step (a wave's copies complete in the order of issue)
-        const bool scales_now = ks % SC_BLOCK == 0 && ks + SC_BLOCK < nk;
-        if (ks + 1 < nk) copy_x(ks + 1);
-        if (ks + 2 < nk) dma_stage((ks >> 1) + 1);
-        if (scales_now) copy_scales(ks / SC_BLOCK + 1);
-        fetch_w(w0, ks);
-        step(w0, ks);
-        if (scales_now) pf_wait_copies<MATS * 4>();
-        else if (ks + 2 < nk) pf_wait_copies<MATS * 2>();
-        else pf_wait_copies<0>();
-        pf_barrier();
-        if (ks + 1 < nk) {
-          if (ks + 2 < nk) copy_x(ks + 2);
-          fetch_w(w1, ks + 1);
-          step(w1, ks + 1);
-          pf_wait_copies<0>();  // this wave's copies (ring stage, activations) have landed
-          pf_barrier();
-        }
+      for (int q = 0; q < XCMAX; ++q) {
+        const int ii = wave + 8 * q;
+        const int slot = ii * 64 + lane, row = slot >> 3, piece = (slot & 7) ^ ((row >> 1) & 7);
+        const int pi = m0 + row;
+        const int pair = pi < p_end ? a.pairs[pi] : 0;
+        xc_src[q] = a.x + (size_t)(pair / a.x_div) * a.K + piece * 8;
+        xc_dst[q] = ii * 1024;
       }
-      // epilogue: D[i][j], j = lane % 32 (weight row), i = 8*(v/4) + 4*(lane/32) + v%4 (token of the 32-token block)
+
+      // the tile with NB token blocks, NB a compile-time constant so that the K loop has no branches
+      auto run = [&](auto nb_c) {
+        constexpr int NB = decltype(nb_c)::value;
+        kx_f32x16 acc[MATS][NB];
 #pragma unroll
-      for (int t = 0; t < NB; ++t)
+        for (int m = 0; m < MATS; ++m)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int po = m0 + t * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
-          if (po < p_end) {
-            uint16_t *out = a.out + (size_t)a.pairs[po] * a.N;
-            if constexpr (DUAL) {
-              if (n0 + trow < a.N) out[n0 + trow] = kx_bf16_rne(kx_swiglu(kx_bfround(acc[0][t][v]), kx_bfround(acc[MATS - 1][t][v])));
-            } else {
+          for (int t = 0; t < NB; ++t)
 #pragma unroll
-              for (int m = 0; m < MATS; ++m)
-                if (n0 + m * BN + trow < a.N) out[n0 + m * BN + trow] = kx_bf16_rne(acc[m][t][v]);
-            }
+            for (int i = 0; i < 16; ++i) acc[m][t][i] = 0.0f;
+        struct WRaw {
+          uint4 q[MATS];  // the group's four packed words
+          float sc[MATS];
+        };
+        constexpr int XC = (NB * 4 + 7) / 8;  // activation copies per wave and K step (every wave issues XC)
+        auto copy_x = [&](int ks) {            // activations of K step ks into tile ks % 2
+#pragma unroll
+          for (int q = 0; q < XC; ++q) pf_copy16_to_lds(xc_src[q] + ks * BK, xs0 + (ks & 1) * XT * 2 + xc_dst[q]);
+        };
+        // this lane's weights of K step ks, from the LDS ring and the staged scales
+        auto fetch_w = [&](WRaw &r, int ks) {
+#pragma unroll
+          for (int m = 0; m < MATS; ++m) {
+            const int q = (ks & 1) * 2 + lh;
+            const uint8_t *st = w_ring + ((ks >> 1) & 1) * MATS * W_STAGE + m * W_STAGE;
+            r.q[m] = *(const uint4 *)(st + (trow * 4 + (q ^ ((trow >> 2) & 3))) * 16);
+            const uint8_t *sb = sc_lds + ((ks / SC_BLOCK) & 1) * (BN * MATS * SC_STRIDE) + (m * BN + trow) * SC_STRIDE;
+            const int el = (ks % SC_BLOCK) * 2 + lh;  // the lane's group among the block's 32
+            r.sc[m] = kx_bf16_f32(*(const uint16_t *)(sb + (((el >> 3) ^ ((trow >> 1) & 3)) * 8 + (el & 7)) * 2));
+          }
+        };
+        auto dequant_j = [&](const WRaw &r, int j, kx_bf16x8 (&b)[MATS]) {
+#pragma unroll
+          for (int m = 0; m < MATS; ++m) {
+            const float sc = r.sc[m];
+            const uint32_t w = j == 0 ? r.q[m].x : j == 1 ? r.q[m].y : j == 2 ? r.q[m].z : r.q[m].w;
+            b[m] = dequant_word(w, sc, sc * 0.0625f, -1032.0f * sc, -72.0f * sc, magic);
+          }
+        };
+        auto read_a = [&](const uint16_t *xs, int j, kx_bf16x8 (&av)[NB]) {
+          const int off = lr * 128 + (((lh * 4 + j) ^ (lr >> 1)) & 7) * 16;  // 128-byte rows, pieces xor-swizzled by the row
+#pragma unroll
+          for (int t = 0; t < NB; ++t) av[t] = *(const kx_bf16x8 *)((const uint8_t *)xs + t * 32 * 128 + off);
+        };
+        constexpr int VPER = (34 * MATS + NB * MATS - 1) / (NB * MATS);  // VALU instructions per MFMA
+        auto mfma_group = [&](const kx_bf16x8 (&av)[NB], const kx_bf16x8 (&b)[MATS], auto with_valu) {
+#pragma unroll
+          for (int t = 0; t < NB; ++t)
+#pragma unroll
+            for (int m = 0; m < MATS; ++m) acc[m][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[t], b[m], acc[m][t], 0, 0, 0);
+          // scheduling: one MFMA, then a share of the VALU work that prepares the next group
+#pragma unroll
+          for (int i = 0; i < NB * MATS; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            if constexpr (decltype(with_valu)::value) __builtin_amdgcn_sched_group_barrier(0x002, VPER, 0);
+          }
+        };
+        // one K step.  MFMA j contracts over columns 8 j .. +7 (lanes 0-31) and 32 + 8 j .. +7 (lanes 32-63); the
+        // operands of group j+1 (LDS reads, dequant) are produced while the matrix cores run group j.
+        auto step = [&](const WRaw &r, int ks) {
+          const uint16_t *xs = xs_lds + (ks & 1) * XT;
+          kx_bf16x8 b0[MATS], b1[MATS], a0[NB], a1[NB];
+          dequant_j(r, 0, b0);
+          read_a(xs, 0, a0);
+          read_a(xs, 1, a1);
+          dequant_j(r, 1, b1);
+          mfma_group(a0, b0, std::true_type{});
+          read_a(xs, 2, a0);
+          dequant_j(r, 2, b0);
+          mfma_group(a1, b1, std::true_type{});
+          read_a(xs, 3, a1);
+          dequant_j(r, 3, b1);
+          mfma_group(a0, b0, std::true_type{});
+          mfma_group(a1, b1, std::false_type{});
+        };
+
+        // prologue: stage 0 of the ring, the first scale block, the first activation tile
+        WRaw w0, w1;
+        copy_scales(0);
+        copy_x(0);
+        dma_stage(0);
+        pf_wait_copies<0>();
+        pf_barrier();
+        for (int ks = 0; ks < nk; ks += 2) {
+          // even step: the other ring stage and the other activation tile were last read behind a barrier.  Order of
+          // issue: activations of the next step, the ring copies, then (every SC_BLOCK steps) the next scale block; the
+          // activations have to land by the end of this step, the copies behind them stay in flight until the end of
+          // the odd step (a wave's copies complete in the order of issue)
+          const bool scales_now = ks % SC_BLOCK == 0 && ks + SC_BLOCK < nk;
+          if (ks + 1 < nk) copy_x(ks + 1);
+          if (ks + 2 < nk) dma_stage((ks >> 1) + 1);
+          if (scales_now) copy_scales(ks / SC_BLOCK + 1);
+          fetch_w(w0, ks);
+          step(w0, ks);
+          if (scales_now) pf_wait_copies<MATS * 4>();
+          else if (ks + 2 < nk) pf_wait_copies<MATS * 2>();
+          else pf_wait_copies<0>();
+          pf_barrier();
+          if (ks + 1 < nk) {
+            if (ks + 2 < nk) copy_x(ks + 2);
+            fetch_w(w1, ks + 1);
+            step(w1, ks + 1);
+            pf_wait_copies<0>();  // this wave's copies (ring stage, activations) have landed
+            pf_barrier();
           }
         }
-    };
-    if (nb == 1) run(std::integral_constant<int, 1>{});
-    else if (nb == 2) run(std::integral_constant<int, 2>{});
-    else if (nb == 3) run(std::integral_constant<int, 3>{});
-    else run(std::integral_constant<int, 4>{});
+        // epilogue: D[i][j], j = lane % 32 (weight row), i = 8*(v/4) + 4*(lane/32) + v%4 (token of the 32-token block)
+#pragma unroll
+        for (int t = 0; t < NB; ++t)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) {
+            const int po = m0 + t * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
+            if (po < p_end) {
+              uint16_t *out = a.out + (size_t)a.pairs[po] * a.N;
+              if constexpr (DUAL) {
+                if (n0 + trow < a.N) out[n0 + trow] = kx_bf16_rne(kx_swiglu(kx_bfround(acc[0][t][v]), kx_bfround(acc[MATS - 1][t][v])));
+              } else {
+#pragma unroll
+                for (int m = 0; m < MATS; ++m)
+                  if (n0 + m * BN + trow < a.N) out[n0 + m * BN + trow] = kx_bf16_rne(acc[m][t][v]);
+              }
+            }
+          }
+      };
+      if (nb == 1) run(std::integral_constant<int, 1>{});
+      else if (nb == 2) run(std::integral_constant<int, 2>{});
+      else if (nb == 3) run(std::integral_constant<int, 3>{});
+      else run(std::integral_constant<int, 4>{});
+    }
   }
 }
 

@@ -33,3 +33,32 @@ def test_every_expert_has_all_tokens(kxlib, ox, path, T):
     ox.ox_moe_layer(C.byref(wo), n.ctypes.data, want.ctypes.data, T, H, I, SI, E, K, 2.827, 0, 0, None, None, None, None, None)
     err = O.max_rel(O.bf16_to_f32(got), O.bf16_to_f32(want))
     assert err < 1e-2, err
+
+
+@pytest.mark.parametrize("path,T", [("decode", t) for t in (65, 128, 129)] + [("prefill", 31)])
+def test_fewer_candidates_than_choices(kxlib, ox, path, T):
+    """Five of eight experts have a bias of -inf: expert 0 stands for the missing choices of every token as well (src/kimi_exec.cu:391-393)
+    and has six pairs per token, more than a tile holds and more than there are tokens."""
+    H, I, SI, E, K = 1024, 1024, 512, 8, 8
+    print(f"masked experts {path} T={T}", flush=True)
+    host, n, x = moe_case(kxlib, H, I, SI, E, K, T, 78)
+    host = dict(host, router_bias=host["router_bias"].copy())
+    host["router_bias"][[1, 2, 4, 6, 7]] = -np.inf
+    cfg = moe_cfg(H, I, SI, E, K)
+    w, bufs = moe_device_weights(host)
+    ws = C.c_void_p()
+    check(kxlib.kx_moe_workspace_create(C.byref(cfg), T, C.byref(ws)))
+    call, flags = (kxlib.kx_moe_prefill_layer, 0) if path == "prefill" else (kxlib.kx_moe_decode_layer, 0x600)
+    views = [C.c_void_p() for _ in range(8)]
+    check(kxlib.kx_moe_workspace_views(ws, *(C.byref(v) for v in views)))
+    for v, width in ((views[6], I), (views[7], H)):                          # what is not written shows
+        check(kxlib.kx_dev_memset(v, 0x7f, T * K * width * 2, None))
+    dn, dx = dev(n), dev(x)
+    check(call(C.byref(cfg), C.byref(w), ws, dn.ptr, dx.ptr, T, flags, None))
+    check(kxlib.kx_sync(None))
+    got = dx.to_numpy(np.uint16, (T, H))
+    check(kxlib.kx_moe_workspace_destroy(ws))
+    want, wo = x.copy(), moe_oracle_weights(host)
+    ox.ox_moe_layer(C.byref(wo), n.ctypes.data, want.ctypes.data, T, H, I, SI, E, K, 2.827, 0, 0, None, None, None, None, None)
+    err = O.max_rel(O.bf16_to_f32(got), O.bf16_to_f32(want))
+    assert err < 1e-2, err
