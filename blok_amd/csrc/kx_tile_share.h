@@ -1,0 +1,90 @@
+// kx_tile_share.h -- which of the tiles of kx_gemm_tile.h a product takes, and how they are shared out over workgroups: host code
+// on sizes alone, in plain C++.
+#pragma once
+#include <stddef.h>
+
+namespace kxtile {
+
+struct TileSize {
+  int tokens, rows;
+  constexpr long sums() const { return (long)tokens * rows; }  // floats that a part of it leaves behind
+  constexpr long of(int t, int r) const { return (long)((t + tokens - 1) / tokens) * ((r + rows - 1) / rows); }
+};
+constexpr TileSize LARGE = {256, 256}, MEDIUM = {128, 128}, SINGLE = {64, 128};
+
+// How a product's tiles are shared out: a workgroup each for the first `whole`, `parts` workgroups with a part of the columns each for
+// every further one, so that no round leaves CUs idle.  The parts have the first ids: as they end, early and unevenly, whole tiles
+// take their places, where behind the whole tiles two of these would share a CU beside an idle one.
+struct Share {
+  int whole, parts;
+  int grid(int tiles) const { return whole + (tiles - whole) * parts; }
+};
+
+// The shortest of: every tile whole; those beyond whole rounds in at most 16 `parts`; all of them in parts.  time(n, p): of n workgroups
+// with a p-th of the columns, for n up to whole rounds of `round` workgroups and beyond.
+template <class Time>
+inline Share share(long tiles, int round, int most_parts, long room, int arrivals, Time time, double *best, int least_parts = 1) {
+  Share s = {(int)tiles, 1};
+  *best = least_parts > 1 ? 1e30 : time(tiles, 1);
+  for (long whole = tiles / round * round, i = 0; i < 2; whole = 0, ++i) {
+    const long rest = tiles - whole;
+    const int most = whole && most_parts > 16 ? 16 : most_parts;
+    for (int p = least_parts > 2 ? least_parts : 2; p <= most && rest > 0 && rest <= arrivals && rest * p <= room; ++p) {
+      const double t = (whole ? time(whole, 1) : 0.0) + time(rest, p);
+      if (t < *best) *best = t, s = {(int)whole, p};
+    }
+    if (whole == 0) break;
+  }
+  return s;
+}
+
+// Which tile, and how it is shared out, for one product of `tokens` x `rows` with `blocks` blocks of 64 columns.
+// Where the medium tiles leave CUs idle they take parts, of at least 16 blocks; beyond that the shorter of two estimates, in
+// us: a round of large tiles takes 12 + 1.6 per block on 256 CUs, of medium ones (two per CU) 4.5 + 1.09; a last round of medium tiles
+// that is not full takes its share of that, but no less than half, the time of one per CU; parts add the time to write their sums and to
+// read those of the others.  Measured against it (us, 32-bit
+// results, large / medium): large tiles in 1.5 rounds, medium ones in 3: 1536 x 16384 x 1024 75 / 69, x 2048 127 / 116, x 4096 228 / 211,
+// x 8192 453 / 434, x 16384 855 / 886; 2048 x 16384 x 2048 150 / 214, 2048 x 8448 x 2048 116 / 94, 2048 x 5120 x 2048 64 / 61, 2048 x 36864 x
+// 7168 1026 / 1265, 2048 x 7168 x 8192 252 / 329, 952 x 7168 x 18432 455 / 353, 700 x 12288 x 16384 379 / 428, 1024 x 36864 x 4096 359 / 345;
+// over 250 products of 300 to 2048 tokens with 2048 to 36864 x 1024 to 16384 the choice is at most 6 % behind the other one.
+// In parts: 300 x 2048 x 8192 71 alone, 32 in four, 100 x 2048 x 8192 73 and 29 in eight, 2048 x 384 x 7168 65 and 32 in four.
+struct Choice {
+  bool large;
+  Share s;
+};
+inline Choice choose(int tokens, int rows, int blocks, size_t part_floats, int arrivals, int cus) {
+  const long medium = MEDIUM.of(tokens, rows), large = LARGE.of(tokens, rows);
+  if (medium <= cus) {
+    long p = cus / medium;
+    if (p > blocks / 16) p = blocks / 16;
+    if ((size_t)p > part_floats / MEDIUM.sums() / medium) p = part_floats / MEDIUM.sums() / medium;
+    return p < 2 || medium > arrivals ? Choice{false, {(int)medium, 1}} : Choice{false, {0, (int)p}};
+  }
+  auto medium_time = [&](long n, int p) {
+    const long full = n * p / (2 * cus), rest = n * p % (2 * cus);
+    const double rounds = p == 1 && full == 0 ? 1.0 : full + (rest == 0 ? 0.0 : rest <= cus ? 0.5 : rest / (2.0 * cus));
+    return rounds * (4.5 + 1.09 * blocks / p) + (p > 1 ? 6.0 + 2.5 * p : 0.0);
+  };
+  auto large_time = [&](long n, int p) { return (n * p + cus - 1) / cus * (12 + 1.6 * blocks / p) + (p > 1 ? 12.0 + 8.0 * p : 0.0); };
+  double tm, tl;
+  const int most = blocks / 16 < 8 ? blocks / 16 : 8;
+  const Share sm = share(medium, 2 * cus, most, part_floats / MEDIUM.sums(), arrivals, medium_time, &tm);
+  const Share sl = share(large, cus, most, part_floats / LARGE.sums(), arrivals, large_time, &tl);
+  return tl < tm ? Choice{true, sl} : Choice{false, sm};
+}
+
+// For the 32-bit tile and blocks of 32 columns.
+inline Share choose_single(int tokens, int rows, int blocks, size_t part_floats, int arrivals, int cus) {
+  const long tiles = SINGLE.of(tokens, rows);
+  auto time = [&](long n, int p) { return (n * p + cus - 1) / cus * (1.5 + 0.97 * blocks / p + (p > 1 ? 2.5 : 0.0)); };
+  // where two workgroups per CU are not filled by whole tiles, never fewer parts than fill them: the sums are as much shorter, and in 32
+  // bits nearer to the exact ones (two parts instead of four were 1 % sooner and 8 % further off over a model of four layers; 64 x 1024 x
+  // 16384 in 16 parts instead of 64 65 % further off)
+  const long room = part_floats / SINGLE.sums(), most = blocks / 8;
+  long least = 2 * cus / tiles < most ? 2 * cus / tiles : most;
+  if (least > room / tiles) least = room / tiles;
+  double best;
+  return share(tiles, cus, (int)most, room, arrivals, time, &best, tiles > arrivals ? 1 : (int)least);
+}
+
+}  // namespace kxtile

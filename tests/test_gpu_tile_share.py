@@ -5,6 +5,7 @@ import pytest
 
 import kagalorn_case as KC
 import kagalorn_oracle as K
+import tile_share as TS
 from test_gpu_kagalorn import BF16_LOGITS, F32_LOGITS
 
 pytestmark = pytest.mark.gpu
@@ -22,3 +23,16 @@ def test_last_round_in_parts(kxlib, tmp_path, dtype, tokens, width, ff, bar):
         first = m.run(ids, [tokens], 1)
         assert KC.logit_error(first, want).max() < bar
         assert (m.run(ids, [tokens], 1) == first).all()
+
+
+def test_more_than_16_parts_in_32_bits(kxlib, tmp_path):
+    """The down product of a decode step: 16 x 512 x 8200, 4 tiles in 32 parts."""
+    cfg = KC.config([KC.delta(heads=4, kv_heads=2, dim=32, vdim=64, ff=8200)], width=512, vocab=300)
+    w = KC.weights(cfg, 8)
+    ids = np.stack([KC.tokens(cfg, 3, 40 + b) for b in range(16)])
+    want = np.stack([K.forward(cfg, w, s) for s in ids], 1)
+    assert TS.choices(TS.build(tmp_path), True, [(16, 512, 8256)], TS.F32) == [(0, 0, 32, 4)]
+    with KC.Model(KC.write(tmp_path, cfg, w), "float32", batch=16, context=3) as m:
+        first = m.run(ids, [1], 16)
+        assert KC.logit_error(first, want).max() < F32_LOGITS
+        assert (m.run(ids, [1], 16) == first).all()

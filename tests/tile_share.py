@@ -1,0 +1,26 @@
+"""The choice of tiles and parts for a product (blok_amd/csrc/kx_tile_share.h), compiled for the host."""
+import os
+import subprocess
+from collections import namedtuple
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CUS = 256
+# scratch of the hybrid decoder in 32 bits, of it and of Kimi-K2 in bf16: floats, counters
+F32, HYBRID, KIMI = (512 * 64 * 128, 512), (256 * 256 * 256, 512), (256 * 256 * 256, 256)
+Choice = namedtuple("Choice", "large whole parts tiles")
+
+
+def build(folder):
+    exe = str(folder / "tile_share")
+    r = subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Wextra", "-Werror", "-I" + os.path.join(os.path.dirname(HERE), "blok_amd", "csrc"),
+                        os.path.join(HERE, "tile_share.cpp"), "-o", exe], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr
+    return exe
+
+
+def choices(exe, f32, products, scratch):
+    """products: (tokens, rows, columns)"""
+    block = 32 if f32 else 64
+    text = "".join(f"{int(f32)} {t} {r} {c // block} {scratch[0]} {scratch[1]} {CUS}\n" for t, r, c in products)
+    out = subprocess.run([exe], input=text, capture_output=True, text=True, timeout=300, check=True).stdout
+    return [Choice(*map(int, line.split())) for line in out.splitlines()]
