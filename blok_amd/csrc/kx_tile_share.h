@@ -20,17 +20,17 @@ struct Share {
   int grid(int tiles) const { return whole + (tiles - whole) * parts; }
 };
 
-// The shortest of: every tile whole; those beyond whole rounds in at most 16 `parts`; all of them in parts.  time(n, p): of n workgroups
-// with a p-th of the columns, for n up to whole rounds of `round` workgroups and beyond.
+// The shortest of: every tile whole; those beyond whole rounds in at most 16 `parts`; all of them in parts.  time(whole, rest, p): of
+// `whole` tiles whole, in whole rounds of `round` where there are others, and `rest` tiles in p parts.
 template <class Time>
 inline Share share(long tiles, int round, int most_parts, long room, int arrivals, Time time, double *best, int least_parts = 1) {
   Share s = {(int)tiles, 1};
-  *best = least_parts > 1 ? 1e30 : time(tiles, 1);
+  *best = least_parts > 1 ? 1e30 : time(tiles, 0, 1);
   for (long whole = tiles / round * round, i = 0; i < 2; whole = 0, ++i) {
     const long rest = tiles - whole;
     const int most = whole && most_parts > 16 ? 16 : most_parts;
     for (int p = least_parts > 2 ? least_parts : 2; p <= most && rest > 0 && rest <= arrivals && rest * p <= room; ++p) {
-      const double t = (whole ? time(whole, 1) : 0.0) + time(rest, p);
+      const double t = time(whole, rest, p);
       if (t < *best) *best = t, s = {(int)whole, p};
     }
     if (whole == 0) break;
@@ -66,17 +66,22 @@ inline Choice choose(int tokens, int rows, int blocks, size_t part_floats, int a
     return rounds * (4.5 + 1.09 * blocks / p) + (p > 1 ? 6.0 + 2.5 * p : 0.0);
   };
   auto large_time = [&](long n, int p) { return (n * p + cus - 1) / cus * (12 + 1.6 * blocks / p) + (p > 1 ? 12.0 + 8.0 * p : 0.0); };
+  auto sum = [](auto time) { return [=](long whole, long rest, int p) { return (whole ? time(whole, 1) : 0.0) + (rest ? time(rest, p) : 0.0); }; };
   double tm, tl;
   const int most = blocks / 16 < 8 ? blocks / 16 : 8;
-  const Share sm = share(medium, 2 * cus, most, part_floats / MEDIUM.sums(), arrivals, medium_time, &tm);
-  const Share sl = share(large, cus, most, part_floats / LARGE.sums(), arrivals, large_time, &tl);
+  const Share sm = share(medium, 2 * cus, most, part_floats / MEDIUM.sums(), arrivals, sum(medium_time), &tm);
+  const Share sl = share(large, cus, most, part_floats / LARGE.sums(), arrivals, sum(large_time), &tl);
   return tl < tm ? Choice{true, sl} : Choice{false, sm};
 }
 
 // For the 32-bit tile and blocks of 32 columns.
 inline Share choose_single(int tokens, int rows, int blocks, size_t part_floats, int arrivals, int cus) {
   const long tiles = SINGLE.of(tokens, rows);
-  auto time = [&](long n, int p) { return (n * p + cus - 1) / cus * (1.5 + 0.97 * blocks / p + (p > 1 ? 2.5 : 0.0)); };
+  auto rounds = [&](long n, int p) { return (n * p + cus - 1) / cus * (1.5 + 0.97 * blocks / p + (p > 1 ? 2.5 : 0.0)); };
+  // Two rounds of parts in front of a single round of whole tiles end so unevenly that CUs are left with two of those beside idle
+  // ones: 464 x 6396 x 1024, 400 tiles, is a seventh slower with the last 144 in three parts each than whole.  Over 1900 products of more
+  // tiles than CUs, 5 to 1024 x 128 to 16000 x 512 to 16384, what is chosen takes 0.85 of the whole tiles' time on average and 1.07 at most.
+  auto time = [&](long whole, long rest, int p) { return whole == cus && rest * p > cus ? 1e30 : rounds(whole, 1) + rounds(rest, p); };
   // where two workgroups per CU are not filled by whole tiles, never fewer parts than fill them: the sums are as much shorter, and in 32
   // bits nearer to the exact ones (two parts instead of four were 1 % sooner and 8 % further off over a model of four layers; 64 x 1024 x
   // 16384 in 16 parts instead of 64 65 % further off)

@@ -28,3 +28,13 @@ def test_32_bit_products_of_few_tiles_fill_two_workgroups_per_cu(exe):
         if got.whole < got.tiles:                                                     # the scratch holds the parts
             assert got.tiles - got.whole <= T.F32[1] and (got.tiles - got.whole) * got.parts * 64 * 128 <= T.F32[0], (t, r, c, got)
             assert got.parts <= max(1, c // 32 // 8), (t, r, c, got)
+
+
+def test_32_bit_parts_beside_one_round_of_whole_tiles_are_one_round(exe):
+    rng = random.Random(6)
+    products = [(464, 6396, 1024), (488, 6250, 2816), (777, 2560, 1024)] + [(_log(rng, 64, 2048), _log(rng, 128, 20000), 64 * _log(rng, 4, 256)) for _ in range(20000)]
+    got = T.choices(exe, True, products, T.F32)
+    assert got[0].parts == got[1].parts == 1 and got[2].whole == T.CUS and got[2].parts == 4
+    for p, c in zip(products, got):
+        if c.whole == T.CUS and c.parts > 1:
+            assert (c.tiles - c.whole) * c.parts <= T.CUS, (p, c)
