@@ -38,3 +38,25 @@ def test_32_bit_parts_beside_one_round_of_whole_tiles_are_one_round(exe):
     for p, c in zip(products, got):
         if c.whole == T.CUS and c.parts > 1:
             assert (c.tiles - c.whole) * c.parts <= T.CUS, (p, c)
+
+
+def test_bf16_products_in_parts_only_where_that_is_sooner(exe):
+    """Products that were measured 11 to 27 % slower in parts (an estimate without the time for the sums) stay whole; those measured
+    sooner have parts: 2048 x 36864 x 7168 1035 us and 1072 whole, 1619 x 2627 x 7424 90 and 104."""
+    whole = [(395, 12951, 7168), (781, 7174, 8000), (965, 6110, 3904), (518, 9182, 8640), (604, 11562, 14528), (348, 15247, 3648), (399, 13619, 7424),
+             (66, 33687, 3392), (137, 23989, 3392), (831, 7193, 3712), (882, 6875, 5696), (461, 12868, 7552), (1501, 4007, 4416)]
+    for scratch in (T.HYBRID, T.KIMI):
+        assert all(c.parts == 1 for c in T.choices(exe, False, whole, scratch))
+        assert T.choices(exe, False, [(2048, 36864, 7168)], scratch) == [(1, 1024, 2, 1152)]
+    assert T.choices(exe, False, [(1619, 2627, 7424)], T.HYBRID)[0].parts > 1
+
+
+def test_bf16_parts_fit_the_scratch(exe):
+    rng = random.Random(7)
+    products = [(_log(rng, 65, 2048), _log(rng, 64, 40000), 64 * _log(rng, 1, 300)) for _ in range(20000)]
+    for scratch in (T.HYBRID, T.KIMI, (256 * 128 * 128, 256), (3000000, 100), (0, 0)):
+        for p, c in zip(products, T.choices(exe, False, products, scratch)):
+            rest, sums = c.tiles - c.whole, 256 * 256 if c.large else 128 * 128
+            assert rest >= 0 and c.parts >= 1 and (c.parts == 1 or rest > 0)
+            if c.parts > 1:
+                assert rest <= scratch[1] and rest * c.parts * sums <= scratch[0] and c.parts <= p[2] // 64 // 16, (p, c, scratch)
