@@ -429,7 +429,7 @@ size_t HybridModel::layout(char *base) {
   slots_of.tiles = (int4 *)at(tiles * sizeof(int4));
   slots_of.n_tiles = (int *)at(4);
   expert_y = (float *)at(expert_slots * W * 4);
-  logits = (float *)at((size_t)logit_rows() * c.vocab * 4);
+  logits = (float *)at((B + logit_rows()) * c.vocab * 4);
   argmax_scratch = (float *)at(KX_ARGMAX_SCRATCH_FLOATS(B) * 4);
   ids = (uint32_t *)at((size_t)max_context * B * 4);
   next = (uint32_t *)at(B * 4);

@@ -43,7 +43,7 @@ struct kx_model {
   int step_tokens = 1;    // tokens (positions x sequences) a step may carry
   char *arena = nullptr;
   uint64_t weight_bytes = 0, cache_bytes = 0, scratch_bytes = 0;
-  float *logits = nullptr, *argmax_scratch = nullptr;                // [logit_rows][vocab], argmax partials
+  float *logits = nullptr, *argmax_scratch = nullptr;                // [max_batch][vocab] of the sampled position, behind them [logit_rows][vocab] for row_logits; argmax partials
   uint32_t *ids = nullptr, *next = nullptr, *history = nullptr;      // [max_context][B], [B], [max_context][B]
   hipStream_t st = nullptr;
   hipEvent_t ev[3] = {nullptr, nullptr, nullptr};

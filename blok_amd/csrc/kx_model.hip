@@ -204,7 +204,7 @@ int layout(const kx_config *c, Plan &p, KimiModel *m) {
   auto *qabs = KX_AT(float *, BT * (size_t)c->heads * KVA * 4);
   auto *partial = KX_AT(float *, kx_mla_partial_floats(att_entries(c), c->heads, c->kv_rank, c->max_context) * 4);
   const size_t expand_bytes = base + p.total - (char *)qabs;  // the two are neighbours
-  auto *logits = KX_AT(float *, B * V * 4);
+  auto *logits = KX_AT(float *, 2 * B * V * 4);  // of the sampled position, and of other places
   auto *argmax_scratch = KX_AT(float *, KX_ARGMAX_SCRATCH_FLOATS(B) * 4);
   auto *ids = KX_AT(uint32_t *, (size_t)c->max_context * B * 4);
   auto *next = KX_AT(uint32_t *, B * 4);

@@ -49,44 +49,25 @@ int extend(kx_model *m, const uint32_t *h_ids, int n, const int32_t *want, int n
     rows.clear();
     at.clear();
     const size_t V = m->vocab;
-    const bool last = i + c == n;
-    bool sampled = false;  // places of which the step itself has left the logits
-    for (int w = 0; w < n_want; ++w) {
-      if (want[w] < i || want[w] >= i + c) continue;
-      if (want[w] == n - 1) {
-        sampled = true;
-        continue;
-      }
-      for (int b = 0; b < B; ++b) {
-        rows.push_back((want[w] - i) * B + b);
-        at.push_back(w * B + b);
-      }
-    }
-    auto copy_sampled = [&]() -> int {
-      for (int w = 0; w < n_want && sampled; ++w)
-        if (want[w] == n - 1) KX_HIP(hipMemcpyAsync(h_logits + (size_t)w * B * V, m->logits, B * V * 4, hipMemcpyDeviceToHost, m->st));
-      sampled = false;
-      return KX_OK;
-    };
-    // behind the sampled rows, where there is room; otherwise over them, and they are made once more
-    const size_t first = last && m->logit_rows() > B ? B : 0, room = m->logit_rows() - first;
-    if (first == 0 && (rc = copy_sampled())) return rc;
-    for (size_t r = 0; r < rows.size(); r += room) {
-      const size_t k = std::min(rows.size() - r, room);
-      if ((rc = m->row_logits(rows.data() + r, (int)k, m->logits + first * V))) return rc;
-      if ((rc = copy_sampled())) return rc;
+    for (int w = 0; w < n_want; ++w)
+      if (want[w] >= i && want[w] < i + c && want[w] != n - 1)
+        for (int b = 0; b < B; ++b) {
+          rows.push_back((want[w] - i) * B + b);
+          at.push_back(w * B + b);
+        }
+    float *const other = m->logits + (size_t)m->max_batch * V;
+    for (size_t r = 0; r < rows.size(); r += m->logit_rows()) {
+      const size_t k = std::min(rows.size() - r, (size_t)m->logit_rows());
+      if ((rc = m->row_logits(rows.data() + r, (int)k, other))) return rc;
       for (size_t j = 0, e; j < k; j = e) {  // rows that lie next to each other on both sides as one
         for (e = j + 1; e < k && at[r + e] == at[r + j] + (int)(e - j);) ++e;
-        KX_HIP(hipMemcpyAsync(h_logits + at[r + j] * V, m->logits + (first + j) * V, (e - j) * V * 4, hipMemcpyDeviceToHost, m->st));
+        KX_HIP(hipMemcpyAsync(h_logits + at[r + j] * V, other + j * V, (e - j) * V * 4, hipMemcpyDeviceToHost, m->st));
       }
       KX_HIP(hipStreamSynchronize(m->st));
     }
-    if ((rc = copy_sampled())) return rc;
-    if (last && first == 0 && !rows.empty()) {  // the sampled position's logits were overwritten; put them back
-      std::vector<int> end(B);
-      for (int b = 0; b < B; ++b) end[b] = (c - 1) * B + b;
-      if ((rc = m->row_logits(end.data(), B, m->logits))) return rc;
-    }
+    // the last place's are those that the step has sampled from
+    for (int w = 0; w < n_want && i + c == n; ++w)
+      if (want[w] == n - 1) KX_HIP(hipMemcpyAsync(h_logits + (size_t)w * B * V, m->logits, B * V * 4, hipMemcpyDeviceToHost, m->st));
   }
   return KX_OK;
 }
