@@ -31,16 +31,17 @@ using namespace kxg;
 // ---- RMSNorm ----------------------------------------------------------------------
 // one 256-thread workgroup per row; thread t owns 8-element chunks t, t+256, ...  A row of a few KB is bound by its trips to
 // memory: the first KEEP chunks of row and weight are asked for together and stay in registers (7168 columns, 12 rows: 5.9 us with a
-// second trip behind the sum, 4.8 to 5.1 so; 2048 rows 12.1 and 11.5).
+// second trip behind the sum, 4.8 to 5.1 so; 2048 rows 13.6 and 12.9).  Shorter rows make the second trip, to the L2 and beside other rows'
+// (2048 rows of 1024, 2048 and 4096 columns: 4.0, 5.4 and 8.2 us so, 5.1, 6.1 and 8.8 with KEEP).
+template <int KEEP>
 __global__ void __launch_bounds__(256) rmsnorm_k(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w,
                                                  uint16_t *__restrict__ y, int n, int x_stride, int y_stride,
                                                  float eps) {
   __shared__ float ws[4];
   const uint16_t *xr = x + (size_t)blockIdx.x * x_stride;
   uint16_t *yr = y + (size_t)blockIdx.x * y_stride;
-  constexpr int KEEP = 4;
   const int chunks = n >> 3;
-  uint4 xs[KEEP], gs[KEEP];
+  uint4 xs[KEEP + 1], gs[KEEP + 1];
 #pragma unroll
   for (int k = 0; k < KEEP; ++k) {
     const int c = min((int)threadIdx.x + k * 256, chunks - 1);
@@ -485,7 +486,8 @@ int kx_rmsnorm_launch(const uint16_t *x, const uint16_t *w, uint16_t *y, int tok
                       int y_stride, float eps, hipStream_t st) {
   KX_REQUIRE(n > 0 && n % 8 == 0, "kx_rmsnorm: n=%d must be a positive multiple of 8", n);
   KX_REQUIRE(tokens > 0, "kx_rmsnorm: tokens=%d must be positive", tokens);
-  hipLaunchKernelGGL(rmsnorm_k, dim3(tokens), dim3(256), 0, st, x, w, y, n, x_stride, y_stride, eps);
+  if (n > 4096) hipLaunchKernelGGL(rmsnorm_k<4>, dim3(tokens), dim3(256), 0, st, x, w, y, n, x_stride, y_stride, eps);
+  else hipLaunchKernelGGL(rmsnorm_k<0>, dim3(tokens), dim3(256), 0, st, x, w, y, n, x_stride, y_stride, eps);
   KX_LAUNCH_CHECK();
   return KX_OK;
 }
