@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include "kx_tile_share.h"
 
 enum {
   KX_EPI_BF16 = 0,        // y = bf(sum)                           matvec_bf16_k
@@ -143,6 +144,11 @@ struct KxDenseArgs {
 inline int kx_pad32(int n) { return (n + 31) & ~31; }
 constexpr size_t KX_DENSE_PART_FLOATS = (size_t)256 * 256 * 256;  // what a device of 256 CUs makes use of: a large tile's sums each
 constexpr int KX_DENSE_ARRIVALS = 256;
+// of it, what products of up to `tokens` tokens with up to `rows` rows (of both matrices) make use of: a medium tile's sums each where
+// their medium tiles leave none of the CUs a second one, and large ones are not taken
+inline size_t kx_dense_part_floats(int tokens, int rows) {
+  return kxtile::MEDIUM.of(tokens, rows) <= 256 ? (size_t)256 * kxtile::MEDIUM.sums() : KX_DENSE_PART_FLOATS;
+}
 int kx_dense_gemm_launch(const KxDenseArgs &a, hipStream_t st);
 // kx_i4mm.hip: the experts of the work list with cnt_lo .. cnt_hi pairs as W4A16 products on the matrix cores with the
 // weights streamed into registers, up to 32 tokens of an expert per pass (passes: grid depth; an expert's pairs beyond

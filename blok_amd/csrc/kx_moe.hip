@@ -17,6 +17,7 @@
 // More tokens: router GEMV, top-k + bucketing, and the shared gate+up GEMV are launches of
 // their own; beyond T*topk = E pairs the routed kernels run as two launches each (experts
 // with one pair, experts with more).
+#include <algorithm>
 #include "kx_common.h"
 #include "kx_dense.h"
 #include "kx_front.h"
@@ -43,6 +44,7 @@ struct kx_moe_workspace {
   uint16_t *eout;     // [T*topk, hidden]
   uint16_t *smid;     // [T, shared_inter]
   uint16_t *sy;       // [T, hidden] shared expert output (prefill path)
+  size_t split_floats[2] = {0, 0};
   float *split_part[2] = {nullptr, nullptr};  // partial sums of dense products that split their columns: of this stream, of the side stream
   int *split_arrived; // [2][KX_DENSE_ARRIVALS] zero between launches
   uint32_t *mid_hand; // [topk, moe_inter] tagged words: one token's mid values inside the resident routed launch
@@ -75,6 +77,10 @@ extern "C" int kx_moe_workspace_create(const kx_config *cfg, int32_t max_tokens,
   ws->max_tokens = max_tokens;
   ws->cfg = *cfg;
   const size_t T = (size_t)max_tokens, E = (size_t)cfg->experts, K = (size_t)cfg->topk;
+  if (max_tokens > 32) {  // the router's rows; the shared expert's gate and up, and down
+    ws->split_floats[0] = kx_dense_part_floats(max_tokens, cfg->experts);
+    ws->split_floats[1] = kx_dense_part_floats(max_tokens, std::max(2 * kx_pad32(cfg->shared_inter), cfg->hidden));
+  }
   struct { void **p; size_t bytes; } allocs[] = {
       {(void **)&ws->logits, T * E * 4}, {(void **)&ws->ids, T * K * 2}, {(void **)&ws->weights, T * K * 4},
       {(void **)&ws->counts, E * 4}, {(void **)&ws->offsets, (E + 1) * 4}, {(void **)&ws->pairs, T * K * 4},
@@ -82,7 +88,7 @@ extern "C" int kx_moe_workspace_create(const kx_config *cfg, int32_t max_tokens,
       {(void **)&ws->mid, T * K * (size_t)cfg->moe_inter * 2}, {(void **)&ws->eout, T * K * (size_t)cfg->hidden * 2},
       {(void **)&ws->smid, T * (size_t)cfg->shared_inter * 2}, {(void **)&ws->sy, T * (size_t)cfg->hidden * 2},
       {(void **)&ws->mid_hand, K * (size_t)cfg->moe_inter * 4}, {(void **)&ws->split_arrived, 2 * KX_DENSE_ARRIVALS * 4},
-      {(void **)&ws->split_part[0], max_tokens > 32 ? KX_DENSE_PART_FLOATS * 4 : 0}, {(void **)&ws->split_part[1], max_tokens > 32 ? KX_DENSE_PART_FLOATS * 4 : 0}};
+      {(void **)&ws->split_part[0], ws->split_floats[0] * 4}, {(void **)&ws->split_part[1], ws->split_floats[1] * 4}};
   for (auto &al : allocs) {
     if (!al.bytes) continue;
     hipError_t e = hipMalloc(al.p, al.bytes);
@@ -455,7 +461,7 @@ extern "C" int kx_moe_prefill_layer(const kx_config *c, const kx_moe_weights *w,
     KxDenseArgs d;
     d.w0 = (const uint16_t *)w0; d.w1 = (const uint16_t *)w1; d.x = x; d.x_stride = cols; d.out = out; d.out_stride = rows; d.mode = mode;
     d.tokens = tokens; d.rows = rows; d.cols = cols;
-    d.part = ws->split_part[side]; d.part_floats = KX_DENSE_PART_FLOATS; d.arrived = ws->split_arrived + side * KX_DENSE_ARRIVALS; d.arrivals = KX_DENSE_ARRIVALS;
+    d.part = ws->split_part[side]; d.part_floats = ws->split_floats[side]; d.arrived = ws->split_arrived + side * KX_DENSE_ARRIVALS; d.arrivals = KX_DENSE_ARRIVALS;
     return kx_dense_gemm_launch(d, side ? ws->side : st);
   };
   if ((rc = dense(w->d_shared_gate, w->d_shared_up, n, ws->smid, KX_GG_BF16, SI, H, 1))) return rc;

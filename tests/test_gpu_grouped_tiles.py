@@ -62,3 +62,18 @@ def test_fewer_candidates_than_choices(kxlib, ox, path, T):
     ox.ox_moe_layer(C.byref(wo), n.ctypes.data, want.ctypes.data, T, H, I, SI, E, K, 2.827, 0, 0, None, None, None, None, None)
     err = O.max_rel(O.bf16_to_f32(got), O.bf16_to_f32(want))
     assert err < 1e-2, err
+
+
+def test_scratch_of_a_small_workspace(kxlib):
+    """The parts of its products' columns: 16 MiB for the router and as much for the shared expert, where the tiles are few."""
+    cfg = moe_cfg(1024, 1024, 512, 32, 4)
+    free, total = [], C.c_size_t()
+    for make in (False, True):
+        ws = C.c_void_p()
+        if make:
+            check(kxlib.kx_moe_workspace_create(C.byref(cfg), 64, C.byref(ws)))
+        free.append(C.c_size_t())
+        check(kxlib.kx_dev_mem_info(C.byref(free[-1]), C.byref(total)))
+        if make:
+            check(kxlib.kx_moe_workspace_destroy(ws))
+    assert free[0].value - free[1].value < 64 << 20, (free[0].value - free[1].value) >> 20
