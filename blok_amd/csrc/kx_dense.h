@@ -151,8 +151,8 @@ inline size_t kx_dense_part_floats(int tokens, int rows) {
 }
 int kx_dense_gemm_launch(const KxDenseArgs &a, hipStream_t st);
 // kx_i4mm.hip: the experts of the work list with cnt_lo .. cnt_hi pairs as W4A16 products on the matrix cores with the
-// weights streamed into registers, up to 32 tokens of an expert per pass (passes: grid depth; an expert's pairs beyond
-// 32 * passes are not computed).  out[pair][N] = W[expert] x[pair / x_div], or swiglu(W0 x, W1 x) with two matrices.
+// weights streamed into registers, up to 32 pairs of an expert per pass (passes: grid depth; the last takes an expert's pairs beyond
+// 32 * passes as well).  out[pair][N] = W[expert] x[pair / x_div], or swiglu(W0 x, W1 x) with two matrices.
 // *done = false (nothing launched) when the shape is not the kernel's.
 int kx_i4mm_launch(bool dual, const uint32_t *w0, const uint16_t *s0, const uint32_t *w1, const uint16_t *s1, const uint16_t *x,
                    uint16_t *out, const int4 *work, const int *pairs, int n_slots, int N, int K, int x_div, size_t expert_w,

@@ -85,7 +85,7 @@ __device__ __forceinline__ uint32_t mm_bf2_to_h2(uint32_t u) {
   return __builtin_bit_cast(uint32_t, h);
 }
 
-// grid (N / 128, experts with work, passes of 32 tokens); 4 waves of 32 rows
+// grid (N / 128, experts with work, passes of 32 pairs); 4 waves of 32 rows
 template <bool DUAL>
 __global__ void __launch_bounds__(MM_WAVES * 64, 2) i4mm_k(MmArgs a) {
   constexpr int MATS = DUAL ? 2 : 1;
@@ -95,141 +95,145 @@ __global__ void __launch_bounds__(MM_WAVES * 64, 2) i4mm_k(MmArgs a) {
   if (rec.x < 0) return;
   const int cnt = rec.z - rec.y;
   if (cnt < a.cnt_lo || cnt > a.cnt_hi) return;
-  const int tok0 = rec.y + 32 * (int)blockIdx.z;
-  if (tok0 >= rec.z) return;
-  const int nt = min(32, rec.z - tok0);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = lane & 31, h = lane >> 5;
-  const int row0 = blockIdx.x * (MM_WAVES * 32) + wave * 32;
-  const int K = a.K, nr = K / MM_RUN;
-  const uint32_t magic = 0x64006400u;
-  uint8_t *wt = mm_lds + 2 * MM_XBUF + wave * (MATS * MM_WTILE);  // this wave's tiles, one per matrix
-  // loads of a run: instruction i takes rows 8 i .. + 7, eight lanes per row
-  const int lrow = lane >> 3, lseg = lane & 7;
-  const uint4 *wp[MATS];
-  wp[0] = (const uint4 *)(a.w0 + (size_t)rec.x * a.expert_w + (size_t)(row0 + lrow) * (K / 8)) + lseg;
-  if (DUAL) wp[1] = (const uint4 *)(a.w1 + (size_t)rec.x * a.expert_w + (size_t)(row0 + lrow) * (K / 8)) + lseg;
-  const size_t wstride8 = (size_t)8 * (K / 8) / 4;  // uint4 between rows 8 apart
-  // scales of the lane's row: groups 8 J + 4 h .. +3 of run J
-  const uint2 *sp[MATS];
-  sp[0] = (const uint2 *)(a.s0 + (size_t)rec.x * a.expert_s + (size_t)(row0 + r) * (K / 32)) + h;
-  if (DUAL) sp[1] = (const uint2 *)(a.s1 + (size_t)rec.x * a.expert_s + (size_t)(row0 + r) * (K / 32)) + h;
-  // activation staging: thread = (token, eighth): blocks of eight columns eighth, eighth + 8, ... of the run
-  const int xt = threadIdx.x >> 3, xe = threadIdx.x & 7;
-  const uint16_t *xrow = nullptr;
-  if (xt < nt) xrow = a.x + (size_t)(a.pairs[tok0 + xt] / a.x_div) * K;
-  uint4 xg[4];
-  auto load_x = [&](int J) {
+  // A pass of 32 pairs; the last of the grid goes on where there are more (an expert that stands for the missing choices of tokens
+  // with too few candidates has several pairs of a token).
+  for (int tok0 = rec.y + 32 * (int)blockIdx.z; tok0 < rec.z; tok0 = blockIdx.z + 1 == gridDim.z ? tok0 + 32 : rec.z) {
+    const int nt = min(32, rec.z - tok0);
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));  // what follows from it is not worked out, and spilled, in front of the loop
+    const int lane = tid & 63, wave = tid >> 6;
+    const int r = lane & 31, h = lane >> 5;
+    const int row0 = blockIdx.x * (MM_WAVES * 32) + wave * 32;
+    const int K = a.K, nr = K / MM_RUN;
+    const uint32_t magic = 0x64006400u;
+    uint8_t *wt = mm_lds + 2 * MM_XBUF + wave * (MATS * MM_WTILE);  // this wave's tiles, one per matrix
+    // loads of a run: instruction i takes rows 8 i .. + 7, eight lanes per row
+    const int lrow = lane >> 3, lseg = lane & 7;
+    const uint4 *wp[MATS];
+    wp[0] = (const uint4 *)(a.w0 + (size_t)rec.x * a.expert_w + (size_t)(row0 + lrow) * (K / 8)) + lseg;
+    if (DUAL) wp[1] = (const uint4 *)(a.w1 + (size_t)rec.x * a.expert_w + (size_t)(row0 + lrow) * (K / 8)) + lseg;
+    const size_t wstride8 = (size_t)8 * (K / 8) / 4;  // uint4 between rows 8 apart
+    // scales of the lane's row: groups 8 J + 4 h .. +3 of run J
+    const uint2 *sp[MATS];
+    sp[0] = (const uint2 *)(a.s0 + (size_t)rec.x * a.expert_s + (size_t)(row0 + r) * (K / 32)) + h;
+    if (DUAL) sp[1] = (const uint2 *)(a.s1 + (size_t)rec.x * a.expert_s + (size_t)(row0 + r) * (K / 32)) + h;
+    // activation staging: thread = (token, eighth): blocks of eight columns eighth, eighth + 8, ... of the run
+    const int xt = tid >> 3, xe = tid & 7;
+    const uint16_t *xrow = nullptr;
+    if (xt < nt) xrow = a.x + (size_t)(a.pairs[tok0 + xt] / a.x_div) * K;
+    uint4 xg[4];
+    auto load_x = [&](int J) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      xg[i] = xrow ? *(const uint4 *)(xrow + J * MM_RUN + (xe + 8 * i) * 8) : make_uint4(0u, 0u, 0u, 0u);
-  };
-  auto store_x = [&](int buf) {
+      for (int i = 0; i < 4; ++i)
+        xg[i] = xrow ? *(const uint4 *)(xrow + J * MM_RUN + (xe + 8 * i) * 8) : make_uint4(0u, 0u, 0u, 0u);
+    };
+    auto store_x = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      // columns 0..7 of the block as f16 pairs (0,1) (2,3) (4,5) (6,7), stored in the order 0, 4, 1, 5, 2, 6, 3, 7
-      const uint32_t p01 = mm_bf2_to_h2(xg[i].x), p23 = mm_bf2_to_h2(xg[i].y), p45 = mm_bf2_to_h2(xg[i].z), p67 = mm_bf2_to_h2(xg[i].w);
-      const uint4 o = make_uint4((p01 & 0xffffu) | (p45 << 16), (p01 >> 16) | (p45 & 0xffff0000u),
-                                 (p23 & 0xffffu) | (p67 << 16), (p23 >> 16) | (p67 & 0xffff0000u));
-      *(uint4 *)(mm_x + buf * MM_XBUF + xt * MM_XPITCH + (xe + 8 * i) * 16) = o;
-    }
-  };
-  // a run's weights as loaded (line layout) and its scales
-  uint4 ga[MATS][4], gb[MATS][4], gc[MATS][4];
-  uint2 sa[MATS], sb[MATS], sc3[MATS];
-  auto load_w = [&](uint4 (&gv)[MATS][4], uint2 (&sv)[MATS], int J) {
+      for (int i = 0; i < 4; ++i) {
+        // columns 0..7 of the block as f16 pairs (0,1) (2,3) (4,5) (6,7), stored in the order 0, 4, 1, 5, 2, 6, 3, 7
+        const uint32_t p01 = mm_bf2_to_h2(xg[i].x), p23 = mm_bf2_to_h2(xg[i].y), p45 = mm_bf2_to_h2(xg[i].z), p67 = mm_bf2_to_h2(xg[i].w);
+        const uint4 o = make_uint4((p01 & 0xffffu) | (p45 << 16), (p01 >> 16) | (p45 & 0xffff0000u),
+                                   (p23 & 0xffffu) | (p67 << 16), (p23 >> 16) | (p67 & 0xffff0000u));
+        *(uint4 *)(mm_x + buf * MM_XBUF + xt * MM_XPITCH + (xe + 8 * i) * 16) = o;
+      }
+    };
+    // a run's weights as loaded (line layout) and its scales
+    uint4 ga[MATS][4], gb[MATS][4], gc[MATS][4];
+    uint2 sa[MATS], sb[MATS], sc3[MATS];
+    auto load_w = [&](uint4 (&gv)[MATS][4], uint2 (&sv)[MATS], int J) {
 #pragma unroll
-    for (int m = 0; m < MATS; ++m) {
+      for (int m = 0; m < MATS; ++m) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) gv[m][i] = mm_stream16(wp[m] + i * wstride8 + J * 8);
-      sv[m] = sp[m][J * 2];
-    }
-  };
-  kx_f32x16 acc[MATS];
-#pragma unroll
-  for (int m = 0; m < MATS; ++m)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
-  // run J from the registers gv: through the wave's LDS tile into the operand layout, then 16 products per matrix
-  auto run = [&](const uint4 (&gv)[MATS][4], const uint2 (&sv)[MATS], int J) {
-    if (J + 1 < nr) load_x(J + 1);
-    uint4 w[MATS][4];
-#pragma unroll
-    for (int m = 0; m < MATS; ++m) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)  // row 8 i + lrow, piece lseg at slot lseg ^ (row % 8)
-        *(uint4 *)(wt + m * MM_WTILE + (8 * i + lrow) * 128 + ((lseg ^ lrow) & 7) * 16) = gv[m][i];
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        for (int i = 0; i < 4; ++i) gv[m][i] = mm_stream16(wp[m] + i * wstride8 + J * 8);
+        sv[m] = sp[m][J * 2];
+      }
+    };
+    kx_f32x16 acc[MATS];
 #pragma unroll
     for (int m = 0; m < MATS; ++m)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) w[m][g] = *(const uint4 *)(wt + m * MM_WTILE + r * 128 + (((4 * h + g) ^ r) & 7) * 16);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    const uint8_t *xb = mm_x + (J & 1) * MM_XBUF + r * MM_XPITCH + h * 256;  // token r, columns 128 h .. of the run
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      kx_h8 bx[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) bx[q] = *(const kx_h8 *)(xb + g * 64 + q * 16);
+      for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
+    // run J from the registers gv: through the wave's LDS tile into the operand layout, then 16 products per matrix
+    auto run = [&](const uint4 (&gv)[MATS][4], const uint2 (&sv)[MATS], int J) {
+      if (J + 1 < nr) load_x(J + 1);
+      uint4 w[MATS][4];
 #pragma unroll
       for (int m = 0; m < MATS; ++m) {
-        const uint32_t sd = (g & 2) ? sv[m].y : sv[m].x;
-        const float sf = kx_bits_f32((g & 1) ? (sd & 0xffff0000u) : (sd << 16));
-        const _Float16 s1 = (_Float16)sf, s16 = (_Float16)(sf * 0.0625f);
-        const kx_h2 sc = {s1, s1}, sc16 = {s16, s16};
-        acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(mm_dequant(w[m][g].x, sc, sc16, magic), bx[0], acc[m], 0, 0, 0);
-        acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(mm_dequant(w[m][g].y, sc, sc16, magic), bx[1], acc[m], 0, 0, 0);
-        acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(mm_dequant(w[m][g].z, sc, sc16, magic), bx[2], acc[m], 0, 0, 0);
-        acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(mm_dequant(w[m][g].w, sc, sc16, magic), bx[3], acc[m], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)  // row 8 i + lrow, piece lseg at slot lseg ^ (row % 8)
+          *(uint4 *)(wt + m * MM_WTILE + (8 * i + lrow) * 128 + ((lseg ^ lrow) & 7) * 16) = gv[m][i];
       }
-    }
-    if (J + 1 < nr) store_x((J + 1) & 1);
-    __syncthreads();
-  };
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+      for (int m = 0; m < MATS; ++m)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) w[m][g] = *(const uint4 *)(wt + m * MM_WTILE + r * 128 + (((4 * h + g) ^ r) & 7) * 16);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      const uint8_t *xb = mm_x + (J & 1) * MM_XBUF + r * MM_XPITCH + h * 256;  // token r, columns 128 h .. of the run
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        kx_h8 bx[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) bx[q] = *(const kx_h8 *)(xb + g * 64 + q * 16);
+#pragma unroll
+        for (int m = 0; m < MATS; ++m) {
+          const uint32_t sd = (g & 2) ? sv[m].y : sv[m].x;
+          const float sf = kx_bits_f32((g & 1) ? (sd & 0xffff0000u) : (sd << 16));
+          const _Float16 s1 = (_Float16)sf, s16 = (_Float16)(sf * 0.0625f);
+          const kx_h2 sc = {s1, s1}, sc16 = {s16, s16};
+          acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(mm_dequant(w[m][g].x, sc, sc16, magic), bx[0], acc[m], 0, 0, 0);
+          acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(mm_dequant(w[m][g].y, sc, sc16, magic), bx[1], acc[m], 0, 0, 0);
+          acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(mm_dequant(w[m][g].z, sc, sc16, magic), bx[2], acc[m], 0, 0, 0);
+          acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(mm_dequant(w[m][g].w, sc, sc16, magic), bx[3], acc[m], 0, 0, 0);
+        }
+      }
+      if (J + 1 < nr) store_x((J + 1) & 1);
+      __syncthreads();
+    };
 
-  // three register sets in rotation: two runs are on their way while one is multiplied
-  load_w(ga, sa, 0);
-  if (1 < nr) load_w(gb, sb, 1);
-  load_x(0);
-  store_x(0);
-  __syncthreads();
-  for (int J = 0; J < nr; J += 3) {
-    if (J + 2 < nr) load_w(gc, sc3, J + 2);
-    run(ga, sa, J);
-    if (J + 1 < nr) {
-      if (J + 3 < nr) load_w(ga, sa, J + 3);
-      run(gb, sb, J + 1);
-    }
-    if (J + 2 < nr) {
-      if (J + 4 < nr) load_w(gb, sb, J + 4);
-      run(gc, sc3, J + 2);
-    }
-  }
-  // D[i][j]: i = weight row 8 (v / 4) + 4 h + v % 4 of the wave's 32, j = token r
-  if (r < nt) {
-    const int pr = a.pairs[tok0 + r];
-    uint16_t *o = a.out + (size_t)pr * a.N + row0 + 4 * h;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      uint16_t v[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float y = acc[0][4 * q + e];
-        if (DUAL) y = kx_swiglu(kx_bfround(y), kx_bfround(acc[MATS - 1][4 * q + e]));
-        v[e] = kx_bf16_rne(y);
+    // three register sets in rotation: two runs are on their way while one is multiplied
+    load_w(ga, sa, 0);
+    if (1 < nr) load_w(gb, sb, 1);
+    load_x(0);
+    store_x(0);
+    __syncthreads();
+    for (int J = 0; J < nr; J += 3) {
+      if (J + 2 < nr) load_w(gc, sc3, J + 2);
+      run(ga, sa, J);
+      if (J + 1 < nr) {
+        if (J + 3 < nr) load_w(ga, sa, J + 3);
+        run(gb, sb, J + 1);
       }
-      *(uint2 *)(o + 8 * q) = make_uint2((uint32_t)v[0] | ((uint32_t)v[1] << 16), (uint32_t)v[2] | ((uint32_t)v[3] << 16));
+      if (J + 2 < nr) {
+        if (J + 4 < nr) load_w(gb, sb, J + 4);
+        run(gc, sc3, J + 2);
+      }
+    }
+    // D[i][j]: i = weight row 8 (v / 4) + 4 h + v % 4 of the wave's 32, j = token r
+    if (r < nt) {
+      const int pr = a.pairs[tok0 + r];
+      uint16_t *o = a.out + (size_t)pr * a.N + row0 + 4 * h;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        uint16_t v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float y = acc[0][4 * q + e];
+          if (DUAL) y = kx_swiglu(kx_bfround(y), kx_bfround(acc[MATS - 1][4 * q + e]));
+          v[e] = kx_bf16_rne(y);
+        }
+        *(uint2 *)(o + 8 * q) = make_uint2((uint32_t)v[0] | ((uint32_t)v[1] << 16), (uint32_t)v[2] | ((uint32_t)v[3] << 16));
+      }
     }
   }
 }
 
 }  // namespace
 
-// The experts of the work list with cnt_lo .. cnt_hi pairs (at most 32 per pass; more take further passes):
+// The experts of the work list with cnt_lo .. cnt_hi pairs (32 per pass):
 // out[pair][N] = W[expert] x[pair / x_div], or, with two matrices, swiglu(W0 x, W1 x).  *done = false, nothing
 // launched, when the shape is not the kernel's.
 int kx_i4mm_launch(bool dual, const uint32_t *w0, const uint16_t *s0, const uint32_t *w1, const uint16_t *s1, const uint16_t *x,

@@ -35,7 +35,7 @@ def test_every_expert_has_all_tokens(kxlib, ox, path, T):
     assert err < 1e-2, err
 
 
-@pytest.mark.parametrize("path,T", [("decode", t) for t in (65, 128, 129)] + [("prefill", 31)])
+@pytest.mark.parametrize("path,T", [("decode", t) for t in (40, 64, 65, 128, 129)] + [("prefill", 31)])
 def test_fewer_candidates_than_choices(kxlib, ox, path, T):
     """Five of eight experts have a bias of -inf: expert 0 stands for the missing choices of every token as well (src/kimi_exec.cu:391-393)
     and has six pairs per token, more than a tile holds and more than there are tokens."""
