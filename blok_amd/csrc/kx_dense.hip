@@ -130,7 +130,7 @@ __global__ void __launch_bounds__(512) gemv_tokblk_route_k(KxGemvArgs a, KxRoute
   __shared__ int s_last;
   __shared__ int s_mask[512];
   __shared__ int s_pos[512];
-  __shared__ uint16_t s_ids[1024];
+  __shared__ uint4 s_ids4[1024 / 8];
   const int tokens = a.tokens, t0 = blockIdx.y * 4, nt = min(4, tokens - t0);
   const float *logits = (const float *)a.out + (size_t)t0 * a.out_stride;
   const int stride = a.out_stride;
@@ -154,9 +154,11 @@ __global__ void __launch_bounds__(512) gemv_tokblk_route_k(KxGemvArgs a, KxRoute
   __syncthreads();
   if (!s_last) return;
   const int n_pairs = tokens * r.topk;
-  for (int p = threadIdx.x; p < n_pairs; p += blockDim.x) s_ids[p] = kx_arrive_load(r.ids + p);
+  uint16_t *s_ids = (uint16_t *)s_ids4;
+  for (int p = threadIdx.x; p < (n_pairs + 7) / 8 * 8; p += blockDim.x) s_ids[p] = p < n_pairs ? kx_arrive_load(r.ids + p) : (uint16_t)0xffff;
   __syncthreads();
-  kxr::bucket_masks(s_ids, tokens, r.topk, r.experts, r.counts, r.offsets, r.pairs, r.work, r.n_active, s_mask, s_pos, r.pair_work);
+  if (!kxr::bucket_masks(s_ids, tokens, r.topk, r.experts, r.counts, r.offsets, r.pairs, r.work, r.n_active, s_mask, s_pos, r.pair_work))
+    kxr::bucket_block(r.ids, n_pairs, r.experts, r.counts, r.offsets, r.pairs, r.work, r.n_active, s_ids4, s_mask, s_pos, true, r.pair_work);
   if (threadIdx.x == 0) kx_arrive_reset(r.counter);
 }
 

@@ -167,11 +167,11 @@ __device__ __forceinline__ void bucket_block(const uint16_t *__restrict__ ids, i
   }
 }
 
-// Bucketing of up to 32 tokens whose ids are distinct within a token (what the top-k gives): one bit per expert and
-// token, so an expert's count and a pair's place among its expert's pairs are population counts, and no thread goes
+// Bucketing of up to 32 tokens whose ids are distinct within a token (what the top-k gives while a token has as many candidates
+// as choices; false otherwise, and bucket_block has to follow): one bit per expert and token, so an expert's count and a pair's place among its expert's pairs are population counts, and no thread goes
 // over all pairs (bucket_block at 256 pairs: 15 us of the 384 threads each scanning them twice).  The results are
 // bucket_block's.  A workgroup of at least E threads, a multiple of 64 and at most 1024; s_mask and s_pos: E ints each.
-__device__ __forceinline__ void bucket_masks(const uint16_t *s_ids, int tokens, int topk, int E, int *__restrict__ counts,
+__device__ __forceinline__ bool bucket_masks(const uint16_t *s_ids, int tokens, int topk, int E, int *__restrict__ counts,
                                              int *__restrict__ offsets, int *__restrict__ pairs, int4 *__restrict__ work,
                                              int *__restrict__ n_active, int *s_mask, int *s_pos,
                                              int4 *__restrict__ pair_work) {
@@ -208,6 +208,7 @@ __device__ __forceinline__ void bucket_masks(const uint16_t *s_ids, int tokens, 
     total += c;
     total_active += a;
   }
+  if (total != n_pairs) return false;  // a token has an id twice; no thread needs the scans' arrays any more
   const int off = base_c + sc - cnt, slot = base_a + sa - act;
   if (tid < E) {
     counts[tid] = cnt;
@@ -229,6 +230,7 @@ __device__ __forceinline__ void bucket_masks(const uint16_t *s_ids, int tokens, 
     if (pair_work) pair_work[pos] = make_int4(id, pos, pos + 1, p);
     if (rank == 0) work[po >> 16] = make_int4(id, o, o + __popc(mm), p);
   }
+  return true;
 }
 
 // top-k of `tokens` tokens (wave w takes tokens w, w + waves, ...), then the bucketing, by one workgroup
@@ -249,10 +251,10 @@ __device__ __forceinline__ void route_block(const float *__restrict__ logits, co
     topk_token<EPL, COHERENT>(logits + (size_t)t * E, bias, ids + (size_t)t * topk, weights + (size_t)t * topk, E, topk,
                               routed_scale, threadIdx.x & 63, s_ids + t * topk);
   __syncthreads();
-  if (MASKS && n_pairs > 64 && tokens <= 32 && n_pairs < 65536 && (blockDim.x & 63) == 0)
-    bucket_masks(s_ids, tokens, topk, E, counts, offsets, pairs, work, n_active, s_cnt, s_act, pair_work);
-  else
-    bucket_block(ids, n_pairs, E, counts, offsets, pairs, work, n_active, s_ids4, s_cnt, s_act, true, pair_work);
+  if (MASKS && n_pairs > 64 && tokens <= 32 && n_pairs < 65536 && (blockDim.x & 63) == 0 &&
+      bucket_masks(s_ids, tokens, topk, E, counts, offsets, pairs, work, n_active, s_cnt, s_act, pair_work))
+    return;
+  bucket_block(ids, n_pairs, E, counts, offsets, pairs, work, n_active, s_ids4, s_cnt, s_act, true, pair_work);
 }
 
 // route_block with the per-lane expert count chosen at run time; COHERENT: the logits were written by other

@@ -1,7 +1,8 @@
 """The list of tiles that the grouped W4A16 GEMMs go over: every expert has exactly T pairs, T on both sides of a 32-token block
-and of a tile's 128 tokens, through the prefill layer (the list is made from 5 tokens on) and through the decode layer with its matrix-core classes (flags 0x600, where
-the list is made from 129 tokens on).  Oracle: the layer in the reference's schedule (src/kimi_exec.cu:835-877); bound: 1e-2 of the
-largest element, which the bf16 roundings of a layer stay below (0.5e-2 measured with other orders of the sums)."""
+and of a tile's 128 tokens, through the prefill layer (the list is made from 5 tokens on) and through the decode layer with its
+matrix-core classes (flags 0x600, where the list is made from 129 tokens on).  Oracle: the layer in the reference's schedule
+(src/kimi_exec.cu:835-877); bound: 1e-2 of the largest element, which the bf16 roundings of a layer stay below (0.5e-2 measured with
+other orders of the sums)."""
 import ctypes as C
 
 import numpy as np
@@ -35,20 +36,21 @@ def test_every_expert_has_all_tokens(kxlib, ox, path, T):
     assert err < 1e-2, err
 
 
-@pytest.mark.parametrize("path,T", [("decode", t) for t in (40, 64, 65, 128, 129)] + [("prefill", 31)])
-def test_fewer_candidates_than_choices(kxlib, ox, path, T):
-    """Five of eight experts have a bias of -inf: expert 0 stands for the missing choices of every token as well (src/kimi_exec.cu:391-393)
+@pytest.mark.parametrize("path,T,E", [("decode", t, 8) for t in (9, 31, 32, 40, 64, 65, 128, 129)] + [("prefill", 31, 8)] +
+                         [("plain", t, e) for t, e in ((1, 8), (4, 8), (9, 80), (10, 80), (32, 8), (64, 8))])
+def test_fewer_candidates_than_choices(kxlib, ox, path, T, E):
+    """All experts but three have a bias of -inf: expert 0 stands for the missing choices of every token as well (src/kimi_exec.cu:391-393)
     and has six pairs per token, more than a tile holds and more than there are tokens."""
-    H, I, SI, E, K = 1024, 1024, 512, 8, 8
-    print(f"masked experts {path} T={T}", flush=True)
+    H, I, SI, K = 1024, 1024, 512, 8
+    print(f"masked experts {path} T={T} E={E}", flush=True)
     host, n, x = moe_case(kxlib, H, I, SI, E, K, T, 78)
     host = dict(host, router_bias=host["router_bias"].copy())
-    host["router_bias"][[1, 2, 4, 6, 7]] = -np.inf
+    host["router_bias"][[e for e in range(E) if e not in (0, 3, 5)]] = -np.inf
     cfg = moe_cfg(H, I, SI, E, K)
     w, bufs = moe_device_weights(host)
     ws = C.c_void_p()
     check(kxlib.kx_moe_workspace_create(C.byref(cfg), T, C.byref(ws)))
-    call, flags = (kxlib.kx_moe_prefill_layer, 0) if path == "prefill" else (kxlib.kx_moe_decode_layer, 0x600)
+    call, flags = (kxlib.kx_moe_prefill_layer, 0) if path == "prefill" else (kxlib.kx_moe_decode_layer, 0x600 if path == "decode" else 0)
     views = [C.c_void_p() for _ in range(8)]
     check(kxlib.kx_moe_workspace_views(ws, *(C.byref(v) for v in views)))
     for v, width in ((views[6], I), (views[7], H)):                          # what is not written shows
