@@ -36,6 +36,25 @@ def test_every_expert_has_all_tokens(kxlib, ox, path, T):
     assert err < 1e-2, err
 
 
+def _run(kxlib, host, n, x, H, I, SI, E, K, T, path, flags):
+    """The layer, with expert outputs that show where nothing is written."""
+    cfg = moe_cfg(H, I, SI, E, K)
+    w, bufs = moe_device_weights(host)
+    ws = C.c_void_p()
+    check(kxlib.kx_moe_workspace_create(C.byref(cfg), T, C.byref(ws)))
+    views = [C.c_void_p() for _ in range(8)]
+    check(kxlib.kx_moe_workspace_views(ws, *(C.byref(v) for v in views)))
+    for v, width in ((views[6], I), (views[7], H)):
+        check(kxlib.kx_dev_memset(v, 0x7f, T * K * width * 2, None))
+    dn, dx = dev(n), dev(x)
+    call = kxlib.kx_moe_prefill_layer if path == "prefill" else kxlib.kx_moe_decode_layer
+    check(call(C.byref(cfg), C.byref(w), ws, dn.ptr, dx.ptr, T, flags, None))
+    check(kxlib.kx_sync(None))
+    got = dx.to_numpy(np.uint16, (T, H))
+    check(kxlib.kx_moe_workspace_destroy(ws))
+    return got
+
+
 @pytest.mark.parametrize("path,T,E", [("decode", t, 8) for t in (9, 31, 32, 40, 64, 65, 128, 129)] + [("prefill", 31, 8)] +
                          [("plain", t, e) for t, e in ((1, 8), (4, 8), (9, 80), (10, 80), (32, 8), (64, 8))])
 def test_fewer_candidates_than_choices(kxlib, ox, path, T, E):
@@ -46,20 +65,35 @@ def test_fewer_candidates_than_choices(kxlib, ox, path, T, E):
     host, n, x = moe_case(kxlib, H, I, SI, E, K, T, 78)
     host = dict(host, router_bias=host["router_bias"].copy())
     host["router_bias"][[e for e in range(E) if e not in (0, 3, 5)]] = -np.inf
-    cfg = moe_cfg(H, I, SI, E, K)
-    w, bufs = moe_device_weights(host)
-    ws = C.c_void_p()
-    check(kxlib.kx_moe_workspace_create(C.byref(cfg), T, C.byref(ws)))
-    call, flags = (kxlib.kx_moe_prefill_layer, 0) if path == "prefill" else (kxlib.kx_moe_decode_layer, 0x600 if path == "decode" else 0)
-    views = [C.c_void_p() for _ in range(8)]
-    check(kxlib.kx_moe_workspace_views(ws, *(C.byref(v) for v in views)))
-    for v, width in ((views[6], I), (views[7], H)):                          # what is not written shows
-        check(kxlib.kx_dev_memset(v, 0x7f, T * K * width * 2, None))
-    dn, dx = dev(n), dev(x)
-    check(call(C.byref(cfg), C.byref(w), ws, dn.ptr, dx.ptr, T, flags, None))
-    check(kxlib.kx_sync(None))
-    got = dx.to_numpy(np.uint16, (T, H))
-    check(kxlib.kx_moe_workspace_destroy(ws))
+    got = _run(kxlib, host, n, x, H, I, SI, E, K, T, path, 0x600 if path == "decode" else 0)
+    want, wo = x.copy(), moe_oracle_weights(host)
+    ox.ox_moe_layer(C.byref(wo), n.ctypes.data, want.ctypes.data, T, H, I, SI, E, K, 2.827, 0, 0, None, None, None, None, None)
+    err = O.max_rel(O.bf16_to_f32(got), O.bf16_to_f32(want))
+    assert err < 1e-2, err
+
+
+@pytest.mark.parametrize("path,T", [("decode", 129), ("decode", 161), ("decode", 300), ("prefill", 161)])
+def test_experts_of_every_class_beside_each_other(kxlib, ox, path, T):
+    """Experts with all tokens, with 1, 2, 3, 33 and 97 of them and with none: those of 1 and 2 pairs are no tiles of the decode layer,
+    another kernel computes them at the same time.  What no kernel writes shows."""
+    H, I, SI, E, K = 1024, 1024, 512, 12, 3
+    print(f"classes {path} T={T}", flush=True)
+    host, n, x = moe_case(kxlib, H, I, SI, E, K, T, 79)
+    order = np.random.default_rng(T).permutation(E)                                 # so that the classes are not in the order of their sizes
+    pick, at = np.zeros((T, E), bool), 0
+    pick[:, order[0]] = True
+    for e, count in zip(order[1:], (1, 2, 3, 33, 97)):
+        pick[(at + np.arange(count)) % T, e] = True
+        at += count
+    for t in range(T):                                                              # the rest to two experts
+        pick[t, order[6:8][:K - pick[t].sum()]] = True
+    assert (pick.sum(1) == K).all() and pick.sum(0)[order[:6]].tolist() == [T, 1, 2, 3, 33, 97] and (pick.sum(0) == 0).sum() >= 4
+    host = dict(host, router_gate=np.zeros((E, H), np.float32), router_bias=np.zeros(E, np.float32))
+    host["router_gate"][np.arange(E), np.arange(E)] = 4.0
+    host["router_gate"] = (host["router_gate"].view(np.uint32) >> 16).astype(np.uint16).reshape(-1)
+    n = n.copy()
+    n[:, :E] = (np.where(pick, 2.0, -2.0).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
+    got = _run(kxlib, host, n, x, H, I, SI, E, K, T, *(("prefill", 0) if path == "prefill" else ("decode", 0x600)))
     want, wo = x.copy(), moe_oracle_weights(host)
     ox.ox_moe_layer(C.byref(wo), n.ctypes.data, want.ctypes.data, T, H, I, SI, E, K, 2.827, 0, 0, None, None, None, None, None)
     err = O.max_rel(O.bf16_to_f32(got), O.bf16_to_f32(want))
