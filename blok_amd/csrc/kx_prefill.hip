@@ -108,7 +108,8 @@ __device__ __forceinline__ kx_bf16x8 dequant_word(uint32_t w, float sc, float sc
 
 // The tiles of up to 128 pairs of every group with at least cnt_lo pairs, {expert, first, last, -}, those of four 32-token
 // blocks first and those of one last (a last round of the short ones ends sooner): tiles of a group in turn, so that workgroups which run at
-// the same time share its weights.  One workgroup, a thread per group; n_tiles[0]: how many.
+// the same time read the same weights, through one L2 where the row tiles are a multiple of 8 (gate and up of 2048 rows), through several
+// where they are not (14 of a down product with 7168).  One workgroup, a thread per group; n_tiles[0]: how many.
 __global__ void __launch_bounds__(1024) grouped_tiles_k(const int4 *__restrict__ work, int n_slots, int cnt_lo, int4 *__restrict__ tiles, int *__restrict__ n_tiles) {
   __shared__ int4 sum[2][1024];
   const int i = threadIdx.x;
