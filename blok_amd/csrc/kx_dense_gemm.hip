@@ -2,10 +2,10 @@
 // logits, W_UV per head, with the epilogues of the mat-vec kernels they stand for (matvec_bf16_k / matvec_bf16_f32_k with
 // add_k, silu_mul_k and the rounding of the logits, src/kimi_exec.cu:248-298, :718-734).
 //
-// The main loop is kx_gemm_tile.h's.  With two matrices (SwiGLU) a tile's rows are blocks of 32 gate rows and their 32 up rows in
+// The main loops are kx_gemm_tile.h's and kx_gemm_turns.h's.  With two matrices (SwiGLU) a tile's rows are blocks of 32 gate rows and their 32 up rows in
 // turn, so that a wave holds both halves of a pair.  Before these tiles the products went through the W4A16 kernel's loop with 64
-// tokens a tile and every lane loading its own row of the matrix: 400 TFLOP/s where these reach 1030 (2048 tokens, gate
-// and up of 2 x 18432 x 7168 with SwiGLU 2.7 ms then).
+// tokens a tile and every lane loading its own row of the matrix: 400 TFLOP/s where these reach 1200 (2048 tokens, gate
+// and up of 2 x 18432 x 7168 with SwiGLU 2.7 ms then, 0.9 now).
 // fp32 sums over exact bf16 products: a tolerance path like every matrix-core path (max-rel 1e-2), not used where tokens
 // have to be identical.
 #include <atomic>
@@ -15,8 +15,6 @@
 #include "kx_math.h"
 
 namespace {
-
-using kxtile::f32x16;
 
 typedef kxtile::Tile<uint16_t, 2, 2, 1, 2, 4> Short;  // 64 tokens x 128 rows: up to 64 tokens
 
@@ -47,7 +45,7 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) dense_gemm_k(
     else return GROUP ? a.pairs[i] : i;
   };
   const int nb = a.cols >> 6;
-  f32x16 acc[TL::MI][TL::NI];
+  typename TL::Sums acc;
   TL::run(lds, kxtile::cut(nb, place.part, place.of), kxtile::cut(nb, place.part + 1, place.of), [&](int r) -> const uint16_t * {
     if (r < TL::BM) return a.x + (size_t)row_of(min(m0 + r, m_end - 1)) * a.x_stride;
     r -= TL::BM;
@@ -55,49 +53,54 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) dense_gemm_k(
     else return w0 + (size_t)min(n0 + r, a.rows - 1) * a.cols;
   }, acc);
   if (!GROUP && place.of > 1 &&
-      !TL::gather(lds, acc, a.part + (size_t)(place.tile - share.whole) * place.of * TL::PART, a.arrived + place.tile - share.whole, place.of, place.part))
+      !kxtile::gather<TL>(lds, acc, a.part + (size_t)(place.tile - share.whole) * place.of * TL::PART, a.arrived + place.tile - share.whole, place.of, place.part))
     return;
-  // block (i, j) of the wave: results t(v) of this lane, in row at(v) of out
-  auto block = [&](int i, int j, auto &&put) {
-    const int c = TL::col(j), n = n0 + (DUAL ? (c >> 6) * 32 + (c & 31) : c);
-    if (n < a.rows) put([&](int v) { return m0 + TL::row(i, v) < m_end; }, [&](int v) { return (size_t)row_of(min(m0 + TL::row(i, v), m_end - 1)) * a.out_stride + n; });
-  };
+  // result c (of a tile's COLS) of block (i, j): in row at(v) of out, if there is one
+  auto result = [&](int j) { const int c = TL::col(j); return n0 + (DUAL ? (c >> 6) * 32 + (c & 31) : c); };
+  auto in = [&](int i, int v) { return m0 + TL::row(i, v) < m_end; };
+  auto at = [&](int i, int v, int n) { return (size_t)row_of(min(m0 + TL::row(i, v), m_end - 1)) * a.out_stride + n; };
+  constexpr int STEP = DUAL ? 32 / TL::SIDE : 1;  // blocks of gate rows in front of their up rows
 #pragma unroll
   for (int i = 0; i < TL::MI; ++i) {
+    if constexpr (MODE == KX_GG_RESID && !DUAL) {  // x = bf(x + bf(y))  (add_k, :248-251); 16 are read before the first is written
 #pragma unroll
-    for (int j = 0; j < TL::NI; j += DUAL ? 2 : 1) {
-      block(i, j, [&](auto &&in, auto &&at) {
+      for (int e0 = 0; e0 < TL::NI * TL::V; e0 += 16) {
+        uint16_t old[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) old[u] = ((const uint16_t *)a.out)[at(i, (e0 + u) % TL::V, min(result((e0 + u) / TL::V), a.rows - 1))];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+          const int j = (e0 + u) / TL::V, v = (e0 + u) % TL::V, n = result(j);
+          if (in(i, v) && n < a.rows) ((uint16_t *)a.out)[at(i, v, n)] = kx_bf16_rne(kx_bf16_f32(old[u]) + kx_bfround(acc[i][j][v]));
+        }
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < TL::NI; ++j) {
+        if (DUAL && j / STEP % 2) continue;
+        const int n = result(j);
+        if (n >= a.rows) continue;
         if constexpr (MODE == KX_GG_KV) {
-          const int n = n0 + TL::col(j), per = a.k_dim + a.v_dim, hd = n / per, d = n - hd * per;
+          const int per = a.k_dim + a.v_dim, hd = n / per, d = n - hd * per;
           const bool key = d < a.k_dim;
           uint16_t *to = key ? (uint16_t *)a.out + d : a.out_v + (d - a.k_dim);
           const int ld = key ? a.k_ld : a.v_ld;
 #pragma unroll
-          for (int v = 0; v < 16; ++v)
-            if (in(v)) {
+          for (int v = 0; v < TL::V; ++v)
+            if (in(i, v)) {
               const int t = m0 + TL::row(i, v), b = t / a.seq;
               to[((size_t)(b * a.heads + hd) * a.cap + t - b * a.seq) * ld] = kx_bf16_rne(acc[i][j][v]);
             }
-        } else if constexpr (DUAL) {
-#pragma unroll
-          for (int v = 0; v < 16; ++v)
-            if (in(v)) ((uint16_t *)a.out)[at(v)] = kx_bf16_rne(kx_swiglu(kx_bfround(acc[i][j][v]), kx_bfround(acc[i][j + 1][v])));
-        } else if constexpr (MODE == KX_GG_RESID) {  // x = bf(x + bf(y))  (add_k, :248-251); all are read before the first is written
-          uint16_t old[16];
-#pragma unroll
-          for (int v = 0; v < 16; ++v) old[v] = ((const uint16_t *)a.out)[at(v)];
-#pragma unroll
-          for (int v = 0; v < 16; ++v)
-            if (in(v)) ((uint16_t *)a.out)[at(v)] = kx_bf16_rne(kx_bf16_f32(old[v]) + kx_bfround(acc[i][j][v]));
         } else {
 #pragma unroll
-          for (int v = 0; v < 16; ++v)
-            if (in(v)) {
-              if constexpr (MODE == KX_GG_BF16) ((uint16_t *)a.out)[at(v)] = kx_bf16_rne(acc[i][j][v]);
-              else ((float *)a.out)[at(v)] = MODE == KX_GG_F32 ? acc[i][j][v] : kx_bfround(acc[i][j][v]);
+          for (int v = 0; v < TL::V; ++v)
+            if (in(i, v)) {
+              if constexpr (DUAL) ((uint16_t *)a.out)[at(i, v, n)] = kx_bf16_rne(kx_swiglu(kx_bfround(acc[i][j][v]), kx_bfround(acc[i][j + STEP][v])));
+              else if constexpr (MODE == KX_GG_BF16) ((uint16_t *)a.out)[at(i, v, n)] = kx_bf16_rne(acc[i][j][v]);
+              else ((float *)a.out)[at(i, v, n)] = MODE == KX_GG_F32 ? acc[i][j][v] : kx_bfround(acc[i][j][v]);
             }
         }
-      });
+      }
     }
   }
 }
@@ -151,5 +154,5 @@ int kx_dense_gemm_launch(const KxDenseArgs &a, hipStream_t st) {
     return launch<Short>(a, {0, (int)p}, st);
   }
   const kxtile::Choice c = kxtile::choose(a.tokens, staged, blocks, room, a.arrivals, cus);
-  return c.large ? launch<kxtile::Large>(a, c.s, st) : launch<kxtile::Medium>(a, c.s, st);
+  return c.large ? launch<kxtile::Large>(a, c.s, st) : c.twin ? launch<kxtile::Twin>(a, c.s, st) : launch<kxtile::Medium>(a, c.s, st);
 }

@@ -14,10 +14,9 @@
 //   -- behind it nobody reads the present block any more, its last operands are in registers --, asks for two more halves
 //   in its place and reads the next block's first operands.
 // What bounds it: a wave reads (MI + NI) KB of operands for MI NI products of 32 cycles, and LDS gives a CU about 128 bytes a
-// cycle: waves of 2 x 4 blocks stay below that with the copies' writes, waves of 2 x 2 do not; and a block of the 256 x 256 tile is
-// 64 KB for 2048 cycles of products and takes about as long to arrive.  2048 x 36864 x 7168 (32-bit result): 1026 us, the copies
-// alone 833, the products alone 710, everything but the copies 795.  A fifth slot, which keeps the queue of copies from
-// running dry, is worth 2 to 8 % to two workgroups per CU with few tiles and costs the large tile 4 %.
+// cycle: waves of 2 x 2 blocks are at that limit with the copies' writes, and every wave asks for its copies between products.  Where
+// the columns are long enough the tiles of kx_gemm_turns.h are sooner, 256 x 256 throughout (2048 x 7168 x 8192 231 us as this loop, 171).
+// A fifth slot, which keeps the queue of copies from running dry, is worth 2 to 8 % to two workgroups per CU with few tiles.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -49,6 +48,9 @@ template <> struct Piece<float> {
 
 template <class T, int WM_, int WN_, int MI_, int NI_, int SLOTS_>
 struct Tile {
+  typedef f32x16 Block;
+  static constexpr int V = 16, SIDE = 32;
+  typedef Block Sums[MI_][NI_];
   static constexpr int COLS = 128 / sizeof(T);  // columns of a block
   static constexpr int SLOTS = SLOTS_, WM = WM_, WN = WN_, MI = MI_, NI = NI_, WAVES = WM * WN, THREADS = WAVES * 64;
   static constexpr int BM = WM * MI * 32, BN = WN * NI * 32, SLOT = (BM > BN ? BM : BN) * 128, LDS = SLOTS * SLOT;
@@ -156,46 +158,55 @@ struct Tile {
     return (((int)threadIdx.x >> 6) / WN * MI + i) * 32 + 8 * (v >> 2) + 4 * (threadIdx.x >> 5 & 1) + (v & 3);
   }
 
-  // The sums of `parts` workgroups that hold a part of the columns each, added in the parts' order by the one that arrives last
-  // (kx_arrive.h); false for the others.  part: parts * PART floats of this tile; arrived: its counter.
-  static __device__ __forceinline__ bool gather(uint8_t *lds, f32x16 (&acc)[MI][NI], float *part, int *arrived, int parts, int p) {
-    int &last = *(int *)lds;  // behind the barrier below nobody reads operands any more
-    uint64_t *at = (uint64_t *)part;
-    constexpr size_t PER = PART / 2;
+};
+
+// The sums of `parts` workgroups that hold a part of the columns each, added in the parts' order by the one that arrives last
+// (kx_arrive.h); false for the others.  part: parts * PART floats of this tile; arrived: its counter.
+template <class TL>
+__device__ __forceinline__ bool gather(uint8_t *lds, typename TL::Sums &acc, float *part, int *arrived, int parts, int p) {
+  int &last = *(int *)lds;  // behind the barrier below nobody reads operands any more
+  uint64_t *at = (uint64_t *)part;
+  constexpr size_t PER = TL::PART / 2;
+  constexpr int H = TL::V / 2, RUN = 8 / H;  // pairs of a block; blocks whose parts are asked for together
 #pragma unroll
-    for (int i = 0; i < MI; ++i)
+  for (int i = 0; i < TL::MI; ++i)
 #pragma unroll
-      for (int j = 0; j < NI; ++j)
+    for (int j = 0; j < TL::NI; ++j)
+#pragma unroll
+      for (int q = 0; q < H; ++q) {
+        const float a = acc[i][j][2 * q], b = acc[i][j][2 * q + 1];
+        kx_arrive_store(at + p * PER + ((i * TL::NI + j) * H + q) * TL::THREADS + threadIdx.x,
+                        (uint64_t)__builtin_bit_cast(uint32_t, a) | (uint64_t)__builtin_bit_cast(uint32_t, b) << 32);
+      }
+  kx_arrive_writes_done();
+  __syncthreads();
+  if (threadIdx.x == 0) last = kx_arrive_is_last(arrived, parts);
+  __syncthreads();
+  if (!last) return false;
+  if (threadIdx.x == 0) kx_arrive_reset(arrived);
+#pragma unroll
+  for (int i = 0; i < TL::MI; ++i)
+#pragma unroll
+    for (int j0 = 0; j0 < TL::NI; j0 += RUN)
+      for (int s = 0; s < parts; ++s) {
+        uint64_t y[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) y[q] = kx_arrive_load(at + s * PER + ((i * TL::NI + j0) * H + q) * TL::THREADS + threadIdx.x);
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-          const float a = acc[i][j][2 * q], b = acc[i][j][2 * q + 1];
-          kx_arrive_store(at + p * PER + ((i * NI + j) * 8 + q) * THREADS + threadIdx.x,
-                          (uint64_t)__builtin_bit_cast(uint32_t, a) | (uint64_t)__builtin_bit_cast(uint32_t, b) << 32);
+          const float a = __builtin_bit_cast(float, (uint32_t)y[q]), b = __builtin_bit_cast(float, (uint32_t)(y[q] >> 32));
+          auto &block = acc[i][j0 + q / H];
+          const int v = 2 * (q % H);
+          block[v] = s ? block[v] + a : a;
+          block[v + 1] = s ? block[v + 1] + b : b;
         }
-    kx_arrive_writes_done();
-    __syncthreads();
-    if (threadIdx.x == 0) last = kx_arrive_is_last(arrived, parts);
-    __syncthreads();
-    if (!last) return false;
-    if (threadIdx.x == 0) kx_arrive_reset(arrived);
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-      for (int j = 0; j < NI; ++j)
-        for (int s = 0; s < parts; ++s) {
-          uint64_t y[8];
-#pragma unroll
-          for (int q = 0; q < 8; ++q) y[q] = kx_arrive_load(at + s * PER + ((i * NI + j) * 8 + q) * THREADS + threadIdx.x);
-#pragma unroll
-          for (int q = 0; q < 8; ++q) {
-            const float a = __builtin_bit_cast(float, (uint32_t)y[q]), b = __builtin_bit_cast(float, (uint32_t)(y[q] >> 32));
-            acc[i][j][2 * q] = s ? acc[i][j][2 * q] + a : a;
-            acc[i][j][2 * q + 1] = s ? acc[i][j][2 * q + 1] + b : b;
-          }
-        }
-    return true;
-  }
-};
+      }
+  return true;
+}
+
+}  // namespace kxtile
+#include "kx_gemm_turns.h"
+namespace kxtile {
 
 // Workgroup id -> work item: consecutive ids go to the chip's eight dies in turn, each with its own L2, so every die takes a
 // run of consecutive items, which share rows of tokens and of the matrix.
@@ -208,7 +219,8 @@ __device__ __forceinline__ int item_of(int id, int n) {
 // in 64 bits cost a workgroup 0.3 us, 2 % of a product of 16 blocks.
 __device__ __forceinline__ int cut(int blocks, int part, int parts) { return (uint32_t)blocks * part / (uint32_t)parts; }
 
-typedef Tile<uint16_t, 4, 2, 2, 4, 4> Large;   // 256 x 256, 8 waves, a CU each
+typedef Turns<false> Large;                    // 256 x 256, 8 waves, a CU each
+typedef Turns<true> Twin;                      // 128 x 128, 8 waves, a CU each
 typedef Tile<uint16_t, 2, 2, 2, 2, 5> Medium;  // 128 x 128, 4 waves, two workgroups per CU
 
 struct Place {
@@ -227,7 +239,7 @@ __device__ __forceinline__ Place place_of(int id, int tiles, Share s) {
 // vector ALU (64 x 64, 4 x 4 a thread) the first, with its activation, took 260 us and was a little further from the 64-bit result.
 typedef Tile<float, 2, 2, 1, 2, 4> Single;
 
-static_assert(Large::BM == LARGE.tokens && Large::BN == LARGE.rows && Medium::BM == MEDIUM.tokens && Medium::BN == MEDIUM.rows &&
+static_assert(Large::BM == LARGE.tokens && Large::BN == LARGE.rows && Medium::BM == MEDIUM.tokens && Medium::BN == MEDIUM.rows && Twin::BM == MEDIUM.tokens && Twin::BN == MEDIUM.rows &&
               Single::BM == SINGLE.tokens && Single::BN == SINGLE.rows, "the rules count other tiles");
 
 }  // namespace kxtile

@@ -9,7 +9,7 @@
 // ones are multiplied; the epilogue stores the product, forms the gated activation of a (gate, up) pair, or updates
 // all residual streams of the row.
 // lin_narrow_k (bf16, up to 64 tokens): all tokens against 64 rows, the columns split over waves and workgroups.
-// lin_gemm_k (bf16, more tokens): tiles of 256 x 256 or 128 x 128 on the matrix cores (kx_gemm_tile.h).
+// lin_gemm_k (bf16, more tokens): tiles of 256 x 256 or 128 x 128 on the matrix cores (kx_gemm_tile.h, kx_gemm_turns.h).
 // In f32 from 5 tokens on tiles of 64 x 128 on the 32-bit matrix instructions; true 32-bit products.
 //
 // Products with experts: up to 4 tokens lin_gemv_k with a matrix per (token, choice), the routing in its prologue, and with
@@ -310,49 +310,53 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) lin_gemm_k(Kx
   }
   x += (size_t)variant_of(a, n0) * a.tokens * x_ld;
   const int nb = a.m.ld / TL::COLS;
-  f32x16 acc[TL::MI][TL::NI];
+  typename TL::Sums acc;
   TL::run(lds, kxtile::cut(nb, at.part, at.of), kxtile::cut(nb, at.part + 1, at.of), [&](int r) {
     return r < TL::BM ? x + source_row<GROUP>(e, tl, r) * x_ld : (const T *)a.m.w + tl.w + (size_t)min(n0 + r - TL::BM, a.m.rows - 1) * a.m.ld;
   }, acc);
   if (!GROUP && at.of > 1 &&
-      !TL::gather(lds, acc, a.part + (size_t)(at.tile - share.whole) * at.of * TL::PART, a.arrived + at.tile - share.whole, at.of, at.part))
+      !kxtile::gather<TL>(lds, acc, a.part + (size_t)(at.tile - share.whole) * at.of * TL::PART, a.arrived + at.tile - share.whole, at.of, at.part))
     return;
 #pragma unroll
   for (int i = 0; i < TL::MI; ++i) {
     if constexpr (EPI == KX_LIN_GLU) {
+      constexpr int STEP = KX_GLU_BLOCK / TL::SIDE;  // blocks of gate rows in front of their up rows
 #pragma unroll
-      for (int j = 0; j < TL::NI; j += 2) {
+      for (int j = 0; j < TL::NI; ++j) {
+        if (j / STEP % 2) continue;
         const int r = n0 + TL::col(j);
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
+        for (int v = 0; v < TL::V; ++v) {
           const int t = tl.m0 + TL::row(i, v);
           if (t < tl.end && r < a.m.rows)
-            put_glu<T>(a, t, (r >> 6) * KX_GLU_BLOCK + (r & 31), acc[i][j][v], acc[i][j + 1][v], GROUP ? e.slot_weight[t] : 1.0f);
+            put_glu<T>(a, t, (r >> 6) * KX_GLU_BLOCK + (r & 31), acc[i][j][v], acc[i][j + STEP][v], GROUP ? e.slot_weight[t] : 1.0f);
         }
       }
-    } else {
+    } else if constexpr (EPI == KX_LIN_F32 || EPI == KX_LIN_HEADS) {
 #pragma unroll
       for (int j = 0; j < TL::NI; ++j) {
         const int r = n0 + TL::col(j);
-        if constexpr (EPI == KX_LIN_F32) {
 #pragma unroll
-          for (int v = 0; v < 16; ++v)
-            if (tl.m0 + TL::row(i, v) < tl.end && r < a.m.rows) put_f32<T>(a, tl.m0 + TL::row(i, v), r, acc[i][j][v]);
-        } else if constexpr (EPI == KX_LIN_HEADS) {
-#pragma unroll
-          for (int v = 0; v < 16; ++v)
-            if (tl.m0 + TL::row(i, v) < tl.end && r < a.m.rows) put_head<T>(a, tl.m0 + TL::row(i, v), r, acc[i][j][v]);
-        } else {
-          constexpr int G = most_streams(EPI) > 2 ? 4 : 16;  // elements read before the first is written
-#pragma unroll
-          for (int v0 = 0; v0 < 16; v0 += G) {
-            Streams<EPI> res[G];
-#pragma unroll
-            for (int v = 0; v < G; ++v) res[v].load(a, min(tl.m0 + TL::row(i, v0 + v), a.tokens - 1), min(r, a.m.rows - 1));
-#pragma unroll
-            for (int v = 0; v < G; ++v)
-              if (tl.m0 + TL::row(i, v0 + v) < a.tokens && r < a.m.rows) res[v].store(a, tl.m0 + TL::row(i, v0 + v), r, acc[i][j][v0 + v]);
+        for (int v = 0; v < TL::V; ++v)
+          if (tl.m0 + TL::row(i, v) < tl.end && r < a.m.rows) {
+            if constexpr (EPI == KX_LIN_F32) put_f32<T>(a, tl.m0 + TL::row(i, v), r, acc[i][j][v]);
+            else put_head<T>(a, tl.m0 + TL::row(i, v), r, acc[i][j][v]);
           }
+      }
+    } else {
+      constexpr int G = most_streams(EPI) > 2 ? 4 : 16;  // elements read before the first is written
+#pragma unroll
+      for (int e0 = 0; e0 < TL::NI * TL::V; e0 += G) {
+        Streams<EPI> res[G];
+#pragma unroll
+        for (int u = 0; u < G; ++u) {
+          const int j = (e0 + u) / TL::V, v = (e0 + u) % TL::V;
+          res[u].load(a, min(tl.m0 + TL::row(i, v), a.tokens - 1), min(n0 + TL::col(j), a.m.rows - 1));
+        }
+#pragma unroll
+        for (int u = 0; u < G; ++u) {
+          const int j = (e0 + u) / TL::V, v = (e0 + u) % TL::V, t = tl.m0 + TL::row(i, v), r = n0 + TL::col(j);
+          if (t < a.tokens && r < a.m.rows) res[u].store(a, t, r, acc[i][j][v]);
         }
       }
     }
@@ -628,6 +632,7 @@ int gemm_launch(const KxLinArgs &a, const KxExpertArgs &e, const T *x, int x_ld,
     if (c.large && a.n_var == 1) return tile_launch<uint16_t, kxtile::Large, EPI, false>(a, e, x, x_ld, c.s, st);  // variants begin at multiples of 128 rows
     // with variants a choice of large tiles is taken as medium ones, whole
     const kxtile::Share whole = {kx_cdiv(a.tokens, kxtile::Medium::BM) * kx_cdiv(a.m.rows, kxtile::Medium::BN), 1};
+    if (c.twin) return tile_launch<uint16_t, kxtile::Twin, EPI, false>(a, e, x, x_ld, c.s, st);
     return tile_launch<uint16_t, kxtile::Medium, EPI, false>(a, e, x, x_ld, c.large ? whole : c.s, st);
   }
 }

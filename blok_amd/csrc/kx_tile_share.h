@@ -38,56 +38,74 @@ inline Share share(long tiles, int round, int most_parts, long room, int arrival
   return s;
 }
 
-// Which tile, and how it is shared out, for one product of `tokens` x `rows` with `blocks` blocks of 64 columns.
-// Where the medium tiles leave CUs idle they take parts, of at least 16 blocks.  Beyond that the tile is the one that is sooner whole, by
-// estimates in us: a round of large tiles takes 12 + 1.6 per block on 256 CUs, of medium ones (two per CU) 4.5 + 1.09; a last round of
-// medium tiles that is not full takes its share of that, but no less than half, the time of one per CU.  Measured against it (us, 32-bit
-// results, large / medium): large tiles in 1.5 rounds, medium ones in 3: 1536 x 16384 x 1024 75 / 69, x 2048 127 / 116, x 4096 228 / 211,
-// x 8192 453 / 434, x 16384 855 / 886; 2048 x 16384 x 2048 150 / 214, 2048 x 8448 x 2048 116 / 94, 2048 x 5120 x 2048 64 / 61, 2048 x 36864 x
-// 7168 1026 / 1265, 2048 x 7168 x 8192 252 / 329, 952 x 7168 x 18432 455 / 353, 700 x 12288 x 16384 379 / 428, 1024 x 36864 x 4096 359 / 345.
-// In parts: 300 x 2048 x 8192 71 alone, 32 in four, 100 x 2048 x 8192 73 and 29 in eight, 2048 x 384 x 7168 65 and 32 in four.
+// Which tile, and how it is shared out, for one product of `tokens` x `rows` with `blocks` blocks of 64 columns, by estimates in us that
+// are fitted to measurements of 22000 products (65 to 2048 x 384 to 40000 x 256 to 18560, 32-bit results).
+// Where the medium tiles leave CUs idle each has a CU to itself, in at least 10 blocks as the twin tile (kx_gemm_turns.h; at 4 blocks
+// it takes 8 % longer than the medium one, at 10 2 % less, at 16 7 % and at 40 19 % less), and they take parts, of at least 16
+// blocks: as many as fill the CUs, or more rounds of shorter ones where that is 5 % sooner (149 x 8548 x 18304, 134 tiles: 153 us whole, 103 in
+// three).  300 x 2048 x 8192 71 alone, 32 in four, 100 x 2048 x 8192 73 and 29 in eight, 2048 x 384 x 7168 65 and 32 in four (medium).
+// Beyond that the tile is the one that is sooner whole, or in parts where that is clearly sooner: what is chosen takes 0.976 of the
+// time of the sooner of whole medium and large tiles over 7000 products, 200 of them more than 3 % longer, and 1.5 % more than the best of
+// every way to share out.  Measured (us, large / medium, whole): 2048 x 16384 x 2048 115 / 147, 2048 x 7168 x 8192 171 / 262, 2048 x 8192 x
+// 2048 58 / 78, 2048 x 4096 x 2048 45 / 40, 1989 x 22265 x 1152 160 / 123, 945 x 32877 x 320 46 / 30; 260 x 11856 x 11904, 279 medium tiles,
+// 196 whole, 116 as twin tiles with the last 23 in six parts.
 struct Choice {
   bool large;
   Share s;
+  bool twin = false;  // of the tiles of 128 x 128 those with two groups of waves
 };
 inline Choice choose(int tokens, int rows, int blocks, size_t part_floats, int arrivals, int cus) {
   const long medium = MEDIUM.of(tokens, rows), large = LARGE.of(tokens, rows);
+  // n workgroups of `per` blocks: rounds of `round` + `block` per block, a last one of `last` and between `lone` and `block`
+  auto rounds = [&](long n, double per, double round, double block, double last, double lone) {
+    const long r = n % cus;
+    return n / cus * (round + block * per) + (r == 0 ? 0.0 : last + (lone + (block - lone) * r / cus) * per);
+  };
   if (medium <= cus) {
-    long p = cus / medium;
-    if (p > blocks / 16) p = blocks / 16;
-    if ((size_t)p > part_floats / MEDIUM.sums() / medium) p = part_floats / MEDIUM.sums() / medium;
-    return p < 2 || medium > arrivals ? Choice{false, {(int)medium, 1}} : Choice{false, {0, (int)p}};
+    const long room = medium > arrivals ? 0 : (long)(part_floats / MEDIUM.sums() / medium), most = room < blocks / 16 ? room : blocks / 16;
+    auto time = [&](long p) { return 3.3 + rounds(medium * p, (double)blocks / p, 6.0, 0.458, 4.4, 0.327) + (p > 1 ? 0.9 + 1.4 * p + 0.009 * medium * p : 0.0); };
+    long p = cus / medium < most ? cus / medium : most;
+    if (p < 1) p = 1;
+    const long fill = p;
+    for (long q = fill + 1; q <= most && medium * q <= 4 * cus; ++q)
+      if (time(q) * 1.05 < time(fill) && time(q) < time(p)) p = q;
+    return {false, p == 1 ? Share{(int)medium, 1} : Share{0, (int)p}, blocks >= 10 * p};
   }
-  const long full = medium / (2 * cus), rest = medium % (2 * cus);
-  const double rounds = full == 0 ? 1.0 : full + (rest == 0 ? 0.0 : rest <= cus ? 0.5 : rest / (2.0 * cus));
-  const bool large_whole = (large + cus - 1) / cus * (12 + 1.6 * blocks) < rounds * (4.5 + 1.09 * blocks);
-  // In parts where that is clearly sooner, by closer estimates (fitted to 4 to 20 ways of sharing out each of 5900 products, 65 to 2048 x
-  // 512 to 40000 x 1024 to 18560): a workgroup that leaves its sums behind, and has them read, costs the memory's time for them, 0.032 us a
-  // medium and 0.07 a large one; a last medium round takes 0.44 of a full one up to a workgroup per CU.  They are off by a tenth: parts have to
-  // gain 15 % of their own time, 12 % of the whole product's where the tile is another one.  Of those products 62 are then more than 3 %
-  // slower than whole, one by 11 %; 1329 are 3 % faster or more, and on average they take 0.973 of the time.  (With the whole tiles' estimate and 6 +
-  // 2.5 per part, 12 + 8 for large ones, 582 were slower, by up to 47 %: 965 x 6110 x 3904 66 whole, 84 in two parts each.)
-  auto medium_rounds = [&](long n, bool parts) {
+  auto whole_large = [&](long n) { return 3.3 + rounds(n, blocks, 13.8, 1.45, 14.8, 0.92); };
+  auto whole_medium = [&](long n) {  // two per CU
+    const double round = 4.3 + (1.0 + 0.0009 * blocks) * blocks, lone = 2.2 + 0.463 * blocks;
     const long f = n / (2 * cus), r = n % (2 * cus);
-    if (f == 0 && !parts) return 0.78 + (r <= cus ? 0.0 : 0.22 * (r - cus) / cus);
-    return f + (r == 0 ? 0.0 : r <= cus ? 0.44 : 0.44 + 0.56 * (r - cus) / cus);
+    return 5.5 + f * round + (r == 0 ? 0.0 : r <= cus ? lone : lone + (round - lone) * (0.59 + 0.28 * (r - cus) / cus));  // a CU with two of the last round
   };
-  auto shared = [&](bool with_large) {
-    return [=](long whole, long n, int p) {
-      const double round = with_large ? 10 + 1.63 * blocks : 4.3 + 1.22 * blocks;
-      const double t = whole == 0 ? 0.0 : round * (with_large ? (double)((whole + cus - 1) / cus) : medium_rounds(whole, n > 0));
-      if (n == 0) return t;
-      const double own = with_large ? (n * p + cus - 1) / cus * 1.63 * blocks / p + 9 * p + 0.07 * n * p : medium_rounds(n * p, true) * 1.22 * blocks / p + 0.032 * n * p;
-      return with_large == large_whole ? t + 1.15 * own : 1.12 * (t + own);
-    };
-  };
+  const bool large_whole = whole_large(large) < whole_medium(medium);
+  // In parts, or in rounds of twin tiles with the last one in parts: a workgroup that leaves its sums behind, and has them read,
+  // costs the memory's time for them, 0.009 us a twin, 0.032 a medium and 0.074 a large one.  The estimates are off by a tenth: parts have to gain 15 %
+  // of their own time, large ones 12 % of the product's where whole ones would be medium; twin tiles 22 % (with 12 % 48
+  // of 1192 products in parts took more than a tenth longer than whole, now 5 of 960), 5 % where they are whole.
   const int most = blocks / 16 < 8 ? blocks / 16 : 8;
-  double tm, tl;
-  const Share sm = share(medium, 2 * cus, most, part_floats / MEDIUM.sums(), arrivals, shared(false), &tm);
-  const Share sl = share(large, cus, most, part_floats / LARGE.sums(), arrivals, shared(true), &tl);
-  // whole tiles only of the size that is sooner whole
-  if (large_whole) return sm.parts > 1 && tm < tl ? Choice{false, sm} : Choice{true, sl};
-  return sl.parts > 1 && tl < tm ? Choice{true, sl} : Choice{false, sm};
+  auto large_time = [&](long n0, long n, int p) {
+    const double t = n0 == 0 ? 0.0 : whole_large(n0);
+    if (n == 0) return t;
+    const double own = rounds(n * p, (double)blocks / p, 21.0, 1.36, 20.5, 0.63) + 0.8 * p + 0.074 * n * p;
+    return large_whole ? t + 1.15 * own : 1.12 * (t + own);
+  };
+  auto medium_time = [&](long n0, long n, int p) {  // a last round takes 0.44 of a full one up to a workgroup per CU
+    const double t = n0 == 0 ? 0.0 : whole_medium(n0);
+    const long wgs = n * p, f = wgs / (2 * cus), r = wgs % (2 * cus);
+    return n == 0 ? t : t + 1.15 * ((f + (r == 0 ? 0.0 : r <= cus ? 0.44 : 0.44 + 0.56 * (r - cus) / cus)) * (1.2 + 0.0009 * blocks) * blocks / p + 0.032 * wgs);
+  };
+  auto twin_time = [&](long n0, long n, int p) {
+    const double t = n0 == 0 ? 0.0 : 3.3 + rounds(n0, blocks, 6.0, 0.458, 4.4, 0.327);
+    return n == 0 ? 1.05 * t : 1.22 * (t + rounds(n * p, (double)blocks / p, 6.0, 0.458, 4.4, 0.327) + 0.9 + 1.4 * p + 0.009 * n * p);
+  };
+  double tm, tl, tt;
+  const Share sm = share(medium, 2 * cus, most, part_floats / MEDIUM.sums(), arrivals, medium_time, &tm);
+  const Share sl = share(large, cus, most, part_floats / LARGE.sums(), arrivals, large_time, &tl);
+  const Share st = share(medium, cus, most, part_floats / MEDIUM.sums(), arrivals, twin_time, &tt);
+  // whole large and medium tiles only of the size that is sooner whole
+  if (!large_whole && sl.parts == 1) tl = 1e30;
+  if (large_whole && sm.parts == 1) tm = 1e30;
+  return tt < tl && tt < tm ? Choice{false, st, true} : tl < tm ? Choice{true, sl} : Choice{false, sm};
 }
 
 // For the 32-bit tile and blocks of 32 columns.

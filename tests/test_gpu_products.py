@@ -136,3 +136,11 @@ def test_large_tiles(kxlib, tokens, rows, cols):
     gv, uv = np.minimum(y[:, :ff], 1.5), np.clip(y[:, ff:2 * ff], -1.5, 1.5)
     want = gv * K.sigmoid(1.702 * gv) * (uv + 1.0)
     assert rel((out.to_numpy(np.uint16, (tokens, ff)).astype(np.uint32) << 16).view(np.float32), want) < 1e-2
+
+
+@pytest.mark.parametrize("tokens, rows, cols", [(300, 1000, 640), (129, 4100, 704), (66, 129, 1280), (2047, 2048, 832), (1793, 8191, 1024), (2048, 7424, 1088)],
+                         ids=["twin, 10 blocks", "twin, 11", "twin, a few", "twin, 13", "large, 16", "large, 17"])
+def test_tiles_whose_groups_take_turns(kxlib, tokens, rows, cols):
+    """Even and odd numbers of blocks, tiles with remainders of tokens and rows, every epilogue: the bars of the large tiles, 32-bit sums of up to
+    1088 products (about 1e-6)."""
+    test_large_tiles(kxlib, tokens, rows, cols)
