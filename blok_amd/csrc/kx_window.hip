@@ -12,6 +12,7 @@
 #include <atomic>
 #include <type_traits>
 #include "kx_common.h"
+#include "kx_lds_copy.h"
 #include "kx_rows.h"
 #include "kx_window.h"
 
@@ -21,6 +22,7 @@ using kxr::Elem;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
@@ -272,35 +274,51 @@ __global__ void __launch_bounds__(MERGE_THREADS) win_merge_k(KxWindowArgs a, int
   }
 }
 
-// ---- bf16, several positions: one head, 128 consecutive positions of one sequence, 4 waves of 32 queries ----
+// ---- bf16, several positions: one head, 128 consecutive positions of one sequence, two groups of 4 waves of 32 queries ----
 // S^T = K Q^T and O^T = V^T P^T, so that a lane holds one query (lane % 32) in both products: the running maximum and
 // denominator are one value per lane, and the weights go from the first product's result into the second product's
-// operand without leaving the registers.  The result layout gives lane (q, h) the keys 8 (v / 4) + 4 h + v % 4 of a tile of
-// 32; the operand layout wants 8 keys in a row per lane, so within 16 keys the V^T tile stores keys 0-3, 8-11 for
-// h = 0 and 4-7, 12-15 for h = 1.  The 8-key pieces of a V^T row are xor-swizzled by the row, which spreads the
-// transposing writes over the banks.  The next tile's rows are on their way to registers while a tile is multiplied;
-// scores are in units of log 2, so that a weight is one exp2.
+// operand without leaving the registers.  The result layout gives lane (q, h) the keys 8 (v / 4) + 4 h + v % 4 of 32; the rows of V that
+// a transposing read (ds_read_b64_tr_b16) gathers for it are those.  Scores are in units of log 2, so that a weight is one exp2.
+// What bounds it: a wave reads 20 KB of keys and values of 192 and 128 columns for 20 products of 32 cycles, and as many cycles of
+// vector arithmetic make the weights of its 32 x 32 scores, so every SIMD has two waves, whose products and weights overlap: group g
+// has half g of every tile's keys, its own maximum, denominator and sums, and the groups' sums meet at the end.  Tiles are
+// copied to LDS two ahead, the second group asking for its share of a tile behind its scores, so that the address path is free
+// when the first one begins.  Workgroups with the most keys come first.
+// 64 heads of 192 and 128, 2048 positions: 382 us with one wave per SIMD and tiles through registers, 184 now; 952 positions behind 2048:
+// 265 and 194; 16 heads of 128, 2048 positions, window 1024: 64 and 49.
 // A key that a query does not see has a weight of zero, and its value is multiplied all the same; zero times a value that is not
 // finite would make the query's output follow a position behind it, or one that its window has left.  So a workgroup whose sums
 // are not all finite makes them once more: in tiles that not every query sees as a whole, such values are replaced by zeros, and
-// added at the end by the queries that see them.  This costs a launch 0 to 4 % (64 heads of 192, 2048 positions behind 952: 612 us, 618
-// with it; 4 sequences, 32 heads of 128, 2048 positions with a window of 4096 behind 3000: 1278 and 1327); looking for such values as
-// each tile is written to LDS took 857.
-constexpr int FQ = 128, FK = 64;
-__device__ __forceinline__ int vt_piece(int d, int piece) { return (piece ^ (d >> 1) ^ (d >> 4)) & 7; }
+// added at the end by the queries that see them.
+constexpr int FQ = 128, FK = 64, FLASH_WAVES = 8;
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) uint8_t LdsByte;
 
 template <int ND, int NV>  // 32-column blocks of a key and of a value
-__global__ void __launch_bounds__(256) win_flash_k(KxWindowArgs a) {
-  constexpr int KSTR = ND * 32 + 8, VSTR = FK + 8;
-  extern __shared__ __attribute__((aligned(16))) uint16_t fl_lds[];
-  __shared__ int odd_s;                 // a sum that is not finite
-  uint16_t *ks = fl_lds;                // [FK][KSTR]
-  uint16_t *vt = ks + FK * KSTR;        // [NV * 32][VSTR]
+struct Flash {
+  static constexpr int KP = ND * 4, VP = NV * 4;  // pieces of 16 bytes of a row
+  static constexpr int KB = FK * KP * 16, TILE = KB + FK * VP * 16, STAGES = 3 * TILE <= 128 * 1024 ? 3 : 2;
+  static constexpr int COPIES = TILE / 1024, CPW = (COPIES + FLASH_WAVES - 1) / FLASH_WAVES;  // of a tile, of a wave
+  static constexpr int KEEP = NV > 1 ? NV / 2 : 1;  // blocks of the result that a group finishes; of one block group 0
+  static constexpr int MERGE = FLASH_WAVES * KEEP * 4096, ENDS = MERGE + FLASH_WAVES * 64 * 8;
+  static constexpr int ODD = STAGES * TILE > ENDS ? STAGES * TILE : ENDS, LDS = ODD + 16;
+  // Where piece p of row r lies in the row: eight consecutive rows read the same piece of a key, four rows the same 64 bytes of
+  // a value, each without meeting in a bank.
+  static __device__ __forceinline__ int key_piece(int r, int p) { return p ^ (ND == 1 ? r >> 1 & 3 : r & 7); }
+  static __device__ __forceinline__ int value_piece(int r, int p) { return p ^ (NV == 1 ? 0 : NV == 2 ? (r >> 1 & 1) * 4 : (r & 3) * 4); }
+};
+
+template <int ND, int NV>
+__global__ void __launch_bounds__(FLASH_WAVES * 64, 2) win_flash_k(KxWindowArgs a) {
+  using F = Flash<ND, NV>;
+  extern __shared__ __attribute__((aligned(16))) uint8_t fl_lds[];
+  LdsByte *const lds = (LdsByte *)fl_lds;
+  int &odd_s = *(int *)(fl_lds + F::ODD);  // a sum that is not finite
   const KxWindowSpec &s = a.s;
   const KxWindowCache &c = a.c;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lq = lane & 31, hh = lane >> 5;
-  const int h = blockIdx.y, b = blockIdx.z, g = h / (s.heads / s.kv_heads);
-  const int i0 = blockIdx.x * FQ, i = i0 + wave * 32 + lq;  // this lane's position of the step
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), me = wave & 3, half = wave >> 2, lq = lane & 31, hh = lane >> 5;
+  const int h = blockIdx.x % s.heads, b = blockIdx.x / s.heads, g = h / (s.heads / s.kv_heads);
+  const int i0 = (gridDim.y - 1 - blockIdx.y) * FQ, i = i0 + me * 32 + lq;  // this lane's position of the step
   const bool live = i < a.positions;
   const int p = a.pos + min(i, a.positions - 1), tok = min(i, a.positions - 1) * (a.tok_batch ? a.tok_batch : a.batch) + b;
   const int p_first = a.pos + i0, p_last = a.pos + min(i0 + FQ, a.positions) - 1;
@@ -315,116 +333,127 @@ __global__ void __launch_bounds__(256) win_flash_k(KxWindowArgs a) {
     for (int kk = 0; kk < ND * 2; ++kk) q[kk] = kk * 16 < c.dp ? *(const bf16x8 *)(qr + kk * 16 + hh * 8) : bf16x8{};
   }
   f32x16 o[NV];
-  float m, z;  // z: of this lane's half of the keys
+  float m, z;  // z: of this lane's half of the group's keys
   const float scale2 = s.scale * 1.44269504088896341f;
 
   // tiles: the blocks the last query sees, then the positions from the first query's window on
   const int tb = (seen_blocks(p_last, s.size, s.pool) + FK - 1) / FK;
   const int j0 = window_lo(p_first, s.size) & ~(FK - 1), tiles = tb + (p_last - j0) / FK + 1;
   // what all and what any of this wave's queries see
-  const int q0 = __builtin_amdgcn_readfirstlane(a.pos + min(i0 + wave * 32, a.positions - 1));
-  const int q1 = __builtin_amdgcn_readfirstlane(a.pos + min(i0 + wave * 32 + 31, a.positions - 1));
+  const int q0 = __builtin_amdgcn_readfirstlane(a.pos + min(i0 + me * 32, a.positions - 1));
+  const int q1 = __builtin_amdgcn_readfirstlane(a.pos + min(i0 + me * 32 + 31, a.positions - 1));
   const int nb0 = seen_blocks(q0, s.size, s.pool), nb1 = seen_blocks(q1, s.size, s.pool), lo0 = window_lo(q0, s.size), lo1 = window_lo(q1, s.size);
   auto first_key = [&](int t) { return t < tb ? t * FK : j0 + (t - tb) * FK; };
   auto seen_by_all = [&](int t) {
     return t < tb ? (t + 1) * FK <= seen_blocks(p_first, s.size, s.pool) : first_key(t) >= window_lo(p_last, s.size) && first_key(t) + FK - 1 <= p_first;
   };
-  constexpr int VT = (FK / 8) * NV * 16, VN = (VT + 255) / 256;  // V is taken by 8 keys x 2 columns
-  u32x4 kreg[ND];
-  uint32_t vreg[VN][8];
+  // This wave's copies of a tile, 1024 bytes of LDS each.  Where there are fewer the last one is made again, so that every wave waits
+  // for the same number.  A row has no more than c.dp and c.vp columns: a piece past them is the last one, which meets zeros of the query or a
+  // result that is not stored.
+  int crow[F::CPW], ccol[F::CPW];
+#pragma unroll
+  for (int y = 0; y < F::CPW; ++y) {
+    const int k = min(wave + FLASH_WAVES * y, F::COPIES - 1);
+    const bool key = k < F::KB / 1024;
+    const int x = (key ? k : k - F::KB / 1024) * 64 + lane, per = key ? F::KP : F::VP, r = x / per;
+    crow[y] = r;
+    ccol[y] = min((key ? F::key_piece(r, x % per) : F::value_piece(r, x % per)) * 8, (key ? c.dp : c.vp) - 8);
+  }
   // Rows of a tile: a window tile starts at a multiple of FK and the ring's length is one, so it does not wrap inside; past the
-  // last block there is nothing to read.  What is read beyond a row's columns or the keys a query sees meets zeros.
-  auto fetch = [&](int t) {
+  // last block there is nothing to read.  What is read beyond the keys a query sees meets zeros.
+  const uint32_t lds0 = (uint32_t)(uintptr_t)lds;
+  auto ask = [&](int t, int stage) {
     const bool pooled = t < tb;
     const int k0 = first_key(t), last = pooled ? c.blocks - 1 - k0 : FK - 1;
     const uint16_t *kr = pooled ? pkc + (size_t)k0 * c.dp : kc + (size_t)(k0 % c.cap) * c.dp;
     const uint16_t *vr = pooled ? pvc + (size_t)k0 * c.vp : vc + (size_t)(k0 % c.cap) * c.vp;
 #pragma unroll
-    for (int y = 0; y < ND; ++y) {
-      const int x = y * 256 + tid, r = x / (ND * 4), d = (x - r * (ND * 4)) * 8;
-      kreg[y] = *(const u32x4 *)(kr + (size_t)min(r, last) * c.dp + min(d, c.dp - 8));
-    }
-#pragma unroll
-    for (int y = 0; y < VN; ++y) {
-      const int x = min(y * 256 + tid, VT - 1), oct = x / (NV * 16), d = min((x - oct * (NV * 16)) * 2, c.vp - 2);
-#pragma unroll
-      for (int r = 0; r < 8; ++r) vreg[y][r] = *(const uint32_t *)(vr + (size_t)min(oct * 8 + r, last) * c.vp + d);
+    for (int y = 0; y < F::CPW; ++y) {
+      const int k = min(wave + FLASH_WAVES * y, F::COPIES - 1);
+      const bool key = k < F::KB / 1024;
+      kx_copy16_to_lds((key ? kr : vr) + (uint32_t)(min(crow[y], last) * (key ? c.dp : c.vp) + ccol[y]), __builtin_amdgcn_readfirstlane(lds0 + stage * F::TILE + k * 1024));
     }
   };
-  auto put = [&](bool as_it_is) {
-    if (!as_it_is)
+  // this lane's operands: pieces of key `half * 32 + lq`, and rows half * 32 + 4 hh + (lane % 16) / 4 of 16 columns of the values
+  int kp[4], vp[NV];
 #pragma unroll
-      for (int y = 0; y < VN; ++y)
+  for (int y = 0; y < 4; ++y) kp[y] = (half * 32 + lq) * (F::KP * 16) + F::key_piece(lq, (2 * y + hh) & (F::KP - 1 < 7 ? 3 : 7)) * 16;
+  const int vrow = 4 * hh + (lane >> 2 & 3);
 #pragma unroll
-        for (int r = 0; r < 8; ++r) vreg[y][r] &= ~(((((vreg[y][r] & 0x7f807f80u) + 0x00800080u) & 0x80008000u) >> 15) * 0xffffu);  // an exponent of all ones carries into the sign's place
-#pragma unroll
-    for (int y = 0; y < ND; ++y) {
-      const int x = y * 256 + tid, r = x / (ND * 4), d = (x - r * (ND * 4)) * 8;
-      *(u32x4 *)(ks + r * KSTR + d) = kreg[y];
-    }
-#pragma unroll
-    for (int y = 0; y < VN; ++y) {
-      const int x = y * 256 + tid, oct = x / (NV * 16), d = (x - oct * (NV * 16)) * 2;
-      if (x >= VT) continue;
-      const uint32_t *w = vreg[y];
-#pragma unroll
-      for (int half = 0; half < 2; ++half) {  // keys 0-3 of the octet, keys 4-7
-        const int at = vt_piece(d, (oct >> 1) * 2 + half) * 8 + (oct & 1) * 4;
-        const uint32_t *k4 = w + 4 * half;
-        *(u32x2 *)(vt + d * VSTR + at) = u32x2{(k4[0] & 0xffffu) | (k4[1] << 16), (k4[2] & 0xffffu) | (k4[3] << 16)};
-        *(u32x2 *)(vt + (d + 1) * VSTR + at) = u32x2{(k4[0] >> 16) | (k4[1] & 0xffff0000u), (k4[2] >> 16) | (k4[3] & 0xffff0000u)};
-      }
-    }
-  };
+  for (int j = 0; j < NV; ++j)
+    vp[j] = F::KB + (half * 32 + vrow) * (F::VP * 16) + F::value_piece(vrow, j * 4) * 16 + (lane >> 4 & 1) * 32 + (lane & 3) * 8;
   auto attend = [&](auto replace) {
 #pragma unroll
     for (int j = 0; j < NV; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v) o[j][v] = 0.0f;
-    m = s.sink ? (a.sinks ? a.sinks[h] * 1.44269504088896341f : 0.0f) : NEG_INF;
-    z = s.sink && hh == 0 ? 1.0f : 0.0f;
-    fetch(0);
+    const bool sink = s.sink && half == 0;
+    m = sink ? (a.sinks ? a.sinks[h] * 1.44269504088896341f : 0.0f) : NEG_INF;
+    z = sink && hh == 0 ? 1.0f : 0.0f;
+#pragma unroll
+    for (int t = 0; t < F::STAGES - 1; ++t)
+      if (t < tiles) ask(t, t);
+    int stage = 0;
     for (int t = 0; t < tiles; ++t) {
       const bool pooled = t < tb;
       const int k0 = first_key(t);
-      __syncthreads();  // the tile before has been multiplied
-      put(!decltype(replace)::value || seen_by_all(t));
-      __syncthreads();
-      fetch(min(t + 1, tiles - 1));
-      const bool none = pooled ? k0 >= nb1 : k0 > q1 || k0 + FK - 1 < lo0;
-      const bool all = pooled ? k0 + FK <= nb0 : k0 >= lo1 && k0 + FK - 1 <= q0;
-      if (none) continue;
-      f32x16 sc[2];
+      if (F::STAGES > 2 && t + 1 < tiles) kx_wait_copies<F::CPW>();
+      else kx_wait_copies<0>();
+      kx_lds_barrier();  // the tile is in LDS for every wave, and the tile before has been multiplied
+      const LdsByte *const at = lds + stage * F::TILE;
+      const int next = stage == 0 ? F::STAGES - 1 : stage - 1;  // of the tile before
+      stage = stage == F::STAGES - 1 ? 0 : stage + 1;
+      if constexpr (decltype(replace)::value) {
+        if (t + F::STAGES - 1 < tiles) ask(t + F::STAGES - 1, next);
+        if (!seen_by_all(t)) {
+          typedef __attribute__((address_space(3))) u32x4 LdsPiece;
+          for (int x = tid; x < FK * F::VP; x += FLASH_WAVES * 64) {
+            LdsPiece *w = (LdsPiece *)(at + F::KB) + x;
+            u32x4 y = *w;
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {
+            for (int e = 0; e < 4; ++e) y[e] &= ~(((((y[e] & 0x7f807f80u) + 0x00800080u) & 0x80008000u) >> 15) * 0xffffu);  // an exponent of all ones carries into the sign's place
+            *w = y;
+          }
+          kx_lds_barrier();
+        }
+      } else {
+        if (half == 0 && t + F::STAGES - 1 < tiles) ask(t + F::STAGES - 1, next);
+      }
+      const int kh = k0 + half * 32;  // this group's first key
+      const bool none = pooled ? kh >= nb1 : kh > q1 || kh + 31 < lo0;
+      const bool all = pooled ? kh + 32 <= nb0 : kh >= lo1 && kh + 31 <= q0;
+      f32x16 sc;
+      if (!none) {
 #pragma unroll
-        for (int v = 0; v < 16; ++v) sc[kt][v] = 0.0f;
+        for (int v = 0; v < 16; ++v) sc[v] = 0.0f;
 #pragma unroll
         for (int kk = 0; kk < ND * 2; ++kk) {
-          const bf16x8 kf = *(const bf16x8 *)(ks + (kt * 32 + lq) * KSTR + kk * 16 + hh * 8);
-          sc[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, q[kk], sc[kt], 0, 0, 0);
+          const bf16x8 kf = *(const __attribute__((address_space(3))) bf16x8 *)(at + kp[kk & 3] + (kk >> 2) * 128);
+          sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, q[kk], sc, 0, 0, 0);
         }
       }
-      const int from = (pooled ? 0 : lo) - k0 - 4 * hh, to = (pooled ? nb - 1 : p) - k0 - 4 * hh;  // the keys this lane's query sees, from its first one on
+      if constexpr (!decltype(replace)::value) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (half == 1 && t + F::STAGES - 1 < tiles) ask(t + F::STAGES - 1, next);
+      }
+      if (none) continue;
+      const int from = (pooled ? 0 : lo) - kh - 4 * hh, to = (pooled ? nb - 1 : p) - kh - 4 * hh;  // the keys this lane's query sees, from its first one on
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) sc[kt][v] *= scale2;
+      for (int v = 0; v < 16; ++v) sc[v] *= scale2;
       if (!all) {
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            const int e = kt * 32 + 8 * (v >> 2) + (v & 3);
-            sc[kt][v] = ((e < from) | (e > to)) ? NEG_INF : sc[kt][v];
-          }
+        for (int v = 0; v < 16; ++v) {
+          const int e = 8 * (v >> 2) + (v & 3);
+          sc[v] = ((e < from) | (e > to)) ? NEG_INF : sc[v];
+        }
       }
       float tm = NEG_INF;
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) tm = fmaxf(tm, sc[kt][v]);
-      tm = fmaxf(tm, __shfl_xor(tm, 32));
+      for (int v = 0; v < 16; ++v) tm = fmaxf(tm, sc[v]);
+      {
+        const auto both = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, tm), __builtin_bit_cast(uint32_t, tm), false, false);
+        tm = fmaxf(__builtin_bit_cast(float, (uint32_t)both[0]), __builtin_bit_cast(float, (uint32_t)both[1]));
+      }
       if (__any(tm > m)) {
         const float m1 = fmaxf(m, tm), al = m == NEG_INF ? 0.0f : __builtin_amdgcn_exp2f(m - m1);
         m = m1;
@@ -436,56 +465,33 @@ __global__ void __launch_bounds__(256) win_flash_k(KxWindowArgs a) {
       }
       const float mm = m == NEG_INF ? 0.0f : m;  // nothing seen so far
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
+      for (int v = 0; v < 16; ++v) {
+        sc[v] = __builtin_amdgcn_exp2f(sc[v] - mm);
+        z += sc[v];
+      }
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          sc[kt][v] = __builtin_amdgcn_exp2f(sc[kt][v] - mm);
-          z += sc[kt][v];
-        }
-#pragma unroll
-      for (int ss = 0; ss < FK / 16; ++ss) {
-        const f32x16 &f = sc[ss >> 1];
-        const int v0 = (ss & 1) * 8;
+      for (int ss = 0; ss < 2; ++ss) {
         uint32_t pw[4];
 #pragma unroll
         for (int y = 0; y < 4; ++y) {
-          const f32x2 two = {f[v0 + 2 * y], f[v0 + 2 * y + 1]};
+          const f32x2 two = {sc[ss * 8 + 2 * y], sc[ss * 8 + 2 * y + 1]};
           pw[y] = __builtin_bit_cast(uint32_t, __builtin_convertvector(two, bf16x2));
         }
         const bf16x8 pf = __builtin_bit_cast(bf16x8, make_uint4(pw[0], pw[1], pw[2], pw[3]));
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
-          const int d = j * 32 + lq;
-          const bf16x8 vf = *(const bf16x8 *)(vt + d * VSTR + vt_piece(d, ss * 2 + hh) * 8);
+          s16x4 v4[2];
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+            v4[u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)(at + vp[j] + (ss * 16 + u * 8) * (F::VP * 16)));
+          const bf16x8 vf = __builtin_bit_cast(bf16x8, __builtin_shufflevector(v4[0], v4[1], 0, 1, 2, 3, 4, 5, 6, 7));
           o[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf, o[j], 0, 0, 0);
         }
       }
     }
   };
-  auto store = [&]() {
-    z += __shfl_xor(z, 32);
-    if (!live) return;
-    const float inv = 1.0f / z;
-    uint16_t *out = (uint16_t *)a.out + (size_t)tok * a.out_ld + h * s.vdim;
-    const float *gate = a.g_off >= 0 ? a.proj + (size_t)tok * a.proj_ld + a.g_off + h * s.vdim : nullptr;
-#pragma unroll
-    for (int j = 0; j < NV; ++j) {
-      float gt[16];
-#pragma unroll
-      for (int v = 0; v < 16; ++v) gt[v] = gate ? gate[min(j * 32 + 8 * (v >> 2) + 4 * hh + (v & 3), s.vdim - 1)] : 0.0f;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) asm volatile("" : "+v"(gt[v]));  // all sixteen are asked for before the first is used
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int d = j * 32 + 8 * (v >> 2) + 4 * hh + (v & 3);
-        const float y = o[j][v] * inv * (gate ? kxr::sigmoid_for<uint16_t>(gt[v]) : 1.0f);
-        if (d < s.vdim) out[d] = kx_bf16_rne(y);
-      }
-    }
-  };
   if (tid == 0) odd_s = 0;
   attend(std::false_type{});
-  store();
   float odd[4] = {};  // zero, unless a sum is not finite
 #pragma unroll
   for (int j = 0; j < NV; ++j)
@@ -501,18 +507,71 @@ __global__ void __launch_bounds__(256) win_flash_k(KxWindowArgs a) {
       for (int t = 0; t < tiles; ++t) {
         if (seen_by_all(t)) continue;
         const bool pooled = t < tb;
-        const int k0 = first_key(t), e1 = min(FK - 1, (pooled ? nb - 1 : p) - k0);
+        const int k0 = first_key(t), e1 = min(half * 32 + 31, (pooled ? nb - 1 : p) - k0);
         const uint16_t *vr = pooled ? pvc + (size_t)k0 * c.vp : vc + (size_t)(k0 % c.cap) * c.vp;
 #pragma unroll 1
-        for (int e = max(0, (pooled ? 0 : lo) - k0); e <= e1; ++e)
+        for (int e = max(half * 32, (pooled ? 0 : lo) - k0); e <= e1; ++e)
 #pragma unroll
           for (int v = 0; v < 16; ++v) {
             const float x = kx_bf16_f32(vr[(size_t)e * c.vp + min(j * 32 + 8 * (v >> 2) + 4 * hh + (v & 3), c.vp - 1)]);
             o[j][v] = __builtin_isfinite(x) ? o[j][v] : o[j][v] + x;
           }
       }
-    store();
+    __syncthreads();  // the tiles are not read any more
   }
+  // the groups' sums meet: each gives what the other finishes
+  z += __shfl_xor(z, 32);
+  const int other = (half ^ 1) * 4 + me;
+  f32x4 *const sums = (f32x4 *)fl_lds;
+  float *const ends = (float *)(fl_lds + F::MERGE);
+#pragma unroll
+  for (int j = 0; j < F::KEEP; ++j)
+#pragma unroll
+    for (int y = 0; y < 4; ++y) {
+      const f32x16 x = NV == 1 ? o[0] : half ? o[j] : o[NV - F::KEEP + j];
+      sums[((wave * F::KEEP + j) * 4 + y) * 64 + lane] = f32x4{x[4 * y], x[4 * y + 1], x[4 * y + 2], x[4 * y + 3]};
+    }
+  ends[(wave * 64 + lane) * 2] = m;
+  ends[(wave * 64 + lane) * 2 + 1] = z;
+  __syncthreads();
+  if (!live || (NV == 1 && half)) return;
+  const float m2 = ends[(other * 64 + lane) * 2], top = fmaxf(m, m2);
+  const float w1 = m == NEG_INF ? 0.0f : __builtin_amdgcn_exp2f(m - top), w2 = m2 == NEG_INF ? 0.0f : __builtin_amdgcn_exp2f(m2 - top);
+  const float inv = 1.0f / __builtin_fmaf(ends[(other * 64 + lane) * 2 + 1], w2, z * w1);
+  uint16_t *out = (uint16_t *)a.out + (size_t)tok * a.out_ld + h * s.vdim;
+  const float *gate = a.g_off >= 0 ? a.proj + (size_t)tok * a.proj_ld + a.g_off + h * s.vdim : nullptr;
+  const bool wide = ((s.vdim | a.out_ld) & 3) == 0 && ((uintptr_t)a.out & 7) == 0 &&
+                    (!gate || (((a.proj_ld | a.g_off) & 3) == 0 && ((uintptr_t)a.proj & 15) == 0));  // four columns at a time
+  f32x4 gt[F::KEEP][4];
+#pragma unroll
+  for (int j = 0; j < F::KEEP; ++j)
+#pragma unroll
+    for (int y = 0; y < 4; ++y) {
+      const int d = (half * F::KEEP + j) * 32 + 8 * y + 4 * hh;
+      if (!gate) continue;
+      if (wide) gt[j][y] = *(const f32x4 *)(gate + min(d, s.vdim - 4));
+      else
+#pragma unroll
+        for (int v = 0; v < 4; ++v) gt[j][y][v] = gate[min(d + v, s.vdim - 1)];
+    }
+#pragma unroll
+  for (int j = 0; j < F::KEEP; ++j)
+#pragma unroll
+    for (int y = 0; y < 4; ++y) {
+      const int d = (half * F::KEEP + j) * 32 + 8 * y + 4 * hh;
+      const f32x16 x = NV > 1 && half ? o[NV - F::KEEP + j] : o[j];
+      const f32x4 x2 = sums[((other * F::KEEP + j) * 4 + y) * 64 + lane];
+      uint16_t r[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) r[v] = kx_bf16_rne(__builtin_fmaf(x2[v], w2, x[4 * y + v] * w1) * inv * (gate ? kxr::sigmoid_for<uint16_t>(gt[j][y][v]) : 1.0f));
+      if (wide && d < s.vdim) {
+        *(u32x2 *)(out + d) = u32x2{r[0] | (uint32_t)r[1] << 16, r[2] | (uint32_t)r[3] << 16};
+      } else {
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          if (d + v < s.vdim) out[d + v] = r[v];
+      }
+    }
 }
 
 // keys per workgroup of win_partial_k: few parts, but enough workgroups
@@ -528,16 +587,16 @@ size_t floats_per_part(const KxWindowSpec &s) { return (size_t)s.heads * (kx_pad
 
 template <int ND>
 int flash_nv(const KxWindowArgs &a, int nv, hipStream_t st) {
-  const dim3 grid(kx_cdiv(a.positions, FQ), a.s.heads, a.batch);
+  const dim3 grid(a.s.heads * a.batch, kx_cdiv(a.positions, FQ));
 #define KX_FLASH(NV)                                                                                                          \
   {                                                                                                                           \
-    const size_t lds = ((size_t)FK * (ND * 32 + 8) + (size_t)NV * 32 * (FK + 8)) * 2;                                         \
+    constexpr int lds = Flash<ND, NV>::LDS;                                                                                   \
     static std::atomic<bool> attr{false};                                                                                     \
     if (!attr) {                                                                                                              \
-      KX_HIP(hipFuncSetAttribute((const void *)win_flash_k<ND, NV>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));   \
+      KX_HIP(hipFuncSetAttribute((const void *)win_flash_k<ND, NV>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));        \
       attr = true;                                                                                                            \
     }                                                                                                                         \
-    hipLaunchKernelGGL((win_flash_k<ND, NV>), grid, dim3(256), lds, st, a);                                                   \
+    hipLaunchKernelGGL((win_flash_k<ND, NV>), grid, dim3(FLASH_WAVES * 64), lds, st, a);                                      \
   }
   if (nv == 1) KX_FLASH(1) else if (nv == 2) KX_FLASH(2) else if (nv <= 4) KX_FLASH(4) else KX_FLASH(8)
 #undef KX_FLASH
