@@ -355,17 +355,39 @@ __global__ void __launch_bounds__(512, 1) grouped_gemm_k(PfArgs a) {
 }
 
 // x[t][r] = bf(x + bf(bf(sum_slot eout[t*topk+slot][r] * w[t][slot]) + sy[t][r]))  (:868-877)
+// W columns per thread, 8 where rows are whole 16-byte pieces; their rows of all slots are asked for together, up to eight.  Bound by the
+// experts' results: 2048 tokens of 8 x 7168 154 us with a column per thread, 57 now.
+template <int W>
 __global__ void __launch_bounds__(256) moe_combine_k(const uint16_t *__restrict__ eout, const float *__restrict__ rw,
                                                      const uint16_t *__restrict__ sy, uint16_t *__restrict__ x, int hidden,
                                                      int topk, uint32_t flags) {
-  const int t = blockIdx.y, r = blockIdx.x * blockDim.x + threadIdx.x;
+  struct alignas(W * 2) Cols {
+    uint16_t v[W];
+  };
+  const int t = blockIdx.y, r = (blockIdx.x * blockDim.x + threadIdx.x) * W;
   if (r >= hidden) return;
-  float acc = 0.0f;
-  for (int k = 0; k < topk; ++k)
-    acc = __builtin_fmaf(kx_bf16_f32(eout[((size_t)t * topk + k) * hidden + r]), rw[(size_t)t * topk + k], acc);
-  const float down = kx_bfround(kx_bfround(acc) + kx_bf16_f32(sy[(size_t)t * hidden + r]));
-  uint16_t *xr = x + (size_t)t * hidden + r;
-  *xr = (flags & 1u) ? kx_bf16_rne(down) : kx_bf16_rne(kx_bf16_f32(*xr) + down);
+  const uint16_t *e = eout + (size_t)t * topk * hidden + r;
+  const Cols s = *(const Cols *)(sy + (size_t)t * hidden + r);
+  Cols *xr = (Cols *)(x + (size_t)t * hidden + r), old = *xr;
+  float acc[W] = {};
+  for (int k0 = 0; k0 < topk; k0 += 8) {
+    Cols y[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) y[k] = *(const Cols *)(e + (size_t)min(k0 + k, topk - 1) * hidden);
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      if (k0 + k < topk) {
+        const float w = rw[(size_t)t * topk + k0 + k];
+#pragma unroll
+        for (int c = 0; c < W; ++c) acc[c] = __builtin_fmaf(kx_bf16_f32(y[k].v[c]), w, acc[c]);
+      }
+  }
+#pragma unroll
+  for (int c = 0; c < W; ++c) {
+    const float down = kx_bfround(kx_bfround(acc[c]) + kx_bf16_f32(s.v[c]));
+    old.v[c] = (flags & 1u) ? kx_bf16_rne(down) : kx_bf16_rne(kx_bf16_f32(old.v[c]) + down);
+  }
+  *xr = old;
 }
 
 }  // namespace
@@ -414,7 +436,9 @@ int kx_grouped_gemm_launch(bool dual, const void *w0, const uint16_t *s0, const 
 
 int kx_moe_combine_launch(const uint16_t *eout, const float *rw, const uint16_t *sy, uint16_t *x, int tokens, int hidden,
                           int topk, uint32_t flags, hipStream_t st) {
-  hipLaunchKernelGGL(moe_combine_k, dim3(kx_cdiv(hidden, 256), tokens), dim3(256), 0, st, eout, rw, sy, x, hidden, topk, flags);
+  const bool pieces = hidden % 8 == 0 && (((uintptr_t)eout | (uintptr_t)sy | (uintptr_t)x) & 15) == 0;
+  if (pieces) hipLaunchKernelGGL(moe_combine_k<8>, dim3(kx_cdiv(hidden, 8 * 256), tokens), dim3(256), 0, st, eout, rw, sy, x, hidden, topk, flags);
+  else hipLaunchKernelGGL(moe_combine_k<1>, dim3(kx_cdiv(hidden, 256), tokens), dim3(256), 0, st, eout, rw, sy, x, hidden, topk, flags);
   KX_LAUNCH_CHECK();
   return KX_OK;
 }
