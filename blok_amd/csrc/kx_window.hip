@@ -7,7 +7,8 @@
 // it norms the query itself, and the workgroup that holds the newest key also norms that key, writes the cache rows
 // and, where a block completes, its means.  win_merge_k merges the parts, adds the sink and applies the output gate.
 // Steps of several positions: win_prep_k norms the projections and writes queries and cache rows, win_pool_k the
-// blocks that complete, and then win_flash_k (bf16; matrix cores) or win_partial_k<T, false> + win_merge_k (f32) attend.
+// blocks that complete, and then win_flash_k (bf16) or win_flash_f32_k attend on the matrix cores, or win_partial_k<T, false> +
+// win_merge_k where neither takes the shape.
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -574,6 +575,226 @@ __global__ void __launch_bounds__(FLASH_WAVES * 64, 2) win_flash_k(KxWindowArgs 
     }
 }
 
+// ---- f32, several positions: one head, 32 consecutive positions of one sequence ----
+// As above with 32-bit products (v_mfma_f32_32x32x2_f32) and without LDS: wave w of four has every fourth tile of 32 keys to itself, from
+// memory into the operands' registers.  Lane (r, h) holds columns 8 k + 4 h .. +3 of key r and of query r, so that the first product
+// meets two of them at a time, in four chains (two where registers are short); its result in register v is the weight of key 8 (v / 4) + 4 h + v % 4, which the second
+// product takes as it is, with NV columns of that key's value from NV r on.  The keys of the next tile are asked for when the scores are
+// made, its values behind the second product.  Bound by the products, 8192 cycles of a SIMD for 32 keys of 128 and 128 columns.
+// The waves' sums meet at the end.  In tiles that not every query sees as a whole a value that is not finite is replaced by
+// zero in the product, and added by the queries that see it.
+// 777 positions, 8 heads of 128: 52 us, 141 in parts of 256 keys on the vector ALU.  The error is no larger: chains are short, and a
+// tile's sums are added to those before it (1.02e-7 to 2.05e-7 for 33 to 2048 positions, 0.96 to 1.00 of the parts').
+constexpr int GQ = 32;
+template <int N> struct Floats { typedef float Type __attribute__((ext_vector_type(N))); };
+
+template <int ND, int NV>
+__global__ void __launch_bounds__(256, 1) win_flash_f32_k(KxWindowArgs a) {
+  typedef typename Floats<NV>::Type Value;
+  constexpr int KP = ND * 4, ENDS = 4 * 4 * NV * 1024, QUERIES = ENDS + 4 * 64 * 8;
+  extern __shared__ __attribute__((aligned(16))) uint8_t fl_lds[];
+  const KxWindowSpec &s = a.s;
+  const KxWindowCache &c = a.c;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lq = lane & 31, hh = lane >> 5;
+  const int h = blockIdx.x % s.heads, b = blockIdx.x / s.heads, g = h / (s.heads / s.kv_heads);
+  const int i0 = (gridDim.y - 1 - blockIdx.y) * GQ, i = i0 + lq;
+  const int p = a.pos + min(i, a.positions - 1), tok = min(i, a.positions - 1) * (a.tok_batch ? a.tok_batch : a.batch) + b;
+  const int p_first = a.pos + i0, p_last = a.pos + min(i0 + GQ, a.positions) - 1;
+  const int nb = seen_blocks(p, s.size, s.pool), lo = window_lo(p, s.size);
+  const size_t head = (size_t)b * s.kv_heads + g;
+  const float *kc = (const float *)c.k + head * c.cap * c.dp, *vc = (const float *)c.v + head * c.cap * c.vp;
+  const float *pkc = (const float *)c.pk + head * c.blocks * c.dp, *pvc = (const float *)c.pv + head * c.blocks * c.vp;
+  f32x4 k[KP];
+  f32x4 *const q = (f32x4 *)(fl_lds + QUERIES) + lane;  // [piece][lane], the same for all waves
+  {
+    const float *qr = (const float *)a.q + (size_t)tok * (a.q_ld ? a.q_ld : (size_t)s.heads * c.dp) + (size_t)h * c.dp;
+    for (int x = wave; x < KP; x += 4) q[x * 64] = x * 8 < c.dp ? *(const f32x4 *)(qr + x * 8 + hh * 4) : f32x4{};
+  }
+  __syncthreads();
+  // tiles: the blocks the last query sees, then the positions from the first query's window on; the ring's length is a multiple of 32
+  const int tb = (seen_blocks(p_last, s.size, s.pool) + 31) / 32;
+  const int j0 = window_lo(p_first, s.size) & ~31, tiles = tb + (p_last - j0) / 32 + 1;
+  auto first_key = [&](int t) { return t < tb ? t * 32 : j0 + (t - tb) * 32; };
+  // past the last block there is nothing to read, and past a row's columns its last ones are read again, which meet zeros of the query or a
+  // result that is not stored
+  auto ask_keys = [&](int t) {
+    const int k0 = first_key(t), last = t < tb ? c.blocks - 1 - k0 : 31;
+    const float *kr = t < tb ? pkc + (size_t)k0 * c.dp : kc + (size_t)(k0 % c.cap) * c.dp;
+    const uint32_t at = min(lq, last) * c.dp + hh * 4;
+#pragma unroll
+    for (int x = 0; x < KP; ++x) k[x] = *(const f32x4 *)(kr + min(x * 8, c.dp - 8) + at);
+  };
+  Value val[16];
+  auto ask_values = [&](int t) {
+    const int k0 = first_key(t), last = t < tb ? c.blocks - 1 - k0 : 31, d = min(lq * NV, c.vp - NV);
+    const float *vr = t < tb ? pvc + (size_t)k0 * c.vp : vc + (size_t)(k0 % c.cap) * c.vp;
+    if (last >= 31) {
+      const uint32_t at = 4 * hh * c.vp + d;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) val[v] = *(const Value *)(vr + (8 * (v >> 2) + (v & 3)) * c.vp + at);
+    } else {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) val[v] = *(const Value *)(vr + (uint32_t)(min(8 * (v >> 2) + 4 * hh + (v & 3), last) * c.vp + d));
+    }
+  };
+  f32x16 o[NV];
+#pragma unroll
+  for (int j = 0; j < NV; ++j)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) o[j][v] = 0.0f;
+  const bool sink = s.sink && wave == 0;
+  float m = sink ? (a.sinks ? a.sinks[h] : 0.0f) : NEG_INF, z = sink && hh == 0 ? 1.0f : 0.0f;  // z: of this lane's half of the keys
+  if (wave < tiles) {
+    ask_keys(wave);
+    ask_values(wave);
+  }
+  for (int t = wave; t < tiles; t += 4) {
+    asm volatile("" ::: "memory");  // the query's pieces are read again for each tile: there are no registers to keep them in
+    const bool pooled = t < tb, more = t + 4 < tiles;
+    const int k0 = first_key(t);
+    f32x16 part[2][4], sc;  // short chains: four products each, of which four are added, and those in their order
+    auto gather = [&](const f32x16 (&four)[4]) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) sc[v] += (four[0][v] + four[1][v]) + (four[2][v] + four[3][v]);
+      asm volatile("" : "+v"(sc));  // here: the sums of all pieces at once have no registers
+    };
+#pragma unroll
+    for (int v = 0; v < 16; ++v) sc[v] = 0.0f;
+#pragma unroll
+    for (int x = 0; x < KP; x += 4) {
+      f32x16(&four)[4] = part[x >> 2 & 1];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) four[e] = f32x16{};
+#pragma unroll
+      for (int y = 0; y < 4; ++y) {
+        const f32x4 qx = q[(x + y) * 64];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) four[e] = __builtin_amdgcn_mfma_f32_32x32x2f32(k[x + y][e], qx[e], four[e], 0, 0, 0);
+      }
+      if (x > 0) gather(part[(x >> 2 & 1) ^ 1]);  // under the products of this one
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    gather(part[(KP / 4 - 1) & 1]);
+#pragma unroll
+    for (int v = 0; v < 16; ++v) sc[v] *= s.scale;
+    if (more) ask_keys(t + 4);
+    const int from = (pooled ? 0 : lo) - k0, to = (pooled ? nb - 1 : p) - k0;  // the keys of the tile that this lane's query sees
+    const bool all = pooled ? k0 + 32 <= seen_blocks(p_first, s.size, s.pool) : k0 >= window_lo(p_last, s.size) && k0 + 31 <= p_first;
+    bool odd = false;
+    if (!all) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int e = 8 * (v >> 2) + 4 * hh + (v & 3);
+        sc[v] = ((e < from) | (e > to)) ? NEG_INF : sc[v];
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+          const bool fine = __builtin_isfinite(val[v][j]);
+          odd |= !fine;
+          val[v][j] = fine ? val[v][j] : 0.0f;
+        }
+      }
+    }
+    float top[4];
+#pragma unroll
+    for (int y = 0; y < 4; ++y) top[y] = fmaxf(fmaxf(sc[y], sc[4 + y]), fmaxf(sc[8 + y], sc[12 + y]));
+    float tm = fmaxf(fmaxf(top[0], top[1]), fmaxf(top[2], top[3]));
+    tm = fmaxf(tm, __shfl_xor(tm, 32));
+    if (__any(tm > m)) {
+      const float m1 = fmaxf(m, tm), al = m == NEG_INF ? 0.0f : kx_expf(m - m1);
+      m = m1;
+      z *= al;
+#pragma unroll
+      for (int j = 0; j < NV; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[j][v] *= al;
+    }
+    const float mm = m == NEG_INF ? 0.0f : m;  // nothing seen so far
+#pragma unroll
+    for (int v = 0; v < 16; ++v) sc[v] = kx_expf(sc[v] - mm);
+#pragma unroll
+    for (int y = 0; y < 4; ++y) top[y] = (sc[y] + sc[4 + y]) + (sc[8 + y] + sc[12 + y]);
+    z += (top[0] + top[1]) + (top[2] + top[3]);
+    constexpr int JW = NV > 1 ? 2 : 1;
+    f32x16 own[2][JW];  // the tile's, two blocks of columns at a time
+    auto keep = [&](int j) {
+#pragma unroll
+      for (int y = 0; y < JW; ++y)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[j + y][v] += own[j / JW & 1][y][v];
+#pragma unroll
+      for (int y = 0; y < JW; ++y) asm volatile("" : "+v"(o[j + y]));
+    };
+#pragma unroll
+    for (int j = 0; j < NV; j += JW) {
+      f32x16(&now)[JW] = own[j / JW & 1];
+#pragma unroll
+      for (int y = 0; y < JW; ++y) now[y] = f32x16{};
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+#pragma unroll
+        for (int y = 0; y < JW; ++y) now[y] = __builtin_amdgcn_mfma_f32_32x32x2f32(val[v][j + y], sc[v], now[y], 0, 0, 0);
+      if (j > 0) keep(j - JW);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    keep(NV - JW);
+    if (__builtin_expect(__any(odd), 0)) {
+      const float *vr = pooled ? pvc + (size_t)k0 * c.vp : vc + (size_t)(k0 % c.cap) * c.vp;
+#pragma unroll 1
+      for (int e = max(0, from); e <= min(31, to); ++e) {
+        int d0 = 4 * hh;
+        asm volatile("" : "+v"(d0));  // the places are worked out here, not kept for the whole kernel
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const Value x = *(const Value *)(vr + (uint32_t)(e * c.vp + min((8 * (v >> 2) + d0 + (v & 3)) * NV, c.vp - NV)));
+#pragma unroll
+          for (int j = 0; j < NV; ++j) o[j][v] = __builtin_isfinite(x[j]) ? o[j][v] : o[j][v] + x[j];
+        }
+      }
+    }
+    if (more) ask_values(t + 4);
+  }
+  // the waves' sums meet: [wave][v / 4][column][lane]
+  z += __shfl_xor(z, 32);
+  f32x4 *const sums = (f32x4 *)fl_lds;
+  float *const ends = (float *)(fl_lds + ENDS);
+#pragma unroll
+  for (int j = 0; j < NV; ++j)
+#pragma unroll
+    for (int y = 0; y < 4; ++y) sums[((wave * 4 + y) * NV + j) * 64 + lane] = f32x4{o[j][4 * y], o[j][4 * y + 1], o[j][4 * y + 2], o[j][4 * y + 3]};
+  ends[(wave * 64 + lane) * 2] = m;
+  ends[(wave * 64 + lane) * 2 + 1] = z;
+  __syncthreads();
+  if (i >= a.positions) return;
+  float mw[4], weight[4], most = NEG_INF, total = 0.0f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) most = fmaxf(most, mw[w] = ends[(w * 64 + lane) * 2]);
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    weight[w] = mw[w] == NEG_INF ? 0.0f : kx_expf(mw[w] - most);
+    total = __builtin_fmaf(ends[(w * 64 + lane) * 2 + 1], weight[w], total);
+  }
+  const float inv = 1.0f / total;
+  const int d0 = (8 * wave + 4 * hh) * NV;  // this lane's 4 NV columns
+  float y[4 * NV];
+#pragma unroll
+  for (int j = 0; j < NV; ++j) {
+    f32x4 sum = {};
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const f32x4 x = sums[((w * 4 + wave) * NV + j) * 64 + lane];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) sum[v] = weight[w] > 0.0f ? __builtin_fmaf(x[v], weight[w], sum[v]) : sum[v];  // a wave without keys has none
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) y[v * NV + j] = sum[v] * inv;
+  }
+  float *out = (float *)a.out + (size_t)tok * a.out_ld + h * s.vdim;
+  const float *gate = a.g_off >= 0 ? a.proj + (size_t)tok * a.proj_ld + a.g_off + h * s.vdim : nullptr;
+#pragma unroll
+  for (int x = 0; x < 4 * NV; ++x)
+    if (d0 + x < s.vdim) out[d0 + x] = y[x] * (gate ? kx_sigmoidf(gate[d0 + x]) : 1.0f);
+}
+
 // keys per workgroup of win_partial_k: few parts, but enough workgroups
 int part_keys(const KxWindowSpec &s, int total, int tokens) {
   const int R = s.heads / s.kv_heads;
@@ -602,6 +823,40 @@ int flash_nv(const KxWindowArgs &a, int nv, hipStream_t st) {
 #undef KX_FLASH
   KX_LAUNCH_CHECK();
   return KX_OK;
+}
+
+template <int ND>
+int flash_f32_nv(const KxWindowArgs &a, int nv, hipStream_t st) {
+  const dim3 grid(a.s.heads * a.batch, kx_cdiv(a.positions, GQ));
+#define KX_FLASH(NV)                                                                                                          \
+  {                                                                                                                           \
+    constexpr int lds = 4 * 4 * NV * 1024 + 4 * 64 * 8 + ND * 4 * 1024;                                                       \
+    static std::atomic<bool> attr{false};                                                                                     \
+    if (!attr) {                                                                                                              \
+      KX_HIP(hipFuncSetAttribute((const void *)win_flash_f32_k<ND, NV>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));    \
+      attr = true;                                                                                                            \
+    }                                                                                                                         \
+    hipLaunchKernelGGL((win_flash_f32_k<ND, NV>), grid, dim3(256), lds, st, a);                                               \
+  }
+  if (nv == 1) KX_FLASH(1) else if (nv == 2) KX_FLASH(2) else KX_FLASH(4)
+#undef KX_FLASH
+  KX_LAUNCH_CHECK();
+  return KX_OK;
+}
+// On the matrix cores where that is sooner.  They take a tile's edges with it, 4 us for 128 keys of 256 columns to every 32 queries of a CU, and
+// 16 us to begin; parts on the vector ALU are workgroups of one token and key head, bound by reading its keys for each, 5.5 TB/s over the chip,
+// and by 0.06 us a token and head where those are few.  Whole operator, 8 heads of 128 on 2 key heads, window 1024 (us, parts / matrix cores): 8 positions
+// 15 / 24, 20 32 / 29, 33 43 / 31, 100 93 / 33, 777 316 / 75; 16 sequences of 50 558 / 35; 16 heads on 4, 2048 1141 / 258.
+bool flash_f32(const KxWindowArgs &a) {
+  const KxWindowSpec &s = a.s;
+  if (a.c.dp > 256 || a.c.vp > 128) return false;
+  if (a.tok_batch || a.q_ld) return true;  // parts know nothing of it
+  const double most = most_keys(s, a.pos + a.positions), mean = 0.5 * (most + most_keys(s, a.pos + 1)), columns = a.c.dp + a.c.vp;
+  const long groups = (long)s.heads * a.batch * kx_cdiv(a.positions, GQ), tokens = (long)a.batch * a.positions;
+  const double keys = (kx_cdiv(groups, std::max(1, kx_device_cus())) - 1) * mean + most;
+  const double flash = 16.0 + keys / 128 * 4.0 * columns / 256;
+  const double parts = 7.0 + tokens * std::max(0.06 * s.heads, mean * columns * 4 * s.kv_heads / 5.5e6);
+  return flash < parts;
 }
 
 int check(const KxWindowArgs &a) {
@@ -650,6 +905,11 @@ int attend(const KxWindowArgs &a, hipStream_t st) {
     const int nd = a.c.dp / 32, nv = a.c.vp / 32;
     return nd == 1 ? flash_nv<1>(a, nv, st) : nd == 2 ? flash_nv<2>(a, nv, st) : nd <= 4 ? flash_nv<4>(a, nv, st)
          : nd <= 6 ? flash_nv<6>(a, nv, st) : flash_nv<8>(a, nv, st);
+  }
+  if (sizeof(T) == 4 && flash_f32(a)) {
+    const int nd = a.c.dp / 32, nv = a.c.vp / 32;
+    return nd == 1 ? flash_f32_nv<1>(a, nv, st) : nd == 2 ? flash_f32_nv<2>(a, nv, st) : nd <= 4 ? flash_f32_nv<4>(a, nv, st)
+         : nd <= 6 ? flash_f32_nv<6>(a, nv, st) : flash_f32_nv<8>(a, nv, st);
   }
   KX_REQUIRE(!a.tok_batch && !a.q_ld, "window attention: a part of a step with keys of %d and values of %d", a.s.dim, a.s.vdim);
   return attend_parts<T>(a, false, st);

@@ -555,3 +555,17 @@ def test_trace_replay(kxlib, models, tmp_path):
     two = json.dumps({"step": 0, "entries": [{"id": "a", "tokens": [1], "want": []}, {"id": "b", "tokens": [1], "want": []}], "end": []})
     r = subprocess.run(cmd, input=two + "\n", capture_output=True, text=True, timeout=400)
     assert r.returncode == 1 and "one request at a time" in r.stderr
+
+
+@pytest.mark.parametrize("heads, kv, dim, vdim, size, pool, batch, cuts", [(4, 2, 32, 32, 40, 8, 2, [97]), (8, 2, 40, 70, 1000, 16, 1, [33, 64]), (4, 4, 190, 120, 64, 4, 1, [31, 130]),
+                                                                           (2, 1, 256, 128, 96, 0, 3, [65, 1, 60]), (3, 3, 128, 20, 33, 32, 2, [200])])
+def test_32_bit_attention_of_prompts(kxlib, heads, kv, dim, vdim, size, pool, batch, cuts):
+    """Tiles of 32 queries and keys with remainders, rings that begin anywhere, keys and values of every width the matrix cores take.  The bar: sums of up to
+    256 products and 260 weights, 2e-6."""
+    n = sum(cuts)
+    w = Window(kxlib, heads, kv, dim, vdim, size, pool, 1, batch=batch, context=n, positions=max(cuts))
+    proj = np.random.default_rng(dim).standard_normal((batch, n, w.cols[-1])).astype(np.float32)
+    got = w.run(proj, cuts, batch)
+    for b in range(batch):
+        assert rel(got[b], w.oracle(proj[b], pool=pool or 1 << 20)) < 2e-6
+    w.close()
