@@ -444,12 +444,13 @@ int expanded(const KxLatentArgs &a, hipStream_t st) {
   const int tokens = a.batch * a.positions, n = a.pos + a.positions, cap = kx_pad(n, 64), dp = kx_pad(s.dim + s.rot_dim, 32), vp = kx_pad(s.vdim, 32);
   hipLaunchKernelGGL(prep_k<T>, dim3(tokens), dim3(256), 0, st, a, dp);
   KX_LAUNCH_CHECK();
-  for (int b = 0; b < a.batch; ++b)
+  const int at_once = (long)a.batch * n > KX_NARROW_TOKENS ? a.batch : 1;  // sequences in one product
+  for (int b = 0; b < a.batch; b += at_once)
     for (int value = 0; value < 2; ++value) {
       const int ld = value ? vp : dp;
       KxLinArgs g;
       g.m = value ? a.uv : a.uk;
-      g.tokens = n;
+      g.tokens = at_once * n;
       g.row.cols = s.kv_rank;
       g.row.x = (const T *)a.rows + (size_t)b * a.cap * kx_latent_row(s);
       g.row.x_ld = kx_latent_row(s);
@@ -458,6 +459,11 @@ int expanded(const KxLatentArgs &a, hipStream_t st) {
       g.mid_ld = ld;
       g.head_dim = value ? s.vdim : s.dim;
       g.head_stride = (size_t)cap * ld;
+      if (at_once > 1) {
+        g.seq = n;
+        g.seq_rows = a.cap;
+        g.seq_out = (size_t)s.heads * cap * ld;
+      }
       int rc = kx_linear_launch(sizeof(T) == 4, g, nullptr, st);
       if (rc) return rc;
     }

@@ -74,6 +74,11 @@ struct KxLinArgs {
   // HEADS: element (t, h * head_dim + d) goes to mid[h * head_stride + t * mid_ld + d]
   int head_dim = 0;
   size_t head_stride = 0;
+  // HEADS of several sequences in one product (seq > 0; more tokens than KX_NARROW_TOKENS): token t is row t % seq of sequence t / seq, whose rows
+  // of x begin seq_rows rows and whose results seq_out elements behind those of the one before.  Three sequences of 701 positions, 2048 x 512:
+  // one launch of 24 us where three took 18 each.
+  int seq = 0;
+  size_t seq_rows = 0, seq_out = 0;
   float *streams = nullptr;  // STREAMS: f32 [tokens][n_streams][m.rows]
   int n_streams = 1;
   const float *mix = nullptr, *outw = nullptr;  // nullptr: identity and ones

@@ -47,9 +47,9 @@ __device__ __forceinline__ void put_f32(const KxLinArgs &a, int t, int r, float 
   else ((T *)a.mid)[(size_t)t * a.mid_ld + r - a.act_from] = Elem<T>::make(gelu<T>(y));
 }
 template <class T>
-__device__ __forceinline__ void put_head(const KxLinArgs &a, int t, int r, float y) {
+__device__ __forceinline__ void put_head(const KxLinArgs &a, size_t at, int r, float y) {  // at: of the token
   const int h = r / a.head_dim;
-  ((T *)a.mid)[h * a.head_stride + (size_t)t * a.mid_ld + r - h * a.head_dim] = Elem<T>::make(y);
+  ((T *)a.mid)[h * a.head_stride + at + r - h * a.head_dim] = Elem<T>::make(y);
 }
 // variant of the activation rows that matrix rows from r on meet
 __device__ __forceinline__ int variant_of(const KxLinArgs &a, int r) {
@@ -239,7 +239,7 @@ lin_gemv_k(KxLinArgs a, KxExpertArgs x) {
       if (finish) {
         if constexpr (EPI == KX_LIN_GLU) put_glu<T>(a, MODE == GV_EXPERT_IN ? pair : tok, unit, red[wave][lane], red[wave][NT + lane], weight);
         else if constexpr (EPI == KX_LIN_F32) put_f32<T>(a, tok, row, red[wave][lane]);
-        else if constexpr (EPI == KX_LIN_HEADS) put_head<T>(a, tok, row, red[wave][lane]);
+        else if constexpr (EPI == KX_LIN_HEADS) put_head<T>(a, (size_t)tok * a.mid_ld, row, red[wave][lane]);
         else res.store(a, tok0 + tok, row, red[wave][lane]);
       }
       asm volatile("" ::: "memory");
@@ -290,6 +290,11 @@ __device__ __forceinline__ size_t source_row(const KxExpertArgs &e, const Tile &
   const int s = min(t.m0 + i, t.end - 1);
   return GROUP && e.gather ? e.gather[s] : s;
 }
+// place of token t of a product of several sequences
+__device__ __forceinline__ size_t of_sequence(const KxLinArgs &a, size_t per_seq, size_t per_token, int t) {
+  const int b = (uint32_t)t / (uint32_t)a.seq;
+  return b * per_seq + (size_t)(t - b * a.seq) * per_token;
+}
 
 template <class T, class TL, int EPI, bool GROUP>
 __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) lin_gemm_k(KxLinArgs a, KxExpertArgs e, const T *__restrict__ x, int x_ld, kxtile::Share share) {
@@ -312,6 +317,7 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) lin_gemm_k(Kx
   const int nb = a.m.ld / TL::COLS;
   typename TL::Sums acc;
   TL::run(lds, kxtile::cut(nb, at.part, at.of), kxtile::cut(nb, at.part + 1, at.of), [&](int r) {
+    if (EPI == KX_LIN_HEADS && !GROUP && a.seq && r < TL::BM) return x + of_sequence(a, a.seq_rows, 1, min(tl.m0 + r, tl.end - 1)) * x_ld;
     return r < TL::BM ? x + source_row<GROUP>(e, tl, r) * x_ld : (const T *)a.m.w + tl.w + (size_t)min(n0 + r - TL::BM, a.m.rows - 1) * a.m.ld;
   }, acc);
   if (!GROUP && at.of > 1 &&
@@ -332,16 +338,23 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) lin_gemm_k(Kx
             put_glu<T>(a, t, (r >> 6) * KX_GLU_BLOCK + (r & 31), acc[i][j][v], acc[i][j + STEP][v], GROUP ? e.slot_weight[t] : 1.0f);
         }
       }
-    } else if constexpr (EPI == KX_LIN_F32 || EPI == KX_LIN_HEADS) {
+    } else if constexpr (EPI == KX_LIN_F32) {
 #pragma unroll
       for (int j = 0; j < TL::NI; ++j) {
         const int r = n0 + TL::col(j);
 #pragma unroll
         for (int v = 0; v < TL::V; ++v)
-          if (tl.m0 + TL::row(i, v) < tl.end && r < a.m.rows) {
-            if constexpr (EPI == KX_LIN_F32) put_f32<T>(a, tl.m0 + TL::row(i, v), r, acc[i][j][v]);
-            else put_head<T>(a, tl.m0 + TL::row(i, v), r, acc[i][j][v]);
-          }
+          if (tl.m0 + TL::row(i, v) < tl.end && r < a.m.rows) put_f32<T>(a, tl.m0 + TL::row(i, v), r, acc[i][j][v]);
+      }
+    } else if constexpr (EPI == KX_LIN_HEADS) {
+#pragma unroll
+      for (int v = 0; v < TL::V; ++v) {
+        const int t = tl.m0 + TL::row(i, v);
+        if (t >= tl.end) continue;
+        const size_t at = a.seq ? of_sequence(a, a.seq_out, a.mid_ld, t) : (size_t)t * a.mid_ld;
+#pragma unroll
+        for (int j = 0; j < TL::NI; ++j)
+          if (n0 + TL::col(j) < a.m.rows) put_head<T>(a, at, n0 + TL::col(j), acc[i][j][v]);
       }
     } else {
       constexpr int G = most_streams(EPI) > 2 ? 4 : 16;  // elements read before the first is written
@@ -488,7 +501,7 @@ __global__ void __launch_bounds__(512, MI == 1 ? 4 : 2) lin_narrow_k(KxLinArgs a
       if constexpr (EPI >= KX_LIN_STREAMS) res.load(a, t, r);
       const float y = value(i >> 6, i & 63);
       if constexpr (EPI == KX_LIN_F32) put_f32<uint16_t>(a, t, r, y);
-      else if constexpr (EPI == KX_LIN_HEADS) put_head<uint16_t>(a, t, r, y);
+      else if constexpr (EPI == KX_LIN_HEADS) put_head<uint16_t>(a, (size_t)t * a.mid_ld, r, y);
       else res.store(a, t, r, y);
     }
   }
@@ -687,6 +700,8 @@ int check_matrix(const KxLinArgs &a) {
   KX_REQUIRE(a.n_streams >= 1 && a.n_streams <= KX_MAX_STREAMS && (a.mix || a.n_streams == 1), "kx_linear: %d streams", a.n_streams);
   KX_REQUIRE(a.epi != KX_LIN_F32 || a.act_from >= a.m.rows || (a.mid && a.mid_ld >= a.m.rows - a.act_from), "kx_linear: no room for %d activations", a.m.rows - a.act_from);
   KX_REQUIRE(a.epi != KX_LIN_HEADS || (a.head_dim > 0 && a.mid), "kx_linear: heads of %d", a.head_dim);
+  KX_REQUIRE(!a.seq || (a.seq > 0 && a.epi == KX_LIN_HEADS && a.row.kind == KX_ROW_PLAIN && a.tokens > KX_NARROW_TOKENS && a.tokens % a.seq == 0), "kx_linear: %d tokens in sequences of %d",
+             a.tokens, a.seq);
   KX_REQUIRE(a.row.kind != KX_ROW_SHIFT || (a.epi == KX_LIN_F32 && a.row.n_streams == 1 && a.row.batch > 0 && a.row.tokens == a.tokens && a.row.prev && a.row.prev_out &&
                                             a.row.prev != a.row.prev_out && a.n_var == a.row.n_mix + 1 && a.n_var <= KX_MAX_VARIANTS),
              "kx_linear: %d mixes of %d tokens", a.row.n_mix, a.row.tokens);
