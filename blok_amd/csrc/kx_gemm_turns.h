@@ -26,15 +26,17 @@
 
 namespace kxtile {
 
-// 16 x 16 blocks of sums: element v of block (i, j) is matrix row col(j), token row(i, v).
-template <bool TWIN>
+// 16 x 16 blocks of sums: element v of block (i, j) is matrix row col(j), token row(i, v).  RI: blocks of tokens of a wave while it
+// multiplies; with fewer than four, tiles of 64 RI x 256 for the ends of lists of rows.
+template <bool TWIN, int RI = 4>
 struct Turns {
   typedef f32x4 Block;
   static constexpr int V = 4, SIDE = 16;
   static constexpr int COLS = 64, THREADS = 512, WAVES_PER_SIMD = 2;
-  static constexpr int BM = TWIN ? 128 : 256, BN = BM;
-  static constexpr int MI = TWIN ? 2 : 4, NI = TWIN ? 4 : 8;       // blocks of a wave when the products are done
-  static constexpr int XS = BM * 128, LDS = TWIN ? 4 * 2 * XS : 2 * 2 * XS;  // bytes of a block's tokens; four blocks, two
+  static_assert(!TWIN || RI == 4, "twin tiles are 128 x 128");
+  static constexpr int BM = TWIN ? 128 : 64 * RI, BN = TWIN ? 128 : 256;
+  static constexpr int MI = TWIN ? 2 : RI, NI = TWIN ? 4 : 8;      // blocks of a wave when the products are done
+  static constexpr int XS = BM * 128, WS = BN * 128, LDS = (TWIN ? 4 : 2) * (XS + WS);  // bytes of a block's tokens, of its rows; four blocks, two
   static constexpr size_t PART = (size_t)BM * BN;
   typedef Block Sums[MI][NI];
 
@@ -42,7 +44,7 @@ struct Turns {
   static __device__ __forceinline__ int member() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6 & 3); }
   static __device__ __forceinline__ int col(int j) { return (TWIN ? (member() & 1) * 64 : group() * 128) + j * 16 + (threadIdx.x & 15); }
   static __device__ __forceinline__ int row(int i, int v) {
-    return (TWIN ? (member() >> 1) * 64 + group() * 32 : member() * 64) + i * 16 + 4 * (threadIdx.x >> 4 & 3) + v;
+    return (TWIN ? (member() >> 1) * 64 + group() * 32 : member() * (16 * RI)) + i * 16 + 4 * (threadIdx.x >> 4 & 3) + v;
   }
 
   static __device__ __forceinline__ void turn() {
@@ -54,14 +56,17 @@ struct Turns {
   static __device__ __forceinline__ void run(uint8_t *lds, int kb0, int kb1, Row row, Sums &out) {
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
     const int lane = threadIdx.x & 63, sub = lane >> 3, g = group(), me = member(), lr = lane & 15, kq = lane >> 4, n = kb1 - kb0;
-    constexpr int RI = 4, RJ = TWIN ? 4 : 8;  // blocks of a wave while it multiplies
-    constexpr int XW = TWIN ? XS : 2 * XS;    // the matrix lies behind the tokens: of the same block, of both
-    // the eight copies of a wave per block, eight rows each.  Whole: tokens or matrix; Twin: four of the tokens and four of the matrix
+    constexpr int RJ = TWIN ? 4 : 8;        // blocks of rows of a wave while it multiplies
+    constexpr int XW = TWIN ? XS : 2 * XS;  // the matrix lies behind the tokens: of the same block, of both
+    // the up to eight copies of a wave per block, eight rows each.  Whole: tokens or matrix; Twin: four of the tokens and four of the matrix
     const uint16_t *src[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) src[i] = row((!TWIN && g ? BM : 0) + (i * 4 + me) * 8 + sub) + kb0 * COLS + ((lane & 7) ^ sub) * 8;
+    for (int i = 0; i < 8; ++i) {
+      const int r = (i * 4 + me) * 8 + sub;
+      src[i] = row(TWIN ? r : g ? BM + r : RI < 4 ? min(r, BM - 1) : r) + kb0 * COLS + ((lane & 7) ^ sub) * 8;
+    }
     auto copy = [&](int b, int base, int i) { kx_copy16_to_lds(src[i] + b * COLS, __builtin_amdgcn_readfirstlane(lds0 + base + (i * 4 + me) * 1024)); };
-    const uint8_t *const xs = lds + ((TWIN ? me >> 1 : me) * 64 + lr) * 128, *const ws = lds + XW + ((TWIN ? (me & 1) * 64 : g * 128) + lr) * 128;
+    const uint8_t *const xs = lds + ((TWIN ? (me >> 1) * 64 : me * (16 * RI)) + lr) * 128, *const ws = lds + XW + ((TWIN ? (me & 1) * 64 : g * 128) + lr) * 128;
     const int p[2] = {(kq ^ (lr & 7)) * 16, ((4 + kq) ^ (lr & 7)) * 16};  // the lane's piece of a row, columns 0 to 31 and 32 to 63
     Block acc[RI][RJ];
 #pragma unroll
@@ -89,14 +94,14 @@ struct Turns {
       constexpr int HALF = BN / 2 * 128;  // of a block of the matrix
       if (g == 0) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) copy(0, 0, i);
+        for (int i = 0; i < 2 * RI; ++i) copy(0, 0, i);
         kx_wait_copies<0>();
       } else {
 #pragma unroll
         for (int i = 0; i < 8; ++i) copy(0, XW, i);
         if (n > 1) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) copy(1, XW + XS, i);
+          for (int i = 0; i < 4; ++i) copy(1, XW + WS, i);
           kx_wait_copies<4>();
         } else {
           kx_wait_copies<0>();
@@ -106,25 +111,25 @@ struct Turns {
       turn();
       if (g == 1) turn();
       for (int b = 0; b < n; ++b) {
-        const int at = (b & 1) * XS, other = at ^ XS;
-        read(0, at, at);
+        const int at = b & 1, other = at ^ 1;
+        read(0, at * XS, at * WS);
         if (b + 1 < n) {
           if (g == 0) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) copy(b + 1, other, i);
+            for (int i = 0; i < RI; ++i) copy(b + 1, other * XS, i);
           } else {
 #pragma unroll
-            for (int i = 4; i < 8; ++i) copy(b + 1, XW + other, i);
+            for (int i = 4; i < 8; ++i) copy(b + 1, XW + other * WS, i);
           }
         }
-        read(1, at, at);
+        read(1, at * XS, at * WS);
         if (g == 0) {
           if (b + 1 < n)
 #pragma unroll
-            for (int i = 4; i < 8; ++i) copy(b + 1, other, i);
+            for (int i = RI; i < 2 * RI; ++i) copy(b + 1, other * XS, i);
         } else if (b + 2 < n) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) copy(b + 2, XW + at, i);
+          for (int i = 0; i < 4; ++i) copy(b + 2, XW + at * WS, i);
           kx_wait_copies<8>();  // group 0's half of block b + 1, asked for a block ago, has come
         } else {
           kx_wait_copies<0>();

@@ -296,24 +296,9 @@ __device__ __forceinline__ size_t of_sequence(const KxLinArgs &a, size_t per_seq
   return b * per_seq + (size_t)(t - b * a.seq) * per_token;
 }
 
+// one tile, or a part of its columns
 template <class T, class TL, int EPI, bool GROUP>
-__global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) lin_gemm_k(KxLinArgs a, KxExpertArgs e, const T *__restrict__ x, int x_ld, kxtile::Share share) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  Tile tl;
-  int n0;
-  kxtile::Place at = {0, 0, 1};
-  if constexpr (GROUP) {
-    if (!tile_of<true>(a, e, TL::BM, tl)) return;
-    n0 = blockIdx.x * TL::BN;
-  } else {
-    const int tm = (a.tokens + TL::BM - 1) / TL::BM;
-    at = kxtile::place_of(blockIdx.x, tm * ((a.m.rows + TL::BN - 1) / TL::BN), share);
-    n0 = at.tile / tm * TL::BN;
-    tl.m0 = at.tile % tm * TL::BM;
-    tl.end = a.tokens;
-    tl.w = 0;
-  }
-  x += (size_t)variant_of(a, n0) * a.tokens * x_ld;
+__device__ __forceinline__ void gemm_tile(uint8_t *lds, const KxLinArgs &a, const KxExpertArgs &e, const T *__restrict__ x, int x_ld, const Tile &tl, int n0, kxtile::Place at, int whole) {
   const int nb = a.m.ld / TL::COLS;
   typename TL::Sums acc;
   TL::run(lds, kxtile::cut(nb, at.part, at.of), kxtile::cut(nb, at.part + 1, at.of), [&](int r) {
@@ -321,7 +306,7 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) lin_gemm_k(Kx
     return r < TL::BM ? x + source_row<GROUP>(e, tl, r) * x_ld : (const T *)a.m.w + tl.w + (size_t)min(n0 + r - TL::BM, a.m.rows - 1) * a.m.ld;
   }, acc);
   if (!GROUP && at.of > 1 &&
-      !kxtile::gather<TL>(lds, acc, a.part + (size_t)(at.tile - share.whole) * at.of * TL::PART, a.arrived + at.tile - share.whole, at.of, at.part))
+      !kxtile::gather<TL>(lds, acc, a.part + (size_t)(at.tile - whole) * at.of * TL::PART, a.arrived + at.tile - whole, at.of, at.part))
     return;
 #pragma unroll
   for (int i = 0; i < TL::MI; ++i) {
@@ -373,6 +358,37 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) lin_gemm_k(Kx
         }
       }
     }
+  }
+}
+
+// Tiles of up to 256 slots of an expert.  Its last one takes the kernel of as many quarters as it fills: 2 of them are as long as two tiles of 128 x 128.
+template <class TL>
+constexpr bool LISTED_LARGE = false;
+template <>
+constexpr bool LISTED_LARGE<kxtile::Large> = true;
+
+template <class T, class TL, int EPI, bool GROUP>
+__global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) lin_gemm_k(KxLinArgs a, KxExpertArgs e, const T *__restrict__ x, int x_ld, kxtile::Share share) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  Tile tl;
+  if constexpr (GROUP) {
+    if (!tile_of<true>(a, e, TL::BM, tl)) return;
+    const int n0 = blockIdx.x * TL::BN;
+    if constexpr (LISTED_LARGE<TL>) {
+      const int n = tl.end - tl.m0;
+      if (n <= 64) return gemm_tile<T, kxtile::Turns<false, 1>, EPI, true>(lds, a, e, x, x_ld, tl, n0, {0, 0, 1}, 0);
+      if (n <= 128) return gemm_tile<T, kxtile::Turns<false, 2>, EPI, true>(lds, a, e, x, x_ld, tl, n0, {0, 0, 1}, 0);
+      if (n <= 192) return gemm_tile<T, kxtile::Turns<false, 3>, EPI, true>(lds, a, e, x, x_ld, tl, n0, {0, 0, 1}, 0);
+    }
+    gemm_tile<T, TL, EPI, true>(lds, a, e, x, x_ld, tl, n0, {0, 0, 1}, 0);
+  } else {
+    const int tm = (a.tokens + TL::BM - 1) / TL::BM;
+    const kxtile::Place at = kxtile::place_of(blockIdx.x, tm * ((a.m.rows + TL::BN - 1) / TL::BN), share);
+    const int n0 = at.tile / tm * TL::BN;
+    tl.m0 = at.tile % tm * TL::BM;
+    tl.end = a.tokens;
+    tl.w = 0;
+    gemm_tile<T, TL, EPI, false>(lds, a, e, x + (size_t)variant_of(a, n0) * a.tokens * x_ld, x_ld, tl, n0, at, share.whole);
   }
 }
 
@@ -639,6 +655,7 @@ int gemm_launch(const KxLinArgs &a, const KxExpertArgs &e, const T *x, int x_ld,
     const kxtile::Share s = GROUP ? kxtile::Share{0, 1} : kxtile::choose_single(a.tokens, a.m.rows, a.m.ld / kxtile::Single::COLS, room, arrivals, cus);
     return tile_launch<float, kxtile::Single, EPI, GROUP>(a, e, x, x_ld, s, st);
   } else if constexpr (GROUP) {
+    if (e.tile_slots > 128) return tile_launch<uint16_t, kxtile::Large, EPI, true>(a, e, x, x_ld, {0, 1}, st);
     return e.tile_slots > 64 ? tile_launch<uint16_t, kxtile::Medium, EPI, true>(a, e, x, x_ld, {0, 1}, st) : tile_launch<uint16_t, SmallSlots, EPI, true>(a, e, x, x_ld, {0, 1}, st, small_slots_lds(a, e));
   } else {
     const kxtile::Choice c = kxtile::choose(a.tokens, a.m.rows, a.m.ld >> 6, room, arrivals, cus);
@@ -751,7 +768,7 @@ int expert_out(const KxLinArgs &a, const KxExpertArgs &e, hipStream_t st) {
 template <class T>
 int expert_gemm(const KxLinArgs &a, const KxExpertArgs &e, const T *x, int x_ld, hipStream_t st) {
   KX_REQUIRE(e.tiles && e.n_tiles && e.max_tiles > 0 && e.max_tiles <= 65535 && a.n_var == 1, "experts: %d tiles", e.max_tiles);
-  KX_REQUIRE(e.tile_slots > 0 && e.tile_slots <= (sizeof(T) == 4 ? 64 : 128), "experts: tiles of %d", e.tile_slots);
+  KX_REQUIRE(e.tile_slots > 0 && e.tile_slots <= (sizeof(T) == 4 ? 64 : 256), "experts: tiles of %d", e.tile_slots);
   KX_REQUIRE(a.epi != KX_LIN_GLU || e.slot_weight, "experts: no weights");
   if (a.epi == KX_LIN_GLU) return gemm_launch<T, KX_LIN_GLU, true>(a, e, x, x_ld, st);
   KX_REQUIRE(a.epi == KX_LIN_F32, "experts: epilogue %d", a.epi);

@@ -740,3 +740,18 @@ def test_trace_replay(kxlib, models, tmp_path):
         assert sorted(os.listdir(out)) == [f"{i}.f32" for i in want]
         for i, ref in want.items():
             assert KC.logit_error(np.fromfile(out / f"{i}.f32", np.float32).reshape(ref.shape), ref).max() < bar, (dtype, i)
+
+
+@pytest.mark.parametrize("tokens", [192, 256, 300, 380, 440])
+def test_experts_with_tiles_of_256_slots(kxlib, tokens):
+    """All tokens to every second of 64 experts: lists of tiles that end in one of one to four quarters, rows of both products that are no multiple of 256."""
+    a = Experts(kxlib, 1300, 620, 64, 32, 64, 0, tokens)
+    a.router[:], a.bias[:] = 0.0, 0.0
+    a.bias[::2] = 3.0
+    a.push()
+    r = np.random.default_rng(tokens)
+    x, rows = r.standard_normal((tokens, 1300)).astype(np.float32), KC.bf16(r.standard_normal((tokens, 64)))
+    got, ids = a.run(x, rows)
+    assert (np.sort(ids, 1) == np.arange(0, 64, 2)).all()
+    assert rel(got, a.oracle(x, rows, ids)) < 2e-2
+    a.close()
