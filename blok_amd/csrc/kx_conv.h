@@ -41,4 +41,37 @@ __device__ __forceinline__ void shift(const KxConvArgs &a, int b, int ch) {
   for (int j = 0; j < keep; ++j) a.hist_out[((size_t)b * keep + j) * a.channels + ch] = input(a, b, a.positions - keep + j, ch, col);
 }
 
+// A channel at a step's only position, of up to FEW taps: its inputs and weights are asked for together.  A loop over any number of taps
+// asks for them one after the other, and that, with the state and the step's numbers asked for behind it, was half of a decode step's
+// recurrent kernels: delta_step_k 12.8 us and 6.2 with all of it in front, ssd_step_k 13.4 and 10.1 (kx_delta.hip, kx_ssd.hip).
+constexpr int FEW = 4;
+struct Channel {
+  float w[FEW], x[FEW], bias;
+};
+__device__ __forceinline__ Channel ask(const KxConvArgs &a, int b, int ch) {
+  Channel c;
+  const int col = column(a, ch);
+  c.bias = a.bias ? a.bias[ch] : 0.0f;
+#pragma unroll
+  for (int j = 0; j < FEW; ++j) {
+    const int t = min(j, a.taps - 1);
+    c.w[j] = a.w[(size_t)ch * a.taps + t];
+    const float *at = t == a.taps - 1 ? a.proj + (size_t)b * a.proj_ld + col : a.hist + ((size_t)b * (a.taps - 1) + t) * a.channels + ch;
+    c.x[j] = *at;  // input(a, b, t - (a.taps - 1), ch, col), without a branch between the loads
+  }
+  return c;
+}
+__device__ __forceinline__ float silu_of(const KxConvArgs &a, const Channel &c) {
+  float v = c.bias;
+#pragma unroll
+  for (int j = 0; j < FEW; ++j)
+    if (j < a.taps) v = __builtin_fmaf(c.w[j], c.x[j], v);
+  return kx_siluf(v);
+}
+__device__ __forceinline__ void shift(const KxConvArgs &a, int b, int ch, const Channel &c) {
+#pragma unroll
+  for (int j = 1; j < FEW; ++j)
+    if (j < a.taps) a.hist_out[((size_t)b * (a.taps - 1) + j - 1) * a.channels + ch] = c.x[j];
+}
+
 }  // namespace kxc

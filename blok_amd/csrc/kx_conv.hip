@@ -30,11 +30,7 @@ __global__ void __launch_bounds__(256) conv_silu_k(KxConvArgs a, float *__restri
       if (i0 + j < i1) raw[(size_t)((i0 + j) * a.batch + b) * C + ch] = kx_siluf(v);
     }
   }
-}
-
-__global__ void __launch_bounds__(256) conv_hist_k(KxConvArgs a) {
-  const int ch = blockIdx.x * 256 + threadIdx.x;
-  if (ch < a.channels) kxc::shift(a, blockIdx.y, ch);
+  if (i1 == a.positions && a.taps > 1) kxc::shift(a, b, ch);
 }
 
 }  // namespace
@@ -48,9 +44,5 @@ int kx_conv_launch(const KxConvArgs &a, float *raw, hipStream_t st) {
   else if (a.taps == 4) hipLaunchKernelGGL(conv_silu_k<4>, grid, dim3(256), 0, st, a, raw);
   else hipLaunchKernelGGL(conv_silu_k<0>, grid, dim3(256), 0, st, a, raw);
   KX_LAUNCH_CHECK();
-  if (a.taps > 1) {
-    hipLaunchKernelGGL(conv_hist_k, dim3(kx_cdiv(a.channels, 256), a.batch), dim3(256), 0, st, a);
-    KX_LAUNCH_CHECK();
-  }
   return KX_OK;
 }

@@ -1,7 +1,8 @@
 // kx_delta.hip -- see kx_delta.h.  Nothing here is less than 32-bit.  No counterpart in the reference, which has no recurrent layer.
 //
 // One token per sequence: delta_step_k.  A workgroup owns 32 columns of one head's state; it convolves and norms the
-// head's q and k itself, reads its columns once, and writes them once.
+// head's q and k itself, reads its columns once, and writes them once.  All it needs from memory is asked
+// for first, and the columns stay in registers (figures in kx_conv.h).
 //
 // Several positions: the convolutions (kx_conv.hip), then blocks of 16 tokens counted from the step's first position.  With S the
 // state before a block, D(i, j) the product of the decays of its tokens i + 1 .. j and G(j) that of tokens 1 .. j,
@@ -44,41 +45,75 @@ __host__ __device__ __forceinline__ KxConvArgs conv_of(const KxDeltaArgs &a) {
   return c;
 }
 
+template <int RPT>  // rows of the state per thread
 __global__ void __launch_bounds__(256) delta_step_k(KxDeltaArgs a, KxConvArgs cv) {
-  extern __shared__ float dl_lds[];
-  __shared__ float red[4];
+  __shared__ float q[8 * RPT], k[8 * RPT], v[SC], red[2][4];
   __shared__ float part[2][8][SC];
   const KxDeltaSpec &s = a.s;
   const int D = s.dim, V = s.vdim, tid = threadIdx.x, slices = (V + SC - 1) / SC;
   const int h = blockIdx.x / slices, c0 = (blockIdx.x - h * slices) * SC, b = blockIdx.y;
-  const int kvh = h / (s.heads / s.kv_heads), nq = s.kv_heads * D;
-  float *q = dl_lds, *k = q + D, *v = k + D, *S = v + SC;  // S [D][SC]
+  const int ratio = s.heads / s.kv_heads, kvh = h / ratio, nq = s.kv_heads * D;
   const int c = tid & (SC - 1), rg = tid / SC, col = min(c0 + c, V - 1);
   float *st = a.state + ((size_t)b * s.heads + h) * D * V;
-  for (int r = rg; r < D; r += 8) S[r * SC + c] = st[(size_t)r * V + col];
-  float qq = 0.0f, kk = 0.0f;
-  for (int x = tid; x < 2 * D; x += 256) {
-    const bool key = x >= D;
-    const int d = key ? x - D : x;
-    const float y = kxc::conv_silu(cv, b, 0, (key ? nq : 0) + kvh * D + d);
-    (key ? k : q)[d] = y;
-    if (key) kk = __builtin_fmaf(y, y, kk);
-    else qq = __builtin_fmaf(y, y, qq);
+  // all that comes from memory is asked for first: what the convolutions need, the numbers of the step, the state
+  auto channel = [&](int x) { return x < D ? kvh * D + x : nq + kvh * D + x - D; };
+  constexpr int CH = (2 * 8 * RPT + 255) / 256;  // channels of q and k per thread
+  const bool few = cv.taps <= kxc::FEW, first = c0 == 0 && h % ratio == 0;
+  kxc::Channel ch[CH], vch;
+  if (few) {
+#pragma unroll
+    for (int y = 0; y < CH; ++y) ch[y] = kxc::ask(cv, b, channel(min(tid + y * 256, 2 * D - 1)));
+    vch = kxc::ask(cv, b, 2 * nq + h * V + min(c0 + (tid & (SC - 1)), V - 1));
   }
-  if (tid < SC) v[tid] = c0 + tid < V ? kxc::conv_silu(cv, b, 0, 2 * nq + h * V + c0 + tid) : 0.0f;
-  qq = kxr::block_sum(qq, red);
-  kk = kxr::block_sum(kk, red);
-  const float qsc = kx_rsqrtf(qq + s.unit_eps) * kx_rsqrtf((float)D), ksc = kx_rsqrtf(kk + s.unit_eps);
   const float *pr = a.proj + (size_t)b * a.proj_ld;
-  const float beta = kx_sigmoidf(pr[a.b_off + h]), g = decay_of(pr[a.a_off + h], a.a_log[h], a.dt_bias[h]);
-  // the convolutions' inputs for the next token: this workgroup's value channels, and q and k once per head of theirs
-  if (s.taps > 1) {
+  const float pb = pr[a.b_off + h], pa = pr[a.a_off + h], a_log = a.a_log[h], dt_bias = a.dt_bias[h];
+  float S[RPT];
+#pragma unroll
+  for (int r = 0; r < RPT; ++r) S[r] = st[(size_t)min(rg + 8 * r, D - 1) * V + col];
+  float qq = 0.0f, kk = 0.0f;
+  auto put = [&](int x, float y) {
+    (x >= D ? k : q)[x >= D ? x - D : x] = y;
+    if (x >= D) kk = __builtin_fmaf(y, y, kk);
+    else qq = __builtin_fmaf(y, y, qq);
+  };
+  // the convolutions, and their inputs for the next token: this workgroup's value channels, and q and k once per head of theirs
+  if (few) {
+#pragma unroll
+    for (int y = 0; y < CH; ++y) {
+      const int x = tid + y * 256;
+      if (x >= 2 * D) continue;
+      put(x, kxc::silu_of(cv, ch[y]));
+      if (first) kxc::shift(cv, b, channel(x), ch[y]);
+    }
+    if (tid < SC) v[tid] = c0 + tid < V ? kxc::silu_of(cv, vch) : 0.0f;
+    if (tid < SC && c0 + tid < V) kxc::shift(cv, b, 2 * nq + h * V + c0 + tid, vch);
+  } else {
+    for (int x = tid; x < 2 * D; x += 256) {
+      put(x, kxc::conv_silu(cv, b, 0, channel(x)));
+      if (first) kxc::shift(cv, b, channel(x));
+    }
+    if (tid < SC) v[tid] = c0 + tid < V ? kxc::conv_silu(cv, b, 0, 2 * nq + h * V + c0 + tid) : 0.0f;
     if (tid < SC && c0 + tid < V) kxc::shift(cv, b, 2 * nq + h * V + c0 + tid);
-    if (c0 == 0 && h % (s.heads / s.kv_heads) == 0)
-      for (int x = tid; x < 2 * D; x += 256) kxc::shift(cv, b, x < D ? kvh * D + x : nq + kvh * D + x - D);
   }
+  qq = kxr::wave_sum(qq);
+  kk = kxr::wave_sum(kk);
+  if ((tid & 63) == 0) {
+    red[0][tid >> 6] = qq;
+    red[1][tid >> 6] = kk;
+  }
+  __syncthreads();
+  qq = kk = 0.0f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    qq += red[0][w];
+    kk += red[1][w];
+  }
+  const float qsc = kx_rsqrtf(qq + s.unit_eps) * kx_rsqrtf((float)D), ksc = kx_rsqrtf(kk + s.unit_eps);
+  const float beta = kx_sigmoidf(pb), g = decay_of(pa, a_log, dt_bias);
   float sk = 0.0f;
-  for (int r = rg; r < D; r += 8) sk = __builtin_fmaf(S[r * SC + c], k[r], sk);
+#pragma unroll
+  for (int r = 0; r < RPT; ++r)
+    if (rg + 8 * r < D) sk = __builtin_fmaf(S[r], k[rg + 8 * r], sk);
   part[0][rg][c] = sk;
   __syncthreads();
   sk = 0.0f;
@@ -86,10 +121,13 @@ __global__ void __launch_bounds__(256) delta_step_k(KxDeltaArgs a, KxConvArgs cv
   for (int j = 0; j < 8; ++j) sk += part[0][j][c];
   const float u = beta * (v[c] - g * (sk * ksc)) * ksc;
   float o = 0.0f;
-  for (int r = rg; r < D; r += 8) {
-    const float n = __builtin_fmaf(k[r], u, g * S[r * SC + c]);
-    o = __builtin_fmaf(n, q[r], o);
-    if (c0 + c < V) st[(size_t)r * V + c0 + c] = n;
+#pragma unroll
+  for (int r = 0; r < RPT; ++r) {
+    const int row = rg + 8 * r;
+    if (row >= D) continue;
+    const float n = __builtin_fmaf(k[row], u, g * S[r]);
+    o = __builtin_fmaf(n, q[row], o);
+    if (c0 + c < V) st[(size_t)row * V + c0 + c] = n;
   }
   part[1][rg][c] = o;
   __syncthreads();
@@ -446,8 +484,10 @@ int kx_delta_launch(const KxDeltaArgs &a, hipStream_t st) {
   KX_REQUIRE(s.dim <= 256, "delta rule: keys of %d columns, at most 256", s.dim);
   KX_REQUIRE(a.batch > 0 && a.positions > 0 && (s.taps == 1 || (a.hist && a.hist_out && a.hist != a.hist_out)), "delta rule: %d x %d tokens", a.batch, a.positions);
   if (a.positions == 1) {
-    const size_t lds = ((size_t)2 * s.dim + SC + (size_t)s.dim * SC) * 4;
-    hipLaunchKernelGGL(delta_step_k, dim3(s.heads * kx_cdiv(s.vdim, SC), a.batch), dim3(256), lds, st, a, conv_of(a));
+    const dim3 grid(s.heads * kx_cdiv(s.vdim, SC), a.batch);
+    if (s.dim <= 64) hipLaunchKernelGGL(delta_step_k<8>, grid, dim3(256), 0, st, a, conv_of(a));
+    else if (s.dim <= 128) hipLaunchKernelGGL(delta_step_k<16>, grid, dim3(256), 0, st, a, conv_of(a));
+    else hipLaunchKernelGGL(delta_step_k<32>, grid, dim3(256), 0, st, a, conv_of(a));
     KX_LAUNCH_CHECK();
     return KX_OK;
   }

@@ -34,19 +34,38 @@ __global__ void __launch_bounds__(256) ssd_step_k(KxSsdArgs a, KxConvArgs cv) {
   const int h = blockIdx.x / slices, c0 = (blockIdx.x - h * slices) * SC, b = blockIdx.y, ratio = s.heads / s.groups, g = h / ratio;
   const int c = tid & (SC - 1), rg = tid / SC, col = min(c0 + c, V - 1), inner = kx_ssd_inner(s);
   float *st = a.state + ((size_t)b * s.heads + h) * N * V;
+  auto channel = [&](int i) { return inner + (i < N ? g * N + i : s.groups * N + g * N + i - N); };
+  constexpr int CH = (2 * 8 * RPT + 255) / 256;  // channels of B and C per thread
+  const bool few = cv.taps <= kxc::FEW, first = c0 == 0 && h % ratio == 0;
+  kxc::Channel ch[CH], xch;
+  if (few) {
+#pragma unroll
+    for (int y = 0; y < CH; ++y) ch[y] = kxc::ask(cv, b, channel(min(tid + y * 256, 2 * N - 1)));
+    xch = kxc::ask(cv, b, h * V + min(c0 + (tid & (SC - 1)), V - 1));
+  }
+  const float pd = a.proj[(size_t)b * a.proj_ld + a.dt_off + h], bias = a.dt_bias[h], a_log = a.a_log[h];
   float S[RPT];
 #pragma unroll
   for (int r = 0; r < RPT; ++r) S[r] = st[(size_t)min(rg + 8 * r, N - 1) * V + col];
-  auto channel = [&](int i) { return inner + (i < N ? g * N + i : s.groups * N + g * N + i - N); };
-  for (int i = tid; i < 2 * N; i += 256) bc[i] = kxc::conv_silu(cv, b, 0, channel(i));
-  if (tid < SC) xs[tid] = c0 + tid < V ? kxc::conv_silu(cv, b, 0, h * V + c0 + tid) : 0.0f;
-  const float dt = step_size(a, b, h), decay = decay_of(a, h, dt);
-  // the convolutions' inputs for the next token: this workgroup's x channels, and B and C once per group
-  if (s.taps > 1) {
+  // the convolutions, and their inputs for the next token: this workgroup's x channels, and B and C once per group
+  if (few) {
+#pragma unroll
+    for (int y = 0; y < CH; ++y) {
+      const int i = tid + y * 256;
+      if (i < 2 * N) bc[i] = kxc::silu_of(cv, ch[y]);
+      if (i < 2 * N && first) kxc::shift(cv, b, channel(i), ch[y]);
+    }
+    if (tid < SC) xs[tid] = c0 + tid < V ? kxc::silu_of(cv, xch) : 0.0f;
+    if (tid < SC && c0 + tid < V) kxc::shift(cv, b, h * V + c0 + tid, xch);
+  } else {
+    for (int i = tid; i < 2 * N; i += 256) {
+      bc[i] = kxc::conv_silu(cv, b, 0, channel(i));
+      if (first) kxc::shift(cv, b, channel(i));
+    }
+    if (tid < SC) xs[tid] = c0 + tid < V ? kxc::conv_silu(cv, b, 0, h * V + c0 + tid) : 0.0f;
     if (tid < SC && c0 + tid < V) kxc::shift(cv, b, h * V + c0 + tid);
-    if (c0 == 0 && h % ratio == 0)
-      for (int i = tid; i < 2 * N; i += 256) kxc::shift(cv, b, channel(i));
   }
+  const float dt = kxr::softplus(pd + bias), decay = kx_expf(-kx_expf(a_log) * dt);
   __syncthreads();
   const float x = xs[c] * dt;
   float y = 0.0f;
