@@ -31,6 +31,10 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 constexpr float NEG_INF = -__builtin_inff();
 constexpr int RB = 4;            // query heads whose values are summed together in win_partial_k
 constexpr int PART_THREADS = 256;
+// Rows of keys and of values that a thread of win_partial_k asks for first: all, of 64 keys of 128 columns.  One token is a chain of waits for
+// memory on few workgroups; with the rows, the numbers under the norms and the query asked for together it has three left.  16 heads of 128
+// on 4 key heads, 384 keys: 13.4 us before and 10.2 now, and win_merge_k, whose sums are asked for ahead of their weights, 4.8 and 3.7.
+constexpr int AHEAD_K = 2, AHEAD_V = 4;
 
 __host__ __device__ __forceinline__ int seen_blocks(int p, int size, int pool) {
   return pool > 0 && p - size + 1 > 0 ? (p - size + 1) / pool : 0;
@@ -100,7 +104,7 @@ template <class T, bool FUSED>
 __global__ void __launch_bounds__(PART_THREADS) win_partial_k(KxWindowArgs a, int tok0, int ch, float *po, float *pm, float *pz) {
   using E = Elem<T>;
   extern __shared__ __attribute__((aligned(16))) float win_lds[];
-  __shared__ float red[4];
+  __shared__ float red[2][4];
   const KxWindowSpec &s = a.s;
   const KxWindowCache &c = a.c;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -122,22 +126,83 @@ __global__ void __launch_bounds__(PART_THREADS) win_partial_k(KxWindowArgs a, in
   const size_t head = (size_t)b * s.kv_heads + g;
   const T *kc = (const T *)c.k + head * c.cap * c.dp, *vc = (const T *)c.v + head * c.cap * c.vp;
   const T *pkc = (const T *)c.pk + head * c.blocks * c.dp, *pvc = (const T *)c.pv + head * c.blocks * c.vp;
+  const int base = p / c.cap * c.cap;  // position j of the window: slot j - base, one ring length more below it
+  auto slot_of = [&](int e) {
+    const int j = lo + e - nb - base;
+    return j < 0 ? j + c.cap : j;
+  };
+  // scores: 8 lanes per key; values: vp / 8 threads per key.  The first rows of both are asked for before anything else.
+  const int l8 = lane & 7, tpk = c.vp >> 3, groups = PART_THREADS / tpk, grp = tid / tpk, col = (tid - grp * tpk) * 8;
+  struct Keys { typename E::Raw x[2]; };  // 128 columns
+  auto key_row = [&](int k0) {
+    const int e = e0 + min(k0 + (lane >> 3), n - 1);
+    return e < nb ? pkc + (size_t)e * c.dp : kc + (size_t)slot_of(e) * c.dp;
+  };
+  auto ask_keys = [&](int k0) {
+    const T *key = key_row(k0);
+    return Keys{{E::cached(key + min(l8 * 8, c.dp - 8)), E::cached(key + min(l8 * 8 + 64, c.dp - 8))}};
+  };
+  auto ask_values = [&](int k) {
+    const int e = e0 + min(k, n - 1);
+    return E::cached((e < nb ? pvc + (size_t)e * c.vp : vc + (size_t)slot_of(e) * c.vp) + col);
+  };
+  Keys kr[AHEAD_K];
+  typename E::Raw vr[AHEAD_V];
+  auto ask_all = [&] {
+#pragma unroll
+    for (int y = 0; y < AHEAD_K; ++y) kr[y] = ask_keys(wave * 8 + 32 * y);
+#pragma unroll
+    for (int y = 0; y < AHEAD_V; ++y) vr[y] = ask_values(grp + groups * y);
+  };
+  ask_all();
   if (FUSED) {
     const float *pr = a.proj + (size_t)tok * a.proj_ld;
     const int nq = s.heads * s.dim, nk = s.kv_heads * s.dim;
     float qs = 1.0f, ks = 1.0f;
-    if (a.q_norm) {
-      float v = 0.0f, w = 0.0f;
-      for (int x = tid; x < nq; x += PART_THREADS) v = __builtin_fmaf(pr[a.q_off + x], pr[a.q_off + x], v);
-      for (int x = tid; x < nk; x += PART_THREADS) w = __builtin_fmaf(pr[a.k_off + x], pr[a.k_off + x], w);
-      qs = kx_rsqrtf(kxr::block_sum(v, red) / (float)nq + a.eps);
-      ks = kx_rsqrtf(kxr::block_sum(w, red) / (float)nk + a.eps);
+    constexpr int UB = 8, UQ = 4;  // numbers of a thread asked for together
+    float qx[UQ], qw[UQ];
+#pragma unroll
+    for (int k = 0; k < UQ; ++k) {
+      const int x = min(tid + k * PART_THREADS, R * c.dp - 1), r = x / c.dp, y = (g * R + r) * s.dim + min(x - r * c.dp, s.dim - 1);
+      qx[k] = pr[a.q_off + y];
+      qw[k] = a.q_norm ? a.q_norm[y] : 1.0f;
     }
-    for (int x = tid; x < R * c.dp; x += PART_THREADS) {
-      const int r = x / c.dp, d = x - r * c.dp, y = (g * R + r) * s.dim + d;
-      float v = d < s.dim ? pr[a.q_off + y] * qs * (a.q_norm ? a.q_norm[y] : 1.0f) : 0.0f;
+    if (a.q_norm) {
+      float u[2][UB], v[2] = {};
+      auto ask = [&](int j, int x0) {
+#pragma unroll
+        for (int k = 0; k < UB; ++k) u[j][k] = pr[(j ? a.k_off : a.q_off) + min(x0 + k * PART_THREADS, (j ? nk : nq) - 1)];
+      };
+      ask(0, tid);
+      ask(1, tid);
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        for (int x0 = tid; x0 < (j ? nk : nq); x0 += UB * PART_THREADS) {
+          if (x0 > tid) ask(j, x0);
+#pragma unroll
+          for (int k = 0; k < UB; ++k)
+            if (x0 + k * PART_THREADS < (j ? nk : nq)) v[j] = __builtin_fmaf(u[j][k], u[j][k], v[j]);
+        }
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        v[j] = kxr::wave_sum(v[j]);
+        if (lane == 0) red[j][wave] = v[j];
+      }
+      __syncthreads();
+      qs = kx_rsqrtf((((red[0][0] + red[0][1]) + red[0][2]) + red[0][3]) / (float)nq + a.eps);
+      ks = kx_rsqrtf((((red[1][0] + red[1][1]) + red[1][2]) + red[1][3]) / (float)nk + a.eps);
+    }
+    auto put = [&](int x, float q, float w) {
+      float v = x - x / c.dp * c.dp < s.dim ? q * qs * w : 0.0f;
       if (sizeof(T) == 2) v = kx_bfround(v);  // the query the other kernels read
       qv[x] = v;
+    };
+#pragma unroll
+    for (int k = 0; k < UQ; ++k)
+      if (tid + k * PART_THREADS < R * c.dp) put(tid + k * PART_THREADS, qx[k], qw[k]);
+    for (int x = tid + UQ * PART_THREADS; x < R * c.dp; x += PART_THREADS) {
+      const int r = x / c.dp, y = (g * R + r) * s.dim + min(x - r * c.dp, s.dim - 1);
+      put(x, pr[a.q_off + y], a.q_norm ? a.q_norm[y] : 1.0f);
     }
     if (e0 + n == total) {  // this workgroup holds the newest key: it writes the cache
       const int slot = p % c.cap;
@@ -150,27 +215,20 @@ __global__ void __launch_bounds__(PART_THREADS) win_partial_k(KxWindowArgs a, in
       __threadfence_block();
       __syncthreads();
       if (s.pool > 0 && (p + 1) % s.pool == 0 && p / s.pool < c.blocks) pool_block<T>(a, head, p / s.pool, tid, PART_THREADS);
+      ask_all();  // the newest key's rows are there now
     }
   } else {
     const T *q = (const T *)a.q + ((size_t)tok * s.heads + g * R) * c.dp;
     for (int x = tid; x < R * c.dp; x += PART_THREADS) qv[x] = E::load(q + x);
   }
   __syncthreads();
-  const int base = p / c.cap * c.cap;  // position j of the window: slot j - base, one ring length more below it
-  auto slot_of = [&](int e) {
-    const int j = lo + e - nb - base;
-    return j < 0 ? j + c.cap : j;
-  };
-  // scores: 8 lanes per key
-  const int l8 = lane & 7;
-  for (int k0 = wave * 8; k0 < n; k0 += 32) {
-    const int e = e0 + min(k0 + (lane >> 3), n - 1);
-    const T *key = e < nb ? pkc + (size_t)e * c.dp : kc + (size_t)slot_of(e) * c.dp;
+  auto scores = [&](int k0, const Keys &first) {
+    const T *key = key_row(k0);
     for (int r0 = 0; r0 < R; r0 += RB) {
       float d[RB] = {};
-      for (int x = l8 * 8; x < c.dp; x += 64) {
+      auto times = [&](const typename E::Raw &raw, int x) {
         float kf[8];
-        E::unpack(kf, E::cached(key + x));
+        E::unpack(kf, raw);
 #pragma unroll
         for (int r = 0; r < RB; ++r) {
           const float *q = qv + min(r0 + r, R - 1) * c.dp + x;
@@ -180,7 +238,11 @@ __global__ void __launch_bounds__(PART_THREADS) win_partial_k(KxWindowArgs a, in
           d[r] = __builtin_fmaf(kf[4], qb.x, d[r]); d[r] = __builtin_fmaf(kf[5], qb.y, d[r]);
           d[r] = __builtin_fmaf(kf[6], qb.z, d[r]); d[r] = __builtin_fmaf(kf[7], qb.w, d[r]);
         }
-      }
+      };
+#pragma unroll
+      for (int y = 0; y < 2; ++y)
+        if (l8 * 8 + 64 * y < c.dp) times(first.x[y], l8 * 8 + 64 * y);
+      for (int x = l8 * 8 + 128; x < c.dp; x += 64) times(E::cached(key + x), x);
 #pragma unroll
       for (int r = 0; r < RB; ++r) {
         d[r] += kxw::dpp_f<kxw::DPP_QUAD_XOR1>(d[r]);
@@ -189,7 +251,11 @@ __global__ void __launch_bounds__(PART_THREADS) win_partial_k(KxWindowArgs a, in
         if (l8 == 0 && r0 + r < R && k0 + (lane >> 3) < n) sc[(r0 + r) * ch + k0 + (lane >> 3)] = d[r] * s.scale;
       }
     }
-  }
+  };
+#pragma unroll
+  for (int y = 0; y < AHEAD_K; ++y)
+    if (wave * 8 + 32 * y < n) scores(wave * 8 + 32 * y, kr[y]);
+  for (int k0 = wave * 8 + 32 * AHEAD_K; k0 < n; k0 += 32) scores(k0, ask_keys(k0));
   __syncthreads();
   for (int r = wave; r < R; r += 4) {
     float m = NEG_INF, z = 0.0f;
@@ -207,22 +273,24 @@ __global__ void __launch_bounds__(PART_THREADS) win_partial_k(KxWindowArgs a, in
     }
   }
   __syncthreads();
-  // weighted values: vp / 8 threads per key
-  const int tpk = c.vp >> 3, groups = PART_THREADS / tpk, grp = tid / tpk, col = (tid - grp * tpk) * 8;
   for (int r0 = 0; r0 < R; r0 += RB) {
     float acc[RB][8] = {};
-    if (grp < groups)
-      for (int k = grp; k < n; k += groups) {
-        const int e = e0 + k;
-        float vf[8];
-        E::unpack(vf, E::cached((e < nb ? pvc + (size_t)e * c.vp : vc + (size_t)slot_of(e) * c.vp) + col));
+    auto times = [&](const typename E::Raw &raw, int k) {
+      float vf[8];
+      E::unpack(vf, raw);
 #pragma unroll
-        for (int r = 0; r < RB; ++r) {
-          const float w = sc[min(r0 + r, R - 1) * ch + k];
+      for (int r = 0; r < RB; ++r) {
+        const float w = sc[min(r0 + r, R - 1) * ch + k];
 #pragma unroll
-          for (int x = 0; x < 8; ++x) acc[r][x] = __builtin_fmaf(w, vf[x], acc[r][x]);
-        }
+        for (int x = 0; x < 8; ++x) acc[r][x] = __builtin_fmaf(w, vf[x], acc[r][x]);
       }
+    };
+    if (grp < groups) {
+#pragma unroll
+      for (int y = 0; y < AHEAD_V; ++y)
+        if (grp + groups * y < n) times(vr[y], grp + groups * y);
+      for (int k = grp + groups * AHEAD_V; k < n; k += groups) times(ask_values(k), k);
+    }
     if (grp < groups)
 #pragma unroll
       for (int r = 0; r < RB; ++r)
@@ -248,15 +316,26 @@ __global__ void __launch_bounds__(MERGE_THREADS) win_merge_k(KxWindowArgs a, int
   const KxWindowSpec &s = a.s;
   const int h = blockIdx.x, tok = tok0 + blockIdx.y, tid = threadIdx.x;
   const size_t row = (size_t)blockIdx.y * parts;
+  constexpr int UB = 8;  // parts asked for together, the first before their weights are known
+  auto ask = [&](float (&x)[UB], int d, int k0) {
+#pragma unroll
+    for (int k = 0; k < UB; ++k) x[k] = po[((row + min(k0 + k, parts - 1)) * s.heads + h) * a.c.vp + d];
+  };
+  auto gate_of = [&](int d) { return a.g_off >= 0 ? a.proj[(size_t)tok * a.proj_ld + a.g_off + h * s.vdim + d] : 0.0f; };
+  const int d0 = min(tid, s.vdim - 1);
+  float x[UB], gate = gate_of(d0);
+  ask(x, d0, 0);
   if (tid < 64) {
     const float sink = a.sinks ? a.sinks[h] : 0.0f;
-    float m = s.sink ? sink : NEG_INF, z = 0.0f;
-    for (int k = tid; k < parts; k += 64) m = fmaxf(m, pm[(row + k) * s.heads + h]);
+    const float m0 = tid < parts ? pm[(row + tid) * s.heads + h] : NEG_INF, z0 = tid < parts ? pz[(row + tid) * s.heads + h] : 0.0f;
+    float m = fmaxf(s.sink ? sink : NEG_INF, m0), z = 0.0f;
+    for (int k = tid + 64; k < parts; k += 64) m = fmaxf(m, pm[(row + k) * s.heads + h]);
     m = kxw::wave_max_f32(m);
     for (int k = tid; k < parts; k += 64) {
-      const float w = kx_expf(pm[(row + k) * s.heads + h] - m);
+      const bool first = k == tid;
+      const float w = kx_expf((first ? m0 : pm[(row + k) * s.heads + h]) - m);
       weight[k] = w;
-      z = __builtin_fmaf(pz[(row + k) * s.heads + h], w, z);
+      z = __builtin_fmaf(first ? z0 : pz[(row + k) * s.heads + h], w, z);
     }
     const float inv = 1.0f / (kxr::wave_sum(z) + (s.sink ? kx_expf(sink - m) : 0.0f));
     for (int k = tid; k < parts; k += 64) weight[k] *= inv;
@@ -264,14 +343,15 @@ __global__ void __launch_bounds__(MERGE_THREADS) win_merge_k(KxWindowArgs a, int
   __syncthreads();
   T *out = (T *)a.out + (size_t)tok * a.out_ld + h * s.vdim;
   for (int d = tid; d < s.vdim; d += MERGE_THREADS) {
-    const float gate = a.g_off >= 0 ? kx_sigmoidf(a.proj[(size_t)tok * a.proj_ld + a.g_off + h * s.vdim + d]) : 1.0f;
+    if (d > tid) gate = gate_of(d);
     float v = 0.0f;
-#pragma unroll 8
-    for (int k = 0; k < parts; ++k) {  // a part without keys has not written its sums
-      const float x = po[((row + k) * s.heads + h) * a.c.vp + d];
-      v = weight[k] > 0.0f ? __builtin_fmaf(x, weight[k], v) : v;
+    for (int k0 = 0; k0 < parts; k0 += UB) {
+      if (d > tid || k0) ask(x, d, k0);
+#pragma unroll
+      for (int k = 0; k < UB; ++k)  // a part without keys has not written its sums
+        if (k0 + k < parts && weight[k0 + k] > 0.0f) v = __builtin_fmaf(x[k], weight[k0 + k], v);
     }
-    out[d] = Elem<T>::make(v * gate);
+    out[d] = Elem<T>::make(a.g_off >= 0 ? v * kx_sigmoidf(gate) : v);
   }
 }
 

@@ -569,3 +569,18 @@ def test_32_bit_attention_of_prompts(kxlib, heads, kv, dim, vdim, size, pool, ba
     for b in range(batch):
         assert rel(got[b], w.oracle(proj[b], pool=pool or 1 << 20)) < 2e-6
     w.close()
+
+
+@pytest.mark.parametrize("f32", [1, 0], ids=["f32", "bf16"])
+@pytest.mark.parametrize("heads, kv, dim, vdim, size, batch, cuts", [(20, 2, 128, 128, 1000, 1, [700, 1, 1, 1]), (4, 4, 136, 72, 300, 40, [331, 1, 1])])
+def test_one_token_with_more_than_is_asked_for_first(kxlib, heads, kv, dim, vdim, size, batch, cuts, f32):
+    """More query columns, parts, keys of a part and columns of a key than a thread asks for ahead.  The bars: 32-bit
+    sums of 136 products and 1000 weights in chains of 64 at most, 2e-6; results rounded to bf16 by at most 2^-9, and as much for queries and keys whose
+    rounding the 32-bit norms decide otherwise."""
+    n = sum(cuts)
+    w = Window(kxlib, heads, kv, dim, vdim, size, 0, f32, batch=batch, context=n, positions=max(cuts))
+    proj = np.random.default_rng(dim).standard_normal((batch, n, w.cols[-1])).astype(np.float32)
+    got = w.run(proj, cuts, batch)
+    for b in {0, batch - 1}:
+        assert rel(got[b][cuts[0]:], w.oracle(proj[b], pool=1 << 20)[cuts[0]:]) < (2e-6 if f32 else 2 ** -8)
+    w.close()
