@@ -144,7 +144,7 @@ __global__ void __launch_bounds__(256) embed_streams_k(const T *__restrict__ emb
                                                        int streams) {
   const T *e = embed + (size_t)ids[blockIdx.x] * ld;
   float *o = x + (size_t)blockIdx.x * streams * width;
-  for (int c = threadIdx.x; c < width; c += 256) {
+  for (int c = blockIdx.y * 256 + threadIdx.x; c < width; c += gridDim.y * 256) {
     float v;
     if constexpr (sizeof(T) == 4) v = e[c];
     else v = kx_bf16_f32(e[c]);
@@ -572,8 +572,9 @@ int HybridModel::step(const uint32_t *d_ids, bool sample, int C) {
   const int T = batch * C, S = c.streams, W = c.width;
   KX_REQUIRE(T > 0 && T <= std::max(step_tokens, max_batch), "%s: a step of %d tokens, at most %d", design(), T, step_tokens);
   const size_t es = f32 ? 4 : 2;
-  if (f32) hipLaunchKernelGGL(embed_streams_k<float>, dim3(T), dim3(256), 0, st, (const float *)embed.w, embed.ld, d_ids, streams, W, S);
-  else hipLaunchKernelGGL(embed_streams_k<uint16_t>, dim3(T), dim3(256), 0, st, (const uint16_t *)embed.w, embed.ld, d_ids, streams, W, S);
+  const dim3 embedded(T, T < 64 ? kx_cdiv(W, 256) : 1);  // few tokens: a column per thread (1 of 2048 columns: 5.9 us in one workgroup, 2.8 in eight)
+  if (f32) hipLaunchKernelGGL(embed_streams_k<float>, embedded, dim3(256), 0, st, (const float *)embed.w, embed.ld, d_ids, streams, W, S);
+  else hipLaunchKernelGGL(embed_streams_k<uint16_t>, embedded, dim3(256), 0, st, (const uint16_t *)embed.w, embed.ld, d_ids, streams, W, S);
   KX_LAUNCH_CHECK();
   for (int i = 0; i < n_layers; ++i) {
     const KxHybridLayer &l = c.layers[i];

@@ -755,3 +755,16 @@ def test_experts_with_tiles_of_256_slots(kxlib, tokens):
     assert (np.sort(ids, 1) == np.arange(0, 64, 2)).all()
     assert rel(got, a.oracle(x, rows, ids)) < 2e-2
     a.close()
+
+
+@pytest.mark.parametrize("width", [100, 101])
+@pytest.mark.parametrize("tokens", [15, 16, 17, 700])
+def test_experts_sorted_and_combined_at_the_edges(kxlib, tokens, width):
+    """The most tokens that the sorting workgroup routes itself, more pairs than it asks for at once, rows that are no multiple of four columns and more experts
+    than rows asked for at once.  The bar is that of 32-bit experts above."""
+    a = Experts(kxlib, width, 40, 40, 24, 64, 1, tokens)
+    r = np.random.default_rng(tokens)
+    x, rows = r.standard_normal((tokens, width)).astype(np.float32), KC.bf16(r.standard_normal((tokens, 64)))
+    got, ids = a.run(x, rows)
+    assert rel(got, a.oracle(x, rows, ids)) < 3e-5
+    a.close()
