@@ -13,6 +13,7 @@
 #include "kx_dense.h"
 #include "kx_gemm_tile.h"
 #include "kx_math.h"
+#include "kx_wave.h"
 
 namespace {
 
@@ -60,6 +61,73 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) dense_gemm_k(
   auto in = [&](int i, int v) { return m0 + TL::row(i, v) < m_end; };
   auto at = [&](int i, int v, int n) { return (size_t)row_of(min(m0 + TL::row(i, v), m_end - 1)) * a.out_stride + n; };
   constexpr int STEP = DUAL ? 32 / TL::SIDE : 1;  // blocks of gate rows in front of their up rows
+  // Blocks of 16 columns are 32 bytes of a row of bf16 results, a quarter of a line, one result to a lane.  Two lanes exchange theirs of two
+  // blocks, so that a store takes 64 bytes of each of its rows (even lanes have two columns of block j, odd lanes two of block j + 1).
+  // Keys and values of 64 heads from 512 columns, 3072 x 16384 164 -> 86 us (one by one is what the tile's short products wait for; 32 columns
+  // to a block took 127); gate and up 2048 x 36864 x 7168 877 -> 848.  Where pairs are not aligned, one by one.
+  if constexpr (TL::SIDE == 16 && !GROUP && (MODE == KX_GG_BF16 || MODE == KX_GG_RESID || MODE == KX_GG_KV)) {
+    if (a.pairs_aligned) {
+      const uint32_t odd = threadIdx.x & 1, order = odd ? 0x03020706u : 0x05040100u;
+      auto pack = [](float lo, float hi) { return (uint32_t)kx_bf16_rne(lo) | (uint32_t)kx_bf16_rne(hi) << 16; };
+      auto exchanged = [&](float lo, float hi) {  // of blocks j and j + 1
+        const uint32_t p = pack(lo, hi), q = kx_f32_bits(kxw::dpp_f<kxw::DPP_QUAD_XOR1>(kx_bits_f32(p)));
+        return __builtin_amdgcn_perm(q, p, order);
+      };
+      constexpr int PAIRS = DUAL ? TL::NI / 4 : TL::NI / 2;
+      auto block = [](int u) { return DUAL ? 4 * u : 2 * u; };
+      int n[PAIRS];
+#pragma unroll
+      for (int u = 0; u < PAIRS; ++u) n[u] = odd ? result(block(u) + 1) - 1 : result(block(u));
+      if constexpr (MODE == KX_GG_KV) {
+        uint16_t *to[PAIRS];
+        int ld[PAIRS];
+#pragma unroll
+        for (int u = 0; u < PAIRS; ++u) {
+          const int per = a.k_dim + a.v_dim, c = min(n[u], a.rows - 2), hd = c / per, d = c - hd * per;
+          const bool key = d < a.k_dim;
+          ld[u] = key ? a.k_ld : a.v_ld;
+          to[u] = (key ? (uint16_t *)a.out + d : a.out_v + (d - a.k_dim)) + (size_t)hd * a.cap * ld[u];
+        }
+#pragma unroll
+        for (int i = 0; i < TL::MI; ++i)
+#pragma unroll
+          for (int v = 0; v < TL::V; ++v) {
+            const int t = m0 + TL::row(i, v), b = t / a.seq;
+            const size_t row = (size_t)b * a.heads * a.cap + t - b * a.seq;
+#pragma unroll
+            for (int u = 0; u < PAIRS; ++u) {
+              const uint32_t y = exchanged(acc[i][2 * u][v], acc[i][2 * u + 1][v]);
+              if (in(i, v) && n[u] < a.rows) *(uint32_t *)(to[u] + row * ld[u]) = y;
+            }
+          }
+      } else {
+#pragma unroll
+        for (int i = 0; i < TL::MI; ++i) {
+          uint32_t old[TL::V][PAIRS];
+          if constexpr (MODE == KX_GG_RESID) {  // x = bf(x + bf(y))  (add_k, :248-251); a block's are read before the first is written
+#pragma unroll
+            for (int v = 0; v < TL::V; ++v)
+#pragma unroll
+              for (int u = 0; u < PAIRS; ++u) old[v][u] = *(const uint32_t *)((const uint16_t *)a.out + at(i, v, min(n[u], a.rows - 2)));
+          }
+#pragma unroll
+          for (int v = 0; v < TL::V; ++v)
+#pragma unroll
+            for (int u = 0; u < PAIRS; ++u) {
+              const int j = block(u);
+              uint32_t y;
+              if constexpr (DUAL)
+                y = exchanged(kx_swiglu(kx_bfround(acc[i][j][v]), kx_bfround(acc[i][j + 2][v])), kx_swiglu(kx_bfround(acc[i][j + 1][v]), kx_bfround(acc[i][j + 3][v])));
+              else y = exchanged(acc[i][j][v], acc[i][j + 1][v]);
+              if constexpr (MODE == KX_GG_RESID)
+                y = pack(kx_bits_f32(old[v][u] << 16) + kx_bits_f32(y << 16), kx_bits_f32(old[v][u] & 0xffff0000u) + kx_bits_f32(y & 0xffff0000u));
+              if (in(i, v) && n[u] < a.rows) *(uint32_t *)((uint16_t *)a.out + at(i, v, n[u])) = y;
+            }
+        }
+      }
+      return;
+    }
+  }
 #pragma unroll
   for (int i = 0; i < TL::MI; ++i) {
     if constexpr (MODE == KX_GG_RESID && !DUAL) {  // x = bf(x + bf(y))  (add_k, :248-251); 16 are read before the first is written
@@ -132,13 +200,16 @@ int launch(const KxDenseArgs &a, kxtile::Share share, hipStream_t st) {
 
 }  // namespace
 
-int kx_dense_gemm_launch(const KxDenseArgs &a, hipStream_t st) {
+int kx_dense_gemm_launch(const KxDenseArgs &args, hipStream_t st) {
+  KxDenseArgs a = args;
   KX_REQUIRE(a.w0 && a.x && a.out && a.tokens > 0 && a.rows > 0, "kx_dense_gemm: tokens=%d rows=%d", a.tokens, a.rows);
   KX_REQUIRE(a.cols > 0 && a.cols % 128 == 0 && a.x_stride >= a.cols && a.x_stride % 8 == 0, "kx_dense_gemm: cols=%d must be a positive multiple of 128", a.cols);
   KX_REQUIRE(a.mode >= KX_GG_BF16 && a.mode <= KX_GG_KV && !((a.w1 || a.work) && a.mode != KX_GG_BF16) && !(a.w1 && a.work), "kx_dense_gemm: out_mode=%d", a.mode);
   KX_REQUIRE(a.mode != KX_GG_KV || (a.seq > 0 && a.tokens % a.seq == 0 && a.heads > 0 && a.rows == a.heads * (a.k_dim + a.v_dim) && a.cap >= a.seq && a.k_ld >= a.k_dim &&
                                     a.v_ld >= a.v_dim && a.out_v),
              "kx_dense_gemm: %d rows for %d heads, %d tokens", a.rows, a.heads, a.tokens);
+  a.pairs_aligned = a.rows % 2 == 0 && (uintptr_t)a.out % 4 == 0 &&
+                    (a.mode == KX_GG_KV ? (a.k_dim | a.v_dim | a.k_ld | a.v_ld) % 2 == 0 && (uintptr_t)a.out_v % 4 == 0 : a.out_stride % 2 == 0);
   if (a.work) {
     KX_REQUIRE(a.pairs && a.groups > 0 && kx_cdiv(a.tokens, kxtile::Medium::BM) <= 65535, "kx_dense_gemm: %d groups", a.groups);
     return launch_as<kxtile::Medium, KX_GG_BF16, false, true>(a, {0, 1}, st);
