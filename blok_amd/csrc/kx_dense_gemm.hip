@@ -128,45 +128,69 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) dense_gemm_k(
       return;
     }
   }
+  // One by one, block by block; row by row where blocks have 16 columns and share a line.  Where a row's results lie, and which lanes have one of
+  // it, is worked out in front of the conditions: behind them the compiler does both again for each result, and a chain of 64 comparisons
+  // is 0.4 us of a product of 8 us.
 #pragma unroll
   for (int i = 0; i < TL::MI; ++i) {
-    if constexpr (MODE == KX_GG_RESID && !DUAL) {  // x = bf(x + bf(y))  (add_k, :248-251); 16 are read before the first is written
+    size_t row[TL::V];
+    uint64_t lanes[TL::V];
+#pragma unroll
+    for (int v = 0; v < TL::V; ++v) {
+      if constexpr (MODE == KX_GG_KV) {
+        const int t = m0 + TL::row(i, v), b = t / a.seq;
+        row[v] = (size_t)b * a.heads * a.cap + t - b * a.seq;
+      } else {
+        row[v] = at(i, v, 0);
+      }
+      lanes[v] = __builtin_amdgcn_ballot_w64(in(i, v));
+      asm volatile("" : "+s"(lanes[v]));
+    }
+    if constexpr (MODE == KX_GG_RESID) {  // x = bf(x + bf(y))  (add_k, :248-251); 16 are read before the first is written
+      uint16_t *const out = (uint16_t *)a.out;
 #pragma unroll
       for (int e0 = 0; e0 < TL::NI * TL::V; e0 += 16) {
         uint16_t old[16];
 #pragma unroll
-        for (int u = 0; u < 16; ++u) old[u] = ((const uint16_t *)a.out)[at(i, (e0 + u) % TL::V, min(result((e0 + u) / TL::V), a.rows - 1))];
+        for (int u = 0; u < 16; ++u) old[u] = out[row[(e0 + u) % TL::V] + min(result((e0 + u) / TL::V), a.rows - 1)];
 #pragma unroll
         for (int u = 0; u < 16; ++u) {
           const int j = (e0 + u) / TL::V, v = (e0 + u) % TL::V, n = result(j);
-          if (in(i, v) && n < a.rows) ((uint16_t *)a.out)[at(i, v, n)] = kx_bf16_rne(kx_bf16_f32(old[u]) + kx_bfround(acc[i][j][v]));
+          if (n < a.rows && __builtin_amdgcn_inverse_ballot_w64(lanes[v])) out[row[v] + n] = kx_bf16_rne(kx_bf16_f32(old[u]) + kx_bfround(acc[i][j][v]));
         }
       }
-    } else {
+    } else if constexpr (MODE == KX_GG_KV) {
 #pragma unroll
       for (int j = 0; j < TL::NI; ++j) {
-        if (DUAL && j / STEP % 2) continue;
-        const int n = result(j);
+        const int n = result(j), per = a.k_dim + a.v_dim, hd = n / per, d = n - hd * per;
         if (n >= a.rows) continue;
-        if constexpr (MODE == KX_GG_KV) {
-          const int per = a.k_dim + a.v_dim, hd = n / per, d = n - hd * per;
-          const bool key = d < a.k_dim;
-          uint16_t *to = key ? (uint16_t *)a.out + d : a.out_v + (d - a.k_dim);
-          const int ld = key ? a.k_ld : a.v_ld;
+        const bool key = d < a.k_dim;
+        const int ld = key ? a.k_ld : a.v_ld;
+        uint16_t *to = (key ? (uint16_t *)a.out + d : a.out_v + (d - a.k_dim)) + (size_t)hd * a.cap * ld;
+#pragma unroll
+        for (int v = 0; v < TL::V; ++v)
+          if (__builtin_amdgcn_inverse_ballot_w64(lanes[v])) to[row[v] * ld] = kx_bf16_rne(acc[i][j][v]);
+      }
+    } else {
+      auto put = [&](int v, int j) {
+        const size_t to = row[v] + result(j);
+        if constexpr (DUAL) ((uint16_t *)a.out)[to] = kx_bf16_rne(kx_swiglu(kx_bfround(acc[i][j][v]), kx_bfround(acc[i][j + STEP][v])));
+        else if constexpr (MODE == KX_GG_BF16) ((uint16_t *)a.out)[to] = kx_bf16_rne(acc[i][j][v]);
+        else ((float *)a.out)[to] = MODE == KX_GG_F32 ? acc[i][j][v] : kx_bfround(acc[i][j][v]);
+      };
+      if constexpr (TL::SIDE == 16) {
+#pragma unroll
+        for (int v = 0; v < TL::V; ++v)
+#pragma unroll
+          for (int j = 0; j < TL::NI; ++j)
+            if (!(DUAL && j / STEP % 2) && result(j) < a.rows && __builtin_amdgcn_inverse_ballot_w64(lanes[v])) put(v, j);
+      } else {
+#pragma unroll
+        for (int j = 0; j < TL::NI; ++j) {
+          if ((DUAL && j / STEP % 2) || result(j) >= a.rows) continue;
 #pragma unroll
           for (int v = 0; v < TL::V; ++v)
-            if (in(i, v)) {
-              const int t = m0 + TL::row(i, v), b = t / a.seq;
-              to[((size_t)(b * a.heads + hd) * a.cap + t - b * a.seq) * ld] = kx_bf16_rne(acc[i][j][v]);
-            }
-        } else {
-#pragma unroll
-          for (int v = 0; v < TL::V; ++v)
-            if (in(i, v)) {
-              if constexpr (DUAL) ((uint16_t *)a.out)[at(i, v, n)] = kx_bf16_rne(kx_swiglu(kx_bfround(acc[i][j][v]), kx_bfround(acc[i][j + STEP][v])));
-              else if constexpr (MODE == KX_GG_BF16) ((uint16_t *)a.out)[at(i, v, n)] = kx_bf16_rne(acc[i][j][v]);
-              else ((float *)a.out)[at(i, v, n)] = MODE == KX_GG_F32 ? acc[i][j][v] : kx_bfround(acc[i][j][v]);
-            }
+            if (__builtin_amdgcn_inverse_ballot_w64(lanes[v])) put(v, j);
         }
       }
     }
