@@ -16,6 +16,7 @@
 #include "kx_lds_copy.h"
 #include "kx_rows.h"
 #include "kx_window.h"
+#include "kx_window_choice.h"
 
 namespace {
 
@@ -665,7 +666,7 @@ __global__ void __launch_bounds__(FLASH_WAVES * 64, 2) win_flash_k(KxWindowArgs 
 // zero in the product, and added by the queries that see it.
 // 777 positions, 8 heads of 128: 52 us, 141 in parts of 256 keys on the vector ALU.  The error is no larger: chains are short, and a
 // tile's sums are added to those before it (1.02e-7 to 2.05e-7 for 33 to 2048 positions, 0.96 to 1.00 of the parts').
-constexpr int GQ = 32;
+using kxwin::GQ;
 template <int N> struct Floats { typedef float Type __attribute__((ext_vector_type(N))); };
 
 template <int ND, int NV>
@@ -923,20 +924,24 @@ int flash_f32_nv(const KxWindowArgs &a, int nv, hipStream_t st) {
   KX_LAUNCH_CHECK();
   return KX_OK;
 }
-// On the matrix cores where that is sooner.  They take a tile's edges with it, 4 us for 128 keys of 256 columns to every 32 queries of a CU, and
-// 16 us to begin; parts on the vector ALU are workgroups of one token and key head, bound by reading its keys for each, 5.5 TB/s over the chip,
-// and by 0.06 us a token and head where those are few.  Whole operator, 8 heads of 128 on 2 key heads, window 1024 (us, parts / matrix cores): 8 positions
-// 15 / 24, 20 32 / 29, 33 43 / 31, 100 93 / 33, 777 316 / 75; 16 sequences of 50 558 / 35; 16 heads on 4, 2048 1141 / 258.
+// Parts of a step's keys: keys of each, how many, and the tokens of a launch.
+struct Parts {
+  int keys, n;
+  size_t per_token, at_once;  // floats; tokens, 0 where the scratch does not hold one's
+};
+Parts parts_of(const KxWindowArgs &a) {
+  const int tokens = a.batch * a.positions, total = most_keys(a.s, a.pos + a.positions), ch = part_keys(a.s, total, tokens), n = kx_cdiv(total, ch);
+  const size_t per_token = n * floats_per_part(a.s);
+  return {ch, n, per_token, std::min<size_t>({(size_t)tokens, a.part_floats / per_token, (size_t)65535})};
+}
 bool flash_f32(const KxWindowArgs &a) {
   const KxWindowSpec &s = a.s;
   if (a.c.dp > 256 || a.c.vp > 128) return false;
   if (a.tok_batch || a.q_ld) return true;  // parts know nothing of it
-  const double most = most_keys(s, a.pos + a.positions), mean = 0.5 * (most + most_keys(s, a.pos + 1)), columns = a.c.dp + a.c.vp;
-  const long groups = (long)s.heads * a.batch * kx_cdiv(a.positions, GQ), tokens = (long)a.batch * a.positions;
-  const double keys = (kx_cdiv(groups, std::max(1, kx_device_cus())) - 1) * mean + most;
-  const double flash = 16.0 + keys / 128 * 4.0 * columns / 256;
-  const double parts = 7.0 + tokens * std::max(0.06 * s.heads, mean * columns * 4 * s.kv_heads / 5.5e6);
-  return flash < parts;
+  const Parts p = parts_of(a);
+  const int most = most_keys(s, a.pos + a.positions);
+  return kxwin::matrix_cores_f32({s.heads, s.kv_heads, a.c.dp + a.c.vp, a.batch, a.positions}, most, 0.5 * (most + most_keys(s, a.pos + 1)), {p.keys, p.n, (long)p.at_once},
+                                 std::max(1, kx_device_cus()));
 }
 
 int check(const KxWindowArgs &a) {
@@ -952,11 +957,9 @@ int check(const KxWindowArgs &a) {
 template <class T>
 int attend_parts(const KxWindowArgs &a, bool fused, hipStream_t st) {
   const KxWindowSpec &s = a.s;
-  const int tokens = a.batch * a.positions, R = s.heads / s.kv_heads;
-  const int total = most_keys(s, a.pos + a.positions), ch = part_keys(s, total, tokens), parts = kx_cdiv(total, ch);
-  const size_t per_token = (size_t)parts * floats_per_part(s);
-  KX_REQUIRE(per_token <= a.part_floats, "window attention: %zu floats of partials, room for %zu", per_token, a.part_floats);
-  const int at_once = (int)std::min<size_t>({(size_t)tokens, a.part_floats / per_token, (size_t)65535});
+  const Parts p = parts_of(a);
+  const int tokens = a.batch * a.positions, R = s.heads / s.kv_heads, ch = p.keys, parts = p.n, at_once = (int)p.at_once;
+  KX_REQUIRE(at_once > 0, "window attention: %zu floats of partials, room for %zu", p.per_token, a.part_floats);
   const size_t lds = ((size_t)R * a.c.dp + (size_t)R * ch + (size_t)(PART_THREADS / (a.c.vp / 8)) * RB * a.c.vp) * 4;
   KX_REQUIRE(lds <= 160 * 1024 - 256, "window attention: %d query heads of %d per key head do not fit a workgroup", R, s.dim);
   static std::atomic<bool> attr{false};

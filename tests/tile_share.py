@@ -10,10 +10,11 @@ F32, HYBRID, KIMI = (512 * 64 * 128, 512), (256 * 256 * 256, 512), (256 * 256 * 
 Choice = namedtuple("Choice", "large whole parts tiles")
 
 
-def build(folder):
-    exe = str(folder / "tile_share")
+def build(folder, name="tile_share"):
+    """tests/<name>.cpp for the host"""
+    exe = str(folder / name)
     r = subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Wextra", "-Werror", "-I" + os.path.join(os.path.dirname(HERE), "blok_amd", "csrc"),
-                        os.path.join(HERE, "tile_share.cpp"), "-o", exe], capture_output=True, text=True, timeout=300)
+                        os.path.join(HERE, name + ".cpp"), "-o", exe], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stderr
     return exe
 
