@@ -101,8 +101,10 @@ __global__ void __launch_bounds__(256) win_pool_k(KxWindowArgs a, int b0) {
 
 // Part `blockIdx.x` of the keys of token tok0 + blockIdx.z for key/value head blockIdx.y: up to ch keys, blocks first.
 // part: [tokens][parts][heads * vp] sums, then [tokens][parts][heads] maxima, then as many denominators.
+// Four waves per SIMD: LDS has room for as many, and with the registers of three long contexts of many sequences are slower (16 sequences of 1000 keys, 16
+// heads of 128, 32 bits: 56 us, 52 so).
 template <class T, bool FUSED>
-__global__ void __launch_bounds__(PART_THREADS) win_partial_k(KxWindowArgs a, int tok0, int ch, float *po, float *pm, float *pz) {
+__global__ void __launch_bounds__(PART_THREADS, 4) win_partial_k(KxWindowArgs a, int tok0, int ch, float *po, float *pm, float *pz) {
   using E = Elem<T>;
   extern __shared__ __attribute__((aligned(16))) float win_lds[];
   __shared__ float red[2][4];
@@ -141,7 +143,10 @@ __global__ void __launch_bounds__(PART_THREADS) win_partial_k(KxWindowArgs a, in
   };
   auto ask_keys = [&](int k0) {
     const T *key = key_row(k0);
-    return Keys{{E::cached(key + min(l8 * 8, c.dp - 8)), E::cached(key + min(l8 * 8 + 64, c.dp - 8))}};
+    Keys k;
+    k.x[0] = E::cached(key + min(l8 * 8, c.dp - 8));
+    if (c.dp > 64) k.x[1] = E::cached(key + min(l8 * 8 + 64, c.dp - 8));
+    return k;
   };
   auto ask_values = [&](int k) {
     const int e = e0 + min(k, n - 1);
@@ -160,7 +165,7 @@ __global__ void __launch_bounds__(PART_THREADS) win_partial_k(KxWindowArgs a, in
     const float *pr = a.proj + (size_t)tok * a.proj_ld;
     const int nq = s.heads * s.dim, nk = s.kv_heads * s.dim;
     float qs = 1.0f, ks = 1.0f;
-    constexpr int UB = 8, UQ = 4;  // numbers of a thread asked for together
+    constexpr int UB = sizeof(T) == 2 ? 8 : 4, UQ = 4;  // numbers of a thread asked for together, as registers allow
     float qx[UQ], qw[UQ];
 #pragma unroll
     for (int k = 0; k < UQ; ++k) {
