@@ -36,8 +36,7 @@ __global__ void __launch_bounds__(256) ssd_step_k(KxSsdArgs a, KxConvArgs cv) {
   float *st = a.state + ((size_t)b * s.heads + h) * N * V;
   auto channel = [&](int i) { return inner + (i < N ? g * N + i : s.groups * N + g * N + i - N); };
   constexpr int CH = (2 * 8 * RPT + 255) / 256;  // channels of B and C per thread
-  // not beside 64 rows of the state: there are no registers for both (16 heads, state 512, 64 sequences 72 us, 78 with everything in front)
-  const bool few = RPT < 64 && cv.taps <= kxc::FEW, first = c0 == 0 && h % ratio == 0;
+  const bool few = cv.taps <= kxc::FEW, first = c0 == 0 && h % ratio == 0;
   kxc::Channel ch[CH], xch;
   if (few) {
 #pragma unroll
