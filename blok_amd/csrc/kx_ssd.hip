@@ -4,6 +4,7 @@
 // reads its columns once, and writes them once.
 // Several positions: the convolutions (kx_conv.hip), ssd_coef_k (the numbers of kx_scan.h's blocks, with dt and the skip
 // weight in them) and kx_scan.hip.
+#include <algorithm>
 #include "kx_common.h"
 #include "kx_conv.h"
 #include "kx_rows.h"
@@ -26,7 +27,8 @@ KxConvArgs conv_of(const KxSsdArgs &a) {
 __device__ __forceinline__ float step_size(const KxSsdArgs &a, size_t tok, int h) { return kxr::softplus(a.proj[tok * a.proj_ld + a.dt_off + h] + a.dt_bias[h]); }
 __device__ __forceinline__ float decay_of(const KxSsdArgs &a, int h, float dt) { return kx_expf(-kx_expf(a.a_log[h]) * dt); }
 
-template <int RPT>  // rows of the state per thread
+// RPT: rows of the state per thread.  AHEAD: the convolutions' inputs are asked for in front of them.
+template <int RPT, bool AHEAD = true>
 __global__ void __launch_bounds__(256) ssd_step_k(KxSsdArgs a, KxConvArgs cv) {
   __shared__ float bc[2 * 8 * RPT], xs[SC], part[8][SC];
   const KxSsdSpec &s = a.s;
@@ -36,7 +38,7 @@ __global__ void __launch_bounds__(256) ssd_step_k(KxSsdArgs a, KxConvArgs cv) {
   float *st = a.state + ((size_t)b * s.heads + h) * N * V;
   auto channel = [&](int i) { return inner + (i < N ? g * N + i : s.groups * N + g * N + i - N); };
   constexpr int CH = (2 * 8 * RPT + 255) / 256;  // channels of B and C per thread
-  const bool few = cv.taps <= kxc::FEW, first = c0 == 0 && h % ratio == 0;
+  const bool few = AHEAD && cv.taps <= kxc::FEW, first = c0 == 0 && h % ratio == 0;
   kxc::Channel ch[CH], xch;
   if (few) {
 #pragma unroll
@@ -162,7 +164,10 @@ int kx_ssd_launch(const KxSsdArgs &a, hipStream_t st) {
     else if (s.state <= 64) hipLaunchKernelGGL(ssd_step_k<8>, grid, dim3(256), 0, st, a, cv);
     else if (s.state <= 128) hipLaunchKernelGGL(ssd_step_k<16>, grid, dim3(256), 0, st, a, cv);
     else if (s.state <= 256) hipLaunchKernelGGL(ssd_step_k<32>, grid, dim3(256), 0, st, a, cv);
-    else hipLaunchKernelGGL(ssd_step_k<64>, grid, dim3(256), 0, st, a, cv);
+    // 64 rows and what is asked for ahead of them leave a SIMD one wave, a CU one workgroup: 24 heads of 32 columns, state 400 (us, all ahead / rows
+    // alone), 8 sequences 10.6 / 14.9, 12 18.9 / 16.5, 64 55 / 43
+    else if ((long)grid.x * grid.y <= std::max(1, kx_device_cus())) hipLaunchKernelGGL(ssd_step_k<64>, grid, dim3(256), 0, st, a, cv);
+    else hipLaunchKernelGGL((ssd_step_k<64, false>), grid, dim3(256), 0, st, a, cv);
     KX_LAUNCH_CHECK();
     return KX_OK;
   }

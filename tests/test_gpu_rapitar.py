@@ -110,6 +110,15 @@ def test_state_space_on_many_workgroups(kxlib):
         d.close()
 
 
+def test_state_space_of_one_token_with_a_workgroup_per_cu_and_more(kxlib):
+    """256 and 258 workgroups of a state of 300 rows, one position at a time: the convolutions' inputs in front of the state, and behind it."""
+    for heads in (128, 129):
+        d = Ssd(kxlib, heads, 40, 300, 1, 4)
+        proj = np.random.default_rng(7).standard_normal((1, 9, d.cols())).astype(np.float32)
+        assert rel(d.run(proj, [1])[0], d.oracle(proj[0])) < 3e-5, heads
+        d.close()
+
+
 def test_state_space_holds_a_write_for_long_and_strong_decays_forget(kxlib):
     heads, vdim, state = 2, 8, 32
     d = Ssd(kxlib, heads, vdim, state, 1, 1)
