@@ -3,6 +3,7 @@
 #pragma once
 #include "kx_linear.h"
 #include "kx_math.h"
+#include "kx_tile_share.h"
 #include "kx_wave.h"
 
 // A step's (token, choice) pairs sorted by expert.
@@ -12,27 +13,26 @@ struct KxExpertSlots {
   int4 *tiles = nullptr;
   int *n_tiles = nullptr;
 };
-// slots per tile of a step (those of the GEMM that will read them), and the most tiles its pairs make.  rows: of the product with
-// fewer of them.  bf16: 256 where an expert has 96 pairs and more on average and a tile of 256 rows each fills the chip a fourth over
-// (the operator with 128 / 256 slots, us: 8 of 64 of 3 x 2048 x 1024 2046 tokens 514 / 470, 1024 tokens 363 / 333, uneven 350 / 372, all to 8
-// experts 222 / 191; of 3 x 1536 x 576 1500 tokens 293 / 261), 128 where it does not (of 3 x 1024 x 512 2046 tokens 227 / 233, 768 to 8 experts 110 / 126;
-// tiles listed by size, the short ones last, lose that an expert's tiles read one matrix at a time: 514 / 530); 32, those of the kernel for few tokens, where it has fewer than 8 and no expert can have
+// slots per tile of a step (those of the GEMM that will read them), and the most tiles its pairs make.  in, out: the matrices of an expert.  bf16: 256 or 128
+// where an expert has 96 pairs and more on average (kx_tile_share.h says which; tiles listed by size, the short ones last, lose that an expert's
+// tiles read one matrix at a time: 8 of 64 of 3 x 2048 x 1024, 2046 tokens 514 / 530); 32, those of the kernel for few tokens, where it has fewer than
+// 8 and no expert can have
 // more than three tiles, each of which reads its matrix again.  The operator with 32 / 64 slots, us: 8 to 8 of 64 of 3 x 2048 x 1024
 // 153 / 180, 63 tokens 211 / 230, all among 8 experts 83 / 90; 4 of 128 of 3 x 4096 x 1536, even 96 tokens 891 / 921, 192 tokens 982 /
 // 985; among 8 experts 96 tokens 174 / 183, 128 tokens 190 / 186, 192 tokens 215 / 187, 255 tokens 239 / 207.
 constexpr int KX_EXPERT_TILE_MIN = 32, KX_EXPERT_TILE_MIN_TOKENS = 3 * KX_EXPERT_TILE_MIN;
-inline int kx_expert_tile(bool f32, int tokens, int top, int experts, int rows, int cus) {
+inline int kx_expert_tile(bool f32, int tokens, int top, int experts, const KxMat &in, const KxMat &out, int cus) {
   const long pairs = (long)tokens * top;
   if (f32) return 64;
-  if (pairs >= 96L * experts) return 4L * experts * ((rows + 255) / 256) >= 5L * cus ? 256 : 128;
+  if (pairs >= 96L * experts) return kxtile::experts_in_large_tiles(pairs, experts, {in.rows, in.ld / KX_LD}, {out.rows, out.ld / KX_LD}, cus) ? 256 : 128;
   return pairs >= 8L * experts || tokens > KX_EXPERT_TILE_MIN_TOKENS ? 64 : KX_EXPERT_TILE_MIN;
 }
 inline int kx_expert_tiles(int tokens, int top, int experts, int tile) {
   const int pairs = tokens * top;
   return (pairs + tile - 1) / tile + (experts < pairs ? experts : pairs);
 }
-// Routes `tokens` tokens (e.logits, e.bias) and sorts the pairs into s, for products of `rows` rows and more; fills in e what kx_expert_gemm_launch reads.
-int kx_expert_route_launch(bool f32, KxExpertArgs &e, const KxExpertSlots &s, int tokens, int rows, hipStream_t st);
+// Routes `tokens` tokens (e.logits, e.bias) and sorts the pairs into s, for products with `in` and `out`; fills in e what kx_expert_gemm_launch reads.
+int kx_expert_route_launch(bool f32, KxExpertArgs &e, const KxExpertSlots &s, int tokens, const KxMat &in, const KxMat &out, hipStream_t st);
 // x[t] += sum_j y[slot of choice j of t], f32 rows of `width`
 int kx_expert_combine_launch(const KxExpertSlots &s, const float *y, float *x, int tokens, int top, int width, hipStream_t st);
 

@@ -110,11 +110,11 @@ __global__ void __launch_bounds__(256) combine_k(KxExpertSlots s, const float *_
 
 }  // namespace
 
-int kx_expert_route_launch(bool f32, KxExpertArgs &e, const KxExpertSlots &s, int tokens, int rows, hipStream_t st) {
+int kx_expert_route_launch(bool f32, KxExpertArgs &e, const KxExpertSlots &s, int tokens, const KxMat &in, const KxMat &out, hipStream_t st) {
   KX_REQUIRE(e.experts > 0 && e.experts <= KX_MAX_EXPERTS && e.top > 0 && e.top <= e.experts && e.top <= KX_MAX_TOP && tokens > 0 && e.logits && e.bias,
              "experts: %d of %d for %d tokens", e.top, e.experts, tokens);
   e.ids = s.ids; e.weights = s.weights;
-  e.tile_slots = kx_expert_tile(f32, tokens, e.top, e.experts, rows, std::max(1, kx_device_cus()));
+  e.tile_slots = kx_expert_tile(f32, tokens, e.top, e.experts, in, out, std::max(1, kx_device_cus()));
   e.max_tiles = kx_expert_tiles(tokens, e.top, e.experts, e.tile_slots);
   e.tiles = s.tiles; e.n_tiles = s.n_tiles; e.slot_weight = s.slot_weight;
   if (tokens <= BUCKET_WAVES) {
@@ -155,7 +155,7 @@ int kx_expert_ff_launch(bool f32, const KxExpertFf &f, int tokens, hipStream_t s
     KX_DO(kx_rows_launch(f32, gu.row, tokens, f.h_buf, gu.m.ld, st));
     h = f.h_buf;
   }
-  KX_DO(kx_expert_route_launch(f32, e, f.s, tokens, std::min(gu.m.rows, f.down.rows), st));
+  KX_DO(kx_expert_route_launch(f32, e, f.s, tokens, gu.m, f.down, st));
   e.gather = f.s.gather;
   KX_DO(kx_expert_gemm_launch(f32, gu, e, h, gu.m.ld, st));
   KX_DO(kx_linear_launch(f32, f.out, f.row_buf, st));

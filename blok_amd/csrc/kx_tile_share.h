@@ -38,6 +38,19 @@ inline Share share(long tiles, int round, int most_parts, long room, int arrival
   return s;
 }
 
+// Whole tiles of a product of `blocks` blocks of 64 columns, without what a launch takes: a last round costs most of a full one.
+inline double large_rounds(double n, int blocks, int cus) {
+  const long f = (long)(n / cus);
+  const double r = n - (double)f * cus;
+  return f * (13.8 + 1.45 * blocks) + (r == 0 ? 0.0 : 14.8 + (0.92 + 0.53 * r / cus) * blocks);
+}
+inline double medium_rounds(double n, int blocks, int cus) {  // two per CU
+  const double round = 4.3 + (1.0 + 0.0009 * blocks) * blocks, lone = 2.2 + 0.463 * blocks;
+  const long f = (long)(n / (2 * cus));
+  const double r = n - 2.0 * f * cus;
+  return f * round + (r == 0 ? 0.0 : r <= cus ? lone : lone + (round - lone) * (0.59 + 0.28 * (r - cus) / cus));  // a CU with two of the last round
+}
+
 // Which tile, and how it is shared out, for one product of `tokens` x `rows` with `blocks` blocks of 64 columns, by estimates in us that
 // are fitted to measurements of 22000 products (65 to 2048 x 384 to 40000 x 256 to 18560, 32-bit results).
 // Where the medium tiles leave CUs idle each has a CU to itself, in at least 10 blocks as the twin tile (kx_gemm_turns.h; at 4 blocks
@@ -71,12 +84,8 @@ inline Choice choose(int tokens, int rows, int blocks, size_t part_floats, int a
       if (time(q) * 1.05 < time(fill) && time(q) < time(p)) p = q;
     return {false, p == 1 ? Share{(int)medium, 1} : Share{0, (int)p}, blocks >= 10 * p};
   }
-  auto whole_large = [&](long n) { return 3.3 + rounds(n, blocks, 13.8, 1.45, 14.8, 0.92); };
-  auto whole_medium = [&](long n) {  // two per CU
-    const double round = 4.3 + (1.0 + 0.0009 * blocks) * blocks, lone = 2.2 + 0.463 * blocks;
-    const long f = n / (2 * cus), r = n % (2 * cus);
-    return 5.5 + f * round + (r == 0 ? 0.0 : r <= cus ? lone : lone + (round - lone) * (0.59 + 0.28 * (r - cus) / cus));  // a CU with two of the last round
-  };
+  auto whole_large = [&](long n) { return 3.3 + large_rounds(n, blocks, cus); };
+  auto whole_medium = [&](long n) { return 5.5 + medium_rounds(n, blocks, cus); };
   const bool large_whole = whole_large(large) < whole_medium(medium);
   // In parts, or in rounds of twin tiles with the last one in parts: a workgroup that leaves its sums behind, and has them read,
   // costs the memory's time for them, 0.009 us a twin, 0.032 a medium and 0.074 a large one.  The estimates are off by a tenth: parts have to gain 15 %
@@ -106,6 +115,25 @@ inline Choice choose(int tokens, int rows, int blocks, size_t part_floats, int a
   if (!large_whole && sl.parts == 1) tl = 1e30;
   if (large_whole && sm.parts == 1) tm = 1e30;
   return tt < tl && tt < tm ? Choice{false, st, true} : tl < tm ? Choice{true, sl} : Choice{false, sm};
+}
+
+// Experts' products in large tiles, whose last one of an expert is computed in quarters, or in medium ones: `pairs` of tokens and experts
+// meet two matrices of every expert.  How the pairs are spread is known on the device alone: even but for remainders.  A tile
+// that is a quarter full takes 0.51 of a full one.  Large ones where they take less than 1.4 of the medium ones' estimate and 15 us a product behind
+// it.  The operator over 1050 steps of 33 to 8192 tokens, 4 to 1000 experts of 3 x 256 to 7168 x 32 to 3000, spread evenly, unevenly and
+// among 4 or 12 of them: what is chosen takes 1.003 of the sooner one's time and 25 of them are more than 3 % longer than in medium tiles
+// or by the rule before (a large tile each for every expert fills the chip a fourth over: 1.040), by 14 % at most.  us, medium / large: 8 of 64 of 3 x
+// 2048 x 1024, 2046 tokens 514 / 470, all among 8 222 / 191, 1024 tokens unevenly 350 / 372; 6 of 384 of 3 x 512 x 32, 8192 tokens 220 / 251; 2 of 16 of
+// 3 x 7168 x 2048, 8192 tokens 2344 / 1918; 2 of 8 of 3 x 4096 x 1536, 1536 tokens 299 / 257.
+struct ExpertMatrix {
+  int rows, blocks;
+};
+inline bool experts_in_large_tiles(long pairs, int experts, ExpertMatrix in, ExpertMatrix out, int cus) {
+  auto tiles = [&](int slots) { const double n = (double)pairs / slots + 0.3 * experts; return n > experts ? n : (double)experts; };
+  const double full = 0.35 + 0.65 * tiles(64) / 4 / tiles(256);
+  auto large = [&](ExpertMatrix m) { return 15.0 + full * large_rounds(tiles(256) * ((m.rows + 255) / 256), m.blocks, cus); };
+  auto medium = [&](ExpertMatrix m) { return medium_rounds(tiles(128) * ((m.rows + 127) / 128), m.blocks, cus); };
+  return large(in) + large(out) < 1.4 * (medium(in) + medium(out));
 }
 
 // For the 32-bit tile and blocks of 32 columns.

@@ -11,6 +11,7 @@ import pytest
 import kagalorn_case as KC
 import rapitar_case as RC
 import rapitar_oracle as R
+import tile_share as TS
 from blok_amd import runtime
 from blok_amd.lib import DevBuf, KxExpertsConfig, KxLatentConfig, KxLinearArgs, KxSsdConfig, KxWkvConfig, check
 from kxt import dev, say
@@ -751,17 +752,19 @@ def test_trace_replay(kxlib, models, tmp_path):
             assert KC.logit_error(np.fromfile(out / f"{i}.f32", np.float32).reshape(ref.shape), ref).max() < bar, (dtype, i)
 
 
-@pytest.mark.parametrize("tokens", [192, 256, 300, 380, 440])
-def test_experts_with_tiles_of_256_slots(kxlib, tokens):
-    """All tokens to every second of 64 experts: lists of tiles that end in one of one to four quarters, rows of both products that are no multiple of 256."""
-    a = Experts(kxlib, 1300, 620, 64, 32, 64, 0, tokens)
+@pytest.mark.parametrize("width, ff, top, tokens", [(1300, 620, 32, 520), (1300, 620, 32, 445), (3000, 129, 32, 608), (3000, 129, 32, 650), (3000, 65, 64, 480), (3000, 65, 64, 520)])
+def test_experts_with_tiles_of_256_slots(kxlib, tmp_path, width, ff, top, tokens):
+    """All tokens to every second of 64 experts, or to all: lists of tiles that end in one of one to four quarters, rows of both products that are no multiple
+    of 256, products of two, three and an even and an odd number of blocks more."""
+    assert TS.experts_large(TS.build(tmp_path, "expert_tiles"), [(tokens, top, 64, width, ff)]) == [True]
+    a = Experts(kxlib, width, ff, 64, top, 64, 0, tokens)
     a.router[:], a.bias[:] = 0.0, 0.0
     a.bias[::2] = 3.0
     a.push()
     r = np.random.default_rng(tokens)
-    x, rows = r.standard_normal((tokens, 1300)).astype(np.float32), KC.bf16(r.standard_normal((tokens, 64)))
+    x, rows = r.standard_normal((tokens, width)).astype(np.float32), KC.bf16(r.standard_normal((tokens, 64)))
     got, ids = a.run(x, rows)
-    assert (np.sort(ids, 1) == np.arange(0, 64, 2)).all()
+    assert (np.sort(ids, 1) == np.arange(0, 64, 64 // top)).all()
     assert rel(got, a.oracle(x, rows, ids)) < 2e-2
     a.close()
 

@@ -60,3 +60,14 @@ def test_bf16_parts_fit_the_scratch(exe):
             assert rest >= 0 and c.parts >= 1 and (c.parts == 1 or rest > 0)
             if c.parts > 1:
                 assert rest <= scratch[1] and rest * c.parts * sums <= scratch[0] and c.parts <= p[2] // 64 // 16, (p, c, scratch)
+
+
+# tokens, experts each of them has, experts, width, ff; us in tiles of 128 and of 256 slots, evenly spread
+EXPERTS = [(8192, 6, 384, 512, 32, 220, 251), (1024, 8, 64, 1536, 576, 209, 217), (8192, 2, 16, 7168, 2048, 2344, 1918), (1536, 2, 8, 4096, 1536, 299, 257), (6000, 2, 8, 768, 3072, 372, 323),
+           (2046, 8, 64, 2048, 1024, 514, 470), (1024, 8, 64, 2048, 1024, 363, 333), (1536, 8, 64, 1536, 576, 269, 249), (1536, 8, 64, 1024, 512, 165, 184)]
+
+
+def test_experts_take_the_tiles_that_are_sooner(tmp_path):
+    """A rule that counts one large tile for every expert takes the slower ones for the first five, by up to 22 %."""
+    for c, large in zip(EXPERTS, T.experts_large(T.build(tmp_path, "expert_tiles"), [c[:5] for c in EXPERTS]), strict=True):
+        assert c[6 if large else 5] <= 1.03 * min(c[5:]), c

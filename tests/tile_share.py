@@ -19,9 +19,26 @@ def build(folder, name="tile_share"):
     return exe
 
 
-def choices(exe, f32, products, scratch):
-    """products: (tokens, rows, columns)"""
+def _answers(exe, f32, products, scratch):
     block = 32 if f32 else 64
     text = "".join(f"{int(f32)} {t} {r} {c // block} {scratch[0]} {scratch[1]} {CUS}\n" for t, r, c in products)
     out = subprocess.run([exe], input=text, capture_output=True, text=True, timeout=300, check=True).stdout
-    return [Choice(*map(int, line.split())) for line in out.splitlines()]
+    return [tuple(map(int, line.split())) for line in out.splitlines()]
+
+
+def choices(exe, f32, products, scratch):
+    """products: (tokens, rows, columns)"""
+    return [Choice(*a[:4]) for a in _answers(exe, f32, products, scratch)]
+
+
+def tiles(exe, products, scratch=(0, 0)):
+    """"large", "twin" or "medium" for bf16 products"""
+    return ["large" if a[0] else "twin" if a[4] else "medium" for a in _answers(exe, False, products, scratch)]
+
+
+def experts_large(exe, cases):
+    """cases: (tokens, top, experts, width, ff); whether their products take tiles of 256 slots where they are not fewer than 96 to an expert"""
+    pad = lambda n, to: (n + to - 1) // to * to
+    text = "".join(f"{t * top} {e} {2 * pad(ff, 32)} {pad(w, 64) // 64} {w} {pad(ff, 64) // 64} {CUS}\n" for t, top, e, w, ff in cases)
+    out = subprocess.run([exe], input=text, capture_output=True, text=True, timeout=300, check=True).stdout
+    return [line == "1" for line in out.split()]
