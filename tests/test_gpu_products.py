@@ -10,6 +10,7 @@ import blok_amd.lib as kxl
 import kagalorn_case as KC
 import kagalorn_oracle as K
 import oracle as O
+import tile_share as TS
 from blok_amd.lib import DevBuf, KxLinearArgs, check
 from kxt import dev, say
 from test_gpu_kagalorn import BF16_LOGITS, F32_LOGITS, _matrix, rel
@@ -93,9 +94,16 @@ def _put(x):
     return dev((np.ascontiguousarray(x, np.float32).view(np.uint32) >> 16).astype(np.uint16))
 
 
-@pytest.mark.parametrize("tokens, rows, cols", [(1985, 8000, 64), (2048, 8192, 128), (1793, 7937, 192)], ids=lambda v: str(v))
-def test_large_tiles(kxlib, tokens, rows, cols):
-    """Tiles of 256 x 256, whole and with remainders of tokens and rows, through every epilogue that a prompt meets."""
+@pytest.fixture(scope="module")
+def rule(tmp_path_factory):
+    return TS.build(tmp_path_factory.mktemp("share"))
+
+
+@pytest.mark.parametrize("tokens, rows, cols, tile", [(1985, 8000, 64, "medium"), (2048, 8192, 128, "medium"), (1793, 7937, 192, "medium"), (2048, 8192, 384, "large"),
+                                                      (1985, 8000, 448, "large"), (1793, 7937, 576, "large")], ids=lambda v: str(v))
+def test_large_tiles(kxlib, rule, tokens, rows, cols, tile):
+    """Tiles of few blocks, 128 x 128 and, from six on, 256 x 256, whole and with remainders of tokens and rows, through every epilogue that a prompt meets."""
+    assert TS.tiles(rule, [(tokens, rows, (cols + 63) // 64 * 64)]) == [tile]
     r = np.random.default_rng(rows)
     w, x = KC.bf16(r.standard_normal((rows, cols)) * cols ** -0.5), KC.bf16(r.standard_normal((tokens, cols)))
     dw, ld = _matrix(w, 0)
@@ -138,9 +146,9 @@ def test_large_tiles(kxlib, tokens, rows, cols):
     assert rel((out.to_numpy(np.uint16, (tokens, ff)).astype(np.uint32) << 16).view(np.float32), want) < 1e-2
 
 
-@pytest.mark.parametrize("tokens, rows, cols", [(300, 1000, 640), (129, 4100, 704), (66, 129, 1280), (2047, 2048, 832), (1793, 8191, 1024), (2048, 7424, 1088)],
-                         ids=["twin, 10 blocks", "twin, 11", "twin, a few", "twin, 13", "large, 16", "large, 17"])
-def test_tiles_whose_groups_take_turns(kxlib, tokens, rows, cols):
+@pytest.mark.parametrize("tokens, rows, cols, tile", [(300, 1000, 640, "twin"), (129, 4100, 704, "twin"), (66, 129, 1280, "twin"), (2047, 2048, 832, "twin"), (1793, 8191, 1024, "large"),
+                                                      (2048, 7424, 1088, "large")], ids=["twin, 10 blocks", "twin, 11", "twin, a few", "twin, 13", "large, 16", "large, 17"])
+def test_tiles_whose_groups_take_turns(kxlib, rule, tokens, rows, cols, tile):
     """Even and odd numbers of blocks, tiles with remainders of tokens and rows, every epilogue: the bars of the large tiles, 32-bit sums of up to
     1088 products (about 1e-6)."""
-    test_large_tiles(kxlib, tokens, rows, cols)
+    test_large_tiles(kxlib, rule, tokens, rows, cols, tile)

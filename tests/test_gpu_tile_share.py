@@ -57,13 +57,15 @@ def strict():
     return kxl.load_library(os.path.join(os.path.dirname(kxl.lib_path()), "libkx_strict.so"))
 
 
-# gate and up: 528 medium tiles, the last 16 shared, and 352 large ones, the last 96; down: all of 72 large tiles shared
-@pytest.mark.parametrize("hidden, inter, tokens, product, choice", [(2048, 16896, 187, "gate and up", (0, 512, 2, 528)), (4096, 11264, 900, "gate and up", (1, 256, 2, 352)),
-                                                                    (3072, 8192, 1300, "down", (1, 0, 3, 72))])
-def test_kimi_shares_large_and_medium_tiles(kxlib, strict, ox, tmp_path, hidden, inter, tokens, product, choice):
+# gate and up: 528 medium tiles, the last 16 shared, 352 large ones, the last 96, and 280 twin ones, the last 24; down: all of 72 large tiles shared
+@pytest.mark.parametrize("hidden, inter, tokens, product, tile, choice",
+                         [(2048, 16896, 187, "gate and up", "medium", (0, 512, 2, 528)), (4096, 11264, 900, "gate and up", "large", (1, 256, 2, 352)),
+                          (3072, 8192, 1300, "down", "large", (1, 0, 3, 72)), (7168, 3584, 515, "gate and up", "twin", (0, 256, 5, 280))])
+def test_kimi_shares_large_and_medium_tiles(kxlib, strict, ox, tmp_path, hidden, inter, tokens, product, tile, choice):
     """A prompt in one step against itself in steps whose products are whole or few-tile ones."""
     shape = (tokens, 2 * inter, hidden) if product == "gate and up" else (tokens, hidden, inter)
-    assert TS.choices(TS.build(tmp_path), False, [shape], TS.KIMI) == [choice]
+    exe = TS.build(tmp_path)
+    assert TS.choices(exe, False, [shape], TS.KIMI) == [choice] and TS.tiles(exe, [shape], TS.KIMI) == [tile]
     cfg = _config(16, 1, tokens + 1)
     cfg.hidden, cfg.dense_inter = hidden, inter
     ids = O.tokens_u32(tokens, cfg.seed, 4, cfg.vocab).reshape(1, tokens)
@@ -81,9 +83,11 @@ def test_kimi_shares_large_and_medium_tiles(kxlib, strict, ox, tmp_path, hidden,
     assert row_err < 2e-2 and log_err < 3e-2
 
 
-@pytest.mark.parametrize("width, ff, tokens, choice", [(2048, 16450, 187, (0, 512, 2, 516)), (4096, 11264, 900, (1, 256, 2, 352))])
-def test_hybrid_decoder_shares_large_and_medium_tiles(kxlib, strict, tmp_path, monkeypatch, width, ff, tokens, choice):
-    assert TS.choices(TS.build(tmp_path), False, [(tokens, 2 * ((ff + 31) // 32 * 32), width)], TS.HYBRID) == [choice]
+@pytest.mark.parametrize("width, ff, tokens, tile, choice", [(2048, 16450, 187, "medium", (0, 512, 2, 516)), (4096, 11264, 900, "large", (1, 256, 2, 352)),
+                                                             (6144, 3290, 515, "twin", (0, 256, 5, 260))])
+def test_hybrid_decoder_shares_large_and_medium_tiles(kxlib, strict, tmp_path, monkeypatch, width, ff, tokens, tile, choice):
+    exe, shape = TS.build(tmp_path), (tokens, 2 * ((ff + 31) // 32 * 32), width)
+    assert TS.choices(exe, False, [shape], TS.HYBRID) == [choice] and TS.tiles(exe, [shape], TS.HYBRID) == [tile]
     cfg = KC.config([KC.delta(heads=4, kv_heads=2, dim=32, vdim=64, ff=ff)], width=width, vocab=300)
     path, ids, got = KC.write(tmp_path / "m", cfg, {}), KC.tokens(cfg, tokens, 5)[None], []
     for lib, cuts in ((kxlib, [tokens]), (strict, [tokens]), (kxlib, [100])):
