@@ -38,7 +38,7 @@ struct KxWindowArgs {
   void *out = nullptr;                    // [tokens][out_ld] of the model's type: heads * vdim, gated
   int out_ld = 0;
   void *q = nullptr;        // scratch [tokens][heads][dp] of the model's type
-  // kx_window_attend on the matrix cores: tokens from one position of a sequence to its next (0: batch) and elements from one
+  // kx_window_attend in bf16 on the matrix cores: tokens from one position of a sequence to its next (0: batch) and elements from one
   // token's queries to the next's (0: heads * dp), where `heads` and `batch` are a part of a step's
   int tok_batch = 0;
   size_t q_ld = 0;

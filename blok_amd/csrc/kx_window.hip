@@ -664,7 +664,7 @@ __global__ void __launch_bounds__(FLASH_WAVES * 64, 2) win_flash_k(KxWindowArgs 
 // ---- f32, several positions: one head, 32 consecutive positions of one sequence ----
 // As above with 32-bit products (v_mfma_f32_32x32x2_f32) and without LDS: wave w of four has every fourth tile of 32 keys to itself, from
 // memory into the operands' registers.  Lane (r, h) holds columns 8 k + 4 h .. +3 of key r and of query r, so that the first product
-// meets two of them at a time, in four chains (two where registers are short); its result in register v is the weight of key 8 (v / 4) + 4 h + v % 4, which the second
+// meets two of them at a time, in four chains; its result in register v is the weight of key 8 (v / 4) + 4 h + v % 4, which the second
 // product takes as it is, with NV columns of that key's value from NV r on.  The keys of the next tile are asked for when the scores are
 // made, its values behind the second product.  Bound by the products, 8192 cycles of a SIMD for 32 keys of 128 and 128 columns.
 // The waves' sums meet at the end.  In tiles that not every query sees as a whole a value that is not finite is replaced by
@@ -684,7 +684,7 @@ __global__ void __launch_bounds__(256, 1) win_flash_f32_k(KxWindowArgs a) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lq = lane & 31, hh = lane >> 5;
   const int h = blockIdx.x % s.heads, b = blockIdx.x / s.heads, g = h / (s.heads / s.kv_heads);
   const int i0 = (gridDim.y - 1 - blockIdx.y) * GQ, i = i0 + lq;
-  const int p = a.pos + min(i, a.positions - 1), tok = min(i, a.positions - 1) * (a.tok_batch ? a.tok_batch : a.batch) + b;
+  const int p = a.pos + min(i, a.positions - 1), tok = min(i, a.positions - 1) * a.batch + b;
   const int p_first = a.pos + i0, p_last = a.pos + min(i0 + GQ, a.positions) - 1;
   const int nb = seen_blocks(p, s.size, s.pool), lo = window_lo(p, s.size);
   const size_t head = (size_t)b * s.kv_heads + g;
@@ -693,7 +693,7 @@ __global__ void __launch_bounds__(256, 1) win_flash_f32_k(KxWindowArgs a) {
   f32x4 k[KP];
   f32x4 *const q = (f32x4 *)(fl_lds + QUERIES) + lane;  // [piece][lane], the same for all waves
   {
-    const float *qr = (const float *)a.q + (size_t)tok * (a.q_ld ? a.q_ld : (size_t)s.heads * c.dp) + (size_t)h * c.dp;
+    const float *qr = (const float *)a.q + ((size_t)tok * s.heads + h) * c.dp;
     for (int x = wave; x < KP; x += 4) q[x * 64] = x * 8 < c.dp ? *(const f32x4 *)(qr + x * 8 + hh * 4) : f32x4{};
   }
   __syncthreads();
@@ -941,8 +941,7 @@ Parts parts_of(const KxWindowArgs &a) {
 }
 bool flash_f32(const KxWindowArgs &a) {
   const KxWindowSpec &s = a.s;
-  if (a.c.dp > 256 || a.c.vp > 128) return false;
-  if (a.tok_batch || a.q_ld) return true;  // parts know nothing of it
+  if (a.c.dp > 256 || a.c.vp > 128 || a.tok_batch || a.q_ld) return false;
   const Parts p = parts_of(a);
   const int most = most_keys(s, a.pos + a.positions);
   return kxwin::matrix_cores_f32({s.heads, s.kv_heads, a.c.dp + a.c.vp, a.batch, a.positions}, most, 0.5 * (most + most_keys(s, a.pos + 1)), {p.keys, p.n, (long)p.at_once},
