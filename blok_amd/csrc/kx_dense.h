@@ -140,7 +140,7 @@ struct KxDenseArgs {
   size_t part_floats = 0;
   int *arrived = nullptr;      // [arrivals], zero between launches
   int arrivals = 0;
-  bool pairs_aligned = false;  // set by the launch: two neighbouring bf16 results are 4 aligned bytes
+  bool pairs_aligned = false;  // set by the launch: two neighbouring bf16 results are 4 aligned bytes (KV: always)
 };
 inline int kx_pad32(int n) { return (n + 31) & ~31; }
 constexpr size_t KX_DENSE_PART_FLOATS = (size_t)256 * 256 * 256;  // what a device of 256 CUs makes use of: a large tile's sums each

@@ -66,7 +66,7 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) dense_gemm_k(
   // Keys and values of 64 heads from 512 columns, 3072 x 16384 164 -> 86 us (one by one is what the tile's short products wait for; 32 columns
   // to a block took 127); gate and up 2048 x 36864 x 7168 877 -> 848.  Where pairs are not aligned, one by one.
   if constexpr (TL::SIDE == 16 && !GROUP && (MODE == KX_GG_BF16 || MODE == KX_GG_RESID || MODE == KX_GG_KV)) {
-    if (a.pairs_aligned) {
+    if (MODE == KX_GG_KV || a.pairs_aligned) {
       const uint32_t odd = threadIdx.x & 1, order = odd ? 0x03020706u : 0x05040100u;
       auto pack = [](float lo, float hi) { return (uint32_t)kx_bf16_rne(lo) | (uint32_t)kx_bf16_rne(hi) << 16; };
       auto exchanged = [&](float lo, float hi) {  // of blocks j and j + 1
@@ -234,6 +234,7 @@ int kx_dense_gemm_launch(const KxDenseArgs &args, hipStream_t st) {
              "kx_dense_gemm: %d rows for %d heads, %d tokens", a.rows, a.heads, a.tokens);
   a.pairs_aligned = a.rows % 2 == 0 && (uintptr_t)a.out % 4 == 0 &&
                     (a.mode == KX_GG_KV ? (a.k_dim | a.v_dim | a.k_ld | a.v_ld) % 2 == 0 && (uintptr_t)a.out_v % 4 == 0 : a.out_stride % 2 == 0);
+  KX_REQUIRE(a.mode != KX_GG_KV || a.pairs_aligned, "kx_dense_gemm: keys of %d and values of %d in rows of %d and %d", a.k_dim, a.v_dim, a.k_ld, a.v_ld);
   if (a.work) {
     KX_REQUIRE(a.pairs && a.groups > 0 && kx_cdiv(a.tokens, kxtile::Medium::BM) <= 65535, "kx_dense_gemm: %d groups", a.groups);
     return launch_as<kxtile::Medium, KX_GG_BF16, false, true>(a, {0, 1}, st);
