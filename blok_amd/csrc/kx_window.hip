@@ -145,7 +145,7 @@ __global__ void __launch_bounds__(PART_THREADS, 4) win_partial_k(KxWindowArgs a,
     const T *key = key_row(k0);
     Keys k;
     k.x[0] = E::cached(key + min(l8 * 8, c.dp - 8));
-    if (c.dp > 64) k.x[1] = E::cached(key + min(l8 * 8 + 64, c.dp - 8));
+    if (sizeof(T) == 2 || c.dp > 64) k.x[1] = E::cached(key + min(l8 * 8 + 64, c.dp - 8));
     return k;
   };
   auto ask_values = [&](int k) {
@@ -154,18 +154,20 @@ __global__ void __launch_bounds__(PART_THREADS, 4) win_partial_k(KxWindowArgs a,
   };
   Keys kr[AHEAD_K];
   typename E::Raw vr[AHEAD_V];
-  auto ask_all = [&] {
+  auto ask_all = [&] {  // in 32 bits, twice the bytes, no row twice: a short context has no second ones
 #pragma unroll
-    for (int y = 0; y < AHEAD_K; ++y) kr[y] = ask_keys(wave * 8 + 32 * y);
+    for (int y = 0; y < AHEAD_K; ++y)
+      if (sizeof(T) == 2 || y == 0 || 32 * y < n) kr[y] = ask_keys(wave * 8 + 32 * y);
 #pragma unroll
-    for (int y = 0; y < AHEAD_V; ++y) vr[y] = ask_values(grp + groups * y);
+    for (int y = 0; y < AHEAD_V; ++y)
+      if (sizeof(T) == 2 || y == 0 || groups * y < n) vr[y] = ask_values(grp + groups * y);
   };
   ask_all();
   if (FUSED) {
     const float *pr = a.proj + (size_t)tok * a.proj_ld;
     const int nq = s.heads * s.dim, nk = s.kv_heads * s.dim;
     float qs = 1.0f, ks = 1.0f;
-    constexpr int UB = sizeof(T) == 2 ? 8 : 4, UQ = 4;  // numbers of a thread asked for together, as registers allow
+    constexpr int UB = 8, UQ = 4;  // numbers of a thread asked for together
     float qx[UQ], qw[UQ];
 #pragma unroll
     for (int k = 0; k < UQ; ++k) {
