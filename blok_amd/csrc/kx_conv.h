@@ -43,7 +43,7 @@ __device__ __forceinline__ void shift(const KxConvArgs &a, int b, int ch) {
 
 // A channel at a step's only position, of up to FEW taps: its inputs and weights are asked for together.  A loop over any number of taps
 // asks for them one after the other, and that, with the state and the step's numbers asked for behind it, was half of a decode step's
-// recurrent kernels: delta_step_k 12.8 us and 6.2 with all of it in front, ssd_step_k 13.4 and 10.1 (kx_delta.hip, kx_ssd.hip).
+// delta_step_k, 12.8 us and 6.2 with all of it in front, and a quarter of ssd_step_k, 13.4 and 10.1 (kx_delta.hip, kx_ssd.hip).
 constexpr int FEW = 4;
 struct Channel {
   float w[FEW], x[FEW], bias;

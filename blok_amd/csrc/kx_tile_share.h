@@ -56,7 +56,7 @@ inline double medium_rounds(double n, int blocks, int cus) {  // two per CU
 // Where the medium tiles leave CUs idle each has a CU to itself, in at least 10 blocks as the twin tile (kx_gemm_turns.h; at 4 blocks
 // it takes 8 % longer than the medium one, at 10 2 % less, at 16 7 % and at 40 19 % less), and they take parts, of at least 16
 // blocks: as many as fill the CUs, or more rounds of shorter ones where that is 5 % sooner (149 x 8548 x 18304, 134 tiles: 153 us whole, 103 in
-// three).  300 x 2048 x 8192 71 alone, 32 in four, 100 x 2048 x 8192 73 and 29 in eight, 2048 x 384 x 7168 65 and 32 in four (medium).
+// three).  300 x 2048 x 8192 53 alone, 28 in five, 100 x 2048 x 8192 52 and 28 in eight, 2048 x 384 x 7168 48 and 29 in five (as medium tiles alone 71, 73 and 65).
 // Beyond that the tile is the one that is sooner whole, or in parts where that is clearly sooner: what is chosen takes 0.976 of the
 // time of the sooner of whole medium and large tiles over 7000 products, 200 of them more than 3 % longer, and 1.5 % more than the best of
 // every way to share out.  Measured (us, large / medium, whole): 2048 x 16384 x 2048 115 / 147, 2048 x 7168 x 8192 171 / 262, 2048 x 8192 x

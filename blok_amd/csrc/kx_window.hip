@@ -374,7 +374,9 @@ __global__ void __launch_bounds__(MERGE_THREADS) win_merge_k(KxWindowArgs a, int
 // copied to LDS two ahead, the second group asking for its share of a tile behind its scores, so that the address path is free
 // when the first one begins.  Workgroups with the most keys come first.
 // 64 heads of 192 and 128, 2048 positions: 382 us with one wave per SIMD and tiles through registers, 184 now; 952 positions behind 2048:
-// 265 and 194; 16 heads of 128, 2048 positions, window 1024: 64 and 49.
+// 265 and 194; 16 heads of 128, 2048 positions, window 1024: 64 and 49.  The whole operator, 16 heads on 4 key heads, 2048 positions, over keys of 32 to 256 and
+// values of 32 to 256 columns takes 0.51 to 0.89 of what it did (256 and 256, whose tiles leave room for two stages and spill 40 bytes a lane, 245 and 125
+// us; 64 and 128 91 and 67; 192 and 32 84 and 74), and 72 other steps 0.49 to 1.00.
 // A key that a query does not see has a weight of zero, and its value is multiplied all the same; zero times a value that is not
 // finite would make the query's output follow a position behind it, or one that its window has left.  So a workgroup whose sums
 // are not all finite makes them once more: in tiles that not every query sees as a whole, such values are replaced by zeros, and
