@@ -415,8 +415,11 @@ __device__ __forceinline__ uint2 mm_read_tr(uint32_t addr) {
   return __builtin_bit_cast(uint2, v);
 }
 // the copies into the tile ring and the fence-free barrier: kx_lds_copy.h (this kernel waits for a tile itself,
-// where it needs it: wait_tile below)
-__device__ __forceinline__ void mm_copy16_to_lds(const void *src, uint32_t lds_base) { kx_copy16_to_lds(src, lds_base); }
+// where it needs it: wait_tile below).  Nontemporal where one position reads the rows: 16 sequences of 32768 positions 131.8 -> 125.9 us.
+__device__ __forceinline__ void mm_copy16_to_lds(const void *src, uint32_t lds_base, bool once) {
+  if (once) kx_copy16_to_lds_once(src, lds_base);
+  else kx_copy16_to_lds(src, lds_base);
+}
 __device__ __forceinline__ void mm_barrier() { kx_lds_barrier(); }
 
 __global__ void __launch_bounds__(512, 1) mla_partial_mfma_k(MlaArgs a) {
@@ -451,6 +454,7 @@ __global__ void __launch_bounds__(512, 1) mla_partial_mfma_k(MlaArgs a) {
   // the sequence repeat its last row.  The lane's places inside a tile do not change from tile to tile: the nine
   // source offsets are kept, and only a tile that reaches past the sequence goes through the row clamp.
   const int cw = wave & 3;
+  const bool once = !a.seqs || (int)gridDim.z == a.seqs;  // positions of a prompt step read the same rows
   int c_off[9];   // elements from the tile's first row
   int c_row[9];
 #pragma unroll
@@ -467,12 +471,12 @@ __global__ void __launch_bounds__(512, 1) mla_partial_mfma_k(MlaArgs a) {
     const uint32_t dst = lds0 + (t % MM_RING) * MM_NAT + cw * 1024;
     if (row0 + MM_T <= seq) {
 #pragma unroll
-      for (int u = 0; u < 9; ++u) mm_copy16_to_lds(src + c_off[u], dst + u * 4096);
+      for (int u = 0; u < 9; ++u) mm_copy16_to_lds(src + c_off[u], dst + u * 4096, once);
     } else {
 #pragma unroll
       for (int u = 0; u < 9; ++u) {
         const int back = max(row0 + c_row[u] - (seq - 1), 0);  // rows past the last one
-        mm_copy16_to_lds(src + c_off[u] - back * MLA_KVA, dst + u * 4096);
+        mm_copy16_to_lds(src + c_off[u] - back * MLA_KVA, dst + u * 4096, once);
       }
     }
   };
