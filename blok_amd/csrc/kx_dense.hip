@@ -313,8 +313,21 @@ int kx_gemv_plan(int epi, KxGemvArgs &a, int *ri) { return gemv_plan(epi, a, *ri
 // route, routed: the router's logits; *routed says whether the launch has also done the routing (gemv_tokblk_route_k)
 static int gemv_launch_impl(int epi, KxGemvArgs a, hipStream_t st, const KxRouteArgs *route, bool *routed) {
   int ri;
-  const int CR = gemv_plan(epi, a, ri, 4);
+  int CR = gemv_plan(epi, a, ri, 4);
   if (CR < 0) return KX_ERR_ARG;
+  // One token and more chunks than workgroups run at once: that many workgroups, which go on to their next chunk with its weights on their way, and
+  // chunks of as many tiles as let the one with the most rows have the fewest.
+  int at_once = 4096;
+  if (a.tokens == 1 && !a.row_block) {
+    const int slots = std::max(1, 1024 / (a.nw * a.rs * 64)) * std::max(1, kx_device_cus()), rt = a.rs * ri;  // 128 registers: 16 waves per CU
+    if (kx_cdiv(a.rows, CR) > slots) {
+      auto most = [&](int nt) { return kx_cdiv(kx_cdiv(a.rows, rt * nt), slots) * nt; };  // tiles of a workgroup
+      for (int nt = a.nt - 1; nt >= 1; --nt)
+        if (most(nt) < most(a.nt)) a.nt = nt;
+      CR = rt * a.nt;
+      at_once = slots;
+    }
+  }
   const int S = a.cols / 512;
   const int mats = epi == KX_EPI_SWIGLU ? 2 : 1;
   const int all_tokens = a.tokens;
@@ -383,7 +396,7 @@ static int gemv_launch_impl(int epi, KxGemvArgs a, hipStream_t st, const KxRoute
     const int chunks = kx_cdiv(a.rows, CR);
     const size_t lds = (size_t)mats * CR * b.tokens * S * sizeof(float);
     KX_REQUIRE(lds <= 160 * 1024, "kx_gemv: %zu bytes of LDS needed", lds);
-    dim3 g(chunks < 4096 ? chunks : 4096), blk(a.nw * a.rs * 64);
+    dim3 g(chunks < at_once ? chunks : at_once), blk(a.nw * a.rs * 64);
     if (mats == 2) launch_ri<2>(b, ri, tt, g, blk, lds, st);
     else launch_ri<1>(b, ri, tt, g, blk, lds, st);
     KX_LAUNCH_CHECK();

@@ -45,6 +45,10 @@ def test_rmsnorm_parity(kxlib, ox, n, tokens):
     (1000, 1536, 13, 0),    # the same, ragged rows and a ragged last token block
     (2048, 512, 9, 0),
     (384, 1024, 70, 1),     # more than 32 tokens: still one launch
+    (131072, 512, 1, 0),    # one token, as many chunks as workgroups run at once
+    (131073, 512, 1, 0),    # and more: chunks of fewer tiles that come out even, two or three to a workgroup, the last one moved back
+    (300001, 512, 1, 1),
+    (66000, 1536, 1, 0),    # workgroups of 768 threads, one to a CU
 ])
 def test_gemv_bf16_parity(kxlib, ox, rows, cols, tokens, f32):
     say(f"gemv_bf16 rows={rows} cols={cols} tokens={tokens} f32={f32}")
