@@ -8,6 +8,8 @@
 // and block numbers stay in registers.  Barriers wait for LDS only: a block's read-outs are still on their way to memory
 // when the next block begins.  With KS = 2 the second half's read-outs go through LDS to the first half's wave, which adds
 // and stores them behind the block's barrier.
+// Up to 128 rows of the state two workgroups fit a CU: 264 registers with a decay per head and 128 rows made that one, and 384 workgroups two
+// rounds (3 sequences of 682 tokens, 64 heads of 128 x 64 135 us, 92 within 256 registers).
 #include <algorithm>
 #include <atomic>
 #include "kx_common.h"
@@ -23,7 +25,7 @@ template <int KT, bool CHANNEL, int KS>
 constexpr size_t lds_floats() { return 2 * (2 * NB * (KT * 16 + 4) + (CHANNEL ? KT * 16 : 0) + (KS > 1 ? 4 / KS * 256 : 0)); }
 
 template <int KT, bool CHANNEL, int KS>  // 16 KT >= dim
-__global__ void __launch_bounds__(256) scan_k(KxScanArgs a) {
+__global__ void __launch_bounds__(256, KT <= 8 ? 2 : 1) scan_k(KxScanArgs a) {
   constexpr int K = KT * 16, KW = KT / KS, COLS = 64 / KS, STR = K + 4, KEYS = 2 * NB * STR, STAGE = KEYS + (CHANNEL ? K : 0), NS = 2 * NB * K / 256, NT = (K + 255) / 256;
   static_assert(KT % KS == 0, "a wave has whole tiles");
   extern __shared__ __attribute__((aligned(16))) float sc_lds[];
