@@ -24,8 +24,6 @@ KxConvArgs conv_of(const KxSsdArgs &a) {
   c.hist = a.hist; c.hist_out = a.hist_out; c.batch = a.batch; c.positions = a.positions;
   return c;
 }
-__device__ __forceinline__ float step_size(const KxSsdArgs &a, size_t tok, int h) { return kxr::softplus(a.proj[tok * a.proj_ld + a.dt_off + h] + a.dt_bias[h]); }
-__device__ __forceinline__ float decay_of(const KxSsdArgs &a, int h, float dt) { return kx_expf(-kx_expf(a.a_log[h]) * dt); }
 
 // RPT: rows of the state per thread.  AHEAD: the convolutions' inputs are asked for in front of them.
 template <int RPT, bool AHEAD = true>
@@ -103,50 +101,77 @@ __host__ __device__ __forceinline__ Work work_of(const KxSsdArgs &a) {
   return w;
 }
 
-// one workgroup per (block, 16 heads of a group): thread (j, i) has the dot product of C_j and B_i, then goes through the heads
+// One workgroup per (block, 16 heads of a group): thread (j, i) has the dot product of C_j and B_i, then goes through the heads.  Bound by the chain of
+// what a workgroup does, so everything from memory is asked for ahead, and products of decays are sixteen factors, ones where a decay is not
+// meant, instead of loops of one LDS read after the other: 3 sequences of 682 tokens, 64 heads in 4 groups, state 128 24.8 us before, 14.1 now, 19 tokens each 22.7
+// and 11.0.
 constexpr int HEADS = 16, BC_COLS = 64;
 __global__ void __launch_bounds__(256) ssd_coef_k(KxSsdArgs a) {
-  __shared__ float bs[NB][BC_COLS + 1], cs[NB][BC_COLS + 1], dt_s[HEADS][NB], a_s[HEADS][NB];
+  __shared__ __attribute__((aligned(16))) float a_s[HEADS][NB];
+  __shared__ float bs[NB][BC_COLS + 1], cs[NB][BC_COLS + 1], dt_s[HEADS][NB];
   const KxSsdSpec &s = a.s;
   const Work w = work_of(a);
   const int tid = threadIdx.x, i = tid & 15, j = tid >> 4, t0 = blockIdx.x * NB, b = blockIdx.z;
   const int ratio = s.heads / s.groups, per = (ratio + HEADS - 1) / HEADS, g = blockIdx.y / per, h0 = g * ratio + (blockIdx.y - g * per) * HEADS;
   const int heads = min(HEADS, (g + 1) * ratio - h0), C = kx_ssd_channels(s), N = s.state, padded = kx_scan_padded(a.positions);
   const float *rows = w.raw + kx_ssd_inner(s) + g * N;
+  constexpr int PER = 2 * NB * BC_COLS / 256;  // of B and C per thread and run of columns
+  float v[PER];
+  auto ask = [&](int n0) {
+#pragma unroll
+    for (int y = 0; y < PER; ++y) {
+      const int x = tid + y * 256, d = min(n0 + x % BC_COLS, N - 1), t = min(t0 + x / BC_COLS % NB, a.positions - 1);
+      v[y] = rows[((size_t)t * a.batch + b) * C + (x >= NB * BC_COLS ? s.groups * N : 0) + d];
+    }
+  };
+  // here a thread is (head, position)
+  const int hh = j, h = h0 + min(hh, heads - 1);
+  const float pd = a.proj[((size_t)min(t0 + i, a.positions - 1) * a.batch + b) * a.proj_ld + a.dt_off + h], bias = a.dt_bias[h], a_log = a.a_log[h];
+  ask(0);
+  const bool mine = t0 + i < a.positions;
+  const float dt = mine ? kxr::softplus(pd + bias) : 0.0f;
+  dt_s[hh][i] = dt;
+  a_s[hh][i] = mine ? kx_expf(-kx_expf(a_log) * dt) : 1.0f;  // a position past the end leaves the state as it is
   float dot = 0.0f;
   for (int n0 = 0; n0 < N; n0 += BC_COLS) {
-    __syncthreads();
-    for (int x = tid; x < 2 * NB * BC_COLS; x += 256) {
-      const int d = n0 + x % BC_COLS, t = x / BC_COLS % NB;
-      const bool c = x >= NB * BC_COLS, in = t0 + t < a.positions && d < N;
-      const float v = in ? rows[((size_t)(t0 + t) * a.batch + b) * C + (c ? s.groups * N : 0) + d] : 0.0f;
-      (c ? cs : bs)[t][x % BC_COLS] = v;
+    if (n0) __syncthreads();
+#pragma unroll
+    for (int y = 0; y < PER; ++y) {
+      const int x = tid + y * 256, t = x / BC_COLS % NB;
+      (x >= NB * BC_COLS ? cs : bs)[t][x % BC_COLS] = t0 + t < a.positions && n0 + x % BC_COLS < N ? v[y] : 0.0f;
     }
+    if (n0 + BC_COLS < N) ask(n0 + BC_COLS);
     __syncthreads();
 #pragma unroll 16
     for (int d = 0; d < BC_COLS; ++d) dot = __builtin_fmaf(cs[j][d], bs[i][d], dot);
   }
-  {
-    const int hh = j, h = h0 + min(hh, heads - 1);  // here a thread is (head, position)
-    const bool in = t0 + i < a.positions;
-    const float dt = in ? step_size(a, (size_t)(t0 + i) * a.batch + b, h) : 0.0f;
-    dt_s[hh][i] = dt;
-    a_s[hh][i] = in ? decay_of(a, h, dt) : 1.0f;  // a position past the end leaves the state as it is
-  }
-  __syncthreads();
+  auto decays = [&](float (&d)[NB], int head) {
+#pragma unroll
+    for (int q = 0; q < NB / 4; ++q) {
+      const float4 f = *(const float4 *)&a_s[head][4 * q];
+      d[4 * q] = f.x; d[4 * q + 1] = f.y; d[4 * q + 2] = f.z; d[4 * q + 3] = f.w;
+    }
+  };
   if (j < heads) {
-    float gamma = 1.0f, end = dt_s[j][i];
-    for (int t = 0; t <= i; ++t) gamma *= a_s[j][t];
-    for (int t = i + 1; t < NB; ++t) end *= a_s[j][t];
+    float d[NB], gamma = 1.0f, end = dt;
+    decays(d, j);
+#pragma unroll
+    for (int t = 0; t < NB; ++t) {
+      gamma *= t <= i ? d[t] : 1.0f;
+      end *= t > i ? d[t] : 1.0f;
+    }
     const size_t at = ((size_t)b * s.heads + h0 + j) * padded + t0 + i;
     w.gamma[at] = gamma;
     w.end[at] = end;
   }
-  for (int hh = 0; hh < heads; ++hh) {
-    float v = dot * dt_s[hh][i];
-    for (int t = i + 1; t <= j; ++t) v *= a_s[hh][t];
-    if (i == j) v += a.skip[h0 + hh];
-    w.inner[(((size_t)b * s.heads + h0 + hh) * padded + t0 + j) * NB + i] = i <= j ? v : 0.0f;
+#pragma unroll 4
+  for (int k = 0; k < heads; ++k) {
+    float d[NB], y = dot * dt_s[k][i];
+    decays(d, k);
+#pragma unroll
+    for (int t = 1; t < NB; ++t) y *= t > i && t <= j ? d[t] : 1.0f;
+    if (i == j) y += a.skip[h0 + k];
+    w.inner[(((size_t)b * s.heads + h0 + k) * padded + t0 + j) * NB + i] = i <= j ? y : 0.0f;
   }
 }
 
