@@ -152,3 +152,33 @@ def test_tiles_whose_groups_take_turns(kxlib, rule, tokens, rows, cols, tile):
     """Even and odd numbers of blocks, tiles with remainders of tokens and rows, every epilogue: the bars of the large tiles, 32-bit sums of up to
     1088 products (about 1e-6)."""
     test_large_tiles(kxlib, rule, tokens, rows, cols, tile)
+
+
+@pytest.mark.parametrize("f32", [0, 1], ids=["bf16", "f32"])
+@pytest.mark.parametrize("tokens", [2, 3, 4])
+@pytest.mark.parametrize("cols, streams, groups, heads", [(96, 1, 1, 3), (1000, 2, 4, 8), (2048, 2, 2, 16), (4097, 3, 1, 17)])
+def test_rows_in_a_launch_of_their_own(kxlib, tokens, cols, streams, groups, heads, f32):
+    """Two to four tokens: with room for them the rows are built in front of the product, without in it, and the results are the same to the bit."""
+    r = np.random.default_rng(cols + tokens)
+    rows = 70
+    w, ld = _matrix(KC.bf16(r.standard_normal((rows, cols)) * cols ** -0.5), f32)
+    vdim = cols // heads
+    x, win = dev(r.standard_normal((tokens, streams, cols)).astype(np.float32)), dev(r.standard_normal(streams).astype(np.float32))
+    norm = dev((1 + 0.3 * r.standard_normal(cols)).astype(np.float32))
+    o, gate = dev(r.standard_normal((tokens, cols)).astype(np.float32)), dev(r.standard_normal((tokens, cols + 5)).astype(np.float32))
+    scratch = DevBuf(tokens * ld * 4)
+    forms = [dict(row_kind=1, streams=streams, groups=groups, d_streams_in=x.ptr, d_in=win.ptr)]
+    if vdim * heads == cols:
+        forms += [dict(row_kind=2, streams=1, groups=1, heads=heads, vdim=vdim, d_o=o.ptr, d_gate=gate.ptr, gate_ld=cols + 5, gate_first=first) for first in (0, 1)]
+    for form in forms:
+        got = []
+        for room in (None, scratch.ptr):
+            out = dev(np.full((tokens, rows), 7.0, np.float32))
+            a = KxLinearArgs(f32=f32, tokens=tokens, rows=rows, cols=cols, ld=ld, eps=1e-5, d_w=w.ptr, d_norm=norm.ptr, epilogue=0, out_ld=rows)
+            for k, v in form.items():
+                setattr(a, k, v)
+            a.d_out = out.ptr
+            check(kxlib.kx_linear_run(C.byref(a), room, None))
+            check(kxlib.kx_sync(None))
+            got.append(out.to_numpy(np.float32, (tokens, rows)))
+        assert np.isfinite(got[0]).all() and (got[0] != 7.0).any() and np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32)), form
