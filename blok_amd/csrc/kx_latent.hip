@@ -254,9 +254,12 @@ __global__ void __launch_bounds__(256) latent_part_k(KxLatentArgs a, Parts p, in
     }
 }
 
-// the parts of one head of one token merged with the sink, OUT_ROWS rows of its W_uv, the gate
-constexpr int OUT_THREADS = 512, OUT_AHEAD = 20;  // OUT_AHEAD: a thread's parts that are asked for before the weights are known
-template <class T>
+// The parts of one head of one token merged with the sink, OUT_ROWS rows of its W_uv, the gate.  AHEAD: a thread's parts that are asked for before the
+// weights are known.  Few parts are all asked for by four: with twenty every thread asks for the last part again and again, and 185 registers leave a CU
+// one workgroup: 8 tokens of 16 heads of 128 rows of 512, 3 parts, 13.3 us with twenty, 6.7 now.
+constexpr int OUT_THREADS = 512, OUT_AHEAD = 20, OUT_FEW = 4;
+__host__ __device__ constexpr int out_shares(int vp) { return vp <= OUT_THREADS ? 4 : vp <= 2 * OUT_THREADS ? 2 : 1; }  // vp / 4 threads hold all columns
+template <class T, int AHEAD>
 __global__ void __launch_bounds__(OUT_THREADS) latent_out_k(KxLatentArgs a, Parts w, int tok0, int vp) {
   using E = Elem<T>;
   extern __shared__ __attribute__((aligned(16))) float lo_lds[];
@@ -266,12 +269,12 @@ __global__ void __launch_bounds__(OUT_THREADS) latent_out_k(KxLatentArgs a, Part
   float *lat = lo_lds, *sum = lat + ld, *weight = sum + 4 * ld, *den = weight + w.parts;  // [ld], [4][ld], [parts], [parts]
   const size_t row = (size_t)blockIdx.y * w.parts;
   // four columns per thread; where fewer threads hold them all, the others take parts of their own
-  const int quads = vp / 4, shares = quads <= OUT_THREADS / 4 ? 4 : quads <= OUT_THREADS / 2 ? 2 : 1, per = OUT_THREADS / shares, share = tid / per, tq = tid - share * per;
+  const int quads = vp / 4, shares = out_shares(vp), per = OUT_THREADS / shares, share = tid / per, tq = tid - share * per;
   const float *po = w.o + (row * s.heads + h) * vp;
   auto part = [&](int k, int x) { return *(const f32x4 *)(po + (size_t)min(k, w.parts - 1) * s.heads * vp + 4 * min(x, quads - 1)); };
-  f32x4 y[OUT_AHEAD];
+  f32x4 y[AHEAD];
 #pragma unroll
-  for (int j = 0; j < OUT_AHEAD; ++j) y[j] = part(share + j * shares, tq);
+  for (int j = 0; j < AHEAD; ++j) y[j] = part(share + j * shares, tq);
   constexpr int RW = OUT_ROWS / (OUT_THREADS / 64);  // rows per wave
   typename E::Raw uv[RW];
   float gate[RW];
@@ -302,12 +305,12 @@ __global__ void __launch_bounds__(OUT_THREADS) latent_out_k(KxLatentArgs a, Part
   __syncthreads();
   for (int x = tq; x < quads; x += per) {
     f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int k0 = share; k0 < w.parts; k0 += OUT_AHEAD * shares) {
+    for (int k0 = share; k0 < w.parts; k0 += AHEAD * shares) {
       if (x != tq || k0 != share)
 #pragma unroll
-        for (int j = 0; j < OUT_AHEAD; ++j) y[j] = part(k0 + j * shares, x);
+        for (int j = 0; j < AHEAD; ++j) y[j] = part(k0 + j * shares, x);
 #pragma unroll
-      for (int j = 0; j < OUT_AHEAD; ++j) {
+      for (int j = 0; j < AHEAD; ++j) {
         const int k = k0 + j * shares;
         const float wt = k < w.parts ? weight[k] : 0.0f;
 #pragma unroll
@@ -432,7 +435,7 @@ int few(const KxLatentArgs &a, hipStream_t st) {
     if (rc) return rc;
     const size_t lds = ((size_t)5 * a.uv.ld + 2 * p.parts) * 4;
     KX_REQUIRE(lds <= 64 * 1024, "latent attention: %d parts of %d columns", p.parts, s.kv_rank);
-    hipLaunchKernelGGL(latent_out_k<T>, dim3(s.heads * kx_cdiv(s.vdim, OUT_ROWS), p.n), dim3(OUT_THREADS), lds, st, a, p, t0, vp);
+    hipLaunchKernelGGL((p.parts <= OUT_FEW * out_shares(vp) ? latent_out_k<T, OUT_FEW> : latent_out_k<T, OUT_AHEAD>), dim3(s.heads * kx_cdiv(s.vdim, OUT_ROWS), p.n), dim3(OUT_THREADS), lds, st, a, p, t0, vp);
     KX_LAUNCH_CHECK();
   }
   return KX_OK;

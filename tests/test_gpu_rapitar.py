@@ -331,6 +331,17 @@ def test_latent_attention_without_room_for_expanded_keys(kxlib, f32):
 
 
 @FORMATS
+@pytest.mark.parametrize("case, context", [((2, 16, 8, 8, 16, 64), 1024), ((2, 16, 8, 8, 16, 600), 128), ((1, 16, 8, 8, 16, 600), 256), ((1, 8, 4, 4, 8, 1100), 64)],
+                         ids=lambda x: "-".join(map(str, x)) if isinstance(x, tuple) else str(x))
+def test_latent_parts_that_are_asked_for_at_once_and_more(kxlib, case, context, f32):
+    """One token at a time across the contexts where its parts become more than a workgroup asks for at once: 16 of 64 keys, 8 of 16 or 32, 4 of 16."""
+    a = Latent(kxlib, *case, f32, context=context + 8, positions=context)
+    rows = np.random.default_rng(11).standard_normal((1, context + 5, a.cols()[-1])).astype(np.float32)
+    assert rel(a.run(rows, [context - 3, 1])[0][-8:], a.oracle(rows[0])[-8:]) < _bar(f32)
+    a.close()
+
+
+@FORMATS
 def test_latent_tiles_one_after_the_other(kxlib, f32):
     """Enough tokens, heads and keys that a workgroup goes through several tiles of keys."""
     a = Latent(kxlib, 24, 16, 8, 8, 16, 64, f32, batch=6, context=640, positions=8)
