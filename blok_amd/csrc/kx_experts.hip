@@ -15,20 +15,31 @@ __global__ void __launch_bounds__(256) route_k(KxExpertArgs e, int tokens) {
 
 // One workgroup: counts per expert, their running sums, tiles, and a slot for every pair.  ROUTE: of up to BUCKET_WAVES tokens, which it routes itself, a
 // wave each.  It is one chain of waits, so a thread asks for PAIRS_AHEAD pairs at once and a wave makes its own running sums.  2046 tokens, 8 experts
-// each: 17.4 us with a pair at a time and sums over LDS, 12.0 now; 8 tokens: 6.5 + 4.2 and a launch between them, 11.8 in one.
+// each: 17.4 us with a pair at a time and sums over LDS, 12.0 now; 8 tokens: 6.5 + 4.2 and a launch between them, 11.8 in one; 10.6 and, with
+// their pairs kept in LDS instead of read back from memory, 9.8.
 constexpr int BUCKET_WAVES = KX_MAX_EXPERTS / 64, PAIRS_AHEAD = 16;
 template <bool ROUTE>
 __global__ void __launch_bounds__(KX_MAX_EXPERTS) bucket_k(KxExpertArgs e, KxExpertSlots s, int tokens) {
   __shared__ int count[KX_MAX_EXPERTS], total[2][BUCKET_WAVES];
+  __shared__ int own_id[ROUTE ? BUCKET_WAVES * KX_MAX_TOP : 1];  // of the pairs it routes itself
+  __shared__ float own_weight[ROUTE ? BUCKET_WAVES * KX_MAX_TOP : 1];
+  static_assert(BUCKET_WAVES * KX_MAX_TOP <= KX_MAX_EXPERTS, "a thread has one pair of those");
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), pairs = tokens * e.top;
   count[tid] = 0;
-  if (ROUTE && wave < tokens)
-    kxe::route_wave(e.logits + (size_t)wave * e.logits_ld, e.bias, e.experts, e.top, e.ids + (size_t)wave * e.top, e.weights + (size_t)wave * e.top);
-  if (ROUTE) __threadfence_block();
+  if (ROUTE && wave < tokens) kxe::route_wave(e.logits + (size_t)wave * e.logits_ld, e.bias, e.experts, e.top, own_id + wave * e.top, own_weight + wave * e.top);
   __syncthreads();
   int id[PAIRS_AHEAD];
   float weight[PAIRS_AHEAD];
   auto ask = [&](int p0) {  // pairs p0 + tid, and so on
+    if constexpr (ROUTE) {
+      id[0] = own_id[min(tid, pairs - 1)];
+      weight[0] = own_weight[min(tid, pairs - 1)];
+      if (tid < pairs) {
+        e.ids[tid] = id[0];
+        e.weights[tid] = weight[0];
+      }
+      return;
+    }
 #pragma unroll
     for (int k = 0; k < PAIRS_AHEAD; ++k)
       if (p0 + k * KX_MAX_EXPERTS < pairs) {
