@@ -7,7 +7,7 @@
 // A GEMV kernel streams the weights once per block of four tokens and is bound by its fma count from about 16 tokens
 // on (every weight meets every token on the VALU), and
 // the prefill GEMM of kx_dense_gemm.hip, built for tiles of 64 tokens and more, leaves most of the chip idle on one of
-// 32.  Here a workgroup of 8 waves owns 32 weight rows and all (up to 32) tokens, the eight waves
+// 32.  Here a workgroup of 8 waves takes tiles of 32 weight rows (16 of each of two matrices) and all (up to 32) tokens, the eight waves
 // split the columns, and their partial 32 x 32 tiles (v_mfma_f32_32x32x16_bf16) are summed through LDS in wave
 // order before the epilogue.
 //
@@ -17,16 +17,20 @@
 // blocks of 256: a copy instruction (global_load_lds_dwordx4, no registers) moves 512 contiguous bytes of two rows,
 // lane (l / 32, l % 32) = (row of the pair, 16-byte slot); the lane fetches piece slot ^ (row % 16) of its row, so
 // that the operand reads -- lane (r, h) wants piece p of row r and finds it in slot p ^ (r % 16) -- fall into different
-// banks.  Blocks go through a ring of 4 stages (3 for two matrices), three (two) blocks in flight behind the one being
+// banks.  Blocks go through a ring of 5 stages (4 with more than 16 tokens), four (three) blocks in flight behind the one being
 // multiplied; each wave issues its share of a block's copies, waits for its own by count (they complete in order),
 // and one barrier per block makes every wave's copies visible and the stage that is overwritten next free.  Wave w
-// multiplies pieces 4w .. 4w+3 of the block (two products per matrix).  The lm_head takes 0.43 ms this way (5.5 TB/s).  The matrix is
-// copied nontemporally (kx_lds_copy.h): a step of 12 sequences through two dense layers of Kimi-K2 and a head 676 -> 628 us.
+// multiplies pieces 4w .. 4w+3 of the block.  The matrix is copied nontemporally (kx_lds_copy.h).
+// LDS leaves a CU one workgroup.  Where there are tiles for half of the CUs and more, every CU has one and an equal share of the rows, whose tiles follow each other
+// through the ring: the next tile's blocks are on their way while a tile's sums are added.  A workgroup per 32 rows instead was 224 for the 7168
+// rows of a down projection and, two matrices at a time, two rounds and a quarter for 18432 rows.  12 tokens, 2 x 18432 x 7168 91.5 us so, 79.3 now; 7168 x
+// 8192 and 7168 x 18432 38.3 on average, and 32768 x 7168 71.8, the three together 32.2 on average of 45.0; a step through two dense layers and a head 624 -> 568 us.
 // The copies are issued from inline asm and the barrier carries no fence: a copy the compiler knows of makes it
 // complete everything in flight before every LDS access it cannot tell from the copy's target.
 //
 // Sums are fp32 over exact bf16 products in another order than the GEMV's: this path is held to the 1e-2 bar, like the
 // other matrix-core paths, and serves batches the token-identity checks do not run on.
+#include <algorithm>
 #include <atomic>
 #include "kx_common.h"
 #include "kx_lds_copy.h"
@@ -49,105 +53,135 @@ template <int N>
 __device__ __forceinline__ void sk_wait_copies() { kx_wait_copies<N>(); }
 __device__ __forceinline__ void sk_barrier() { kx_lds_barrier(); }
 
-template <bool DUAL>
+// FEW: up to 16 tokens, half the copies of tokens and a stage more.  DUAL: a tile is 16 rows of each matrix.
+template <bool DUAL, bool FEW>
+struct Skinny {
+  static constexpr int NS = FEW ? 5 : 4;             // stages
+  static constexpr int XC = FEW ? 1 : 2, CPW = 2 + XC;  // copy instructions per wave and block: two of the matrix, XC of the tokens
+  static constexpr int ROWS = DUAL ? 16 : 32;        // rows of the result per tile
+  static constexpr uint32_t TILE = 32 * 512, STAGE = TILE + (FEW ? 16 : 32) * 512, PART = NS * STAGE;
+  static constexpr size_t LDS = PART + 8 * 16 * 32 * sizeof(float);  // the ring, and the waves' sums of 16 tokens
+};
+
+template <bool DUAL, bool FEW>
 __global__ void __launch_bounds__(512) skinny_staged_k(SkinnyArgs a) {
-  constexpr int MATS = DUAL ? 2 : 1;
-  constexpr int TILES = MATS + 1;            // weight tiles and the activation tile of a stage, 16 KB each
-  constexpr int NS = DUAL ? 3 : 4;           // stages
-  constexpr int CPW = TILES * 2;             // copy instructions per wave and block (16 per tile over 8 waves)
-  constexpr uint32_t TILE = 32 * 512, STAGE = TILES * TILE;
+  using K = Skinny<DUAL, FEW>;
+  constexpr int NS = K::NS, CPW = K::CPW, ROWS = K::ROWS;
   extern __shared__ __attribute__((aligned(16))) uint8_t sk_lds[];
   const uint32_t lds0 = (uint32_t)(uintptr_t)sk_lds;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 31, h = lane >> 5;
-  const int row0 = blockIdx.x * 32;
   const int nb = a.cols >> 8;  // blocks of 256 columns
-  // this wave's copies of a block: instruction u moves rows 2 i, 2 i + 1 of tile t, (t, i) = ((8 u + wave) / 16, .. % 16)
-  const uint16_t *csrc[CPW];
-  uint32_t cdst[CPW];
+  const int row_end = (int)((long)a.rows * (blockIdx.x + 1) / gridDim.x);
+  int row0 = (int)((long)a.rows * blockIdx.x / gridDim.x);  // of the tile that is multiplied
+  const int total = (row_end - row0 + ROWS - 1) / ROWS * nb;
+  // this wave's copies of a block: instruction i moves staged rows 2 i and 2 i + 1
+  const uint16_t *wsrc[2], *xsrc[K::XC];
+  auto rows_from = [&](int first) {
 #pragma unroll
-  for (int u = 0; u < CPW; ++u) {
-    const int idx = u * 8 + wave, t = idx >> 4, i = idx & 15;
-    const int row = 2 * i + h, piece = r ^ (row & 15);
-    const uint16_t *base = t == MATS ? a.x + (size_t)min(row, a.tokens - 1) * a.x_stride
-                                     : (t == 0 ? a.w0 : a.w1) + (size_t)min(row0 + row, a.rows - 1) * a.cols;
-    csrc[u] = base + piece * 8;
-    cdst[u] = t * TILE + i * 1024;
-  }
-  auto copy_block = [&](int b) {
-    const uint32_t st = lds0 + (uint32_t)(b % NS) * STAGE;
-#pragma unroll
-    for (int u = 0; u < CPW; ++u) {
-      const uint32_t to = __builtin_amdgcn_readfirstlane(st + cdst[u]);
-      if (u < 2 * MATS) kx_copy16_to_lds_once(csrc[u] + b * 256, to);  // the matrices
-      else kx_copy16_to_lds(csrc[u] + b * 256, to);
+    for (int u = 0; u < 2; ++u) {
+      const int row = 2 * (u * 8 + wave) + h;
+      wsrc[u] = (DUAL && u ? a.w1 : a.w0) + (size_t)min(first + (DUAL ? row & 15 : row), row_end - 1) * a.cols + (r ^ (row & 15)) * 8;
     }
   };
-  kx_f32x16 acc[MATS];
 #pragma unroll
-  for (int m = 0; m < MATS; ++m)
+  for (int u = 0; u < K::XC; ++u) {
+    const int row = 2 * (u * 8 + wave) + h;
+    xsrc[u] = a.x + (size_t)min(row, a.tokens - 1) * a.x_stride + (r ^ (row & 15)) * 8;
+  }
+  int copy_row = row0, copy_block = 0, copy_stage = 0;  // what is asked for next
+  rows_from(copy_row);
+  auto copy_next = [&]() {
+    const uint32_t st = lds0 + (uint32_t)copy_stage * K::STAGE + wave * 1024;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[m][v] = 0.0f;
+    for (int u = 0; u < 2; ++u) kx_copy16_to_lds_once(wsrc[u] + copy_block * 256, __builtin_amdgcn_readfirstlane(st + u * 8192));
+#pragma unroll
+    for (int u = 0; u < K::XC; ++u) kx_copy16_to_lds(xsrc[u] + copy_block * 256, __builtin_amdgcn_readfirstlane(st + K::TILE + u * 8192));
+    copy_stage = copy_stage == NS - 1 ? 0 : copy_stage + 1;
+    if (++copy_block == nb) {
+      copy_block = 0;
+      rows_from(copy_row += ROWS);
+    }
+  };
+  kx_f32x16 acc;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
   // operand reads of this lane: piece 4 wave + 2 q + h of row r sits in slot piece ^ (r % 16)
   uint32_t roff[2];
 #pragma unroll
-  for (int q = 0; q < 2; ++q) roff[q] = (uint32_t)r * 512 + (uint32_t)((4 * wave + 2 * q + h) ^ (r & 15)) * 16;
+  for (int q = 0; q < 2; ++q) roff[q] = (uint32_t)((4 * wave + 2 * q + h) ^ (r & 15)) * 16;
+  const uint32_t wrow = (uint32_t)r * 512, xrow = K::TILE + (uint32_t)(FEW ? r & 15 : r) * 512;  // tokens 16 to 31 of FEW: nobody's
 
 #pragma unroll
-  for (int b = 0; b < NS - 1; ++b)
-    if (b < nb) copy_block(b);
-  for (int b = 0; b < nb; ++b) {
-    // this wave's copies of block b have landed when at most those of the blocks behind it are in flight
-    const int behind = min(nb - 1 - b, NS - 2);
-    if (behind >= 2) sk_wait_copies<2 * CPW>();
+  for (int k = 0; k < NS - 1; ++k)
+    if (k < total) copy_next();
+  int stage = 0, block = 0;
+  for (int k = 0; k < total; ++k) {
+    // this wave's copies of block k have landed when at most those of the blocks behind it are in flight; stores of the last tile's
+    // results, which are counted with them, make it wait for more
+    const int behind = min(total - 1 - k, NS - 2);
+    if (NS > 4 && behind >= 3) sk_wait_copies<3 * CPW>();
+    else if (behind >= 2) sk_wait_copies<2 * CPW>();
     else if (behind == 1) sk_wait_copies<CPW>();
     else sk_wait_copies<0>();
-    sk_barrier();  // every wave's copies of block b are in LDS; every wave is done with block b - 1
-    if (b + NS - 1 < nb) copy_block(b + NS - 1);  // into the stage block b - 1 was read from
-    const uint8_t *st = sk_lds + (uint32_t)(b % NS) * STAGE;
+    sk_barrier();  // every wave's copies of block k are in LDS; every wave is done with block k - 1
+    if (k + NS - 1 < total) copy_next();  // into the stage block k - 1 was read from
+    const uint8_t *st = sk_lds + (uint32_t)stage * K::STAGE;
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const kx_bf16x8 xv = *(const kx_bf16x8 *)(st + MATS * TILE + roff[q]);
+    for (int q = 0; q < 2; ++q)
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const kx_bf16x8 *)(st + xrow + roff[q]), *(const kx_bf16x8 *)(st + wrow + roff[q]), acc, 0, 0, 0);
+    stage = stage == NS - 1 ? 0 : stage + 1;
+    if (++block < nb) continue;
+    block = 0;
+    // the tile's sums, 16 tokens at a time; the barriers of a tile's blocks, two at least, lie between its reads here and the next one's writes
+    float(*part)[16][32] = (float(*)[16][32])(sk_lds + K::PART);
 #pragma unroll
-      for (int m = 0; m < MATS; ++m) {
-        const kx_bf16x8 wv = *(const kx_bf16x8 *)(st + m * TILE + roff[q]);
-        acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xv, wv, acc[m], 0, 0, 0);
+    for (int p = 0; p < (FEW ? 1 : 2); ++p) {
+      if (p) sk_barrier();
+#pragma unroll
+      for (int v = 0; v < 8; ++v) part[wave][8 * (v >> 2) + 4 * h + (v & 3)][r] = acc[8 * p + v];
+      sk_barrier();
+      const int rr = threadIdx.x % ROWS, t = threadIdx.x / ROWS, row = row0 + rr, tok = 16 * p + t;
+      if (t >= 16 || row >= row_end || tok >= a.tokens) continue;
+      auto sum = [&](int c) {
+        float y = part[0][t][c];
+#pragma unroll
+        for (int w = 1; w < 8; ++w) y += part[w][t][c];
+        return y;
+      };
+      const float y = sum(rr);
+      const size_t o = (size_t)tok * a.out_stride + row;
+      if (DUAL) {
+        ((uint16_t *)a.out)[o] = kx_bf16_rne(kx_swiglu(kx_bfround(y), kx_bfround(sum(rr + 16))));
+      } else if (a.mode == KX_GG_BF16) {
+        ((uint16_t *)a.out)[o] = kx_bf16_rne(y);
+      } else if (a.mode == KX_GG_F32) {
+        ((float *)a.out)[o] = y;
+      } else if (a.mode == KX_GG_F32_OF_BF16) {
+        ((float *)a.out)[o] = kx_bfround(y);
+      } else {  // x = bf(x + bf(y))  (add_k, :248-251)
+        uint16_t *xo = (uint16_t *)a.out + o;
+        *xo = kx_bf16_rne(kx_bf16_f32(*xo) + kx_bfround(y));
       }
     }
+    row0 += ROWS;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
   }
-  sk_barrier();  // the ring is free: it takes the partial tiles
-  float(*part)[8][32][32] = (float(*)[8][32][32])sk_lds;
-#pragma unroll
-  for (int m = 0; m < MATS; ++m)
-#pragma unroll
-    for (int v = 0; v < 16; ++v) part[m][wave][8 * (v >> 2) + 4 * h + (v & 3)][r] = acc[m][v];
-  __syncthreads();
-  for (int idx = threadIdx.x; idx < 32 * 32; idx += 512) {
-    const int rr = idx & 31, t = idx >> 5;
-    const int row = row0 + rr;
-    if (row >= a.rows || t >= a.tokens) continue;
-    float y[MATS];
-#pragma unroll
-    for (int m = 0; m < MATS; ++m) {
-      float sum = part[m][0][t][rr];
-#pragma unroll
-      for (int w = 1; w < 8; ++w) sum += part[m][w][t][rr];
-      y[m] = sum;
-    }
-    const size_t o = (size_t)t * a.out_stride + row;
-    if (DUAL) {
-      ((uint16_t *)a.out)[o] = kx_bf16_rne(kx_swiglu(kx_bfround(y[0]), kx_bfround(y[MATS - 1])));
-    } else if (a.mode == KX_GG_BF16) {
-      ((uint16_t *)a.out)[o] = kx_bf16_rne(y[0]);
-    } else if (a.mode == KX_GG_F32) {
-      ((float *)a.out)[o] = y[0];
-    } else if (a.mode == KX_GG_F32_OF_BF16) {
-      ((float *)a.out)[o] = kx_bfround(y[0]);
-    } else {  // x = bf(x + bf(y))  (add_k, :248-251)
-      uint16_t *xo = (uint16_t *)a.out + o;
-      *xo = kx_bf16_rne(kx_bf16_f32(*xo) + kx_bfround(y[0]));
-    }
+}
+
+template <bool DUAL, bool FEW>
+int skinny(const SkinnyArgs &a, hipStream_t st) {
+  using K = Skinny<DUAL, FEW>;
+  static std::atomic<bool> attr{false};  // setting it twice from two threads is harmless
+  if (!attr) {
+    KX_HIP(hipFuncSetAttribute((const void *)skinny_staged_k<DUAL, FEW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)K::LDS));
+    attr = true;
   }
+  const int tiles = kx_cdiv(a.rows, K::ROWS), cus = std::max(1, kx_device_cus());
+  hipLaunchKernelGGL((skinny_staged_k<DUAL, FEW>), dim3(2 * tiles > cus ? std::min(cus, a.rows) : tiles), dim3(512), K::LDS, st, a);
+  KX_LAUNCH_CHECK();
+  return KX_OK;
 }
 
 }  // namespace
@@ -162,17 +196,8 @@ int kx_skinny_gemm_launch(bool dual, const uint16_t *w0, const uint16_t *w1, con
   SkinnyArgs a;
   a.w0 = w0; a.w1 = w1; a.x = x; a.out = out; a.rows = rows; a.cols = cols; a.tokens = tokens; a.x_stride = x_stride;
   a.out_stride = out_stride; a.mode = out_mode;
-  const dim3 g((unsigned)kx_cdiv(rows, 32));
-  const size_t lds = (size_t)(dual ? 3 * 3 : 4 * 2) * 32 * 512;  // the ring: stages x tiles x 16 KB
-  static std::atomic<bool> attr{false};  // setting it twice from two threads is harmless
-  if (!attr) {
-    KX_HIP(hipFuncSetAttribute((const void *)skinny_staged_k<false>, hipFuncAttributeMaxDynamicSharedMemorySize, 4 * 2 * 32 * 512));
-    KX_HIP(hipFuncSetAttribute((const void *)skinny_staged_k<true>, hipFuncAttributeMaxDynamicSharedMemorySize, 3 * 3 * 32 * 512));
-    attr = true;
-  }
-  if (dual) hipLaunchKernelGGL(skinny_staged_k<true>, g, dim3(512), lds, st, a);
-  else hipLaunchKernelGGL(skinny_staged_k<false>, g, dim3(512), lds, st, a);
-  KX_LAUNCH_CHECK();
-  *done = true;
-  return KX_OK;
+  const bool few = tokens <= 16;
+  const int rc = dual ? few ? skinny<true, true>(a, st) : skinny<true, false>(a, st) : few ? skinny<false, true>(a, st) : skinny<false, false>(a, st);
+  *done = rc == KX_OK;
+  return rc;
 }

@@ -114,3 +114,26 @@ def test_a_model_takes_the_memory_that_its_size_is_given_as(kxlib):
     taken = before - _free(kxlib)
     km.close()
     assert taken < sum(p.value for p in parts) + (64 << 20)
+
+
+@pytest.mark.parametrize("batch", [5, 16, 17, 32])
+@pytest.mark.parametrize("ff, vocab", [(8704, 9001), (2048, 4097), (4608, 33000)], ids=["two and three tiles a workgroup", "a tile or a few rows each", "five tiles"])
+def test_products_of_a_batch_on_as_many_workgroups_as_run_at_once(kxlib, ox, batch, ff, vocab):
+    """One position of 5 to 32 sequences a step, 16 and 17 on either side of the kernel's two forms: rows that do not come out even on 256 workgroups, against the
+    same model's GEMVs.  The bars are those of long steps."""
+    prompt = 6
+    cfg = _config(16, batch, prompt + 4)
+    cfg.dense_inter, cfg.vocab = ff, vocab
+    ids = O.tokens_u32(batch * prompt, cfg.seed, 4, cfg.vocab).reshape(batch, prompt)
+    km = KxModel(kxlib, cfg)
+    got = []
+    for exact in (15, 0):
+        check(kxlib.kx_model_set_exact(km.h, exact))
+        check(kxlib.kx_model_set_prefill_chunk(km.h, 1))
+        rc, out, _ = km.generate(ids, 1)
+        assert rc == 0, kxlib.kx_last_error()
+        got.append((O.bf16_to_f32(np.stack([km.latent(1, b, prompt) for b in range(batch)])).astype(np.float64), km.logits(batch)))
+    km.close()
+    (rows, logits), (rows1, logits1) = got
+    assert np.abs(rows1 - rows).max() / np.abs(rows).max() < 2e-2
+    assert max(O.max_rel(logits1[b], logits[b]) for b in range(batch)) < 3e-2
