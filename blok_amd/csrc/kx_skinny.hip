@@ -24,7 +24,7 @@
 // LDS leaves a CU one workgroup.  Where there are tiles for half of the CUs and more, every CU has one and an equal share of the rows, whose tiles follow each other
 // through the ring: the next tile's blocks are on their way while a tile's sums are added.  A workgroup per 32 rows instead was 224 for the 7168
 // rows of a down projection and, two matrices at a time, two rounds and a quarter for 18432 rows.  12 tokens, 2 x 18432 x 7168 91.5 us so, 79.3 now; 7168 x
-// 8192 and 7168 x 18432 38.3 on average, and 32768 x 7168 71.8, the three together 32.2 on average of 45.0; a step through two dense layers and a head 624 -> 568 us.
+// 8192, 7168 x 18432, 12288 x 1536 (two each) and 32768 x 7168 35.7 on average, 32.2 now; a step through two dense layers and a head 624 -> 568 us.
 // The copies are issued from inline asm and the barrier carries no fence: a copy the compiler knows of makes it
 // complete everything in flight before every LDS access it cannot tell from the copy's target.
 //
@@ -47,6 +47,7 @@ struct SkinnyArgs {
   const uint16_t *x;        // bf16 [tokens, x_stride]
   void *out;                // [tokens, out_stride]: bf16, or f32 (see mode)
   int rows, cols, tokens, x_stride, out_stride, mode;
+  int share, extra;         // rows of a workgroup, one more for the first `extra`
 };
 
 template <int N>
@@ -72,8 +73,8 @@ __global__ void __launch_bounds__(512) skinny_staged_k(SkinnyArgs a) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 31, h = lane >> 5;
   const int nb = a.cols >> 8;  // blocks of 256 columns
-  const int row_end = (int)((long)a.rows * (blockIdx.x + 1) / gridDim.x);
-  int row0 = (int)((long)a.rows * blockIdx.x / gridDim.x);  // of the tile that is multiplied
+  const int bx = blockIdx.x, row_end = min((bx + 1) * a.share + min(bx + 1, a.extra), a.rows);
+  int row0 = bx * a.share + min(bx, a.extra);  // of the tile that is multiplied
   const int total = (row_end - row0 + ROWS - 1) / ROWS * nb;
   // this wave's copies of a block: instruction i moves staged rows 2 i and 2 i + 1
   const uint16_t *wsrc[2], *xsrc[K::XC];
@@ -171,7 +172,7 @@ __global__ void __launch_bounds__(512) skinny_staged_k(SkinnyArgs a) {
 }
 
 template <bool DUAL, bool FEW>
-int skinny(const SkinnyArgs &a, hipStream_t st) {
+int skinny(SkinnyArgs a, hipStream_t st) {
   using K = Skinny<DUAL, FEW>;
   static std::atomic<bool> attr{false};  // setting it twice from two threads is harmless
   if (!attr) {
@@ -179,7 +180,10 @@ int skinny(const SkinnyArgs &a, hipStream_t st) {
     attr = true;
   }
   const int tiles = kx_cdiv(a.rows, K::ROWS), cus = std::max(1, kx_device_cus());
-  hipLaunchKernelGGL((skinny_staged_k<DUAL, FEW>), dim3(2 * tiles > cus ? std::min(cus, a.rows) : tiles), dim3(512), K::LDS, st, a);
+  const int even = std::min(cus, a.rows), grid = 2 * tiles > cus ? even : tiles;
+  a.share = grid == even ? a.rows / even : K::ROWS;
+  a.extra = grid == even ? a.rows % even : 0;
+  hipLaunchKernelGGL((skinny_staged_k<DUAL, FEW>), dim3(grid), dim3(512), K::LDS, st, a);
   KX_LAUNCH_CHECK();
   return KX_OK;
 }
