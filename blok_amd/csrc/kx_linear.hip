@@ -4,7 +4,7 @@
 // decoder whose shapes come from its config.json: nothing here asks for a multiple of 512 columns.
 //
 // lin_gemv_k (up to 4 tokens): a workgroup of 8 waves builds the activation rows in LDS (kx_rows.h: residual streams
-// and norm, or the gated read-out of the delta rule) while the first weight loads are under way, then every wave
+// and norm, or the gated read-out of the delta rule; of several tokens a launch in front does) while the first weight loads are under way, then every wave
 // streams two rows of the matrix at a time, 8 columns per lane and load, the next pieces in flight while the present
 // ones are multiplied; the epilogue stores the product, forms the gated activation of a (gate, up) pair, or updates
 // all residual streams of the row.
@@ -419,13 +419,15 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) lin_gemm_k(Kx
 // through four Rapitar layers of width 2048 13.55 -> 12.40 ms.
 constexpr int NARROW_ROWS = 64, NARROW_MAX_SPLITS = 16;
 template <int MI, int EPI, bool GROUP>
-__global__ void __launch_bounds__(512, MI == 1 ? 4 : 2) lin_narrow_k(KxLinArgs a, KxExpertArgs e, const uint16_t *__restrict__ x, int x_ld, int splits) {
+__global__ void __launch_bounds__(512, MI == 1 ? 4 : 2) lin_narrow_k(KxLinArgs a, KxExpertArgs e, const uint16_t *__restrict__ x, int x_ld, int splits, bool once, int share, int extra) {
   constexpr int ROWS = NARROW_ROWS + 32 * MI, HALF = ROWS * 128, STAGE = 2 * HALF, NS = MI == 1 ? 3 : 4, CPW = 2 + MI;
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   __shared__ int last_one;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lr = lane & 31, h = lane >> 5, n0 = blockIdx.x * NARROW_ROWS, part = GROUP ? 0 : blockIdx.y;
+  const int lr = lane & 31, h = lane >> 5, part = GROUP ? 0 : blockIdx.y;
+  // share rows each, the first `extra` workgroups one more (divisions in 64 bits here cost a workgroup 0.5 us)
+  const int bx = blockIdx.x, n0 = bx * share + min(bx, extra), n1 = min(n0 + share + (bx < extra), a.m.rows);
   Tile tl;
   if (!tile_of<GROUP>(a, e, 0, tl)) return;
   const int m0 = tl.m0, tokens = tl.end - m0;
@@ -443,7 +445,7 @@ __global__ void __launch_bounds__(512, MI == 1 ? 4 : 2) lin_narrow_k(KxLinArgs a
     if (i < 2) {
       const int q = wave * 2 + i, row = (q & 7) * 8 + sub;
       half[i] = q >> 3;
-      src[i] = (const uint16_t *)a.m.w + tl.w + (size_t)min(n0 + row, a.m.rows - 1) * a.m.ld + ((lane & 7) ^ sub) * 8;
+      src[i] = (const uint16_t *)a.m.w + tl.w + (size_t)min(n0 + row, n1 - 1) * a.m.ld + ((lane & 7) ^ sub) * 8;
       dst[i] = half[i] * HALF + (q & 7) * 1024;
     } else {
       const int q = min(wave + 8 * (i - 2), 2 * groups - 1);
@@ -459,7 +461,7 @@ __global__ void __launch_bounds__(512, MI == 1 ? 4 : 2) lin_narrow_k(KxLinArgs a
     for (int i = 0; i < CPW; ++i) {
       const uint16_t *const from = src[i] + min(2 * b + half[i], nh - 1) * 64;
       const uint32_t to = __builtin_amdgcn_readfirstlane(st + dst[i]);
-      if (i < 2) kx_copy16_to_lds_once(from, to);  // the matrix
+      if (i < 2 && once) kx_copy16_to_lds_once(from, to);  // the matrix
       else kx_copy16_to_lds(from, to);
     }
   };
@@ -532,7 +534,7 @@ __global__ void __launch_bounds__(512, MI == 1 ? 4 : 2) lin_narrow_k(KxLinArgs a
   } else {
     for (int i = threadIdx.x; i < outs; i += 512) {
       const int t = m0 + (i >> 6), r = n0 + (i & 63);
-      if (r >= a.m.rows) continue;
+      if (r >= n1) continue;
       Streams<EPI> res;
       if constexpr (EPI >= KX_LIN_STREAMS) res.load(a, Streams<EPI>::of(a, t), r);
       const float y = value(i >> 6, i & 63);
@@ -616,6 +618,19 @@ int narrow_splits(const KxLinArgs &a, int groups) {
   s = (int)std::min<size_t>(s, a.part_floats / ((size_t)groups * NARROW_ROWS * a.tokens));
   return s < 2 || groups > a.arrivals ? 1 : s;
 }
+// Workgroups with equal shares of the rows, one per CU or as many as fill whole rounds of two, where groups of 64 rows would leave CUs with one beside others
+// with two, or with none: 8 tokens, 17472 x 2048, 273 groups 21.8 us, 512 workgroups 18.9.  The columns' parts, and with them the sums, stay as they are.
+// Not for matrices for less than half of the CUs, nor for parts of less than 1024 columns, where starts and ends of the workgroups count for more than
+// their rows (9344 x 2048 in three parts 12.2 and 12.3; models of 1024 columns 1 % longer).
+int narrow_even(const KxLinArgs &a, int groups, int splits) {
+  const long cus = std::max(1, kx_device_cus()), all = (long)groups * splits;
+  if (2 * all <= cus || a.m.ld < 1024 * splits) return groups;
+  const long target = all <= cus ? cus : (all + 2 * cus - 1) / (2 * cus) * 2 * cus;
+  const int even = (int)std::min<long>(target / splits, a.m.rows);
+  if (even <= groups || (splits > 1 && (even > a.arrivals || (size_t)even * splits * NARROW_ROWS * a.tokens > a.part_floats))) return groups;
+  return even;
+}
+constexpr size_t ONCE = (size_t)24 << 20, ONCE_EXPERTS = (size_t)192 << 20;  // bytes of a matrix, of all experts' ones
 template <int EPI, bool GROUP>
 int narrow_launch(const KxLinArgs &a, const KxExpertArgs &e, const uint16_t *x, int x_ld, hipStream_t st) {
   static std::atomic<bool> attr{false};
@@ -625,11 +640,21 @@ int narrow_launch(const KxLinArgs &a, const KxExpertArgs &e, const uint16_t *x, 
     if constexpr (!GROUP) KX_HIP(hipFuncSetAttribute((const void *)lin_narrow_k<2, EPI, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds[1]));
     attr = true;
   }
-  const int groups = kx_cdiv(a.m.rows, NARROW_ROWS), splits = GROUP ? 1 : narrow_splits(a, groups);
+  int groups = kx_cdiv(a.m.rows, NARROW_ROWS);
+  const int splits = GROUP ? 1 : narrow_splits(a, groups);
+  int share = NARROW_ROWS, extra = 0;  // rows of a workgroup
+  if (!GROUP && EPI != KX_LIN_GLU && a.n_var == 1) {
+    const int even = narrow_even(a, groups, splits);
+    if (even > groups) groups = even, share = a.m.rows / even, extra = a.m.rows % even;
+  }
   const dim3 grid(groups, GROUP ? e.max_tiles : splits);
-  if constexpr (GROUP) hipLaunchKernelGGL((lin_narrow_k<1, EPI, true>), grid, dim3(512), lds[0], st, a, e, x, x_ld, splits);
-  else if (a.tokens <= 32) hipLaunchKernelGGL((lin_narrow_k<1, EPI, false>), grid, dim3(512), lds[0], st, a, e, x, x_ld, splits);
-  else hipLaunchKernelGGL((lin_narrow_k<2, EPI, false>), grid, dim3(512), lds[1], st, a, e, x, x_ld, splits);
+  // Nontemporal copies leave nothing for the next step, and the weights of small models lie in the memory-side cache of 256 MB from step to step: they are for matrices
+  // that a model which fits there does not have (copied so, models of 1024 columns took 2 to 5 % longer a step).
+  const size_t bytes = (GROUP ? (size_t)e.experts * e.stride : (size_t)a.m.rows * a.m.ld) * 2;
+  const bool once = bytes >= (GROUP ? ONCE_EXPERTS : ONCE);
+  if constexpr (GROUP) hipLaunchKernelGGL((lin_narrow_k<1, EPI, true>), grid, dim3(512), lds[0], st, a, e, x, x_ld, splits, once, share, extra);
+  else if (a.tokens <= 32) hipLaunchKernelGGL((lin_narrow_k<1, EPI, false>), grid, dim3(512), lds[0], st, a, e, x, x_ld, splits, once, share, extra);
+  else hipLaunchKernelGGL((lin_narrow_k<2, EPI, false>), grid, dim3(512), lds[1], st, a, e, x, x_ld, splits, once, share, extra);
   KX_LAUNCH_CHECK();
   return KX_OK;
 }

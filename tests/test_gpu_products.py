@@ -182,3 +182,31 @@ def test_rows_in_a_launch_of_their_own(kxlib, tokens, cols, streams, groups, hea
             check(kxlib.kx_sync(None))
             got.append(out.to_numpy(np.float32, (tokens, rows)))
         assert np.isfinite(got[0]).all() and (got[0] != 7.0).any() and np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32)), form
+
+
+@pytest.mark.parametrize("tokens", [5, 33, 64])
+@pytest.mark.parametrize("rows, cols", [(8192, 1024), (8193, 1024), (8256, 1088), (16387, 1600), (16448, 2100), (33001, 1024), (40000, 1030)])
+def test_few_tokens_on_workgroups_with_equal_shares(kxlib, rows, cols, tokens):
+    """Rows for half of the CUs and more, one column part: one workgroup per CU, rounds of two per CU, shares of 32 to 64 rows that do not come out even, stored and
+    through two streams.  32-bit sums of bf16 products."""
+    r = np.random.default_rng(rows)
+    w, x = KC.bf16(r.standard_normal((rows, cols)) * cols ** -0.5), KC.bf16(r.standard_normal((tokens, cols)))
+    y = x @ w.T
+    dw, ld = _matrix(w, 0)
+    dx, scratch = _matrix(x, 0)[0], DevBuf(64)
+    base = dict(f32=0, tokens=tokens, rows=rows, cols=cols, ld=ld, row_kind=0, groups=1, d_w=dw.ptr, d_x=dx.ptr, x_ld=ld)
+    out = dev(np.full((tokens, rows + 1), 7.0, np.float32))
+    a = KxLinearArgs(**base, streams=1, epilogue=0, out_ld=rows + 1)
+    a.d_out = out.ptr
+    check(kxlib.kx_linear_run(C.byref(a), scratch.ptr, None))
+    check(kxlib.kx_sync(None))
+    got = out.to_numpy(np.float32, (tokens, rows + 1))
+    assert rel(got[:, :rows], y) < 1e-5 and (got[:, rows:] == 7.0).all()
+    s0 = r.standard_normal((tokens, 2, rows)).astype(np.float32)
+    mix, ow = r.standard_normal((2, 2)).astype(np.float32), r.standard_normal(2).astype(np.float32)
+    ds, dm, do = dev(s0), dev(mix), dev(ow)
+    a = KxLinearArgs(**base, streams=2, epilogue=2, d_mix=dm.ptr, d_outw=do.ptr)
+    a.d_out = ds.ptr
+    check(kxlib.kx_linear_run(C.byref(a), scratch.ptr, None))
+    check(kxlib.kx_sync(None))
+    assert rel(ds.to_numpy(np.float32, s0.shape), K.hyper_write(s0.transpose(1, 0, 2).astype(np.float64), mix, ow, y.astype(np.float64)).transpose(1, 0, 2)) < 1e-5
