@@ -20,6 +20,7 @@
 #include "kx_common.h"
 #include "kx_dense.h"
 #include "kx_gemv_body.h"
+#include "kx_gemv_chunks.h"
 #include "kx_math.h"
 #include "kx_route.h"
 #include "kx_wave.h"
@@ -316,14 +317,12 @@ static int gemv_launch_impl(int epi, KxGemvArgs a, hipStream_t st, const KxRoute
   int CR = gemv_plan(epi, a, ri, 4);
   if (CR < 0) return KX_ERR_ARG;
   // One token and more chunks than workgroups run at once: that many workgroups, which go on to their next chunk with its weights on their way, and
-  // chunks of as many tiles as let the one with the most rows have the fewest.
+  // chunks of as many tiles as make the launch shortest (kx_gemv_chunks.h).
   int at_once = 4096;
   if (a.tokens == 1 && !a.row_block) {
     const int slots = std::max(1, 1024 / (a.nw * a.rs * 64)) * std::max(1, kx_device_cus()), rt = a.rs * ri;  // 128 registers: 16 waves per CU
     if (kx_cdiv(a.rows, CR) > slots) {
-      auto most = [&](int nt) { return kx_cdiv(kx_cdiv(a.rows, rt * nt), slots) * nt; };  // tiles of a workgroup
-      for (int nt = a.nt - 1; nt >= 1; --nt)
-        if (most(nt) < most(a.nt)) a.nt = nt;
+      a.nt = kxgemv::chunk_tiles(a.rows, rt, a.nt, slots);
       CR = rt * a.nt;
       at_once = slots;
     }
