@@ -618,18 +618,6 @@ int narrow_splits(const KxLinArgs &a, int groups) {
   s = (int)std::min<size_t>(s, a.part_floats / ((size_t)groups * NARROW_ROWS * a.tokens));
   return s < 2 || groups > a.arrivals ? 1 : s;
 }
-// Workgroups with equal shares of the rows, one per CU or as many as fill whole rounds of two, where groups of 64 rows would leave CUs with one beside others
-// with two, or with none: 8 tokens, 17472 x 2048, 273 groups 21.8 us, 512 workgroups 18.9.  The columns' parts, and with them the sums, stay as they are.
-// Not for matrices for less than half of the CUs, nor for parts of less than 1024 columns, where starts and ends of the workgroups count for more than
-// their rows (9344 x 2048 in three parts 12.2 and 12.3; models of 1024 columns 1 % longer).
-int narrow_even(const KxLinArgs &a, int groups, int splits) {
-  const long cus = std::max(1, kx_device_cus()), all = (long)groups * splits;
-  if (2 * all <= cus || a.m.ld < 1024 * splits) return groups;
-  const long target = all <= cus ? cus : (all + 2 * cus - 1) / (2 * cus) * 2 * cus;
-  const int even = (int)std::min<long>(target / splits, a.m.rows);
-  if (even <= groups || (splits > 1 && (even > a.arrivals || (size_t)even * splits * NARROW_ROWS * a.tokens > a.part_floats))) return groups;
-  return even;
-}
 constexpr size_t ONCE = (size_t)24 << 20, ONCE_EXPERTS = (size_t)192 << 20;  // bytes of a matrix, of all experts' ones
 template <int EPI, bool GROUP>
 int narrow_launch(const KxLinArgs &a, const KxExpertArgs &e, const uint16_t *x, int x_ld, hipStream_t st) {
@@ -643,8 +631,10 @@ int narrow_launch(const KxLinArgs &a, const KxExpertArgs &e, const uint16_t *x, 
   int groups = kx_cdiv(a.m.rows, NARROW_ROWS);
   const int splits = GROUP ? 1 : narrow_splits(a, groups);
   int share = NARROW_ROWS, extra = 0;  // rows of a workgroup
-  if (!GROUP && EPI != KX_LIN_GLU && a.n_var == 1) {
-    const int even = narrow_even(a, groups, splits);
+  if (!GROUP && EPI != KX_LIN_GLU && a.n_var == 1) {  // GLU: blocks of gate and up; variants begin at multiples of 128 rows
+    const bool parts = splits > 1;
+    const int even = kxtile::even_groups(a.m.rows, a.m.ld, groups, splits, parts ? a.part_floats / ((size_t)NARROW_ROWS * a.tokens) : (size_t)-1, parts ? a.arrivals : a.m.rows,
+                                         std::max(1, kx_device_cus()));
     if (even > groups) groups = even, share = a.m.rows / even, extra = a.m.rows % even;
   }
   const dim3 grid(groups, GROUP ? e.max_tiles : splits);

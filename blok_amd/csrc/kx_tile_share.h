@@ -154,4 +154,20 @@ inline Share choose_single(int tokens, int rows, int blocks, size_t part_floats,
   return share(tiles, cus, (int)most, room, arrivals, time, &best, tiles > arrivals ? 1 : (int)least);
 }
 
+// Workgroups, each with all tokens (5 to 64), an equal share of the rows and one of `parts` parts of the columns, for a product whose rows make `groups` groups of
+// 64: as many as fill whole rounds of one per CU.  Groups of 64 rows leave CUs with one beside others with two, or with none.  us, groups of 64 / shares:
+// 17472 x 2048, 5 tokens 22.2 / 18.7 (273 to 512), 64 tokens 30.9 / 28.1; 9344 x 2048, 64 tokens 16.1 / 15.1 (146 to 256); 40000 x 2048 38.7 / 37.4 and 50.3 /
+// 50.0 (625 to 768); 11003 x 2048 in two parts, 32 tokens 17.4 / 15.6 (344 to 512).  A workgroup copies 64 rows' places whatever its share is, so more
+// rounds than that take longer, also where a CU holds two (up to 32 tokens): 40000 x 1024 as 1024 workgroups 23.3 at 32 tokens and 35.9 at 64, 20.9 and
+// 30.2 as 768; 33000 x 2048 52.6 and 46.2.  The columns' parts, and with them the sums, stay as they are.
+// Not for matrices for less than half of the CUs, nor for parts of less than 1024 columns, where starts and ends of the workgroups count for more than
+// their rows (9344 x 2048 in three parts 12.2 and 12.3; models of 1024 columns 1 % longer).
+// room: workgroups whose sums the scratch of the parts holds; arrivals: counters of groups.
+inline int even_groups(int rows, int cols, int groups, int parts, size_t room, int arrivals, int cus) {
+  const long all = (long)groups * parts;
+  if (2 * all <= cus || cols < 1024 * parts) return groups;
+  const long even = (all + cus - 1) / cus * cus / parts, n = even < rows ? even : rows;
+  return n <= groups || n > arrivals || (size_t)(n * parts) > room ? groups : (int)n;
+}
+
 }  // namespace kxtile
