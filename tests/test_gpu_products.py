@@ -210,3 +210,31 @@ def test_few_tokens_on_workgroups_with_equal_shares(kxlib, rows, cols, tokens):
     check(kxlib.kx_linear_run(C.byref(a), scratch.ptr, None))
     check(kxlib.kx_sync(None))
     assert rel(ds.to_numpy(np.float32, s0.shape), K.hyper_write(s0.transpose(1, 0, 2).astype(np.float64), mix, ow, y.astype(np.float64)).transpose(1, 0, 2)) < 1e-5
+
+
+@pytest.mark.parametrize("vocab, width", [(11003, 2048), (15003, 2048), (7003, 4096), (4003, 8192)], ids=["two parts of 256 shares", "nearly whole groups", "four of 128", "eight of 64"])
+def test_equal_shares_with_parts_of_the_columns(kxlib, strict, tmp_path, monkeypatch, vocab, width):
+    """A head whose rows come out uneven on the shares, with its columns in parts as well: partial sums and counters of arrivals are numbered by shares.  The layer
+    adds nothing, so the head's rows are the normed embeddings and every logit is compared with its 64-bit sum: a rounding of a row's element to the other bf16
+    value moves a logit by about 1e-4 of their root mean square, sums of 32 bits by less.  The same bits whoever comes last, and in both forms of the hand-over."""
+    cfg = KC.config([KC.delta(heads=1, kv_heads=1, dim=8, vdim=8, ff=None)], width=width, vocab=vocab, streams=1, groups=1)
+    w = KC.weights(cfg, vocab)
+    w["l0.mix.o"][:] = 0.0
+    for k in ("in", "out", "mix"):
+        w["l0.hc1." + k][:] = 1.0
+    path, batches = KC.write(tmp_path, cfg, w), (5, 32, 33, 64)
+    ids = KC.tokens(cfg, 64, 7)
+    x = w["embed"][ids]
+    x = KC.bf16(x / np.sqrt((x * x).mean(-1, keepdims=True) + 1e-5) * w["final.norm"]).astype(np.float64)
+    want = x @ w["head"].T
+    got = []
+    for lib in (kxlib, strict):
+        monkeypatch.setattr(KC, "kx", lambda lib=lib: lib)
+        with KC.Model(path, "bfloat16", batch=64, context=4) as m:
+            for b in batches + batches:
+                m.restart(b)
+                got.append(m.extend(ids[:b, None])[0])
+    for i, y in enumerate(got):
+        b = batches[i % 4]
+        assert np.abs(y - want[:b]).max() < 2e-3 * np.sqrt((want * want).mean()), (b, i)
+        assert np.array_equal(y.view(np.uint32), got[i % 4].view(np.uint32)), (b, i)
