@@ -33,6 +33,7 @@
 #include "kx_dense.h"
 #include "kx_math.h"
 #include "kx_mla.h"
+#include "kx_read_once.h"
 #include "kx_wave.h"
 
 // ---- host: YaRN frequencies, rope table, score scale ---------------------------------
@@ -219,6 +220,7 @@ struct MlaArgs {
                           // several positions of n sequences): z = i * n + b is position i of sequence b; it reads
                           // cache block b and attends seq - (grid z / n - 1) + i positions, the last position all `seq`
   size_t seq_stride;      // elements between sequences in the cache
+  bool once;              // rows are read once and copied nontemporally
   float rs, mscale;
 };
 
@@ -415,7 +417,8 @@ __device__ __forceinline__ uint2 mm_read_tr(uint32_t addr) {
   return __builtin_bit_cast(uint2, v);
 }
 // the copies into the tile ring and the fence-free barrier: kx_lds_copy.h (this kernel waits for a tile itself,
-// where it needs it: wait_tile below).  Nontemporal where one position reads the rows: 16 sequences of 32768 positions 131.8 -> 125.9 us.
+// where it needs it: wait_tile below).  Nontemporal where one position reads the rows of a cache that is large enough (kx_read_once.h): 16 sequences of 32768
+// positions 135.9 -> 129.4 us.
 __device__ __forceinline__ void mm_copy16_to_lds(const void *src, uint32_t lds_base, bool once) {
   if (once) kx_copy16_to_lds_once(src, lds_base);
   else kx_copy16_to_lds(src, lds_base);
@@ -454,7 +457,6 @@ __global__ void __launch_bounds__(512, 1) mla_partial_mfma_k(MlaArgs a) {
   // the sequence repeat its last row.  The lane's places inside a tile do not change from tile to tile: the nine
   // source offsets are kept, and only a tile that reaches past the sequence goes through the row clamp.
   const int cw = wave & 3;
-  const bool once = !a.seqs || (int)gridDim.z == a.seqs;  // positions of a prompt step read the same rows
   int c_off[9];   // elements from the tile's first row
   int c_row[9];
 #pragma unroll
@@ -471,12 +473,12 @@ __global__ void __launch_bounds__(512, 1) mla_partial_mfma_k(MlaArgs a) {
     const uint32_t dst = lds0 + (t % MM_RING) * MM_NAT + cw * 1024;
     if (row0 + MM_T <= seq) {
 #pragma unroll
-      for (int u = 0; u < 9; ++u) mm_copy16_to_lds(src + c_off[u], dst + u * 4096, once);
+      for (int u = 0; u < 9; ++u) mm_copy16_to_lds(src + c_off[u], dst + u * 4096, a.once);
     } else {
 #pragma unroll
       for (int u = 0; u < 9; ++u) {
         const int back = max(row0 + c_row[u] - (seq - 1), 0);  // rows past the last one
-        mm_copy16_to_lds(src + c_off[u] - back * MLA_KVA, dst + u * 4096, once);
+        mm_copy16_to_lds(src + c_off[u] - back * MLA_KVA, dst + u * 4096, a.once);
       }
     }
   };
@@ -833,7 +835,7 @@ int kx_mla_partials_launch(const kx_config *c, const uint16_t *cache, size_t seq
   // takes 190-360 us per layer at 32 sequences of 1100 positions)
   const bool use_mfma = kernel == KX_MLA_MATRIX_CORES || (kernel == KX_MLA_AUTO && c->heads == 64 && (seq >= 2048 || (batch >= 5 && seq >= 128)));
   MlaArgs a;
-  a.cache = cache; a.qabs = qabs; a.heads = c->heads; a.seq = seq; a.seq_stride = seq_stride; a.seqs = seqs;
+  a.once = false; a.cache = cache; a.qabs = qabs; a.heads = c->heads; a.seq = seq; a.seq_stride = seq_stride; a.seqs = seqs;
   a.span_tiles = use_mfma ? mfma_span_tiles(seq, batch) : kx_mla_span_tiles(seq);
   const int tiles = (seq + 63) / 64;
   a.spans = (tiles + a.span_tiles - 1) / a.span_tiles;
@@ -883,6 +885,7 @@ int kx_mla_partials_launch(const kx_config *c, const uint16_t *cache, size_t seq
       KX_HIP(hipFuncSetAttribute((const void *)mla_partial_mfma_k, hipFuncAttributeMaxDynamicSharedMemorySize, MM_LDS));
       mfma_attr = true;
     }
+    a.once = (!seqs || batch == seqs) && kxonce::latent((size_t)batch * seq * MLA_KVA * 2);  // positions of a prompt step read the same rows
     hipLaunchKernelGGL(mla_partial_mfma_k, dim3(a.spans, 1, batch), dim3(512), MM_LDS, st, a);
     KX_LAUNCH_CHECK();
     out->pm = a.pm; out->pz = a.pz; out->po = a.po; out->spans = a.spans;
