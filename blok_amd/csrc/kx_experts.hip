@@ -173,6 +173,7 @@ int kx_expert_ff_launch(bool f32, const KxExpertFf &f, int tokens, hipStream_t s
   KxLinArgs down;
   down.m = f.down;
   down.tokens = tokens;
+  down.model_bytes = f.gu.model_bytes;
   down.row.cols = f.down.cols;
   down.out = f.y;
   down.out_ld = f.down.rows;

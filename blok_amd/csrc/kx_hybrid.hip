@@ -119,6 +119,7 @@ struct HybridModel : kx_model {
   int fill(const KxTensorMap &files, const kx_open_options &o);
   int pack(const Slot &s, const void *src, bool src_f32);
   int logits_of(const float *x, const int *map, int n, float *d_out);
+  size_t matrix_bytes = 0;  // of the weights that a step goes through
   void split(KxLinArgs &g) const;
   int product(KxLinArgs &g, void *row_buf) const;
 };
@@ -383,6 +384,7 @@ size_t HybridModel::layout(char *base) {
   part_of(head, 0, 0, "head", c.vocab, W, -1, sg);
   for (auto &t : turns) t.second.first = (float2 *)at((size_t)max_context * (t.first.first / 2) * sizeof(float2));
   weight_bytes = p.total;
+  matrix_bytes = weight_bytes - (size_t)embed.rows * embed.ld * es;
 
   for (size_t i = 0; i < c.layers.size(); ++i) {
     const KxHybridLayer &l = c.layers[i];
@@ -528,6 +530,7 @@ int HybridModel::restart(int batch_) {
 void HybridModel::split(KxLinArgs &g) const {
   g.part = split_part; g.part_floats = split_floats;
   g.arrived = split_arrived; g.arrivals = SPLIT_GROUPS;
+  g.model_bytes = matrix_bytes;
 }
 int HybridModel::product(KxLinArgs &g, void *row_buf) const {
   split(g);
@@ -667,7 +670,7 @@ int HybridModel::step(const uint32_t *d_ids, bool sample, int C) {
     if (experts) {
       KxExpertFf f;
       read(f.gu, w.gu, w.norm1, w.hc[0]);
-      f.gu.limit = l.limit; f.gu.alpha = l.alpha; f.gu.bias = l.bias;
+      f.gu.limit = l.limit; f.gu.alpha = l.alpha; f.gu.bias = l.bias; f.gu.model_bytes = matrix_bytes;
       split(out);
       f.out = out;
       f.down = w.down; f.gu_stride = w.gu_stride; f.down_stride = w.down_stride;

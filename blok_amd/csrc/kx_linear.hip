@@ -21,6 +21,7 @@
 #include "kx_experts.h"
 #include "kx_gemm_tile.h"
 #include "kx_linear.h"
+#include "kx_read_once.h"
 #include "kx_rows.h"
 
 namespace {
@@ -415,8 +416,7 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) lin_gemm_k(Kx
 // multiplies 16 columns of each half for row block w % 2, so that four waves hold sums of the same outputs, which meet in LDS.
 // With several parts the sums go to memory and the workgroup that arrives last (kx_arrive.h) adds the parts in their order,
 // whoever it is, and runs the epilogue: results do not depend on timing.  Token rows past the last are never copied: what the
-// LDS holds there only feeds sums that are not stored.  The matrix is copied nontemporally, whole lines of it (kx_lds_copy.h): 24 steps of 8 sequences
-// through four Rapitar layers of width 2048 13.55 -> 12.40 ms.
+// LDS holds there only feeds sums that are not stored.  Large matrices are copied nontemporally, whole lines of them (kx_read_once.h).
 constexpr int NARROW_ROWS = 64, NARROW_MAX_SPLITS = 16;
 template <int MI, int EPI, bool GROUP>
 __global__ void __launch_bounds__(512, MI == 1 ? 4 : 2) lin_narrow_k(KxLinArgs a, KxExpertArgs e, const uint16_t *__restrict__ x, int x_ld, int splits, bool once, int share, int extra) {
@@ -618,7 +618,6 @@ int narrow_splits(const KxLinArgs &a, int groups) {
   s = (int)std::min<size_t>(s, a.part_floats / ((size_t)groups * NARROW_ROWS * a.tokens));
   return s < 2 || groups > a.arrivals ? 1 : s;
 }
-constexpr size_t ONCE = (size_t)24 << 20, ONCE_EXPERTS = (size_t)192 << 20;  // bytes of a matrix, of all experts' ones
 template <int EPI, bool GROUP>
 int narrow_launch(const KxLinArgs &a, const KxExpertArgs &e, const uint16_t *x, int x_ld, hipStream_t st) {
   static std::atomic<bool> attr{false};
@@ -638,10 +637,7 @@ int narrow_launch(const KxLinArgs &a, const KxExpertArgs &e, const uint16_t *x, 
     if (even > groups) groups = even, share = a.m.rows / even, extra = a.m.rows % even;
   }
   const dim3 grid(groups, GROUP ? e.max_tiles : splits);
-  // Nontemporal copies leave nothing for the next step, and the weights of small models lie in the memory-side cache of 256 MB from step to step: they are for matrices
-  // that a model which fits there does not have (copied so, models of 1024 columns took 2 to 5 % longer a step).
-  const size_t bytes = (GROUP ? (size_t)e.experts * e.stride : (size_t)a.m.rows * a.m.ld) * 2;
-  const bool once = bytes >= (GROUP ? ONCE_EXPERTS : ONCE);
+  const bool once = GROUP ? kxonce::experts((size_t)e.experts * e.stride * 2, a.model_bytes) : kxonce::matrix((size_t)a.m.rows * a.m.ld * 2, a.model_bytes);
   if constexpr (GROUP) hipLaunchKernelGGL((lin_narrow_k<1, EPI, true>), grid, dim3(512), lds[0], st, a, e, x, x_ld, splits, once, share, extra);
   else if (a.tokens <= 32) hipLaunchKernelGGL((lin_narrow_k<1, EPI, false>), grid, dim3(512), lds[0], st, a, e, x, x_ld, splits, once, share, extra);
   else hipLaunchKernelGGL((lin_narrow_k<2, EPI, false>), grid, dim3(512), lds[1], st, a, e, x, x_ld, splits, once, share, extra);

@@ -92,6 +92,7 @@ struct KimiModel : kx_model {
   int *route_distinct = nullptr;   // [n_layers] distinct experts of the last step
   float *route_history = nullptr;  // record level 2: router logits of every position, [n_layers][max_context][max_batch][experts]
   kx_moe_workspace *moe_ws = nullptr;
+  size_t matrix_bytes = 0;  // of the weights that a step goes through: all but the embedding and the rope table
   uint32_t exact = 0;     // kx_model_set_exact: KX_EXACT_* parts that keep the bit-reproducible kernels at every batch size
 
   ~KimiModel() override;
@@ -322,7 +323,7 @@ int KimiModel::step(const uint32_t *d_ids, bool sample, int C) {
     if (g.tokens <= 32) {  // one tile: the kernel built for it
       bool done = false;
       int rc2 = kx_skinny_gemm_launch(dual, g.w0, dual ? g.w1 : nullptr, g.x, g.x_stride, g.out, g.out_stride, mode, g.tokens, g.rows,
-                                      g.cols, &done, st);
+                                      g.cols, m->matrix_bytes, &done, st);
       if (rc2 || done) return rc2;
     }
     KxDenseArgs d = split;
@@ -537,6 +538,7 @@ static int model_new(const kx_config *cfg, const char *who, KimiModel **out) {
   m->c = *cfg;
   m->n_layers = cfg->n_layers; m->hidden = cfg->hidden; m->vocab = cfg->vocab; m->max_batch = cfg->max_batch;
   m->max_context = cfg->max_context; m->eos_id = cfg->eos_id; m->step_tokens = STEP_TOKENS;
+  m->matrix_bytes = p.weights - ((size_t)cfg->vocab * cfg->hidden + (size_t)cfg->max_context * cfg->qk_rope) * 2;
   m->weight_bytes = p.weights; m->cache_bytes = p.cache; m->scratch_bytes = p.scratch;
   hipError_t e = hipMalloc((void **)&m->arena, p.total);
   if (e != hipSuccess) {

@@ -284,11 +284,12 @@ static int moe_layer_body(const kx_config *c, const kx_moe_weights *w, kx_moe_wo
     KX_HIP(hipEventRecord(ws->fork, st));
     KX_HIP(hipStreamWaitEvent(ws->side, ws->fork, 0));
     forked = true;
-    if ((rc = kx_skinny_gemm_launch(true, s.w0, s.w1, s.x, s.x_stride, s.out, s.out_stride, KX_GG_BF16, tokens, s.rows, s.cols,
+    const size_t layer_bytes = ((size_t)E * c->moe_inter * 27 / 16 + (size_t)c->shared_inter * 6 + (size_t)E * 2) * H;  // 4 bits and a scale of 32; the model's are more
+    if ((rc = kx_skinny_gemm_launch(true, s.w0, s.w1, s.x, s.x_stride, s.out, s.out_stride, KX_GG_BF16, tokens, s.rows, s.cols, layer_bytes,
                                     &shared_up_done, ws->side))) return rc;
     if (shared_up_done &&
         (rc = kx_skinny_gemm_launch(false, (const uint16_t *)w->d_shared_down, nullptr, ws->smid, c->shared_inter, ws->sy, H, KX_GG_BF16,
-                                    tokens, H, c->shared_inter, &shared_down_done, ws->side))) return rc;
+                                    tokens, H, c->shared_inter, layer_bytes, &shared_down_done, ws->side))) return rc;
   }
   bool paired = (flags & KX_MOE_HEAD_DONE) && tokens == 1 && norm_w && !mm;  // the caller's launch has done this step
   if (!paired && (rc = kx_gemv_pair_route_launch(s, g, (const float *)w->d_router_bias, ws->ids, ws->weights, E, K, c->routed_scale,

@@ -20,7 +20,7 @@
 // banks.  Blocks go through a ring of 5 stages (4 with more than 16 tokens), four (three) blocks in flight behind the one being
 // multiplied; each wave issues its share of a block's copies, waits for its own by count (they complete in order),
 // and one barrier per block makes every wave's copies visible and the stage that is overwritten next free.  Wave w
-// multiplies pieces 4w .. 4w+3 of the block.  The matrix is copied nontemporally (kx_lds_copy.h).
+// multiplies pieces 4w .. 4w+3 of the block.  Matrices of large models are copied nontemporally (kx_read_once.h).
 // LDS leaves a CU one workgroup.  Where there are tiles for half of the CUs and more, every CU has one and an equal share of the rows, whose tiles follow each other
 // through the ring: the next tile's blocks are on their way while a tile's sums are added.  A workgroup per 32 rows instead was 224 for the 7168
 // rows of a down projection and, two matrices at a time, two rounds and a quarter for 18432 rows.  12 tokens, 2 x 18432 x 7168 91.5 us so, 79.3 now; 7168 x
@@ -36,6 +36,7 @@
 #include "kx_lds_copy.h"
 #include "kx_dense.h"
 #include "kx_math.h"
+#include "kx_read_once.h"
 
 namespace {
 
@@ -54,7 +55,7 @@ template <int N>
 __device__ __forceinline__ void sk_wait_copies() { kx_wait_copies<N>(); }
 __device__ __forceinline__ void sk_barrier() { kx_lds_barrier(); }
 
-// FEW: up to 16 tokens, half the copies of tokens and a stage more.  DUAL: a tile is 16 rows of each matrix.
+// FEW: up to 16 tokens, half the copies of tokens and a stage more.  DUAL: a tile is 16 rows of each matrix.  ONCE (of the kernel): matrices are copied nontemporally.
 template <bool DUAL, bool FEW>
 struct Skinny {
   static constexpr int NS = FEW ? 5 : 4;             // stages
@@ -64,7 +65,7 @@ struct Skinny {
   static constexpr size_t LDS = PART + 8 * 16 * 32 * sizeof(float);  // the ring, and the waves' sums of 16 tokens
 };
 
-template <bool DUAL, bool FEW>
+template <bool DUAL, bool FEW, bool ONCE>
 __global__ void __launch_bounds__(512) skinny_staged_k(SkinnyArgs a) {
   using K = Skinny<DUAL, FEW>;
   constexpr int NS = K::NS, CPW = K::CPW, ROWS = K::ROWS;
@@ -95,7 +96,12 @@ __global__ void __launch_bounds__(512) skinny_staged_k(SkinnyArgs a) {
   auto copy_next = [&]() {
     const uint32_t st = lds0 + (uint32_t)copy_stage * K::STAGE + wave * 1024;
 #pragma unroll
-    for (int u = 0; u < 2; ++u) kx_copy16_to_lds_once(wsrc[u] + copy_block * 256, __builtin_amdgcn_readfirstlane(st + u * 8192));
+    for (int u = 0; u < 2; ++u) {
+      const uint16_t *const from = wsrc[u] + copy_block * 256;
+      const uint32_t to = __builtin_amdgcn_readfirstlane(st + u * 8192);
+      if constexpr (ONCE) kx_copy16_to_lds_once(from, to);
+      else kx_copy16_to_lds(from, to);
+    }
 #pragma unroll
     for (int u = 0; u < K::XC; ++u) kx_copy16_to_lds(xsrc[u] + copy_block * 256, __builtin_amdgcn_readfirstlane(st + K::TILE + u * 8192));
     copy_stage = copy_stage == NS - 1 ? 0 : copy_stage + 1;
@@ -171,19 +177,19 @@ __global__ void __launch_bounds__(512) skinny_staged_k(SkinnyArgs a) {
   }
 }
 
-template <bool DUAL, bool FEW>
+template <bool DUAL, bool FEW, bool ONCE>
 int skinny(SkinnyArgs a, hipStream_t st) {
   using K = Skinny<DUAL, FEW>;
   static std::atomic<bool> attr{false};  // setting it twice from two threads is harmless
   if (!attr) {
-    KX_HIP(hipFuncSetAttribute((const void *)skinny_staged_k<DUAL, FEW>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)K::LDS));
+    KX_HIP(hipFuncSetAttribute((const void *)skinny_staged_k<DUAL, FEW, ONCE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)K::LDS));
     attr = true;
   }
   const int tiles = kx_cdiv(a.rows, K::ROWS), cus = std::max(1, kx_device_cus());
   const int even = std::min(cus, a.rows), grid = 2 * tiles > cus ? even : tiles;
   a.share = grid == even ? a.rows / even : K::ROWS;
   a.extra = grid == even ? a.rows % even : 0;
-  hipLaunchKernelGGL((skinny_staged_k<DUAL, FEW>), dim3(grid), dim3(512), K::LDS, st, a);
+  hipLaunchKernelGGL((skinny_staged_k<DUAL, FEW, ONCE>), dim3(grid), dim3(512), K::LDS, st, a);
   KX_LAUNCH_CHECK();
   return KX_OK;
 }
@@ -193,7 +199,7 @@ int skinny(SkinnyArgs a, hipStream_t st) {
 // One tile of up to 32 tokens against a bf16 matrix (two for SwiGLU).  Returns KX_OK with *done = false, having
 // launched nothing, when the shape is not the kernel's (cols not a multiple of 512, more than 32 tokens).
 int kx_skinny_gemm_launch(bool dual, const uint16_t *w0, const uint16_t *w1, const uint16_t *x, int x_stride, void *out,
-                          int out_stride, int out_mode, int tokens, int rows, int cols, bool *done, hipStream_t st) {
+                          int out_stride, int out_mode, int tokens, int rows, int cols, size_t model_bytes, bool *done, hipStream_t st) {
   *done = false;
   if (tokens < 1 || tokens > 32 || rows < 1 || cols < 512 || cols % 512 || x_stride % 8 || x_stride < cols || (dual && !w1)) return KX_OK;
   KX_REQUIRE(out_mode >= KX_GG_BF16 && out_mode <= KX_GG_RESID && !(dual && out_mode != KX_GG_BF16), "kx_skinny_gemm: out_mode=%d", out_mode);
@@ -201,7 +207,9 @@ int kx_skinny_gemm_launch(bool dual, const uint16_t *w0, const uint16_t *w1, con
   a.w0 = w0; a.w1 = w1; a.x = x; a.out = out; a.rows = rows; a.cols = cols; a.tokens = tokens; a.x_stride = x_stride;
   a.out_stride = out_stride; a.mode = out_mode;
   const bool few = tokens <= 16;
-  const int rc = dual ? few ? skinny<true, true>(a, st) : skinny<true, false>(a, st) : few ? skinny<false, true>(a, st) : skinny<false, false>(a, st);
+  int rc;
+  if (kxonce::layers(model_bytes)) rc = dual ? few ? skinny<true, true, true>(a, st) : skinny<true, false, true>(a, st) : few ? skinny<false, true, true>(a, st) : skinny<false, false, true>(a, st);
+  else rc = dual ? few ? skinny<true, true, false>(a, st) : skinny<true, false, false>(a, st) : few ? skinny<false, true, false>(a, st) : skinny<false, false, false>(a, st);
   *done = rc == KX_OK;
   return rc;
 }
