@@ -79,7 +79,7 @@ __global__ void __launch_bounds__(KX_MAX_EXPERTS) bucket_k(KxExpertArgs e, KxExp
     }
   const int slot0 = at - n, tile0 = tile_at - tiles;
   if (tid == KX_MAX_EXPERTS - 1) *s.n_tiles = tile_at;
-  for (int i = 0; i < tiles; ++i) s.tiles[tile0 + i] = make_int4(tid, slot0 + i * e.tile_slots, min(e.tile_slots, n - i * e.tile_slots), 0);
+  for (int i = 0; i < tiles; ++i) s.tiles[tile0 + i] = make_int4(tid, slot0 + i * e.tile_slots, min(e.tile_slots, n - i * e.tile_slots), tiles);
   count[tid] = slot0;
   __syncthreads();
   for (int p0 = 0; p0 < pairs; p0 += AT_ONCE) {

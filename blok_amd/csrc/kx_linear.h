@@ -109,7 +109,7 @@ struct KxExpertArgs {
   const void *mid = nullptr;
   int mid_ld = 0;
   // many tokens: (token, choice) pairs sorted by expert; tiles of consecutive ones, each of one expert
-  const int4 *tiles = nullptr;       // {expert, first slot, slots, -}
+  const int4 *tiles = nullptr;       // {expert, first slot, slots, tiles of the expert}
   const int *n_tiles = nullptr;
   int max_tiles = 0, tile_slots = 0;
   const int *gather = nullptr;       // slot -> row of x (nullptr: the slot itself)

@@ -276,6 +276,7 @@ __global__ void __launch_bounds__(512) row_k(KxRowArgs a, T *out, int ld) {
 struct Tile {
   int m0, end;  // rows of the result
   size_t w;     // offset of the matrix
+  bool alone;   // the matrix is read for this tile only
 };
 template <bool GROUP>
 __device__ __forceinline__ bool tile_of(const KxLinArgs &a, const KxExpertArgs &e, int bm, Tile &t) {
@@ -285,10 +286,12 @@ __device__ __forceinline__ bool tile_of(const KxLinArgs &a, const KxExpertArgs &
     t.m0 = r.y;
     t.end = r.y + r.z;
     t.w = (size_t)r.x * e.stride;
+    t.alone = r.w == 1;
   } else {
     t.m0 = blockIdx.y * bm;  // bm 0: all tokens
     t.end = a.tokens;
     t.w = 0;
+    t.alone = true;
   }
   return true;
 }
@@ -417,6 +420,8 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) lin_gemm_k(Kx
 // With several parts the sums go to memory and the workgroup that arrives last (kx_arrive.h) adds the parts in their order,
 // whoever it is, and runs the epilogue: results do not depend on timing.  Token rows past the last are never copied: what the
 // LDS holds there only feeds sums that are not stored.  Large matrices are copied nontemporally, whole lines of them (kx_read_once.h).
+// Not those of an expert with several tiles, which find its rows in the L2: 40 tokens to the same 4 of 128 experts of 3 x 4096 x 1536 101.8 us so, 88.7 now, 96 tokens 139.5
+// and 119.2; 96 tokens spread unevenly 264.6 and 242.3.
 constexpr int NARROW_ROWS = 64, NARROW_MAX_SPLITS = 16;
 template <int MI, int EPI, bool GROUP>
 __global__ void __launch_bounds__(512, MI == 1 ? 4 : 2) lin_narrow_k(KxLinArgs a, KxExpertArgs e, const uint16_t *__restrict__ x, int x_ld, int splits, bool once, int share, int extra) {
@@ -431,6 +436,7 @@ __global__ void __launch_bounds__(512, MI == 1 ? 4 : 2) lin_narrow_k(KxLinArgs a
   Tile tl;
   if (!tile_of<GROUP>(a, e, 0, tl)) return;
   const int m0 = tl.m0, tokens = tl.end - m0;
+  const bool nt = once && tl.alone;
   x += (size_t)variant_of(a, n0) * a.tokens * x_ld;
   const int nh = a.m.ld >> 6, nb = (nh + 1) >> 1;  // halves, blocks
   const int b0 = (int)((long)nb * part / splits), b1 = (int)((long)nb * (part + 1) / splits);
@@ -461,7 +467,7 @@ __global__ void __launch_bounds__(512, MI == 1 ? 4 : 2) lin_narrow_k(KxLinArgs a
     for (int i = 0; i < CPW; ++i) {
       const uint16_t *const from = src[i] + min(2 * b + half[i], nh - 1) * 64;
       const uint32_t to = __builtin_amdgcn_readfirstlane(st + dst[i]);
-      if (i < 2 && once) kx_copy16_to_lds_once(from, to);  // the matrix
+      if (i < 2 && nt) kx_copy16_to_lds_once(from, to);  // the matrix
       else kx_copy16_to_lds(from, to);
     }
   };

@@ -780,6 +780,24 @@ def test_experts_with_tiles_of_256_slots(kxlib, tmp_path, width, ff, top, tokens
     a.close()
 
 
+def test_experts_of_a_large_layer_with_one_to_three_tiles(kxlib):
+    """Matrices beyond the memory-side cache.  One expert has every token, in one, two and three tiles, the others a few each, in one.  The bar is that of the others in bf16; a
+    repeated run has the same bits but for the order of an expert's slots, which no sum depends on."""
+    a = Experts(kxlib, 2048, 1056, 32, 2, 64, 0, 96)
+    a.bias[:] = 0.0
+    a.bias[5] = 30.0
+    a.push()
+    r = np.random.default_rng(2)
+    for n in (20, 40, 96):
+        x, rows = r.standard_normal((n, 2048)).astype(np.float32), KC.bf16(r.standard_normal((n, 64)))
+        got, ids = a.run(x, rows)
+        again, _ = a.run(x, rows)
+        assert (ids[:, 0] == 5).all() and np.bincount(ids[:, 1], minlength=32).max() <= 32
+        assert rel(got, a.oracle(x, rows, ids)) < 2e-2, n
+        assert np.array_equal(got.view(np.uint32), again.view(np.uint32)), n
+    a.close()
+
+
 @pytest.mark.parametrize("width", [100, 101])
 @pytest.mark.parametrize("tokens", [15, 16, 17, 700])
 def test_experts_sorted_and_combined_at_the_edges(kxlib, tokens, width):
