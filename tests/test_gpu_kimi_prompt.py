@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import oracle as O
-from blok_amd.lib import check, default_config
+from blok_amd.lib import DevBuf, check, default_config
 from kxt import say
 from test_gpu_model import KxModel
 
@@ -137,3 +137,33 @@ def test_products_of_a_batch_on_as_many_workgroups_as_run_at_once(kxlib, ox, bat
     (rows, logits), (rows1, logits1) = got
     assert np.abs(rows1 - rows).max() / np.abs(rows).max() < 2e-2
     assert max(O.max_rel(logits1[b], logits[b]) for b in range(batch)) < 3e-2
+
+
+@pytest.mark.parametrize("batch", [5, 16, 17, 32])
+@pytest.mark.parametrize("vocab", [8449, 4097, 33000], ids=["shares of 33 and 34", "of 16 and 17", "of 128 and 129"])
+def test_head_and_residual_of_a_batch_element_by_element(kxlib, vocab, batch):
+    """A last tile of one row, and rows that do not come out even.  Every logit against its 64-bit sum over the device's own normed row: sums of 32 bits and a rounding to bf16, which
+    may fall to the other side.  The residual rows, which every projection adds to, against those of the GEMVs: 2^-8 at each of four sums, and what the layers before differ by."""
+    cfg = _config(16, batch, 8)
+    cfg.dense_inter, cfg.vocab = 8704, vocab
+    ids = O.tokens_u32(batch * 3, cfg.seed, 4, vocab).reshape(batch, 3)
+    km = KxModel(kxlib, cfg)
+    check(kxlib.kx_model_set_prefill_chunk(km.h, 1))
+    hidden = []
+    for exact in (15, 0):
+        check(kxlib.kx_model_set_exact(km.h, exact))
+        check(kxlib.kx_prefill(km.h, ids.ctypes.data, batch, 3))
+        hidden.append(km.hidden(batch))
+    logits = km.logits(batch)
+    km.close()
+    H = cfg.hidden
+    norm, head, dn = DevBuf(2 * H), DevBuf(2 * H * vocab), DevBuf(2 * H * batch)
+    check(kxlib.kx_fill_affine_bf16(norm.ptr, H, cfg.seed, 2, 1.0, 0.02, None))
+    check(kxlib.kx_fill_normal_bf16(head.ptr, H * vocab, cfg.seed, 3, cfg.init_sigma, 0, None))
+    dx = DevBuf.from_numpy(hidden[1])
+    check(kxlib.kx_rmsnorm(dx.ptr, norm.ptr, dn.ptr, batch, H, cfg.rms_eps, None))
+    check(kxlib.kx_sync(None))
+    f64 = lambda b, shape: O.bf16_to_f32(b.to_numpy(np.uint16, shape)).astype(np.float64)
+    want = f64(dn, (batch, H)) @ f64(head, (vocab, H)).T
+    assert O.elem_err(logits, want) < 5e-3
+    assert O.elem_err(*map(O.bf16_to_f32, hidden[::-1])) < 2e-2

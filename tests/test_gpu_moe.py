@@ -277,3 +277,36 @@ def test_moe_errors(kxlib):
     assert kxlib.kx_moe_decode_layer(C.byref(cfg), C.byref(w), ws, b.ptr, b.ptr, 5, 0, None) != 0
     assert b"tokens" in kxlib.kx_last_error()
     check(kxlib.kx_moe_workspace_destroy(ws))
+
+
+@pytest.mark.parametrize("tokens", [5, 16, 17, 32])
+@pytest.mark.parametrize("hidden, shared, experts", [(3072, 3072, 8), (5120, 5120, 64), (9216, 512, 40)], ids=["shares of 12", "of 20: a tile and four rows", "of 36, two blocks"])
+def test_products_of_a_shared_expert_element_by_element(kxlib, hidden, shared, experts, tokens):
+    """Products of 5 to 32 tokens on a workgroup per CU, in both of their forms (up to 16 tokens, more) and with either kind of copies.  Routed experts with scales of zero leave
+    the shared expert alone, and with the identity as its down projection the layer's output is the gated rows themselves.  An element's sums may round to the other bf16 value,
+    2^-8 of it, in gate, in up and in the result."""
+    H, SI, E = hidden, shared, experts
+    r = np.random.default_rng(H + tokens)
+    bf = lambda shape, s: O.f32_to_bf16(s * r.standard_normal(shape, np.float32))
+    packed, scales = np.zeros(E * 1024 * H // 8, np.uint32), np.zeros(E * 1024 * H // 32, np.uint16)
+    host = {"router_gate": np.zeros(E * H, np.uint16), "router_bias": np.zeros(E, np.float32), "shared_gate": bf((SI, H), H ** -0.5), "shared_up": bf((SI, H), H ** -0.5),
+            "shared_down": O.f32_to_bf16(np.eye(H, dtype=np.float32)) if H == SI else bf((H, SI), SI ** -0.5)}
+    for k in ("gate", "up", "down"):
+        host[k + "_packed"], host[k + "_scale"] = packed, scales
+    n = bf((tokens, H), 1.0)
+    f64 = lambda a: O.bf16_to_f32(a).astype(np.float64)
+    rounded = lambda y: f64(O.f32_to_bf16(np.ascontiguousarray(y, np.float32)))
+    gate, up = rounded(f64(n) @ f64(host["shared_gate"]).T), rounded(f64(n) @ f64(host["shared_up"]).T)
+    want = rounded(rounded(gate / (1 + np.exp(-gate))) * up)
+    if H != SI:
+        want = want @ f64(host["shared_down"]).T
+    cfg = moe_cfg(H, 1024, SI, E, 2)
+    w, bufs = moe_device_weights(host)
+    ws = C.c_void_p()
+    check(kxlib.kx_moe_workspace_create(C.byref(cfg), tokens, C.byref(ws)))
+    dn, dx = dev(n), dev(bf((tokens, H), 1.0))
+    check(kxlib.kx_moe_decode_layer(C.byref(cfg), C.byref(w), ws, dn.ptr, dx.ptr, tokens, 0x201, None))
+    check(kxlib.kx_sync(None))
+    got = O.bf16_to_f32(dx.to_numpy(np.uint16, (tokens, H)))
+    check(kxlib.kx_moe_workspace_destroy(ws))
+    assert O.elem_err(got, want) < 2e-2
