@@ -17,9 +17,9 @@ struct KxExpertSlots {
 // where an expert has 96 pairs and more on average (kx_tile_share.h says which; tiles listed by size, the short ones last, lose that an expert's
 // tiles read one matrix at a time: 8 of 64 of 3 x 2048 x 1024, 2046 tokens 514 / 530); 32, those of the kernel for few tokens, where it has fewer than
 // 8 and no expert can have
-// more than three tiles, each of which reads its matrix again.  The operator with 32 / 64 slots, us: 8 to 8 of 64 of 3 x 2048 x 1024
-// 153 / 180, 63 tokens 211 / 230, all among 8 experts 83 / 90; 4 of 128 of 3 x 4096 x 1536, even 96 tokens 891 / 921, 192 tokens 982 /
-// 985; among 8 experts 96 tokens 174 / 183, 128 tokens 190 / 186, 192 tokens 215 / 187, 255 tokens 239 / 207.
+// more than three tiles, each of which reads its matrix again.  The operator with 32 / 64 slots, us: 8 tokens to 8 of 64 of 3 x 2048 x 1024
+// 124 / 169, 63 tokens 183 / 223, all among 8 experts 75 / 81, among 16 95 / 84; 4 of 128 of 3 x 4096 x 1536, even 96 tokens 831 / 917, 192 tokens 898 /
+// 955; among 8 experts 96 tokens 152 / 159, 128 tokens 170 / 168, 192 tokens 187 / 162, 255 tokens 222 / 187.
 constexpr int KX_EXPERT_TILE_MIN = 32, KX_EXPERT_TILE_MIN_TOKENS = 3 * KX_EXPERT_TILE_MIN;
 inline int kx_expert_tile(bool f32, int tokens, int top, int experts, const KxMat &in, const KxMat &out, int cus) {
   const long pairs = (long)tokens * top;

@@ -22,7 +22,7 @@ __device__ __forceinline__ void kx_copy16_to_lds(const void *src, uint32_t lds_b
 }
 // The same for what one workgroup reads once: nontemporal, for copies that ask for whole 128-byte lines.  1.1 GB of matrix rows, 8 rows of 128
 // bytes an instruction, arrive at 6.9 to 7.0 TB/s, at 6.1 without; half lines at 5.4, and 6.1 without.  Rows that several workgroups read
-// are for kx_copy16_to_lds, which leaves them in the L2.
+// are for kx_copy16_to_lds, which leaves them in the L2, and so is what the memory-side cache holds from one pass to the next (kx_read_once.h).
 __device__ __forceinline__ void kx_copy16_to_lds_once(const void *src, uint32_t lds_base) {
   uint32_t m0_saved;
   asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off nt\n\ts_mov_b32 m0, %0"

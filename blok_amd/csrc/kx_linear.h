@@ -117,8 +117,9 @@ struct KxExpertArgs {
 };
 constexpr int KX_MAX_EXPERTS = 1024, KX_MAX_TOP = 64;
 
-// f32: the model's type is float, else bf16.  row_buf: tokens * m.ld elements of scratch, where the rows of a step of
-// more than KX_GEMV_TOKENS tokens are built (not used for PLAIN).
+// f32: the model's type is float, else bf16.  row_buf: tokens * m.ld elements of scratch per variant of the rows, where those of other kinds than PLAIN are built: of a step
+// of more than KX_GEMV_TOKENS tokens always, of fewer also where they do not fit a workgroup, and of two (NORM) or three (GATED) tokens and more where row_buf is given
+// and at a multiple of 16 bytes.  Without it the product builds the rows of up to KX_GEMV_TOKENS tokens itself.  The results are the same.
 constexpr int KX_GEMV_TOKENS = 4;
 // bf16: up to this many tokens the matrix is streamed by workgroups that hold all tokens
 constexpr int KX_NARROW_TOKENS = 64;

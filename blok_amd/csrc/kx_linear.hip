@@ -8,7 +8,7 @@
 // streams two rows of the matrix at a time, 8 columns per lane and load, the next pieces in flight while the present
 // ones are multiplied; the epilogue stores the product, forms the gated activation of a (gate, up) pair, or updates
 // all residual streams of the row.
-// lin_narrow_k (bf16, up to 64 tokens): all tokens against 64 rows, the columns split over waves and workgroups.
+// lin_narrow_k (bf16, up to 64 tokens): all tokens against up to 64 rows, the columns split over waves and workgroups.
 // lin_gemm_k (bf16, more tokens): tiles of 256 x 256 or 128 x 128 on the matrix cores (kx_gemm_tile.h, kx_gemm_turns.h).
 // In f32 from 5 tokens on tiles of 64 x 128 on the 32-bit matrix instructions; true 32-bit products.
 //
@@ -412,7 +412,7 @@ __global__ void __launch_bounds__(TL::THREADS, TL::WAVES_PER_SIMD) lin_gemm_k(Kx
 }
 
 // ---- bf16 products of few tokens ----
-// Bound by the stream of the matrix.  A workgroup of 8 waves owns 64 rows (with GLU rows a block of gate and its block of up),
+// Bound by the stream of the matrix.  A workgroup of 8 waves owns a share of up to 64 rows (kxtile::even_groups; with GLU rows a block of gate and its block of up),
 // all tokens, and one of `splits` parts of the columns, so that a matrix of few rows still has a workgroup or two for every CU:
 // a tile per 128 rows alone is 16 workgroups for 2048 rows (90 us for 8 tokens against 2048 x 10240; 11 us here).  The columns
 // are walked in blocks of 128, each two halves of 64 in the layout of the tiles above, through a ring of NS blocks; wave w
@@ -714,7 +714,8 @@ int linear_epi(const KxLinArgs &a, void *row_buf, hipStream_t st) {
       // Rows of several tokens are built by a launch of their own, a workgroup per token: in the product's, where a workgroup builds them one after the other, each takes 3
       // us that the matrix waits.  The rows are the same.  us, before / now: 4 tokens of two normed streams 16384 x 2048 26.9 / 20.2, 6208 x
       // 2048 21.6 / 13.9, 4096 x 1024 14.6 / 10.9, a gated read-out 2048 x 2048 13.2 / 10.2; two tokens 19.4 / 18.3, 14.2 / 12.4 and 9.5 / 9.5, but the
-      // gated one 8.5 / 9.1.
+      // gated one 8.5 / 9.1.  Small products gain as well, one stream, two tokens and four: 256 x 256 7.7 / 7.5 and 12.7 / 9.4, 768 x 768 8.6 / 8.1 and 13.7 / 9.8, 64 x 2048 9.1 /
+      // 8.5 and 14.9 / 10.0; in 32 bits 256 x 256 8.7 / 8.3 and 13.8 / 10.4, 768 x 768 10.2 / 9.9 and 15.5 / 11.6, 8192 x 2048 29.1 / 24.0 and 39.5 / 26.6.
       if (row_buf && (uintptr_t)row_buf % 16 == 0 && ((nt > 1 && a.row.kind == KX_ROW_NORM) || (nt == 4 && a.row.kind == KX_ROW_GATED))) {
         const int rc = rows_launch<T>(a.row, a.tokens, (T *)row_buf, a.m.ld, st);
         if (rc) return rc;
