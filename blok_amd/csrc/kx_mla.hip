@@ -219,8 +219,8 @@ struct MlaArgs {
   int seqs;               // 0: grid index z is sequence z, which attends `seq` positions.  n > 0 (a prefill step of
                           // several positions of n sequences): z = i * n + b is position i of sequence b; it reads
                           // cache block b and attends seq - (grid z / n - 1) + i positions, the last position all `seq`
+  bool once;              // rows are read once and copied nontemporally; in front of seq_stride, where it makes the arguments no longer
   size_t seq_stride;      // elements between sequences in the cache
-  bool once;              // rows are read once and copied nontemporally
   float rs, mscale;
 };
 
