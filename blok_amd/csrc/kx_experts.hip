@@ -5,6 +5,7 @@
 #include <algorithm>
 #include "kx_common.h"
 #include "kx_experts.h"
+#include "kx_read_once.h"
 
 namespace {
 
@@ -149,7 +150,7 @@ int kx_expert_combine_launch(const KxExpertSlots &s, const float *y, float *x, i
 
 int kx_expert_ff_launch(bool f32, const KxExpertFf &f, int tokens, hipStream_t st) {
   KxLinArgs gu = f.gu;
-  gu.model_bytes = std::max(f.gu.model_bytes, (size_t)f.e.experts * (f.gu_stride + f.down_stride) * (f32 ? 4 : 2));  // these at the least
+  gu.model_mb = std::max(f.gu.model_mb, kxonce::megabytes((size_t)f.e.experts * (f.gu_stride + f.down_stride) * (f32 ? 4 : 2)));  // these at the least
   gu.epi = KX_LIN_GLU;
   gu.mid = f.mid;
   gu.mid_ld = f.down.ld;
@@ -174,7 +175,7 @@ int kx_expert_ff_launch(bool f32, const KxExpertFf &f, int tokens, hipStream_t s
   KxLinArgs down;
   down.m = f.down;
   down.tokens = tokens;
-  down.model_bytes = gu.model_bytes;
+  down.model_mb = gu.model_mb;
   down.row.cols = f.down.cols;
   down.out = f.y;
   down.out_ld = f.down.rows;

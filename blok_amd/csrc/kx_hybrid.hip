@@ -25,6 +25,7 @@
 #include "kx_load.h"
 #include "kx_math.h"
 #include "kx_model.h"
+#include "kx_read_once.h"
 #include "kx_safetensors.h"
 
 namespace {
@@ -530,7 +531,7 @@ int HybridModel::restart(int batch_) {
 void HybridModel::split(KxLinArgs &g) const {
   g.part = split_part; g.part_floats = split_floats;
   g.arrived = split_arrived; g.arrivals = SPLIT_GROUPS;
-  g.model_bytes = matrix_bytes;
+  g.model_mb = kxonce::megabytes(matrix_bytes);
 }
 int HybridModel::product(KxLinArgs &g, void *row_buf) const {
   split(g);
@@ -670,7 +671,7 @@ int HybridModel::step(const uint32_t *d_ids, bool sample, int C) {
     if (experts) {
       KxExpertFf f;
       read(f.gu, w.gu, w.norm1, w.hc[0]);
-      f.gu.limit = l.limit; f.gu.alpha = l.alpha; f.gu.bias = l.bias; f.gu.model_bytes = matrix_bytes;
+      f.gu.limit = l.limit; f.gu.alpha = l.alpha; f.gu.bias = l.bias; f.gu.model_mb = kxonce::megabytes(matrix_bytes);
       split(out);
       f.out = out;
       f.down = w.down; f.gu_stride = w.gu_stride; f.down_stride = w.down_stride;

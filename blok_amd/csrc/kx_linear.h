@@ -91,7 +91,7 @@ struct KxLinArgs {
   size_t part_floats = 0;
   int *arrived = nullptr;    // [arrivals], zero between launches
   int arrivals = 0;
-  size_t model_bytes = 0;    // of all matrices of the model (kx_read_once.h); 0: there are no others
+  int model_mb = 0;          // of all matrices of the model (kx_read_once.h), in 2^20 bytes, rounded up; 0: there are no others.  The arguments are no longer with it
 };
 constexpr int KX_MAX_STREAMS = 8;
 

@@ -643,7 +643,7 @@ int narrow_launch(const KxLinArgs &a, const KxExpertArgs &e, const uint16_t *x, 
     if (even > groups) groups = even, share = a.m.rows / even, extra = a.m.rows % even;
   }
   const dim3 grid(groups, GROUP ? e.max_tiles : splits);
-  const bool once = GROUP ? kxonce::experts((size_t)e.experts * e.stride * 2, a.model_bytes) : kxonce::matrix((size_t)a.m.rows * a.m.ld * 2, a.model_bytes);
+  const bool once = GROUP ? kxonce::experts((size_t)e.experts * e.stride * 2, (size_t)a.model_mb << 20) : kxonce::matrix((size_t)a.m.rows * a.m.ld * 2, (size_t)a.model_mb << 20);
   if constexpr (GROUP) hipLaunchKernelGGL((lin_narrow_k<1, EPI, true>), grid, dim3(512), lds[0], st, a, e, x, x_ld, splits, once, share, extra);
   else if (a.tokens <= 32) hipLaunchKernelGGL((lin_narrow_k<1, EPI, false>), grid, dim3(512), lds[0], st, a, e, x, x_ld, splits, once, share, extra);
   else hipLaunchKernelGGL((lin_narrow_k<2, EPI, false>), grid, dim3(512), lds[1], st, a, e, x, x_ld, splits, once, share, extra);

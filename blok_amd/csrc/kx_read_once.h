@@ -17,6 +17,7 @@ inline bool latent(size_t bytes) { return bytes >= LATENT; }
 // 8.3 / 8.7 and 9.6 / 9.1, 8192 x 2048 10.3 / 11.6 and 12.1 / 11.8, 16384 x 2048 13.0 / 15.0 and 17.2 / 15.8.  24 steps of Kimi-K2 layers of 2048 columns, 32 sequences,
 // 189 MB 3.19 / 3.58 ms, 314 MB 6.17 / 6.11; of 7168 columns, 2.1 GB, 12 sequences 13.71 / 12.69.
 constexpr size_t MODEL = (size_t)256 << 20;
+inline int megabytes(size_t bytes) { return (int)((bytes + ((size_t)1 << 20) - 1) >> 20); }
 inline bool layers(size_t model) { return model > MODEL; }
 // Of larger models of the hybrid decoder the smaller matrices are left to the cache, which the larger ones pass by.  32 steps, all plain / all nontemporal / by the
 // matrix: Kagalorn, 8 sequences, 333 MB 9.30 / 9.22 / 9.02 ms, 568 MB 11.01 / 10.48 / 10.37; Rapitar, 265 MB 8.24 / 8.43 / 8.22, 1 GB 13.26 / 12.25 / 12.25.
